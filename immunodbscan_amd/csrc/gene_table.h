@@ -1,0 +1,121 @@
+// gene_table.h — the multi-name automaton of the gene-call scan (host code).
+//
+// A. V. Aho and M. J. Corasick ("Efficient string matching: an aid to
+// bibliographic search", CACM 1975) over the gene names: one pass over a call
+// string's bytes, one table lookup per byte, finds every name that occurs in
+// it.  Bytes are first mapped to classes (class 0: bytes that occur in no
+// name, which lead back to the root), so that a row of the table holds one
+// entry per class instead of 256.
+//
+// A table row is the state's `ncls` transitions and then its list head
+// (stride = ncls + 1).  A transition is the target row's offset in entries
+// (state * stride).  States at which some name ends are numbered last: their
+// offsets are out_min and above, so that the walk needs no flag bits.  The
+// list head is 0 or 1 + the index of the first node of the names that end at
+// the state: node = gene | next << 16, next in the same encoding; a state's
+// own names come first and are followed by its suffix states'.
+//
+// Byte 0 is always in class 0, so that a walk may run over zero bytes past a
+// string's end: names that hold a zero byte are not taken.
+#pragma once
+#include <stdint.h>
+
+#include <algorithm>
+#include <cstddef>
+#include <vector>
+
+struct idb_gene_table {
+    uint32_t ncls = 0, stride = 0, entries = 0;
+    uint32_t out_min = 0;           // offset of the first state that ends a name (entries: none)
+    uint32_t max_len = 0;           // longest usable name
+    uint8_t cls[256] = {};          // class of a byte value
+    std::vector<uint32_t> trans;
+    std::vector<uint32_t> nodes;
+};
+
+#define IDB_GENE_NAME_MAX 1024u     // longer names never match
+
+// False when the table would hold more than `cap` entries or a name holds a
+// zero byte.
+inline bool idb_gene_table_build(uint32_t n_genes, const uint8_t *genes, const uint64_t *gene_off,
+                                 const uint32_t *gene_len, uint32_t cap, idb_gene_table &t)
+{
+    t = idb_gene_table();
+    t.ncls = 1;
+    for (uint32_t g = 0; g < n_genes; ++g) {
+        const uint32_t L = gene_len[g];
+        if (L == 0 || L > IDB_GENE_NAME_MAX) continue;
+        if (L > t.max_len) t.max_len = L;
+        for (uint32_t k = 0; k < L; ++k) {
+            const uint8_t b = genes[gene_off[g] + k];
+            if (!b) return false;
+            if (!t.cls[b]) t.cls[b] = (uint8_t)t.ncls++;  // (at most 255 values)
+        }
+    }
+    const uint32_t st = t.stride = t.ncls + 1u;
+    if (st > cap) return false;
+    t.trans.reserve(std::min<size_t>(cap, 8192u));
+    t.trans.assign(st, 0u);
+    std::vector<uint32_t> tail;  // per state: 1 + its own last node, 0 without
+    tail.push_back(0u);
+    uint32_t states = 1;
+    for (uint32_t g = 0; g < n_genes; ++g) {
+        const uint32_t L = gene_len[g];
+        if (L == 0 || L > IDB_GENE_NAME_MAX) continue;
+        uint32_t s = 0;
+        for (uint32_t k = 0; k < L; ++k) {
+            const size_t at = (size_t)s * st + t.cls[genes[gene_off[g] + k]];
+            if (!t.trans[at]) {
+                if ((uint64_t)(states + 1u) * st > cap) return false;
+                t.trans[at] = states++;
+                t.trans.resize((size_t)states * st, 0u);
+                tail.push_back(0u);
+            }
+            s = t.trans[at];
+        }
+        t.nodes.push_back(g);
+        uint32_t &head = t.trans[(size_t)s * st + t.ncls];
+        if (tail[s]) t.nodes[tail[s] - 1u] |= (uint32_t)t.nodes.size() << 16;
+        else head = (uint32_t)t.nodes.size();
+        tail[s] = (uint32_t)t.nodes.size();
+    }
+    t.entries = states * st;
+    // breadth first: missing edges from the suffix state's finished row, and
+    // the suffix state's list behind the state's own
+    std::vector<uint32_t> fail(states, 0u), queue;
+    queue.reserve(states);
+    for (uint32_t c = 0; c < t.ncls; ++c)
+        if (t.trans[c]) queue.push_back(t.trans[c]);
+    for (size_t q = 0; q < queue.size(); ++q) {
+        const uint32_t s = queue[q];
+        uint32_t *row = &t.trans[(size_t)s * st];
+        const uint32_t *frow = &t.trans[(size_t)fail[s] * st];
+        for (uint32_t c = 0; c < t.ncls; ++c) {
+            if (row[c]) {
+                fail[row[c]] = frow[c];
+                queue.push_back(row[c]);
+            } else {
+                row[c] = frow[c];
+            }
+        }
+        if (tail[s]) t.nodes[tail[s] - 1u] |= frow[t.ncls] << 16;
+        else row[t.ncls] = frow[t.ncls];
+    }
+    // states without a name to report first, then the others
+    std::vector<uint32_t> at(states);
+    uint32_t quiet = 0, loud = 0;
+    for (uint32_t s = 0; s < states; ++s) quiet += t.trans[(size_t)s * st + t.ncls] == 0u;
+    t.out_min = quiet * st;
+    loud = quiet;
+    quiet = 0;
+    for (uint32_t s = 0; s < states; ++s) at[s] = (t.trans[(size_t)s * st + t.ncls] ? loud++ : quiet++) * st;
+    std::vector<uint32_t> out(t.entries);
+    for (uint32_t s = 0; s < states; ++s) {
+        const uint32_t *from = &t.trans[(size_t)s * st];
+        uint32_t *to = &out[at[s]];
+        for (uint32_t c = 0; c < t.ncls; ++c) to[c] = at[from[c]];
+        to[t.ncls] = from[t.ncls];
+    }
+    t.trans.swap(out);
+    return true;
+}

@@ -39,6 +39,7 @@
 #include "../../include/idb.h"
 #include "idb_internal.h"
 #include "copy_pool.h"
+#include "gene_table.h"
 
 // ---------------------------------------------------------------------------
 // Scratch of the allocation-free runs: one static device array, which every
@@ -214,48 +215,6 @@ __device__ __forceinline__ uint64_t fin64(uint64_t z)
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     return z ^ (z >> 31);
-}
-
-// Bytes k .. k+15 of a row of length L as one 16-byte value, zero past the
-// row's end.  Every load stays inside the row: a short tail is read as the
-// row's last 16 bytes and shifted down, rows under 16 bytes byte by byte.
-// Unaligned 16-byte global loads are legal on gfx950.
-__device__ __forceinline__ uint4 row16(const uint8_t *s, uint32_t L, uint32_t k)
-{
-    uint4 v;
-    if (k + 16 <= L) {
-        __builtin_memcpy(&v, s + k, 16);
-        return v;
-    }
-    const uint32_t r = L - k;  // 1 .. 15 bytes left
-    uint64_t lo = 0, hi = 0;
-    if (L >= 16) {
-        uint64_t t[2];
-        __builtin_memcpy(t, s + L - 16, 16);
-        const uint32_t sh = 8 * (16 - r);  // 8 .. 120 bits
-        if (sh >= 64) {
-            lo = t[1] >> (sh - 64);
-        } else {
-            lo = (t[0] >> sh) | (t[1] << (64 - sh));
-            hi = t[1] >> sh;
-        }
-    } else {
-        for (uint32_t b = 0; b < r; ++b) {
-            const uint64_t c = s[k + b];
-            if (b < 8) lo |= c << (8 * b); else hi |= c << (8 * (b - 8));
-        }
-    }
-    v.x = (uint32_t)lo;
-    v.y = (uint32_t)(lo >> 32);
-    v.z = (uint32_t)hi;
-    v.w = (uint32_t)(hi >> 32);
-    return v;
-}
-
-__device__ __forceinline__ uint32_t byte_of(const uint4 &v, uint32_t b)
-{
-    const uint32_t w = b < 8 ? (b < 4 ? v.x : v.y) : (b < 12 ? v.z : v.w);
-    return (w >> (8 * (b & 3))) & 0xFFu;
 }
 
 __global__ void k_fill_rid(const uint32_t *rstart, uint32_t n_reps, uint32_t n, uint32_t *rid)
@@ -2166,31 +2125,6 @@ int idb_gene_bitsets_gpu(idb_ctx *c, uint32_t mem, uint32_t n, const uint8_t *ca
     try {
         check(c, hipSetDevice(c->device), "hipSetDevice");
         hipStream_t s = c->stream;
-        // headers and 4-byte words of the names (names that cannot match get
-        // len = 0xFFFFFFFF: empty, or longer than the reference's 1024-thread
-        // launch allows, cuda/BitsetVector.inl:204)
-        std::vector<idb_gene_hdr> hdr(std::max(n_genes, 1u));
-        std::vector<uint32_t> words(1, 0u);
-        for (uint32_t g = 0; g < n_genes; ++g) {
-            const uint32_t gl = gene_len[g];
-            if (gl == 0 || gl > 1024) {
-                hdr[g] = {0u, 0u, 0xFFFFFFFFu, 0u};
-                continue;
-            }
-            const uint32_t woff = (uint32_t)words.size();
-            for (uint32_t k = 0; k < gl; k += 4) {
-                uint32_t v = 0;
-                for (uint32_t b = 0; b < 4 && k + b < gl; ++b) v |= (uint32_t)genes[gene_off[g] + k + b] << (8 * b);
-                words.push_back(v);
-            }
-            uint32_t last = 0;
-            for (uint32_t b = 0; b < 4 && b < gl; ++b) last |= (uint32_t)genes[gene_off[g] + gl - std::min(gl, 4u) + b] << (8 * b);
-            hdr[g] = {words[woff], last, gl, woff};
-        }
-        idb_gene_hdr *hd = buf<idb_gene_hdr>(c, S_GHDR, hdr.size());
-        uint32_t *wd = buf<uint32_t>(c, S_GWORDS, words.size());
-        check(c, hipMemcpyAsync(hd, hdr.data(), sizeof(idb_gene_hdr) * hdr.size(), hipMemcpyHostToDevice, s), "gene copy");
-        check(c, hipMemcpyAsync(wd, words.data(), sizeof(uint32_t) * words.size(), hipMemcpyHostToDevice, s), "gene copy");
         const uint8_t *cd = calls;
         const uint64_t *od = call_off;
         const uint32_t *ld = call_len;
@@ -2204,8 +2138,79 @@ int idb_gene_bitsets_gpu(idb_ctx *c, uint32_t mem, uint32_t n, const uint8_t *ca
             ld = stage_in<uint32_t>(c, S_GLEN, call_len, n, mem);
             outd = buf<int32_t>(c, S_GOUT, (size_t)n * width);
         }
-        check(c, idb_launch_gene_bitsets(cd, od, ld, n, hd, wd, (uint32_t)words.size(), n_genes, outd, width, s),
-              "gene bitset launch");
+        // The automaton while building its table costs less than testing every
+        // name: measured, the per-name kernel takes 0.45 us per name (a wave's
+        // walk over the names) + 0.081 ns per call and name, the automaton
+        // about 11 us + 4.5 ns per table entry (mostly its construction on the
+        // host).  104 V genes: 58 against 70 us from 100 calls on, 74 us
+        // against 8.75 ms at 1M; 37 D genes: even at 5,000 calls; 6 J genes:
+        // from about 15,000 calls (31.5 against 36.6 us at 20,000).
+        const int64_t worth = 100ll * n_genes + (int64_t)((uint64_t)n * n_genes * 18u / 1000u) - 2500;
+        const uint32_t cap = (uint32_t)std::max<int64_t>(0, std::min<int64_t>(IDB_GENE_TABLE_MAX, worth));
+        // (host copies that the stream may still read at the end of their block)
+        idb_gene_table t;
+        std::vector<uint8_t> big;
+        std::vector<idb_gene_hdr> hdr;
+        std::vector<uint32_t> words;
+        if (n_genes && idb_gene_table_build(n_genes, genes, gene_off, gene_len, cap, t)) {
+            const bool narrow = t.entries <= IDB_GENE_TABLE_NARROW && t.nodes.size() <= 4096;
+            const size_t nodes_at = 256, trans_at = (nodes_at + 4 * t.nodes.size() + 15) & ~(size_t)15;
+            const size_t bytes = trans_at + (narrow ? ((size_t)t.entries + 1) / 2 * 4 : 4 * (size_t)t.entries + 4);
+            // built in the pinned staging area when it fits (the previous
+            // call's upload has ended: calls are synchronous)
+            uint8_t *h = (uint8_t *)c->pinned + IDB_STAGE_BYTES;
+            if (bytes > IDB_STAGE_BYTES) {
+                big.resize(bytes);
+                h = big.data();
+            }
+            std::memcpy(h, t.cls, sizeof(t.cls));
+            if (!t.nodes.empty()) std::memcpy(h + nodes_at, t.nodes.data(), 4 * t.nodes.size());
+            // offsets in bytes; list heads as they are
+            auto fill = [&](auto *e) {
+                for (uint32_t r = 0; r < t.entries; r += t.stride) {
+                    for (uint32_t k = 0; k < t.ncls; ++k)
+                        e[r + k] = (std::decay_t<decltype(*e)>)(t.trans[r + k] * (uint32_t)sizeof(*e));
+                    e[r + t.ncls] = (std::decay_t<decltype(*e)>)t.trans[r + t.ncls];
+                }
+                if (t.entries & 1u) e[t.entries] = 0;
+            };
+            if (narrow) fill((uint16_t *)(h + trans_at));
+            else fill((uint32_t *)(h + trans_at));
+            uint8_t *dev = buf<uint8_t>(c, S_GHDR, bytes);
+            check(c, hipMemcpyAsync(dev, h, bytes, hipMemcpyHostToDevice, s), "gene table copy");
+            check(c, idb_launch_gene_scan(cd, od, ld, n, dev, (const uint32_t *)(dev + nodes_at), dev + trans_at, narrow,
+                                          t.ncls, t.entries, t.out_min, (uint32_t)t.nodes.size(), t.max_len, outd, width,
+                                          s),
+                  "gene scan launch");
+        } else {
+            // headers and 4-byte words of the names (names that cannot match get
+            // len = 0xFFFFFFFF: empty, or longer than the reference's 1024-thread
+            // launch allows, cuda/BitsetVector.inl:204)
+            hdr.resize(std::max(n_genes, 1u));
+            words.assign(1, 0u);
+            for (uint32_t g = 0; g < n_genes; ++g) {
+                const uint32_t gl = gene_len[g];
+                if (gl == 0 || gl > 1024) {
+                    hdr[g] = {0u, 0u, 0xFFFFFFFFu, 0u};
+                    continue;
+                }
+                const uint32_t woff = (uint32_t)words.size();
+                for (uint32_t k = 0; k < gl; k += 4) {
+                    uint32_t v = 0;
+                    for (uint32_t b = 0; b < 4 && k + b < gl; ++b) v |= (uint32_t)genes[gene_off[g] + k + b] << (8 * b);
+                    words.push_back(v);
+                }
+                uint32_t last = 0;
+                for (uint32_t b = 0; b < 4 && b < gl; ++b) last |= (uint32_t)genes[gene_off[g] + gl - std::min(gl, 4u) + b] << (8 * b);
+                hdr[g] = {words[woff], last, gl, woff};
+            }
+            idb_gene_hdr *hd = buf<idb_gene_hdr>(c, S_GHDR, hdr.size());
+            uint32_t *wd = buf<uint32_t>(c, S_GWORDS, words.size());
+            check(c, hipMemcpyAsync(hd, hdr.data(), sizeof(idb_gene_hdr) * hdr.size(), hipMemcpyHostToDevice, s), "gene copy");
+            check(c, hipMemcpyAsync(wd, words.data(), sizeof(uint32_t) * words.size(), hipMemcpyHostToDevice, s), "gene copy");
+            check(c, idb_launch_gene_bitsets(cd, od, ld, n, hd, wd, (uint32_t)words.size(), n_genes, outd, width, s),
+                  "gene bitset launch");
+        }
         if (mem == IDB_MEM_HOST)
             check(c, hipMemcpyAsync(out, outd, sizeof(int32_t) * (size_t)n * width, hipMemcpyDeviceToHost, s),
                   "bitset copy");
@@ -2214,6 +2219,10 @@ int idb_gene_bitsets_gpu(idb_ctx *c, uint32_t mem, uint32_t n, const uint8_t *ca
         (void)hipGetLastError();
         (void)hipStreamSynchronize(c->stream);
         return f.code;
+    } catch (const std::exception &e) {
+        (void)hipStreamSynchronize(c->stream);
+        c->err = e.what();
+        return IDB_ERR_OOM;
     }
     return IDB_OK;
 }

@@ -1,8 +1,17 @@
 // R2 gene bitsets on the device: bit g of row i is set iff gene name g occurs
 // as a contiguous substring of call string i (cuda/BitsetVector.inl:151-175).
 // The reference launches one grid per gene (find_string_occurences,
-// cuda/BitsetVector.inl:181-209); here one wave takes one call string and
-// tests every gene against it:
+// cuda/BitsetVector.inl:181-209).  Two kernels here:
+//
+// k_gene_scan walks the multi-name automaton of gene_table.h, one call string
+// per lane, one table lookup per byte whatever the number of names.  The
+// table sits in LDS as 16-bit entries when it has at most 32,768 (104 V gene
+// names make 7,248 entries, 14.5 KB), else in global memory as 32-bit
+// ones.
+//
+// k_gene_bitsets, where building the table would cost more than it saves (few
+// names and calls, or very long names): one wave takes one call string
+// and tests every gene against it:
 //   * the string is staged in the wave's LDS window, 2048 bytes at a time,
 //     with start positions advancing 1024 at a time (names longer than 1024
 //     bytes never match, as in the reference whose launch of more than 1024
@@ -15,9 +24,168 @@
 //   * the gene headers (the first 512) and the name words (when they fit in
 //     2048 words) are staged in LDS once per block and read by broadcast; the
 //     row's bit words collect in LDS and leave with one store per word.
+#include <algorithm>
+
 #include "idb_internal.h"
+#include "gene_table.h"
 
 namespace {
+
+constexpr uint32_t GS_LONG = 2048;           // longer call strings are walked by a whole wave
+
+// A lane's walk over one call string, with offsets in bytes (one add-shift
+// per lookup).  A byte where a name ends only notes the state, in a queue of
+// four in registers pushed without a branch; the queue is emptied when a
+// lane's is full and at the end of the string.  (Following the lists at once
+// costs the whole wave their latency at nearly every byte: with two alleles
+// per call some lane has one.)  NW > 0: the row's bit words are in w[];
+// NW == 0: they are in global memory (atomic, so that several lanes may walk
+// one row).
+template <typename TE, int NW>
+struct GeneWalk {
+    static constexpr int SH = sizeof(TE) == 2 ? 1 : 2;
+    const char *tr;
+    const uint8_t *cls;
+    const uint32_t *nodes;
+    uint32_t head_at, out_min;    // byte offsets: list head within a row, first state that ends a name
+    int32_t *out;                 // NW == 0: the row's words
+    uint32_t s = 0, cnt = 0;
+    uint32_t q[4] = {};           // the states noted, newest first (16-bit tables: two per word)
+    uint32_t w[NW ? NW : 1] = {};
+
+    __device__ __forceinline__ uint32_t at(uint32_t o) const { return *(const TE *)(tr + o); }
+    __device__ __forceinline__ void flush()
+    {
+        for (; cnt; --cnt) {
+            uint32_t st;
+            if (sizeof(TE) == 2) {
+                st = q[0] & 0xFFFFu;
+                q[0] = __builtin_amdgcn_alignbit(q[1], q[0], 16);
+                q[1] >>= 16;
+            } else {
+                st = q[0];
+                q[0] = q[1];
+                q[1] = q[2];
+                q[2] = q[3];
+            }
+            for (uint32_t n = at(st + head_at); n;) {
+                const uint32_t v = nodes[n - 1u], g = v & 0xFFFFu, bit = 1u << (g & 31u);
+                n = v >> 16;
+                if (NW) {
+#pragma unroll
+                    for (int k = 0; k < NW; ++k)
+                        if ((g >> 5) == (uint32_t)k) w[k] |= bit;
+                } else {
+                    atomicOr((uint32_t *)out + (g >> 5), bit);
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void step(uint32_t byte)
+    {
+        s = at(s + ((uint32_t)cls[byte] << SH));
+        if (cnt == 4u) flush();
+        const bool end = s >= out_min;
+        if (sizeof(TE) == 2) {
+            const uint32_t hi = __builtin_amdgcn_alignbit(q[1], q[0], 16), lo = (q[0] << 16) | s;
+            q[1] = end ? hi : q[1];
+            q[0] = end ? lo : q[0];
+        } else {
+#pragma unroll
+            for (int k = 3; k > 0; --k) q[k] = end ? q[k - 1] : q[k];
+            q[0] = end ? s : q[0];
+        }
+        cnt += end ? 1u : 0u;
+    }
+};
+
+// One call string per lane.  The bound is the chain of dependent lookups (a
+// byte's row depends on the byte before), so the chip is filled with as many
+// lanes as fit; neighbouring lanes read neighbouring strings 16 bytes at a
+// time, so every line of the calls is fetched once.  1M calls of 46.7 bytes
+// against 104 names: 8,666 us for the per-name kernel, 51 us here (20M VALU
+// wave instructions, 33 us of issue; 47 MB of calls at the copy rate: 14 us).
+// A string longer than GS_LONG is cut into 64 segments walked by the lanes of
+// its wave, each starting max_len - 1 bytes early at the root state (a name
+// that ends in the segment starts no earlier).
+template <typename TE, int NW>
+__global__ __launch_bounds__(1024) void k_gene_scan(const uint8_t *calls, const uint64_t *off, const uint32_t *len,
+                                                    uint32_t n, const uint8_t *__restrict__ cls_g,
+                                                    const TE *__restrict__ tr_g, const uint32_t *__restrict__ nodes_g,
+                                                    uint32_t ncls, uint32_t entries, uint32_t out_min, uint32_t n_nodes,
+                                                    uint32_t max_len, int32_t *out, uint32_t width,
+                                                    uint32_t wide_store)
+{
+    extern __shared__ uint32_t gs_lds[];
+    constexpr bool IN_LDS = sizeof(TE) == 2;
+    const uint8_t *cls = (const uint8_t *)gs_lds;        // 256 bytes, then the table
+    for (uint32_t k = threadIdx.x; k < 64; k += blockDim.x) gs_lds[k] = ((const uint32_t *)cls_g)[k];
+    if (IN_LDS)
+        for (uint32_t k = threadIdx.x; k < (entries + 1) / 2; k += blockDim.x)
+            gs_lds[64 + k] = ((const uint32_t *)tr_g)[k];
+    // (16-bit tables: the nodes follow in LDS)
+    uint32_t *nodes_l = gs_lds + 64 + (entries + 1) / 2;
+    if (IN_LDS)
+        for (uint32_t k = threadIdx.x; k < n_nodes; k += blockDim.x) nodes_l[k] = nodes_g[k];
+    __syncthreads();
+    const char *tr = IN_LDS ? (const char *)(gs_lds + 64) : (const char *)tr_g;
+    const uint32_t head_at = ncls * sizeof(TE), out_b = out_min * sizeof(TE);
+    const uint32_t *nodes = IN_LDS ? nodes_l : nodes_g;
+    const uint32_t lane = __lane_id();
+    const uint32_t step = gridDim.x * blockDim.x;
+    // whole waves stay together: `base` is the wave's first row
+    for (uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < n; base += step) {
+        const uint32_t row = base + lane;
+        const bool valid = row < n;
+        const uint32_t L = valid ? len[row] : 0u;
+        const uint8_t *src = calls + (valid ? off[row] : 0ull);
+        int32_t *ro = out + (size_t)row * width;
+        if (!NW && valid)
+            for (uint32_t k = 0; k < width; ++k) ro[k] = 0;
+        const bool is_long = L > GS_LONG;
+        if (!NW) __threadfence();  // the zeros are in place before any bit is set
+        GeneWalk<TE, NW> wk{tr, cls, nodes, head_at, out_b, ro};
+        if (!is_long) {
+            uint4 nx = L ? row16(src, L, 0) : make_uint4(0, 0, 0, 0);
+            for (uint32_t k0 = 0; k0 < L; k0 += 16) {
+                const uint4 v = nx;
+                if (k0 + 16 < L) nx = row16(src, L, k0 + 16);
+                // bytes past the string's end are zero and lead to the root
+#pragma unroll
+                for (uint32_t b = 0; b < 16; ++b) wk.step(byte_of(v, b));
+            }
+            wk.flush();
+        }
+        for (uint64_t lm = __ballot(is_long); lm; lm &= lm - 1ull) {
+            const int o = __builtin_ctzll(lm);
+            const uint32_t Lo = (uint32_t)__shfl((int)L, o, 64);
+            const uint64_t so = __shfl((unsigned long long)(valid ? off[row] : 0ull), o, 64);
+            const uint32_t seg = (Lo + 63u) / 64u;
+            const uint64_t a = (uint64_t)lane * seg, e = min((uint64_t)Lo, a + seg);
+            GeneWalk<TE, NW> lw{tr, cls, nodes, head_at, out_b, out + (size_t)(base + (uint32_t)o) * width};
+            for (uint64_t k = a > max_len - 1u ? a - (max_len - 1u) : 0u; k < e; ++k) lw.step(calls[so + k]);
+            lw.flush();
+            if (NW) {
+#pragma unroll
+                for (int k = 0; k < NW; ++k) {
+#pragma unroll
+                    for (int d = 32; d > 0; d >>= 1) lw.w[k] |= (uint32_t)__shfl_xor((int)lw.w[k], d, 64);
+                    if ((int)lane == o) wk.w[k] = lw.w[k];
+                }
+            }
+        }
+        const uint32_t *w = wk.w;
+        if (NW && valid) {
+            if (NW == 4 && wide_store) {
+                *(uint4 *)ro = make_uint4(w[0], w[1], w[2], w[3]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < NW; ++k)
+                    if ((uint32_t)k < width) ro[k] = (int32_t)w[k];
+            }
+        }
+    }
+}
 
 constexpr uint32_t GSEG = 1024;              // start positions per window
 constexpr uint32_t GWIN = 2 * GSEG;          // window bytes
@@ -153,5 +321,44 @@ hipError_t idb_launch_gene_bitsets(const uint8_t *calls, const uint64_t *off, co
     else
         hipLaunchKernelGGL(k_gene_bitsets<false>, dim3((uint32_t)blocks), dim3(64 * GWPB), 0, s, calls, off, len, n,
                            hdr, gw, n_words, n_genes, out, width);
+    return hipGetLastError();
+}
+
+uint32_t idb_gene_scan_blocks(uint32_t n, uint32_t threads, size_t lds)
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    (void)hipGetLastError();
+    // blocks that fit a CU by threads (2,048) and LDS (160 KB)
+    const uint32_t fit = std::max<uint32_t>(1u, std::min<uint32_t>(2048u / threads, (uint32_t)(163840u / (lds + 512u))));
+    return (uint32_t)std::min<uint64_t>(((uint64_t)n + threads - 1) / threads, (uint64_t)fit * cus);
+}
+
+// blob: the class map (256 bytes), the nodes, the table (16-bit entries when
+// they go to LDS), each 16-byte aligned
+hipError_t idb_launch_gene_scan(const uint8_t *calls, const uint64_t *off, const uint32_t *len, uint32_t n,
+                                const uint8_t *cls, const uint32_t *nodes, const void *trans, bool narrow,
+                                uint32_t ncls, uint32_t entries, uint32_t out_min, uint32_t n_nodes, uint32_t max_len,
+                                int32_t *out, uint32_t width, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    const size_t lds = 256 + (narrow ? ((size_t)entries + 1) / 2 * 4 + 4 * (size_t)n_nodes : 0);
+    // a bigger table shares one copy among more waves, so that a CU stays full
+    const uint32_t threads = lds <= 19000 ? 256u : (lds <= 39000 ? 512u : 1024u);
+    const dim3 grid(idb_gene_scan_blocks(n, threads, lds)), block(threads);
+    const uint32_t wide = width == 4 && ((uintptr_t)out & 15u) == 0 ? 1u : 0u;
+#define IDB_GS(TE, NW)                                                                                            \
+    hipLaunchKernelGGL((k_gene_scan<TE, NW>), grid, block, lds, s, calls, off, len, n, cls, (const TE *)trans,    \
+                       nodes, ncls, entries, out_min, n_nodes, max_len, out, width, wide)
+    if (narrow) {
+        if (width <= 4) IDB_GS(uint16_t, 4);
+        else IDB_GS(uint16_t, 0);
+    } else {
+        if (width <= 4) IDB_GS(uint32_t, 4);
+        else IDB_GS(uint32_t, 0);
+    }
+#undef IDB_GS
     return hipGetLastError();
 }

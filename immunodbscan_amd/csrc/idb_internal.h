@@ -40,6 +40,8 @@
 struct idb_gene_hdr {
     uint32_t w0, w1, len, woff;
 };
+#define IDB_GENE_TABLE_NARROW 32768u    // entries of a table that goes to LDS (16-bit byte offsets)
+#define IDB_GENE_TABLE_MAX (1u << 20)   // entries of the largest table that is built
 #define IDB_GENE_MAX_WIDTH 256u   // bit words per row (8,192 gene names)
 
 // Entry order for runs of up to IDB_SORT_SMALL_MAX entries: stable radix
@@ -148,6 +150,48 @@ struct idb_pair_args {
     uint32_t tune_wpb, tune_grid_mul, no_xcd_order;
 };
 
+// Bytes k .. k+15 of a row of length L as one 16-byte value, zero past the
+// row's end.  Every load stays inside the row: a short tail is read as the
+// row's last 16 bytes and shifted down, rows under 16 bytes byte by byte.
+// Unaligned 16-byte global loads are legal on gfx950.
+__device__ __forceinline__ uint4 row16(const uint8_t *s, uint32_t L, uint32_t k)
+{
+    uint4 v;
+    if (k + 16 <= L) {
+        __builtin_memcpy(&v, s + k, 16);
+        return v;
+    }
+    const uint32_t r = L - k;  // 1 .. 15 bytes left
+    uint64_t lo = 0, hi = 0;
+    if (L >= 16) {
+        uint64_t t[2];
+        __builtin_memcpy(t, s + L - 16, 16);
+        const uint32_t sh = 8 * (16 - r);  // 8 .. 120 bits
+        if (sh >= 64) {
+            lo = t[1] >> (sh - 64);
+        } else {
+            lo = (t[0] >> sh) | (t[1] << (64 - sh));
+            hi = t[1] >> sh;
+        }
+    } else {
+        for (uint32_t b = 0; b < r; ++b) {
+            const uint64_t c = s[k + b];
+            if (b < 8) lo |= c << (8 * b); else hi |= c << (8 * (b - 8));
+        }
+    }
+    v.x = (uint32_t)lo;
+    v.y = (uint32_t)(lo >> 32);
+    v.z = (uint32_t)hi;
+    v.w = (uint32_t)(hi >> 32);
+    return v;
+}
+
+__device__ __forceinline__ uint32_t byte_of(const uint4 &v, uint32_t b)
+{
+    const uint32_t w = b < 8 ? (b < 4 ? v.x : v.y) : (b < 12 ? v.z : v.w);
+    return (w >> (8 * (b & 3))) & 0xFFu;
+}
+
 // LDS bytes one wave of the Myers kernels needs: Peq columns, the edge
 // staging slots, the Myers queue (2 * IDB_TILE 16-bit entries), the per-tile
 // count accumulators of queries and targets, and the tile's query records.
@@ -172,6 +216,10 @@ hipError_t idb_launch_pair_distances(const uint8_t *seq, const uint64_t *off, co
 hipError_t idb_launch_gene_bitsets(const uint8_t *calls, const uint64_t *off, const uint32_t *len, uint32_t n,
                                    const idb_gene_hdr *hdr, const uint32_t *gw, uint32_t n_words, uint32_t n_genes,
                                    int32_t *out, uint32_t width, hipStream_t s);
+hipError_t idb_launch_gene_scan(const uint8_t *calls, const uint64_t *off, const uint32_t *len, uint32_t n,
+                                const uint8_t *cls, const uint32_t *nodes, const void *trans, bool narrow,
+                                uint32_t ncls, uint32_t entries, uint32_t out_min, uint32_t n_nodes, uint32_t max_len,
+                                int32_t *out, uint32_t width, hipStream_t s);
 // Cluster growth over the count pass's pairs (rewrites the pair list in place).
 struct idb_union_args {
     const uint32_t *pe;           // per row: one of its entries | core flag << 31; IDB_NONE without entries

@@ -14,10 +14,11 @@
 //
 // Weights are bfloat16 copies of float32 master weights (Adam keeps the
 // master copy); activations are bfloat16, all products accumulate in float32.
-// The three convolutions, their data gradients and their weight gradients run
-// on one MFMA GEMM kernel (v_mfma_f32_32x32x16_bf16) whose operand loaders
-// gather im2col windows straight from the activations, so no im2col matrix is
-// ever materialised.  Row m of an activation matrix is position m % P of
+// Embeddings come from one fused kernel (k_encode).  In training, the three
+// convolutions, their data gradients and their weight gradients run on one
+// MFMA GEMM kernel (v_mfma_f32_32x32x16_bf16) whose operand loaders gather
+// im2col windows straight from the activations, so no im2col matrix is ever
+// materialised.  Row m of an activation matrix is position m % P of
 // sequence m / P; positions at or past the sequence's length are zero after
 // every layer (each row is convolved with its own zero padding).
 #include <algorithm>
@@ -34,6 +35,7 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t T = 5, NTOK = 32, C0 = 32, C = 128, D = 64;
 constexpr float GELU_K = 0.7978845608028654f;  // sqrt(2 / pi)
@@ -265,21 +267,13 @@ struct EpConvFwd {
         const int32_t lim = (int32_t)len[row0 / PP] - (int32_t)(row0 % PP + pl);  // rows d < lim are letters
         const size_t base = (size_t)(row0 + pl) * C + col;
         uint16_t *a = A + base;
-        if (H) {
-            uint16_t *h = H + base;
+        uint16_t *h = H + base;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int32_t d = (r >> 2) * 8 + (r & 3);
-                const float x = v[r] + b;
-                h[d * C] = f2bf(x);
-                a[d * C] = d < lim ? f2bf(gelu(x)) : (uint16_t)0;
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int32_t d = (r >> 2) * 8 + (r & 3);
-                a[d * C] = d < lim ? f2bf(gelu(v[r] + b)) : (uint16_t)0;
-            }
+        for (int r = 0; r < 16; ++r) {
+            const int32_t d = (r >> 2) * 8 + (r & 3);
+            const float x = v[r] + b;
+            h[d * C] = f2bf(x);
+            a[d * C] = d < lim ? f2bf(gelu(x)) : (uint16_t)0;
         }
     }
 };
@@ -390,7 +384,7 @@ __global__ void k_embed(const uint8_t *btok, const uint32_t *blen, uint32_t nseq
 // Head: mean over the sequence's letters, projection, L2 norm.  One wave per
 // sequence: lanes hold channels l and l + 64, then output l.
 __global__ void k_head_fwd(const uint16_t *A3, const uint32_t *blen, uint32_t nseq, uint32_t P, const uint16_t *wp_b,
-                           const uint16_t *bp, float *pool, float *u, float *z, uint16_t *zb)
+                           const uint16_t *bp, float *pool, float *u, float *z)
 {
     __shared__ float sp[4][C];
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -406,10 +400,8 @@ __global__ void k_head_fwd(const uint16_t *A3, const uint32_t *blen, uint32_t ns
         a1 *= inv;
         sp[w][lane] = a0;
         sp[w][lane + 64] = a1;
-        if (pool) {
-            pool[(size_t)s * C + lane] = a0;
-            pool[(size_t)s * C + lane + 64] = a1;
-        }
+        pool[(size_t)s * C + lane] = a0;
+        pool[(size_t)s * C + lane + 64] = a1;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         float acc = bf2f(bp[lane]);
         for (uint32_t o = 0; o < C; ++o) acc += bf2f(wp_b[(size_t)lane * C + o]) * sp[w][o];
@@ -417,10 +409,8 @@ __global__ void k_head_fwd(const uint16_t *A3, const uint32_t *blen, uint32_t ns
 #pragma unroll
         for (int k = 32; k > 0; k >>= 1) ss += __shfl_xor(ss, k, 64);
         const float nrm = fmaxf(sqrtf(ss), 1e-6f);
-        const float zz = acc / nrm;
-        if (u) u[(size_t)s * D + lane] = acc;
-        if (z) z[(size_t)s * D + lane] = zz;
-        if (zb) zb[(size_t)s * D + lane] = f2bf(zz);
+        u[(size_t)s * D + lane] = acc;
+        z[(size_t)s * D + lane] = acc / nrm;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     }
 }
@@ -559,6 +549,320 @@ __global__ void k_adam(float *th, const float *g, float *m, float *v, uint32_t n
     }
 }
 
+// ---------------------------------------------------------------------------
+// Inference: the whole encoder in one kernel.
+//
+// A block takes a tile of EM = 256 activation rows and keeps them in LDS
+// through all three convolutions (layer by layer, in place), so neither
+// activations nor im2col windows touch HBM.  Sequences are packed back to
+// back with two zero rows between them: a 5-tap window reaches two rows, so
+// that is the zero padding of both neighbours, and no row is spent on
+// positions past a sequence's end (protein rows average 15 of 32 positions,
+// 24-150-letter rows 87 of 160).  Products run transposed (channels x rows):
+// a lane then holds four consecutive channels of one row, which leave as one
+// 8-byte LDS store, and validity is one bit per lane.
+//   4 waves of 64 channels x 128 rows: per 16-deep k step 8 MFMAs (256
+// cycles) take 4 row fragments from LDS (50% of its bandwidth over the 4
+// waves) and 2 weight fragments from L2, packed so that a wave reads 1 KB
+// in a row.  128 accumulators leave room for 2 waves per SIMD; at 71 KB of
+// activations two blocks share a CU, so one block's GELU (as many VALU cycles
+// as the MFMAs take) overlaps the other's products.
+// The k order and the arithmetic of every output are those of the training
+// forward pass (k_gemm), bit for bit.
+// Measured: 200k protein rows (packed 1.25 Tflop) 5.22 -> 1.52 ms, 825 TFLOP/s
+// (a large bf16 product reaches 1,214 here); 20k rows of 24-150 letters
+// 2.98 -> 0.81 ms.
+constexpr uint32_t EM = 256, EST = C + 8;         // rows per tile; LDS row stride (272 bytes: conflict-free)
+constexpr uint32_t EPW = 1024;                    // sequences per packing window
+constexpr uint32_t EGRP = 8;                      // sequences per round of the head
+constexpr uint32_t EKS1 = T * C0 / 16, EKS = T * C / 16;  // k steps of layer 1, of layers 2 and 3
+constexpr size_t EPACK = (size_t)(EKS1 + 2 * EKS) * 4 * 64 * 8;  // packed weights (bfloat16)
+
+// Greedy packing of consecutive sequences into tiles, window by window:
+// tiles (first sequence, count) in any order, and every sequence's first row
+// within its tile.  At most EM + 2 rows per tile counting each sequence's two
+// zero rows (the last two lie in the tile's zero border).
+__global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t n, uint32_t P, uint2 *tiles,
+                                                  uint32_t *n_tiles, uint16_t *rstart)
+{
+    __shared__ uint32_t S[EPW + 1], cut[EPW + 1], part[4], base_s;
+    __shared__ uint16_t nxt[EPW];
+    const uint32_t w0 = blockIdx.x * EPW, m = min(EPW, n - w0), tid = threadIdx.x, lane = tid & 63;
+    constexpr uint32_t PER = EPW / 256;
+    uint32_t v[PER], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < PER; ++k) {
+        const uint32_t i = tid * PER + k;
+        v[k] = i < m ? min(len[w0 + i], P) + 2u : 0u;
+        sum += v[k];
+    }
+    uint32_t inc = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = (uint32_t)__shfl_up((int)inc, o, 64);
+        if (lane >= (uint32_t)o) inc += t;
+    }
+    if (lane == 63) part[tid >> 6] = inc;
+    __syncthreads();
+    uint32_t at = inc - sum;
+    for (uint32_t w = 0; w < (tid >> 6); ++w) at += part[w];
+#pragma unroll
+    for (uint32_t k = 0; k < PER; ++k) {
+        S[tid * PER + k] = at;
+        at += v[k];
+    }
+    if (tid == 255) S[EPW] = at;
+    __syncthreads();
+    // the tile that starts at sequence i ends before nxt[i]
+    for (uint32_t i = tid; i < m; i += 256) {
+        uint32_t lo = i + 1, hi = m;  // S[lo] - S[i] fits (one sequence always does)
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (S[mid] - S[i] <= EM + 2u) lo = mid; else hi = mid - 1;
+        }
+        nxt[i] = (uint16_t)lo;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t c = 0;
+        for (uint32_t i = 0; i < m; i = nxt[i]) cut[c++] = i;
+        cut[c] = m;
+        part[0] = c;
+        base_s = atomicAdd(n_tiles, c);
+    }
+    __syncthreads();
+    const uint32_t c = part[0];
+    for (uint32_t t = tid; t < c; t += 256) tiles[base_s + t] = make_uint2(w0 + cut[t], cut[t + 1] - cut[t]);
+    for (uint32_t i = tid; i < m; i += 256) {
+        uint32_t lo = 0, hi = c;  // last tile that starts at or before i
+        while (lo + 1 < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (cut[mid] <= i) lo = mid; else hi = mid;
+        }
+        rstart[w0 + i] = (uint16_t)(S[i] - S[cut[lo]]);
+    }
+}
+
+// Weights in the order the encoder's waves read them: per layer and k step,
+// four 32-channel fragments of 64 lanes x 8 values; then the projection as
+// (input pair, output) words.
+__global__ void k_enc_pack(const uint16_t *theta_b, uint16_t *dst, uint32_t *wp2)
+{
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < EPACK; i += gridDim.x * blockDim.x) {
+        const uint32_t e = i & 7u, ln = (i >> 3) & 63u, ct = (i >> 9) & 3u;
+        uint32_t ks = i >> 11, cin = C0, o = O_W1;
+        if (ks >= EKS1) {
+            ks -= EKS1;
+            cin = C;
+            o = O_W2;
+            if (ks >= EKS) {
+                ks -= EKS;
+                o = O_W3;
+            }
+        }
+        dst[i] = theta_b[o + (ct * 32 + (ln & 31u)) * (T * cin) + ks * 16 + (ln >> 5) * 8 + e];
+    }
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < C / 2 * D; i += gridDim.x * blockDim.x) {
+        const uint32_t d = i % D, o = 2 * (i / D);
+        wp2[i] = (uint32_t)theta_b[O_WP + d * C + o] | ((uint32_t)theta_b[O_WP + d * C + o + 1] << 16);
+    }
+}
+
+struct EncArgs {
+    const uint8_t *seq;
+    const uint64_t *off;
+    const uint32_t *len;
+    const uint2 *tiles;
+    const uint32_t *n_tiles;
+    const uint16_t *rstart;
+    const uint8_t *vocab;
+    const uint16_t *theta_b, *pack;
+    const uint32_t *wp2;
+    uint32_t P;
+    float *z;        // either may be null
+    uint16_t *zb;
+};
+
+// One convolution over the tile: acc = W x window, CIN input channels.
+template <uint32_t CIN>
+__device__ __forceinline__ void enc_conv(const uint16_t *X, const u32x4 *wp, uint32_t lane, f32x16 (&acc)[2][4])
+{
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    constexpr uint32_t KT = CIN / 16, AHEAD = 2;  // k steps per tap; weight fragments loaded ahead
+    const uint16_t *xr = X + (lane & 31u) * EST + (lane >> 5) * 8;
+    u32x4 wq[AHEAD][2];
+#pragma unroll
+    for (uint32_t a = 0; a < AHEAD; ++a) {
+        wq[a][0] = wp[a * 256];
+        wq[a][1] = wp[a * 256 + 64];
+    }
+#pragma unroll 1
+    for (uint32_t t = 0; t < T; ++t) {
+        const uint16_t *xt = xr + t * EST;
+        const u32x4 *wt = wp + t * KT * 256;
+#pragma unroll
+        for (uint32_t c = 0; c < KT; ++c) {
+            bf16x8 w0 = __builtin_bit_cast(bf16x8, wq[c % AHEAD][0]), w1 = __builtin_bit_cast(bf16x8, wq[c % AHEAD][1]);
+            // (past the layer's last step: the next layer's first fragments,
+            // or the buffer's padding)
+            wq[c % AHEAD][0] = wt[(c + AHEAD) * 256];
+            wq[c % AHEAD][1] = wt[(c + AHEAD) * 256 + 64];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bf16x8 x = *(const bf16x8 *)(xt + j * 32 * EST + c * 16);
+                acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0, x, acc[0][j], 0, 0, 0);
+                acc[1][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1, x, acc[1][j], 0, 0, 0);
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
+{
+    __shared__ __align__(16) uint16_t X[(EM + 4) * EST];
+    __shared__ __align__(16) float bias[3 * C];
+    __shared__ __align__(16) float sp[EGRP][C];
+    __shared__ uint32_t s_len[EM / 2 + 2];
+    __shared__ uint16_t s_row[EM / 2 + 2];
+    __shared__ uint64_t s_off[EM / 2 + 2];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t wc = wave & 1u, wr = wave >> 1;  // this wave's 64 channels and 128 rows
+    for (uint32_t i = tid; i < 3 * C; i += 256) {
+        const uint32_t l = i / C, c = i % C;
+        bias[i] = bf2f(a.theta_b[(l == 0 ? O_B1 : (l == 1 ? O_B2 : O_B3)) + c]);
+    }
+    // the zero border: two rows before the tile and two after
+    for (uint32_t i = tid; i < 4 * EST; i += 256) X[(i < 2 * EST ? 0 : EM * EST) + i] = 0;
+    const uint32_t nt = *a.n_tiles;
+    for (uint32_t ti = blockIdx.x; ti < nt; ti += gridDim.x) {
+        const uint2 t = a.tiles[ti];
+        const uint32_t first = t.x, cnt = t.y;  // cnt <= EM / 2 + 1: two rows at least per sequence
+        __syncthreads();
+        if (tid < cnt) {
+            s_len[tid] = min(a.len[first + tid], a.P);
+            s_row[tid] = a.rstart[first + tid];
+            s_off[tid] = a.off[first + tid];
+        }
+        __syncthreads();
+        {
+            // embedding: thread = row
+            uint32_t lo = 0, hi = cnt;
+            while (lo + 1 < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (s_row[mid] <= tid) lo = mid; else hi = mid;
+            }
+            const uint32_t p = tid - s_row[lo];
+            u32x4 e[4] = {};
+            if (p < s_len[lo]) {
+                const u32x4 *src = (const u32x4 *)(a.theta_b + O_EMB + (uint32_t)a.vocab[a.seq[s_off[lo] + p]] * C0);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) e[k] = src[k];
+            }
+            u32x4 *dst = (u32x4 *)(X + (tid + 2) * EST);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) dst[k] = e[k];
+        }
+        // validity of this lane's four rows (row wr * 128 + 32 j + lane % 32)
+        uint32_t valid = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t row = wr * 128 + 32 * j + (lane & 31u);
+            uint32_t lo = 0, hi = cnt;
+            while (lo + 1 < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (s_row[mid] <= row) lo = mid; else hi = mid;
+            }
+            if (row - s_row[lo] < s_len[lo]) valid |= 1u << j;
+        }
+        __syncthreads();
+        const uint16_t *Xw = X + wr * 128 * EST;
+        const u32x4 *wp = (const u32x4 *)a.pack + wc * 128 + lane;
+#pragma unroll 1
+        for (uint32_t l = 0; l < 3; ++l) {
+            f32x16 acc[2][4];
+            if (l == 0) enc_conv<C0>(Xw, wp, lane, acc);
+            else enc_conv<C>(Xw, wp + (EKS1 + (l - 1) * EKS) * 256, lane, acc);
+            __syncthreads();  // every wave has read the layer's input
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t ch = wc * 64 + i * 32 + 8 * q + 4 * (lane >> 5);
+                    const float4 b = *(const float4 *)(bias + l * C + ch);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float g0 = gelu(acc[i][j][4 * q] + b.x), g1 = gelu(acc[i][j][4 * q + 1] + b.y),
+                                    g2 = gelu(acc[i][j][4 * q + 2] + b.z), g3 = gelu(acc[i][j][4 * q + 3] + b.w);
+                        const bool v = (valid >> j) & 1u;
+                        uint2 o;
+                        o.x = v ? (uint32_t)f2bf(g0) | ((uint32_t)f2bf(g1) << 16) : 0u;
+                        o.y = v ? (uint32_t)f2bf(g2) | ((uint32_t)f2bf(g3) << 16) : 0u;
+                        *(uint2 *)(X + (2 + wr * 128 + 32 * j + (lane & 31u)) * EST + ch) = o;
+                    }
+                }
+            __syncthreads();
+        }
+        // head, EGRP sequences a round: mean over the letters (a wave per
+        // sequence, two channels per lane), projection, L2 norm
+        for (uint32_t s0 = 0; s0 < cnt; s0 += EGRP) {
+#pragma unroll
+            for (uint32_t r = 0; r < EGRP / 4; ++r) {
+                const uint32_t s = s0 + r * 4 + wave;
+                if (s < cnt) {
+                    const uint32_t L = s_len[s];
+                    const uint16_t *src = X + (2 + s_row[s]) * EST + 2 * lane;
+                    float a0 = 0.f, a1 = 0.f;
+                    for (uint32_t p = 0; p < L; ++p) {
+                        const uint32_t v = *(const uint32_t *)(src + p * EST);
+                        a0 += bf2f((uint16_t)v);
+                        a1 += bf2f((uint16_t)(v >> 16));
+                    }
+                    const float inv = L ? 1.f / (float)L : 0.f;
+                    a0 *= inv;
+                    a1 *= inv;
+                    *(float2 *)(&sp[r * 4 + wave][2 * lane]) = make_float2(a0, a1);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            float u[EGRP / 4];
+            const float b0 = bf2f(a.theta_b[O_BP + lane]);
+#pragma unroll
+            for (uint32_t r = 0; r < EGRP / 4; ++r) u[r] = b0;
+#pragma unroll 4
+            for (uint32_t o = 0; o < C; o += 4) {
+                const uint32_t wa = a.wp2[(o / 2) * D + lane], wb = a.wp2[(o / 2 + 1) * D + lane];
+#pragma unroll
+                for (uint32_t r = 0; r < EGRP / 4; ++r) {
+                    const float4 p4 = *(const float4 *)(&sp[r * 4 + wave][o]);
+                    u[r] += bf2f((uint16_t)wa) * p4.x;
+                    u[r] += bf2f((uint16_t)(wa >> 16)) * p4.y;
+                    u[r] += bf2f((uint16_t)wb) * p4.z;
+                    u[r] += bf2f((uint16_t)(wb >> 16)) * p4.w;
+                }
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < EGRP / 4; ++r) {
+                const uint32_t s = s0 + r * 4 + wave;
+                float ss = u[r] * u[r];
+#pragma unroll
+                for (int k = 32; k > 0; k >>= 1) ss += __shfl_xor(ss, k, 64);
+                const float nrm = fmaxf(sqrtf(ss), 1e-6f);
+                const float zz = u[r] / nrm;
+                if (s < cnt) {
+                    if (a.z) a.z[(size_t)(first + s) * D + lane] = zz;
+                    if (a.zb) a.zb[(size_t)(first + s) * D + lane] = f2bf(zz);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
+    }
+}
+
 uint32_t nblocks(uint64_t n, uint32_t bs = 256)
 {
     uint64_t b = (n + bs - 1) / bs;
@@ -593,7 +897,6 @@ struct idb_encoder {
     std::string err;
     // workspace
     uint32_t cap_seq = 0;
-    bool cap_train = false;
     uint8_t *btok = nullptr;
     uint32_t *blen = nullptr, *brows = nullptr;
     uint16_t *X0 = nullptr, *A[3] = {nullptr, nullptr, nullptr}, *H[3] = {nullptr, nullptr, nullptr};
@@ -605,6 +908,18 @@ struct idb_encoder {
     uint32_t *tlen = nullptr;
     uint32_t tok_cap = 0;
     uint8_t *vocab_d = nullptr;
+    // inference: weights in the fused kernel's order (packed again when the
+    // parameters have changed), and the packing of the current rows
+    uint16_t *pack = nullptr;
+    uint32_t *wp2 = nullptr;
+    bool pack_stale = true;
+    uint2 *tiles = nullptr;
+    uint16_t *rstart = nullptr;
+    uint32_t *n_tiles = nullptr;
+    uint32_t plan_cap = 0;
+    float *zbuf = nullptr;
+    uint32_t zbuf_cap = 0;
+    uint32_t enc_blocks = 0;
     std::vector<void *> fixed, ws;  // parameter and workspace allocations
 };
 
@@ -626,35 +941,31 @@ void free_workspace(idb_encoder *e)
     e->cap_seq = 0;
 }
 
-void ensure_workspace(idb_encoder *e, uint32_t nseq, bool train)
+// Workspace of a training step over nseq sequences.
+void ensure_workspace(idb_encoder *e, uint32_t nseq)
 {
-    if (nseq <= e->cap_seq && (!train || e->cap_train)) return;
+    if (nseq <= e->cap_seq) return;
     free_workspace(e);
     const size_t M = (size_t)nseq * e->P;
     e->btok = dalloc<uint8_t>(e->ws, M);
     e->blen = dalloc<uint32_t>(e->ws, nseq);
     e->brows = dalloc<uint32_t>(e->ws, nseq);
     e->X0 = dalloc<uint16_t>(e->ws, M * C0);
-    e->A[0] = dalloc<uint16_t>(e->ws, M * C);
-    e->A[1] = dalloc<uint16_t>(e->ws, M * C);
-    e->A[2] = train ? dalloc<uint16_t>(e->ws, M * C) : e->A[0];
+    for (int l = 0; l < 3; ++l) {
+        e->A[l] = dalloc<uint16_t>(e->ws, M * C);
+        e->H[l] = dalloc<uint16_t>(e->ws, M * C);
+    }
     e->pool = dalloc<float>(e->ws, (size_t)nseq * C);
     e->u = dalloc<float>(e->ws, (size_t)nseq * D);
     e->z = dalloc<float>(e->ws, (size_t)nseq * D);
-    if (train) {
-        for (int l = 0; l < 3; ++l) e->H[l] = dalloc<uint16_t>(e->ws, M * C);
-        e->dHa = dalloc<uint16_t>(e->ws, M * C);
-        e->dHb = dalloc<uint16_t>(e->ws, M * C);
-        e->dX0 = dalloc<float>(e->ws, M * C0);
-        e->dz = dalloc<float>(e->ws, (size_t)nseq * D);
-        e->du = dalloc<float>(e->ws, (size_t)nseq * D);
-        e->y = dalloc<float>(e->ws, nseq / 2 + 1);
-        e->loss = dalloc<float>(e->ws, 1);
-    } else {
-        for (int l = 0; l < 3; ++l) e->H[l] = nullptr;
-    }
+    e->dHa = dalloc<uint16_t>(e->ws, M * C);
+    e->dHb = dalloc<uint16_t>(e->ws, M * C);
+    e->dX0 = dalloc<float>(e->ws, M * C0);
+    e->dz = dalloc<float>(e->ws, (size_t)nseq * D);
+    e->du = dalloc<float>(e->ws, (size_t)nseq * D);
+    e->y = dalloc<float>(e->ws, nseq / 2 + 1);
+    e->loss = dalloc<float>(e->ws, 1);
     e->cap_seq = nseq;
-    e->cap_train = train;
 }
 
 void refresh_transposed(idb_encoder *e)
@@ -665,11 +976,55 @@ void refresh_transposed(idb_encoder *e)
         hipLaunchKernelGGL(k_transpose_w, dim3(nblocks((size_t)C * T * cins[l])), dim3(256), 0, e->stream,
                            e->theta_b + offs[l], cins[l], e->wt[l]);
     hcheck(hipGetLastError(), "transpose launch");
+    e->pack_stale = true;
 }
 
-// Forward over the batch in e->btok / e->blen (nseq, a multiple of 4).
+// Embeddings of rows [0, n) of device data by the fused kernel, on e->stream:
+// float32 (z) and/or bfloat16 (zb), 64 per row.
+void embed_fused(idb_encoder *e, const uint8_t *seq, const uint64_t *off, const uint32_t *len, uint32_t n, float *z,
+                 uint16_t *zb)
+{
+    if (n == 0) return;
+    hipStream_t s = e->stream;
+    if (!e->pack) {
+        // (AHEAD fragments are read past the last layer's end)
+        uint16_t *pack = dalloc<uint16_t>(e->fixed, EPACK + 2 * 2048);
+        e->wp2 = dalloc<uint32_t>(e->fixed, C / 2 * D);
+        e->n_tiles = dalloc<uint32_t>(e->fixed, 1);
+        hcheck(hipMemsetAsync(pack, 0, (EPACK + 2 * 2048) * sizeof(uint16_t), s), "memset");
+        int dev = 0, cus = 0, per_cu = 0;
+        hcheck(hipGetDevice(&dev), "device");
+        hcheck(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device");
+        hcheck(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_encode, 256, 0), "occupancy");
+        e->enc_blocks = (uint32_t)(std::max(per_cu, 1) * cus);
+        e->pack = pack;
+    }
+    if (e->pack_stale) {
+        hipLaunchKernelGGL(k_enc_pack, dim3(256), dim3(256), 0, s, e->theta_b, e->pack, e->wp2);
+        e->pack_stale = false;
+    }
+    if (n > e->plan_cap) {
+        hcheck(hipStreamSynchronize(s), "sync");
+        (void)hipFree(e->tiles);
+        (void)hipFree(e->rstart);
+        e->tiles = nullptr;
+        e->rstart = nullptr;
+        e->plan_cap = 0;
+        hcheck(hipMalloc(&e->tiles, sizeof(uint2) * (size_t)n), "hipMalloc");
+        hcheck(hipMalloc(&e->rstart, sizeof(uint16_t) * (size_t)n), "hipMalloc");
+        e->plan_cap = n;
+    }
+    hcheck(hipMemsetAsync(e->n_tiles, 0, sizeof(uint32_t), s), "memset");
+    hipLaunchKernelGGL(k_enc_plan, dim3((n + EPW - 1) / EPW), dim3(256), 0, s, len, n, e->P, e->tiles, e->n_tiles,
+                       e->rstart);
+    const EncArgs a{seq, off, len, e->tiles, e->n_tiles, e->rstart, e->vocab_d, e->theta_b, e->pack, e->wp2, e->P, z, zb};
+    hipLaunchKernelGGL(k_encode, dim3(std::min(e->enc_blocks, n)), dim3(256), 0, s, a);
+    hcheck(hipGetLastError(), "encoder launch");
+}
+
+// Training forward pass over the batch in e->btok / e->blen (nseq, a multiple of 4).
 template <uint32_t PP>
-void forward_p(idb_encoder *e, uint32_t nseq, bool train, uint16_t *zb_out)
+void forward_p(idb_encoder *e, uint32_t nseq)
 {
     hipStream_t s = e->stream;
     const uint32_t M = nseq * PP;
@@ -679,24 +1034,24 @@ void forward_p(idb_encoder *e, uint32_t nseq, bool train, uint16_t *zb_out)
     uint32_t cin = C0;
     const uint32_t offs[3] = {O_W1, O_W2, O_W3}, boff[3] = {O_B1, O_B2, O_B3};
     for (int l = 0; l < 3; ++l) {
-        uint16_t *out = train ? e->A[l] : e->A[l & 1];
+        uint16_t *out = e->A[l];
         LdConv<PP> la{in, cin, M, 0};
         LdRows lb{e->theta_b + offs[l], T * cin, C};
-        EpConvFwd<PP> ep{e->theta_b + boff[l], e->blen, train ? e->H[l] : nullptr, out};
+        EpConvFwd<PP> ep{e->theta_b + boff[l], e->blen, e->H[l], out};
         hipLaunchKernelGGL((k_gemm<LdConv<PP>, LdRows, EpConvFwd<PP>>), dim3((M + GM - 1) / GM, 1, 1), dim3(256), 0, s,
                            la, lb, ep, M, C, T * cin, T * cin);
         in = out;
         cin = C;
     }
     hipLaunchKernelGGL(k_head_fwd, dim3(nblocks(nseq, 4)), dim3(256), 0, s, in, e->blen, nseq, PP, e->theta_b + O_WP,
-                       e->theta_b + O_BP, train ? e->pool : nullptr, train ? e->u : nullptr, e->z, zb_out);
+                       e->theta_b + O_BP, e->pool, e->u, e->z);
     hcheck(hipGetLastError(), "encoder forward launch");
 }
 
-void forward(idb_encoder *e, uint32_t nseq, bool train, uint16_t *zb_out)
+void forward(idb_encoder *e, uint32_t nseq)
 {
-    if (e->P == 160) forward_p<160>(e, nseq, train, zb_out);
-    else forward_p<32>(e, nseq, train, zb_out);
+    if (e->P == 160) forward_p<160>(e, nseq);
+    else forward_p<32>(e, nseq);
 }
 
 // Backward of sum(dz . z) into e->grad (zeroed here).
@@ -802,7 +1157,7 @@ float step(idb_encoder *e, const uint32_t *pairs_d, const float *labels_d, const
                        e->y, labels_d);
     hipLaunchKernelGGL(k_gather_rows, dim3(nblocks(nseq)), dim3(256), 0, s, e->tok, e->tlen, e->brows, nseq, e->P,
                        e->btok, e->blen);
-    forward(e, nseq, true, nullptr);
+    forward(e, nseq);
     hcheck(hipMemsetAsync(e->loss, 0, sizeof(float), s), "memset");
     hcheck(hipMemsetAsync(e->dz, 0, sizeof(float) * (size_t)nseq * D, s), "memset");
     hipLaunchKernelGGL(k_pair_loss, dim3(nblocks(nb, 4)), dim3(256), 0, s, e->z, e->y, nb, margin, inv_b, e->dz, e->loss);
@@ -834,31 +1189,15 @@ int guard(idb_encoder *e, F &&f)
 }  // namespace
 
 // Embeddings (bfloat16, 64 per row) of rows [0, n) for the learned pair
-// kernel; chunked so the workspace stays bounded.
+// kernel.
 hipError_t idb_encoder_embed_rows(idb_encoder *e, const uint8_t *seq, const uint64_t *off, const uint32_t *len,
                                   uint32_t n, uint16_t *zb, hipStream_t s)
 {
-    idb_dataset d{};
-    d.n_rows = n;
-    d.mem = IDB_MEM_DEVICE;
-    d.seq = seq;
-    d.off = off;
-    d.len = len;
     const int rc = guard(e, [&] {
         hipStream_t keep = e->stream;
         e->stream = s;
         try {
-            tokenize(e, &d);
-            // 32768 rows of 32 positions per chunk: activations of 1M positions
-            const uint32_t chunk = round4(32768u * 32u / e->P);
-            ensure_workspace(e, std::min(round4(n), chunk), false);
-            for (uint32_t first = 0; first < n; first += chunk) {
-                const uint32_t nb = round4(std::min(chunk, n - first));
-                hipLaunchKernelGGL(k_iota_rows, dim3(nblocks(nb)), dim3(256), 0, s, first, n, nb, e->brows);
-                hipLaunchKernelGGL(k_gather_rows, dim3(nblocks(nb)), dim3(256), 0, s, e->tok, e->tlen, e->brows, nb,
-                                   e->P, e->btok, e->blen);
-                forward(e, nb, false, zb + (size_t)first * D);
-            }
+            embed_fused(e, seq, off, len, n, nullptr, zb);
         } catch (...) {
             e->stream = keep;
             throw;
@@ -947,6 +1286,9 @@ void idb_encoder_destroy(idb_encoder *e)
     for (void *p : e->ws) (void)hipFree(p);
     (void)hipFree(e->tok);
     (void)hipFree(e->tlen);
+    (void)hipFree(e->tiles);
+    (void)hipFree(e->rstart);
+    (void)hipFree(e->zbuf);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
 }
@@ -982,17 +1324,20 @@ int idb_encoder_embed(idb_encoder *e, const idb_dataset *d, float *z_host)
     return guard(e, [&] {
         DevData dd;
         const idb_dataset *dv = device_view(d, dd, e->stream);
-        tokenize(e, dv);
-        const uint32_t n = d->n_rows, chunk = round4(32768u * 32u / e->P);
-        ensure_workspace(e, std::min(round4(std::max(n, 1u)), chunk), false);
-        std::vector<float> buf;
+        // a million rows (256 MB of embeddings) at a time
+        const uint32_t n = d->n_rows, chunk = 1u << 20;
+        if (std::min(n, chunk) > e->zbuf_cap) {
+            hcheck(hipStreamSynchronize(e->stream), "sync");
+            (void)hipFree(e->zbuf);
+            e->zbuf = nullptr;
+            e->zbuf_cap = 0;
+            hcheck(hipMalloc(&e->zbuf, sizeof(float) * D * std::min(n, chunk)), "hipMalloc");
+            e->zbuf_cap = std::min(n, chunk);
+        }
         for (uint32_t first = 0; first < n; first += chunk) {
-            const uint32_t cnt = std::min(chunk, n - first), nb = round4(cnt);
-            hipLaunchKernelGGL(k_iota_rows, dim3(nblocks(nb)), dim3(256), 0, e->stream, first, n, nb, e->brows);
-            hipLaunchKernelGGL(k_gather_rows, dim3(nblocks(nb)), dim3(256), 0, e->stream, e->tok, e->tlen, e->brows, nb,
-                               e->P, e->btok, e->blen);
-            forward(e, nb, false, nullptr);
-            hcheck(hipMemcpyAsync(z_host + (size_t)first * D, e->z, sizeof(float) * cnt * D, hipMemcpyDeviceToHost,
+            const uint32_t cnt = std::min(chunk, n - first);
+            embed_fused(e, dv->seq, dv->off + first, dv->len + first, cnt, e->zbuf, nullptr);
+            hcheck(hipMemcpyAsync(z_host + (size_t)first * D, e->zbuf, sizeof(float) * cnt * D, hipMemcpyDeviceToHost,
                                   e->stream), "copy");
         }
         hcheck(hipStreamSynchronize(e->stream), "sync");
@@ -1011,7 +1356,7 @@ int idb_encoder_loss_grad(idb_encoder *e, const idb_dataset *d, const uint32_t *
         tokenize(e, dv);
         const uint32_t *pd = dd.up(pairs, 2 * (size_t)n_pairs, e->stream);
         const float *ld = dd.up(labels, n_pairs, e->stream);
-        ensure_workspace(e, round4(2 * n_pairs), true);
+        ensure_workspace(e, round4(2 * n_pairs));
         *loss = step(e, pd, ld, nullptr, 0, n_pairs, n_pairs, margin, 1.f / (float)n_pairs, true);
         hcheck(hipMemcpyAsync(grad_host, e->grad, sizeof(float) * N_PARAMS, hipMemcpyDeviceToHost, e->stream), "copy");
         hcheck(hipStreamSynchronize(e->stream), "sync");
@@ -1032,7 +1377,7 @@ int idb_encoder_train(idb_encoder *e, const idb_dataset *d, const uint32_t *pair
         const uint32_t *pd = dd.up(pairs, 2 * (size_t)n_pairs, e->stream);
         const float *ld = dd.up(labels, n_pairs, e->stream);
         const uint32_t B = tp->batch_pairs;
-        ensure_workspace(e, round4(2 * B), true);
+        ensure_workspace(e, round4(2 * B));
         std::vector<uint32_t> order(n_pairs);
         std::iota(order.begin(), order.end(), 0u);
         std::mt19937_64 rng(tp->seed);

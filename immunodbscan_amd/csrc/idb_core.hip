@@ -38,6 +38,7 @@
 
 #include "../../include/idb.h"
 #include "idb_internal.h"
+#include "mxfeat.h"
 #include "copy_pool.h"
 #include "gene_table.h"
 
@@ -78,7 +79,7 @@ enum Slot {
     S_LAB, S_RANK, S_RFLAG, S_QBCNT, S_BFLAG, S_TLUT_C, S_SMALL, S_WORK, S_TMP,
     S_OUT_CID, S_OUT_CORE, S_OUT_COP, S_OUT_UNQ, S_OUT_CNT, S_USTART, S_EDGES, S_ENT, S_FILL, S_ZB, S_PAIRS,
     S_DIST, S_CNT2, S_EQG, S_RSCNT, S_PE, S_PARE, S_CMINE, S_GCALLS, S_GOFF, S_GLEN, S_GOUT, S_GHDR, S_GWORDS,
-    S_ELOW, S_SCAN, S_ROWREC, S_COUNT
+    S_ELOW, S_SCAN, S_ROWREC, S_META, S_FEAT, S_VREC, S_INV, S_CNTE, S_ECORE, S_COUNT
 };
 
 struct idb_ctx {
@@ -430,7 +431,8 @@ __global__ void k_membership(const uint32_t *uniq, const uint32_t *num, const in
 // (lb = bits of the longest row).
 __global__ void k_emit_entries(const uint32_t *uniq, const uint32_t *num, const uint64_t *eoff, const int32_t *vb,
                                uint32_t vw, const int32_t *jb, uint32_t jw, const uint32_t *len, const uint32_t *rid,
-                               uint32_t single, uint32_t gj, uint32_t gvj, uint32_t lb, uint64_t *ekey, uint32_t *erow)
+                               uint32_t single, uint32_t gj, uint32_t gvj, uint32_t lb, uint64_t *ekey, uint32_t *erow,
+                               uint4 *rrec)
 {
     const uint32_t U = num[0];
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < U; k += gridDim.x * blockDim.x) {
@@ -438,6 +440,7 @@ __global__ void k_emit_entries(const uint32_t *uniq, const uint32_t *num, const 
         const uint64_t r = rid ? rid[u] : 0u;
         const uint64_t L = len[u];
         uint64_t o = eoff[k];
+        if (rrec) rrec[2 * (size_t)u].w = (uint32_t)o;  // where the row's entries are listed
         if (single) {
             ekey[o] = (r << lb) | L;
             erow[o] = u;
@@ -464,13 +467,6 @@ __global__ void k_emit_entries(const uint32_t *uniq, const uint32_t *num, const 
     }
 }
 
-// Word k of a gene bitset restricted to the genes below gene g.
-__device__ __forceinline__ uint32_t below_gene(uint32_t w, uint32_t k, uint32_t g)
-{
-    if (k * 32 >= g) return 0u;
-    return (k * 32 + 32 > g) ? (w & ((1u << (g - k * 32)) - 1u)) : w;
-}
-
 // Residues mod 16 of the set bits of `w` below gene `g` (all bits when g is
 // ~0u), folded into a 16-bit mask.
 __device__ __forceinline__ uint32_t gene_residues(const int32_t *w, uint32_t nw, uint32_t g)
@@ -492,8 +488,8 @@ __global__ void k_fill_entries(const uint64_t *ekey, const uint32_t *erow, uint3
                                const uint8_t *cmap, uint32_t pad, uint32_t S, uint32_t HW, uint32_t bits,
                                const int16_t *tlut_c, const int16_t *tlut_f, uint32_t pres, uint32_t group_len, uint32_t lb,
                                uint16_t *elen, idb_entry *ent, uint32_t *ecodes, uint32_t *epk, uint8_t *bflag,
-                               uint32_t *eqg, uint32_t *pe, uint32_t *par_e, uint32_t *cmin_e, uint4 *elow,
-                               const uint4 *rrec)
+                               uint32_t *eqg, uint32_t *eqm, uint32_t *pe, uint32_t *par_e, uint32_t *cmin_e,
+                               uint4 *elow, const uint4 *rrec)
 {
     __shared__ uint8_t cm[256];
     __shared__ uint32_t qgc[256 * IDB_QGRAM_WORDS];  // one 64-byte 3-gram count row per thread
@@ -623,6 +619,20 @@ __global__ void k_fill_entries(const uint64_t *ekey, const uint32_t *erow, uint3
             uint4 *dst = (uint4 *)(eqg + (size_t)e * IDB_QGRAM_WORDS);
             for (uint32_t w = 0; w < IDB_QGRAM_WORDS / 4; ++w)
                 dst[w] = make_uint4(row[4 * w], row[4 * w + 1], row[4 * w + 2], row[4 * w + 3]);
+        }
+        if (eqm) {
+            // 3-gram level masks (learned runs)
+            uint32_t g[6] = {0u, 0u, 0u, 0u, 0u, 0u}, hist = 0;
+            for (uint32_t k0 = 0; k0 < L; k0 += 16) {
+                const uint4 v = row16(s, L, k0);
+                for (uint32_t b = 0; b < 16 && k0 + b < L; ++b) {
+                    hist = ((hist << 2) | (cm[byte_of(v, b)] & 3u)) & 63u;
+                    if (k0 + b >= 2) idb_qmask_add(g, hist);
+                }
+            }
+            uint4 *dst = (uint4 *)(eqm + (size_t)e * IDB_QMASK_WORDS);
+            dst[0] = make_uint4(g[0], g[1], g[2], g[3]);
+            dst[1] = make_uint4(g[4], g[5] & IDB_MX_NT_L3HI, 0u, 0u);
         }
         if (epk && bits == 5) {
             // six 5-bit letters per word (bits 0..29), trailing fields zero
@@ -775,8 +785,14 @@ __global__ void k_size_tiles(const uint32_t *num, const uint32_t *qboff, const u
 
 __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, const uint32_t *bstart, uint32_t E,
                              const uint16_t *elen, const uint16_t *hilen, uint32_t banded, uint32_t split,
-                             const uint64_t *ekey, uint32_t lb, uint32_t gvj, const uint64_t *toff, idb_tile *tiles)
+                             const uint64_t *ekey, uint32_t lb, uint32_t gvj, const uint64_t *toff, idb_tile *tiles,
+                             uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t chunk_base)
 {
+    // the pair list's chunks that belong to the count pass's waves
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < chunk_base; i += gridDim.x * blockDim.x) {
+        chunk_fill[i] = 0u;
+        if (i == 0) *n_chunks = chunk_base;
+    }
     const uint32_t B = nb_dev[0];
     const uint32_t QB = qboff[B];
     for (uint32_t qb = blockIdx.x * blockDim.x + threadIdx.x; qb < QB; qb += gridDim.x * blockDim.x) {
@@ -806,6 +822,15 @@ __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, cons
             t.shape = qn | (tn << 8) | ((J == q.I ? 1u : 0u) << 16);
             tiles[o++] = t;
         }
+    }
+}
+
+// The pair list's starting state (k_emit_tiles writes it too).
+__global__ void k_chunk_start(uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t base)
+{
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < base; i += gridDim.x * blockDim.x) {
+        chunk_fill[i] = 0u;
+        if (i == 0) *n_chunks = base;
     }
 }
 
@@ -1140,7 +1165,7 @@ struct StageRanges {
 // tiles twice (counts restored from a snapshot in between) and the fastest by
 // HIP events is kept for this kernel and shape class (kernel, words, code
 // width, filter, alphabet, log2 tiles) for the context's lifetime.
-void autotune(idb_ctx *c, idb_pair_args &a, uint32_t N, uint32_t W, bool ham, bool learned, uint32_t *small,
+void autotune(idb_ctx *c, idb_pair_args &a, uint32_t N, uint32_t E, uint32_t W, bool ham, bool learned, uint32_t *small,
               unsigned long long *work)
 {
     uint32_t lt = 0;
@@ -1149,25 +1174,30 @@ void autotune(idb_ctx *c, idb_pair_args &a, uint32_t N, uint32_t W, bool ham, bo
     auto it = c->tuned.find(key);
     if (it == c->tuned.end()) {
         hipStream_t s = c->stream;
-        int32_t *snap = buf<int32_t>(c, S_CNT2, N);
-        check(c, hipMemcpyAsync(snap, a.cnt, sizeof(int32_t) * N, hipMemcpyDeviceToDevice, s), "tune snapshot");
+        // the pass's count output: per entry or per row
+        int32_t *acc = a.cnt_e ? a.cnt_e : a.cnt;
+        const size_t nacc = a.cnt_e ? E : N;
+        int32_t *snap = buf<int32_t>(c, S_CNT2, nacc);
+        check(c, hipMemcpyAsync(snap, acc, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s), "tune snapshot");
         idb_ctx::Tuned best{0, 0, 0, 0};
         float best_ms = 1e30f;
         uint32_t trials = 0;
+        const uint32_t base = a.chunk_base;
+        a.chunk_base = 0;  // trials start from an empty list
         for (uint32_t wpb : {1u, 2u, 4u})
             for (uint32_t mul : {1u, 2u, 4u, 8u})
                 for (uint32_t nx : {0u, 1u}) {
                     a.tune_wpb = wpb;
                     a.tune_grid_mul = mul;
                     a.no_xcd_order = nx;
-                    check(c, hipMemcpyAsync(a.cnt, snap, sizeof(int32_t) * N, hipMemcpyDeviceToDevice, s), "tune reset");
+                    check(c, hipMemcpyAsync(acc, snap, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s), "tune reset");
                     check(c, hipMemsetAsync(small + 12, 0, sizeof(uint32_t), s), "tune reset");
                     check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "tune reset");
                     // best of two runs per shape
                     float ms = 1e30f;
                     for (int rep = 0; rep < 2; ++rep) {
                         if (rep) {
-                            check(c, hipMemcpyAsync(a.cnt, snap, sizeof(int32_t) * N, hipMemcpyDeviceToDevice, s),
+                            check(c, hipMemcpyAsync(acc, snap, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s),
                                   "tune reset");
                             check(c, hipMemsetAsync(small + 12, 0, sizeof(uint32_t), s), "tune reset");
                             check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "tune reset");
@@ -1190,9 +1220,12 @@ void autotune(idb_ctx *c, idb_pair_args &a, uint32_t N, uint32_t W, bool ham, bo
                     }
                 }
         best.trials = trials;
-        check(c, hipMemcpyAsync(a.cnt, snap, sizeof(int32_t) * N, hipMemcpyDeviceToDevice, s), "tune reset");
+        check(c, hipMemcpyAsync(acc, snap, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s), "tune reset");
         check(c, hipMemsetAsync(small + 12, 0, sizeof(uint32_t), s), "tune reset");
         check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "tune reset");
+        a.chunk_base = base;
+        if (base)
+            hipLaunchKernelGGL(k_chunk_start, dim3(blocks_for(base)), dim3(256), 0, s, a.n_chunks, a.chunk_fill, base);
         it = c->tuned.emplace(key, best).first;
     }
     a.tune_wpb = it->second.wpb;
@@ -1430,12 +1463,13 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
     uint32_t B = 0, T = 0;
     idb_pair_args a{};
     idb_union_args ua{};
+    idb_mx_rows_args mr{};
     if (E > 0) {
         uint64_t *ekey = buf<uint64_t>(c, S_EKEY, E), *ekey2 = buf<uint64_t>(c, S_EKEY2, E);
         uint32_t *erow = buf<uint32_t>(c, S_EROW, E), *erow2 = buf<uint32_t>(c, S_EROW2, E);
         const uint32_t lb = std::max(1u, bits_for(maxlen));
         hipLaunchKernelGGL(k_emit_entries, dim3(blocks_for(U)), dim3(256), 0, s, uniq, num, eoff, vb, vw, jb, jw, len, rid,
-                           single, gj, gvj, lb, ekey, erow);
+                           single, gj, gvj, lb, ekey, erow, rrec);
         const uint64_t max_bucket = single ? std::max(n_reps, 1u) : gvj64 * std::max(n_reps, 1u);
         const unsigned ebits = lb + bits_for(max_bucket);
         bool sorted = false, in_first = false;
@@ -1454,30 +1488,71 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         const uint64_t *skey = in_first ? ekey : ekey2;
         const uint32_t *srow = in_first ? erow : erow2;
         uint16_t *elen = buf<uint16_t>(c, S_ELEN, E);
-        idb_entry *ent = buf<idb_entry>(c, S_ENT, E);
         uint8_t *bflag = buf<uint8_t>(c, S_BFLAG, E);
-        uint32_t *ecodes = ham ? nullptr : buf<uint32_t>(c, S_ECODES, (size_t)E * (S / 4));
-        uint32_t *epk = ham ? buf<uint32_t>(c, S_EPK, (size_t)E * HW) : nullptr;
-        // Levenshtein codes are padded with a sentinel letter K whose Peq row
-        // stays zero, so a Peq read for a letter past a row's end stays in
-        // range (with all 256 byte values present code 0 is used; only the
-        // one-word count kernel reads letters past a row's end, and it runs
-        // for alphabets of at most 31 letters)
-        const uint32_t pad = (!ham && K < 256) ? K : 0u;
+        uint32_t *par_e = buf<uint32_t>(c, S_PARE, E), *cmin_e = buf<uint32_t>(c, S_CMINE, E);
         // The absent-letter filter pays off where random letter matches are
         // rare (protein alphabets); with 4 letters nearly every pair passes.
         const bool filt = !ham && W == 1 && K >= 8 && K <= 31;
-        // Nucleotide rows: the 3-gram profile bound (learned runs apply it to their proposals).
+        // Nucleotide rows: the 3-gram bound (learned runs apply it to their proposals).
         const bool qgram = !ham && K <= 4 && maxlen >= 16;
-        uint32_t *eqg = qgram ? buf<uint32_t>(c, S_EQG, (size_t)E * IDB_QGRAM_WORDS) : nullptr;
-        uint32_t *par_e = buf<uint32_t>(c, S_PARE, E), *cmin_e = buf<uint32_t>(c, S_CMINE, E);
+        // Fixed thresholds of a few edits: bound on the matrix cores, verified
+        // on bit planes (idb_mx.hip).  Not in allocation-free calls: an entry
+        // takes a few bytes more there than in the other passes, and what fits
+        // their scratch has to stay the same.
+        const bool mx = !ham && !single && !learned && !c->noalloc && p->abs_k >= 0 && vw + jw <= 4 &&
+                        ((filt && K <= IDB_MX_MAX_LETTERS && p->abs_k <= 3) || (qgram && p->abs_k <= 4));
         // The count passes test the canonical bucket on the entries' own
         // genes below the bucket's (V words, then J words), when they fit
         // four words.
         uint4 *elow = (!single && !learned && vw + jw <= 4) ? buf<uint4>(c, S_ELOW, E) : nullptr;
-        hipLaunchKernelGGL(k_fill_entries, dim3(blocks_for(E)), dim3(256), 0, s, skey, srow, E, seq, off, copies, vb, vw,
-                           jb, jw, single, gj, gvj, cmap, pad, S, HW, bits, tlut_c, tlut_f, filt ? 1u : 0u,
-                           ham ? 1u : 0u, lb, elen, ent, ecodes, epk, bflag, eqg, pe, par_e, cmin_e, elow, rrec);
+        idb_entry *ent = nullptr;
+        uint32_t *ecodes = nullptr, *epk = nullptr, *eqg = nullptr;
+        if (mx) {
+            const uint32_t planes = qgram ? 2u : 5u, words = W <= 3 ? W : (W <= 5 ? 5u : 8u);
+            const size_t vs = qgram ? 2 * words + 1 : 8;
+            idb_mx_fill_args f{skey, srow, E, seq, vw, jw, gj, gvj, cmap, planes, K, words, (int32_t)tc[0], lb, elen,
+                               buf<uint32_t>(c, S_META, E), buf<uint32_t>(c, S_FEAT, (size_t)E * (qgram ? 24 : 8)),
+                               buf<uint32_t>(c, S_VREC, (size_t)E * vs), bflag, buf<uint32_t>(c, S_INV, E), buf<int32_t>(c, S_CNTE, E), par_e, cmin_e, elow, rrec};
+            check(c, idb_launch_mx_fill(f, s), "entry launch");
+            a.e_feat = f.feat;
+            a.e_meta = f.meta;
+            a.e_vrec = f.vrec;
+            a.cnt_e = f.cnt_e;
+            a.e_row = srow;
+            a.n_entries = E;
+            mr.uniq = uniq;
+            mr.num = num;
+            mr.eoff = eoff;
+            mr.inv = f.inv;
+            mr.cnt_e = f.cnt_e;
+            mr.copies = copies;
+            mr.n = N;
+            mr.min_pts = (int32_t)p->min_pts;
+            mr.cnt = cnt;
+            mr.pe = pe;
+            mr.ecore = buf<uint8_t>(c, S_ECORE, E);
+            mr.par_e = par_e;
+            mr.n_cores = small + IDB_SMALL_CORES;
+            ua.ecore = mr.ecore;
+            ua.erow = srow;
+            a.mx_planes = planes;
+            a.mx_words = words;
+        } else {
+            ent = buf<idb_entry>(c, S_ENT, E);
+            ecodes = ham ? nullptr : buf<uint32_t>(c, S_ECODES, (size_t)E * (S / 4));
+            epk = ham ? buf<uint32_t>(c, S_EPK, (size_t)E * HW) : nullptr;
+            // Levenshtein codes are padded with a sentinel letter K whose Peq row
+            // stays zero, so a Peq read for a letter past a row's end stays in
+            // range (with all 256 byte values present code 0 is used; only the
+            // one-word count kernel reads letters past a row's end, and it runs
+            // for alphabets of at most 31 letters)
+            const uint32_t pad = (!ham && K < 256) ? K : 0u;
+            eqg = qgram ? buf<uint32_t>(c, S_EQG, (size_t)E * IDB_QGRAM_WORDS) : nullptr;
+            hipLaunchKernelGGL(k_fill_entries, dim3(blocks_for(E)), dim3(256), 0, s, skey, srow, E, seq, off, copies, vb,
+                               vw, jb, jw, single, gj, gvj, cmap, pad, S, HW, bits, tlut_c, tlut_f, filt ? 1u : 0u,
+                               ham ? 1u : 0u, lb, elen, ent, ecodes, epk, bflag, learned ? nullptr : eqg,
+                               learned ? eqg : nullptr, pe, par_e, cmin_e, elow, rrec);
+        }
         ua.pe = pe;
         ua.par_e = par_e;
         ua.cmin_e = cmin_e;
@@ -1516,8 +1591,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                                              " are not supported (split the largest V/J bucket)");
         T = (uint32_t)T64;
         idb_tile *tiles = buf<idb_tile>(c, S_TILES, std::max<uint32_t>(T, 1u));
-        hipLaunchKernelGGL(k_emit_tiles, dim3(blocks_for(bqt[1])), dim3(256), 0, s, qboff, num + 1, bstart, E, elen, hilen,
-                           banded ? 1u : 0u, qsplit, skey, lb, gvj, toff, tiles);
         a.tiles = tiles;
         a.n_tiles = T;
         a.ent = ent;
@@ -1569,6 +1642,15 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         a.edges = buf<uint2>(c, S_EDGES, edge_cap);
         a.chunk_fill = buf<uint32_t>(c, S_FILL, a.max_chunks);
         a.n_chunks = small + 12;
+        // Waves own their first chunk (learned runs may repeat their pass and
+        // start from an empty list); at most a quarter of the list is given
+        // out this way, so that partly filled chunks do not make it overflow.
+        a.chunk_base = learned ? 0u
+                               : std::min<uint32_t>((uint32_t)std::min<uint64_t>(4ull * T, 32768u),
+                                                    a.max_chunks / 4);
+        hipLaunchKernelGGL(k_emit_tiles, dim3(blocks_for(std::max<uint64_t>(bqt[1], a.chunk_base))), dim3(256), 0, s,
+                           qboff, num + 1, bstart, E, elen, hilen, banded ? 1u : 0u, qsplit, skey, lb, gvj, toff, tiles,
+                           a.n_chunks, a.chunk_fill, a.chunk_base);
         if (learned) {
             // embeddings of every row, then proposals verified by Myers
             uint16_t *zb = buf<uint16_t>(c, S_ZB, (size_t)N * 64);
@@ -1614,7 +1696,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         check(c, hipMemcpyAsync(c->xfer + 3 * ob, unq_o, sizeof(uint32_t) * N, hipMemcpyDeviceToHost, c->side),
               "output copy");
     }
-    if (E > 0 && T > 0 && (p->flags & IDB_FLAG_AUTOTUNE)) autotune(c, a, N, W, ham, learned, small, work);
+    if (E > 0 && T > 0 && (p->flags & IDB_FLAG_AUTOTUNE)) autotune(c, a, N, E, W, ham, learned, small, work);
     // Learned runs stay uncaptured: when their pair list overflows, the host
     // grows it and runs the learned pass again (below).
     const bool graph = (p->flags & IDB_FLAG_GRAPH) && !(x && x->pairs_out) && !learned;
@@ -1630,8 +1712,13 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             else check(c, ham ? idb_launch_count_hamming(a, s) : idb_launch_count_myers(a, W, s), "count kernel launch");
             if (!g) check(c, hipEventRecord(c->kev[1], s), "event record");
         }
-        hipLaunchKernelGGL(k_core_flags, dim3(blocks_for(N)), dim3(256), 0, s, cnt, N, (int32_t)p->min_pts, core, pe,
-                           small);
+        if (mr.inv) {
+            mr.core = core;
+            check(c, idb_launch_mx_rows(mr, s), "row launch");
+        } else {
+            hipLaunchKernelGGL(k_core_flags, dim3(blocks_for(N)), dim3(256), 0, s, cnt, N, (int32_t)p->min_pts, core,
+                               pe, small);
+        }
         if (!g && early_out) {
             check(c, hipEventRecord(c->side_ev[1], s), "event record");
             check(c, hipStreamWaitEvent(c->side, c->side_ev[1], 0), "side wait");
@@ -1702,11 +1789,20 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                               "pairs copy");
                         check(c, hipStreamSynchronize(s), "pairs sync");
                     }
+                    // a list of entries: their rows
+                    std::vector<uint32_t> er;
+                    if (ua.ecore) {
+                        er.resize(E);
+                        check(c, hipMemcpyAsync(er.data(), ua.erow, sizeof(uint32_t) * E, hipMemcpyDeviceToHost, s),
+                              "pairs copy");
+                        check(c, hipStreamSynchronize(s), "pairs sync");
+                    }
                     uint64_t k = 0;
                     for (uint32_t ch = 0; ch < n_chunks; ++ch)
                         for (uint32_t i = 0; i < fill[ch]; ++i, ++k) {
                             if (k >= x->pairs_cap) continue;
-                            const uint2 e = ed[((size_t)ch << a.chunk_log2) + i];
+                            uint2 e = ed[((size_t)ch << a.chunk_log2) + i];
+                            if (ua.ecore) e = make_uint2(er[e.x], er[e.y]);
                             x->pairs_out[2 * k] = std::min(e.x, e.y);
                             x->pairs_out[2 * k + 1] = std::max(e.x, e.y);
                         }

@@ -90,6 +90,7 @@ hipError_t idb_sort_small(uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1
 #define IDB_MAX_LEN 65535u
 #define IDB_ENC_P 32              // letters per row the encoder reads
 #define IDB_QGRAM_WORDS 16        // 3-gram profile: 64 byte counts per row
+#define IDB_QMASK_WORDS 8         // 3-gram level masks (learned runs): 3 x 64 bits, padded
 
 struct idb_tile {
     uint32_t q0;                  // first query entry
@@ -135,16 +136,26 @@ struct idb_pair_args {
     uint32_t *par;                // fuse pass: union-find parents
     uint32_t *bmin;               // fuse pass: border claims
     unsigned long long *work;     // [0] gated pairs, [1] neighbour pairs, [2] fuse pairs, [3] gated letters,
-                                  // [4] edges, [5] Myers pairs, [6] Myers letters
+                                  // [5] Myers pairs, [6] Myers letters
     uint2 *edges;                 // count pass: neighbour pairs (x, y) in chunks, may be null
     uint32_t *chunk_fill;         // pairs written into each chunk
     uint32_t *n_chunks;           // chunks handed out (counts past max_chunks on overflow)
     uint32_t max_chunks;          // capacity in chunks
+    uint32_t chunk_base;          // chunks 0 .. chunk_base - 1 belong to the waves of that number (counted in n_chunks)
     uint32_t chunk_log2;          // pairs per chunk = 1 << chunk_log2 (>= IDB_TILE)
     uint32_t fuse_if_overflow;    // fuse pass: run only when the pair list overflowed
     int32_t t_const;              // >= 0: every pair's count-pass threshold (absolute mode); -1 otherwise
     const uint16_t *zb;           // learned filter: bfloat16 embedding (64) per row
     float min_sim;                // learned filter: proposal threshold on z_x . z_y
+    // matrix-core passes (idb_mx.hip), null otherwise: 4-bit features, length |
+    // lower-gene flag << 16, records (protein rows: 5 planes, row, copies,
+    // length per entry; nucleotide rows: plane word w of entry e at
+    // w * n_entries + e, then the copies), rows
+    const uint32_t *e_feat, *e_meta, *e_vrec, *e_row;
+    uint32_t n_entries;
+    uint32_t mx_planes, mx_words; // planes per letter (5 or 2), words per plane
+    int32_t *cnt_e;               // their count output, per entry; their pair list holds entries
+    uint32_t sub_log2;            // tiles are taken in 2^sub_log2 parts of their queries
     // launch shape (0 = default): waves per block, grid = resident blocks x
     // grid_mul, and plain block order instead of the XCD-grouped one
     uint32_t tune_wpb, tune_grid_mul, no_xcd_order;
@@ -192,6 +203,26 @@ __device__ __forceinline__ uint32_t byte_of(const uint4 &v, uint32_t b)
     return (w >> (8 * (b & 3))) & 0xFFu;
 }
 
+// Word k of a gene bitset restricted to the genes below gene g.
+__device__ __forceinline__ uint32_t below_gene(uint32_t w, uint32_t k, uint32_t g)
+{
+    if (k * 32 >= g) return 0u;
+    return (k * 32 + 32 > g) ? (w & ((1u << (g - k * 32)) - 1u)) : w;
+}
+
+// Counts one more 3-gram (0..63) in the level masks of a nucleotide row:
+// g[2k], g[2k+1] = the 3-grams seen at least k + 1 times, k = 0, 1, 2.
+__device__ __forceinline__ void idb_qmask_add(uint32_t (&g)[6], uint32_t gram)
+{
+    const uint32_t bit = 1u << (gram & 31u), lo = gram < 32u ? bit : 0u, hi = gram < 32u ? 0u : bit;
+    g[4] |= g[2] & lo;
+    g[5] |= g[3] & hi;
+    g[2] |= g[0] & lo;
+    g[3] |= g[1] & hi;
+    g[0] |= lo;
+    g[1] |= hi;
+}
+
 // LDS bytes one wave of the Myers kernels needs: Peq columns, the edge
 // staging slots, the Myers queue (2 * IDB_TILE 16-bit entries), the per-tile
 // count accumulators of queries and targets, and the tile's query records.
@@ -213,6 +244,49 @@ hipError_t idb_launch_fuse_hamming(const idb_pair_args &a, hipStream_t s);
 hipError_t idb_launch_count_learned(const idb_pair_args &a, hipStream_t s);
 hipError_t idb_launch_pair_distances(const uint8_t *seq, const uint64_t *off, const uint32_t *len, const uint2 *pairs,
                                      unsigned long long n, uint32_t W, uint32_t ham, uint32_t *dist, hipStream_t s);
+// The matrix-core count and fuse passes (idb_mx.hip) and their entry arrays.
+#define IDB_MX_MAX_LETTERS 30u    // alphabet of the one-word (protein) form
+struct idb_mx_fill_args {
+    const uint64_t *ekey;
+    const uint32_t *erow;
+    uint32_t E;
+    const uint8_t *seq;
+    uint32_t vw, jw, gj, gvj;
+    const uint8_t *cmap;
+    uint32_t planes, K, W;
+    int32_t t;
+    uint32_t lb;
+    uint16_t *elen;
+    uint32_t *meta, *feat, *vrec;
+    uint8_t *bflag;
+    uint32_t *inv;                // entry of each (row, gene pair), rows in order (first index: row record word 3)
+    int32_t *cnt_e;
+    uint32_t *par_e, *cmin_e;
+    uint4 *elow;
+    const uint4 *rrec;
+};
+struct idb_mx_rows_args {
+    const uint32_t *uniq, *num;
+    const uint64_t *eoff;
+    const uint32_t *inv;
+    const int32_t *cnt_e;
+    const uint32_t *copies;
+    uint32_t n;
+    int32_t min_pts;
+    int32_t *cnt, *core;
+    uint32_t *pe;
+    uint8_t *ecore;
+    uint32_t *par_e, *n_cores;
+};
+hipError_t idb_launch_mx_fill(const idb_mx_fill_args &f, hipStream_t s);
+hipError_t idb_launch_mx_rows(const idb_mx_rows_args &r, hipStream_t s);
+hipError_t idb_launch_mx_count(const idb_pair_args &a, hipStream_t s);
+hipError_t idb_launch_mx_fuse(const idb_pair_args &a, hipStream_t s);
+// Launch helpers (idb_pairs.hip).
+uint32_t idb_resident_blocks(const void *kernel, uint32_t block, size_t shm);
+uint32_t idb_grid_for(uint32_t n_tiles, uint32_t wpb, uint32_t resident, uint32_t mul);
+uint32_t idb_count_grid(const idb_pair_args &a, uint32_t n_tiles, uint32_t wpb, uint32_t resident);
+uint32_t idb_pick_wpb(const idb_pair_args &a, uint32_t most);
 hipError_t idb_launch_gene_bitsets(const uint8_t *calls, const uint64_t *off, const uint32_t *len, uint32_t n,
                                    const idb_gene_hdr *hdr, const uint32_t *gw, uint32_t n_words, uint32_t n_genes,
                                    int32_t *out, uint32_t width, hipStream_t s);
@@ -229,6 +303,8 @@ struct idb_union_args {
     uint32_t *par;                // per row: set to the component minimum for core rows
     uint32_t *bmin;               // per row: border claims
     const uint32_t *rep;          // per row: representative (for the depth histogram)
+    const uint8_t *ecore;         // per entry: its row's core flag, when the pair list holds entries (else null)
+    const uint32_t *erow;         // per entry: its row
     uint32_t *depth_hist;         // 51 bins of union-find depths, or null (no histogram)
 };
 hipError_t idb_launch_union_edges(const idb_pair_args &a, const idb_union_args &u, hipStream_t s);

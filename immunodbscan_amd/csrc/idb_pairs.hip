@@ -35,236 +35,10 @@
 #include <type_traits>
 
 #include "idb_internal.h"
+#include "idb_pairs_dev.h"
 #include "pairdist.h"
 
 namespace {
-
-__device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
-
-__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-__device__ __forceinline__ uint32_t rl(uint32_t v, uint32_t lane) { return __builtin_amdgcn_readlane(v, lane); }
-
-__device__ __forceinline__ uint32_t ld_agent(const uint32_t *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ uint32_t uf_find(uint32_t *par, uint32_t x)
-{
-    uint32_t p = ld_agent(par + x);
-    while (p != x) {
-        const uint32_t gp = ld_agent(par + p);
-        if (gp != p) {
-            // path halving: gp is an ancestor of x, so the shortcut is safe
-            __hip_atomic_store(par + x, gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        x = p;
-        p = gp;
-    }
-    return x;
-}
-
-// Link the larger root under the smaller one.  After a failed exchange the
-// larger of the two roots strictly decreases, so the loop ends.
-__device__ void uf_union(uint32_t *par, uint32_t a, uint32_t b)
-{
-    a = uf_find(par, a);
-    b = uf_find(par, b);
-    while (a != b) {
-        if (a < b) {
-            const uint32_t t = a;
-            a = b;
-            b = t;
-        }
-        uint32_t expected = a;
-        if (__hip_atomic_compare_exchange_strong(par + a, &expected, b, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT))
-            return;
-        a = uf_find(par, expected);
-        b = uf_find(par, b);
-    }
-}
-
-__device__ __forceinline__ int lowest_common(const int32_t *a, const int32_t *b, uint32_t w)
-{
-    for (uint32_t k = 0; k < w; ++k) {
-        const uint32_t m = (uint32_t)(a[k] & b[k]);
-        if (m) return (int)(k * 32 + __builtin_ctz(m));
-    }
-    return -1;
-}
-
-// Exact canonical-bucket test from the bitsets (single-bucket mode: the V/J
-// gate of cuda/BitsetVector.inl:214-237).
-__device__ bool pair_in_bucket(const idb_pair_args &a, uint32_t x, uint32_t y, uint32_t bucket)
-{
-    const int32_t *vx = a.vbits + (size_t)x * a.vw, *vy = a.vbits + (size_t)y * a.vw;
-    const int32_t *jx = a.jbits + (size_t)x * a.jw, *jy = a.jbits + (size_t)y * a.jw;
-    const int lv = lowest_common(vx, vy, a.vw), lj = lowest_common(jx, jy, a.jw);
-    if (a.single_bucket) return lv >= 0 && lj >= 0;
-    return lv == (int)(bucket / a.gj) && lj == (int)(bucket % a.gj);
-}
-
-// The signature holds the residues mod 16 of the genes in question (canonical
-// mode: genes below the bucket's; single-bucket mode: all genes).  Canonical
-// mode: no common V residue and no common J residue -> no common lower gene ->
-// canonical.  Single-bucket mode: no common V (or J) residue -> no common gene
-// -> the gate fails.  Otherwise the bitsets decide.
-__device__ __forceinline__ bool gate_pair(const idb_pair_args &a, bool chk_x, bool chk_y, uint32_t sx, uint32_t sy,
-                                          uint32_t x, uint32_t y, uint32_t bucket)
-{
-    if (!(a.single_bucket || (chk_x && chk_y))) return true;
-    const uint32_t c = sx & sy;
-    if (a.single_bucket) {
-        if ((c & 0xFFFFu) == 0u || (c >> 16) == 0u) return false;
-    } else if (c == 0u) {
-        return true;
-    }
-    return pair_in_bucket(a, x, y, bucket);
-}
-
-// Neighbour pairs are staged per wave in LDS (IDB_TILE entries) and appended
-// to a chunk of the edge list that the wave owns; a new chunk costs one
-// atomic on the chunk counter, so that counter sees one atomic per chunk
-// instead of one per hit or per stage.  Past the capacity the counter keeps
-// growing and the pairs are dropped, so the overflow is visible and the fuse
-// pass over the tiles runs instead.
-struct EdgeStage {
-    uint2 *buf;       // this wave's IDB_TILE staging slots
-    uint32_t n;       // staged pairs (wave-uniform)
-    uint32_t chunk;   // the wave's current chunk, IDB_NONE before the first
-    uint32_t fill;    // pairs written into it
-    uint32_t total;   // pairs this wave produced
-};
-
-// This block's copy of the run's statistics counters.
-__device__ __forceinline__ unsigned long long *work_copy(const idb_pair_args &a)
-{
-    return a.work + IDB_WORK_U64 * (blockIdx.x & (IDB_WORK_COPIES - 1u));
-}
-
-__device__ __forceinline__ void close_chunk(const idb_pair_args &a, const EdgeStage &st, uint32_t lane)
-{
-    if (st.chunk != IDB_NONE && st.chunk < a.max_chunks && lane == 0) a.chunk_fill[st.chunk] = st.fill;
-}
-
-__device__ __forceinline__ void flush_edges(const idb_pair_args &a, EdgeStage &st, uint32_t lane)
-{
-    if (st.n == 0) return;
-    if (st.chunk == IDB_NONE || st.fill + st.n > (1u << a.chunk_log2)) {
-        close_chunk(a, st, lane);
-        uint32_t c = 0;
-        if (lane == 0) c = atomicAdd(a.n_chunks, 1u);
-        st.chunk = __shfl(c, 0, 64);
-        st.fill = 0;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    if (st.chunk < a.max_chunks && lane < st.n)
-        a.edges[((size_t)st.chunk << a.chunk_log2) + st.fill + lane] = st.buf[lane];
-    st.fill += st.n;
-    st.total += st.n;
-    st.n = 0;
-}
-
-__device__ __forceinline__ void stage_edges(const idb_pair_args &a, EdgeStage &st, bool keep, uint32_t x, uint32_t y,
-                                            uint32_t lane)
-{
-    const unsigned long long km = __ballot(keep);
-    if (!km || !a.edges) return;
-    const uint32_t cnt = (uint32_t)__popcll(km);
-    if (st.n + cnt > IDB_TILE) flush_edges(a, st, lane);
-    if (keep) {
-        const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)km, 0u));
-        st.buf[st.n + below] = make_uint2(x, y);
-    }
-    st.n += cnt;
-}
-
-// End of a count-pass wave: last stage, last chunk's fill, pair total.
-__device__ __forceinline__ void finish_edges(const idb_pair_args &a, EdgeStage &st, uint32_t lane)
-{
-    if (!a.edges) return;
-    flush_edges(a, st, lane);
-    close_chunk(a, st, lane);
-    if (lane == 0 && st.total && a.work) atomicAdd(work_copy(a) + 4, (unsigned long long)st.total);
-}
-
-// Fuse pass launched behind the union step without a host decision: it runs
-// only when the pair list overflowed.
-__device__ __forceinline__ bool fuse_skipped(const idb_pair_args &a)
-{
-    return a.fuse_if_overflow && *(volatile const uint32_t *)a.n_chunks <= a.max_chunks;
-}
-
-// The grid holds only as many waves as can be resident at once (no partly
-// empty second round of waves trails the launch); wave w takes tiles w,
-// w + waves, w + 2 waves, ...  A shared tile counter balances better in
-// principle, but its device-scope atomics wait behind the pass's other
-// atomics: measured on the 200k-row workload, claiming tiles (one counter per
-// XCD, half of the tiles static) made the count pass slower, not faster.
-__device__ __forceinline__ uint32_t next_tile(uint32_t ti, uint32_t total_waves) { return ti + total_waves; }
-
-// The Myers count pass deals the rounds back and forth: wave w takes
-// position w of even rounds and position waves - 1 - w of odd ones, so a wave
-// that drew from a heavy stretch of one round draws from the other end of
-// the next (3% off the 200k-row count pass).  n_tiles past the end.
-__device__ __forceinline__ uint32_t step_tile(uint32_t ti, uint32_t total_waves, uint32_t n_tiles)
-{
-    if (ti >= n_tiles) return n_tiles;
-    const uint32_t r = ti / total_waves, pos = ti % total_waves;
-    const uint64_t nx = (uint64_t)(r + 1) * total_waves + (total_waves - 1 - pos);
-    return nx < n_tiles ? (uint32_t)nx : n_tiles;
-}
-
-// Blocks are dealt to the 8 XCDs round-robin; renumber them so that each XCD
-// starts on a contiguous run of tiles (neighbouring tiles share query blocks).
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
-{
-    const uint32_t per = nb / 8, rem = nb % 8, x = b % 8, k = b / 8;
-    return x < rem ? x * (per + 1) + k : rem * (per + 1) + (x - rem) * per + k;
-}
-
-__device__ __forceinline__ int32_t t_of(uint32_t t2, bool fuse)
-{
-    return fuse ? (int32_t)(int16_t)(t2 >> 16) : (int32_t)(int16_t)(t2 & 0xFFFFu);
-}
-
-__device__ __forceinline__ idb_entry load_entry(const idb_entry *e)
-{
-    const uint4 *p = (const uint4 *)e;
-    const uint4 a = p[0], b = p[1];
-    idb_entry r;
-    r.row = a.x;
-    r.cp = a.y;
-    r.len_chk = a.z;
-    r.t2 = a.w;
-    r.len = b.x;
-    r.pres1 = b.y;
-    r.pres2 = b.z;
-    r.sig = b.w;
-    return r;
-}
-
-// A tile record: the list is read-only during a pass and the index is
-// wave-uniform, so this is a scalar load (waited on by lgkmcnt, which keeps
-// it clear of the vector loads in flight).
-__device__ __forceinline__ idb_tile tile_rec(const idb_pair_args &a, uint32_t ti)
-{
-    typedef const __attribute__((address_space(4))) uint32_t *const_words;
-    const const_words w = (const_words)a.tiles + 4 * (size_t)ti;
-    idb_tile t;
-    t.q0 = w[0];
-    t.t0 = w[1];
-    t.bucket = w[2];
-    t.shape = w[3];
-    return t;
-}
 
 // What a Myers tile needs from global memory, loaded one tile ahead: the
 // record, this lane's query and target entries and, for one-word rows
@@ -702,7 +476,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FILT == 2 &
     constexpr uint32_t QG_WORDS = FILT == 2 ? IDB_TILE * IDB_QGRAM_WORDS : 0u;
     uint32_t *peq = lds + (size_t)wib * (idb_myers_lds_per_wave(K, W) / sizeof(uint32_t) + QG_WORDS);
     uint32_t *qg = peq + idb_myers_lds_per_wave(K, W) / sizeof(uint32_t);
-    EdgeStage est{(uint2 *)(peq + K * W * 64), 0u, IDB_NONE, 0u, 0u};
     uint16_t *queue = (uint16_t *)(peq + K * W * 64 + 2 * IDB_TILE);
     int32_t *qacc = (int32_t *)(peq + K * W * 64 + 3 * IDB_TILE);
     int32_t *tacc = qacc + IDB_TILE;
@@ -712,6 +485,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FILT == 2 &
     // consecutive tiles (often of one query block, with similar work) go to
     // different blocks and so to different CUs, not to the waves of one block
     const uint32_t wave0 = (a.no_xcd_order ? blockIdx.x : xcd_block(blockIdx.x, gridDim.x)) + wib * gridDim.x;
+    EdgeStage est = edge_stage(a, (uint2 *)(peq + K * W * 64), FUSE ? IDB_NONE : wave0);
     unsigned long long gated = 0, hits = 0, gletters = 0, mpairs = 0, mletters = 0;
     unsigned long long glane = 0, gllane = 0;  // per-lane gated pairs and target letters (constant threshold)
 
@@ -1214,7 +988,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t K = a.K;
     uint32_t *peq = lds + (size_t)wib * (idb_count1_lds_per_wave(K) / sizeof(uint32_t));
-    EdgeStage est{(uint2 *)(peq + K * 64), 0u, IDB_NONE, 0u, 0u};
     uint16_t *queue = (uint16_t *)(peq + K * 64 + 2 * IDB_TILE);
     int32_t *qacc = (int32_t *)(peq + K * 64 + 3 * IDB_TILE);
     int32_t *tacc = qacc + IDB_TILE;
@@ -1222,6 +995,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     uint4 *gqc = gq + IDB_TILE;  // query codes, two uint4 per query
     const uint32_t total_waves = gridDim.x * wpb;
     const uint32_t wave0 = (a.no_xcd_order ? blockIdx.x : xcd_block(blockIdx.x, gridDim.x)) + wib * gridDim.x;
+    EdgeStage est = edge_stage(a, (uint2 *)(peq + K * 64), wave0);
     const int32_t t_const = a.t_const;
     const bool exact_low = a.e_low != nullptr;
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
@@ -1550,10 +1324,10 @@ __global__ __launch_bounds__(256) void k_pairs_learned(idb_pair_args a, uint32_t
     const uint32_t K = a.K;
     // per wave: Peq, edge stage, queue, count accumulators, query records,
     // then (3-gram bound) the tile's query and target profiles
-    const uint32_t QGW = a.qgram_filter ? 2u * IDB_TILE * IDB_QGRAM_WORDS : 0u;
+    const uint32_t QGW = a.qgram_filter ? 2u * IDB_TILE * IDB_QMASK_WORDS : 0u;
     uint32_t *peq = lds + (size_t)wib * (idb_myers_lds_per_wave(K, W) / sizeof(uint32_t) + QGW);
     uint32_t *qgp = peq + idb_myers_lds_per_wave(K, W) / sizeof(uint32_t);
-    uint32_t *tgp = qgp + IDB_TILE * IDB_QGRAM_WORDS;
+    uint32_t *tgp = qgp + IDB_TILE * IDB_QMASK_WORDS;
     EdgeStage est{(uint2 *)(peq + K * W * 64), 0u, IDB_NONE, 0u, 0u};
     uint16_t *queue = (uint16_t *)(peq + K * W * 64 + 2 * IDB_TILE);
     int32_t *qacc = (int32_t *)(peq + K * W * 64 + 3 * IDB_TILE);
@@ -1577,12 +1351,12 @@ __global__ __launch_bounds__(256) void k_pairs_learned(idb_pair_args a, uint32_t
         tacc[lane] = 0;
         if (a.qgram_filter) {
             // profiles of the tile's queries and targets (64 bytes each)
-            const uint4 *qs = (const uint4 *)(a.e_qg + (size_t)(tile.q0 + (lane < qn ? lane : 0u)) * IDB_QGRAM_WORDS);
-            const uint4 *ts = (const uint4 *)(a.e_qg + (size_t)p * IDB_QGRAM_WORDS);
+            const uint4 *qs = (const uint4 *)(a.e_qg + (size_t)(tile.q0 + (lane < qn ? lane : 0u)) * IDB_QMASK_WORDS);
+            const uint4 *ts = (const uint4 *)(a.e_qg + (size_t)p * IDB_QMASK_WORDS);
 #pragma unroll
-            for (int k = 0; k < (int)IDB_QGRAM_WORDS / 4; ++k) {
-                ((uint4 *)(qgp + lane * IDB_QGRAM_WORDS))[k] = qs[k];
-                ((uint4 *)(tgp + lane * IDB_QGRAM_WORDS))[k] = ts[k];
+            for (int k = 0; k < (int)IDB_QMASK_WORDS / 4; ++k) {
+                ((uint4 *)(qgp + lane * IDB_QMASK_WORDS))[k] = qs[k];
+                ((uint4 *)(tgp + lane * IDB_QMASK_WORDS))[k] = ts[k];
             }
         }
         // rows of the 32-row halves this lane feeds into the MFMAs
@@ -1621,7 +1395,7 @@ __global__ __launch_bounds__(256) void k_pairs_learned(idb_pair_args a, uint32_t
                         cand |= 1ull << ((2 * i + j) * 16 + r);
                 }
         // target fields of the two target columns this lane holds
-        uint32_t tm[2], tt2[2], tsig[2], ty[2], tp1[2];
+        uint32_t tm[2], tt2[2], tsig[2], ty[2], tp1[2], tp2[2];
         bool tchk[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -1633,6 +1407,7 @@ __global__ __launch_bounds__(256) void k_pairs_learned(idb_pair_args a, uint32_t
             tsig[j] = (uint32_t)__shfl((int)te.sig, src, 64);
             ty[j] = (uint32_t)__shfl((int)te.row, src, 64);
             tp1[j] = (uint32_t)__shfl((int)te.pres1, src, 64);
+            tp2[j] = (uint32_t)__shfl((int)te.pres2, src, 64);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         bool peq_ready = false;
@@ -1676,24 +1451,26 @@ __global__ __launch_bounds__(256) void k_pairs_learned(idb_pair_args a, uint32_t
                                           j ? tsig[1] : tsig[0], q.row, j ? ty[1] : ty[0], tile.bucket);
                 proposed = ok;
                 if (ok && a.band_filter) {
-                    const uint32_t p1 = j ? tp1[1] : tp1[0];
-                    const uint32_t lbx = __builtin_popcount(q.pres1 & ~p1);
-                    const uint32_t lby = __builtin_popcount(p1 & ~q.pres1);
+                    // letters present at least once and at least twice, as
+                    // the fixed-threshold exact pass counts them
+                    const uint32_t p1 = j ? tp1[1] : tp1[0], p2 = j ? tp2[1] : tp2[0];
+                    const uint32_t lbx = __builtin_popcount(q.pres1 & ~p1) + __builtin_popcount(q.pres2 & ~p2);
+                    const uint32_t lby = __builtin_popcount(p1 & ~q.pres1) + __builtin_popcount(p2 & ~q.pres2);
                     ok = (int32_t)(lbx > lby ? lbx : lby) <= t;
                 } else if (ok && a.qgram_filter) {
-                    // the exact 3-gram bound, as the exact pass applies it
-                    const uint4 *qv = (const uint4 *)(qgp + qi * IDB_QGRAM_WORDS);
-                    const uint4 *tv = (const uint4 *)(tgp + tl * IDB_QGRAM_WORDS);
-                    uint32_t l1 = 0;
+                    // the 3-gram bound over three levels, likewise
+                    const uint4 *qv = (const uint4 *)(qgp + qi * IDB_QMASK_WORDS);
+                    const uint4 *tv = (const uint4 *)(tgp + tl * IDB_QMASK_WORDS);
+                    uint32_t nx = 0, ny = 0;
 #pragma unroll
-                    for (int k = 0; k < (int)IDB_QGRAM_WORDS / 4; ++k) {
+                    for (int k = 0; k < 2; ++k) {
                         const uint4 x4 = qv[k], y4 = tv[k];
-                        l1 = __builtin_amdgcn_sad_u8(x4.x, y4.x, l1);
-                        l1 = __builtin_amdgcn_sad_u8(x4.y, y4.y, l1);
-                        l1 = __builtin_amdgcn_sad_u8(x4.z, y4.z, l1);
-                        l1 = __builtin_amdgcn_sad_u8(x4.w, y4.w, l1);
+                        nx += __builtin_popcount(x4.x & ~y4.x) + __builtin_popcount(x4.y & ~y4.y) +
+                              __builtin_popcount(x4.z & ~y4.z) + __builtin_popcount(x4.w & ~y4.w);
+                        ny += __builtin_popcount(y4.x & ~x4.x) + __builtin_popcount(y4.y & ~x4.y) +
+                              __builtin_popcount(y4.z & ~x4.z) + __builtin_popcount(y4.w & ~x4.w);
                     }
-                    ok = (int32_t)l1 <= 6 * t;
+                    ok = (int32_t)max(nx, ny) <= 3 * t;
                 }
             }
             gated += __popcll(__ballot(proposed));
@@ -1929,7 +1706,10 @@ __global__ __launch_bounds__(256) void k_count_ham(idb_pair_args a, uint32_t wpb
     __shared__ int32_t qacc_s[4][IDB_TILE];
     __shared__ uint2 qinfo_s[4][IDB_TILE];              // query row, copies
     __shared__ uint4 qw_s[4][IDB_TILE * QS / 4];        // query words, QS per query
-    EdgeStage est{stage[wib], 0u, IDB_NONE, 0u, 0u};
+    __shared__ unsigned long long stat_sum[3];
+    if (threadIdx.x < 3) stat_sum[threadIdx.x] = 0;
+    __syncthreads();
+    EdgeStage est = edge_stage(a, stage[wib], wave0);
     int32_t *qacc = qacc_s[wib];
     uint2 *qinfo = qinfo_s[wib];
     uint4 *qw = qw_s[wib];
@@ -2058,11 +1838,7 @@ __global__ __launch_bounds__(256) void k_count_ham(idb_pair_args a, uint32_t wpb
     }
     finish_edges(a, est, lane);
     const unsigned long long gated = wave_sum_u64(glane), gletters = wave_sum_u64(gllane), hits = wave_sum_u64(hlane);
-    if (lane == 0 && a.work) {
-        atomicAdd(work_copy(a) + 0, gated);
-        atomicAdd(work_copy(a) + 1, hits);
-        atomicAdd(work_copy(a) + 3, gletters);
-    }
+    add_stats<3>(a, stat_sum, {0u, 1u, 3u}, {gated, hits, gletters}, lane);
 }
 
 // Cluster growth over the recorded pairs, in entry space.  The union-find
@@ -2141,16 +1917,32 @@ __device__ __forceinline__ bool pairs_overflowed(const uint32_t *n_chunks, uint3
 
 constexpr uint32_t PE_CORE = 0x80000000u;
 
-__global__ void k_union_to_entries(uint2 *edges, const uint32_t *fill, const uint32_t *n_chunks, uint32_t max_chunks,
-                                   uint32_t chunk_log2, const uint32_t *pe, uint32_t *par_e, uint32_t *bmin)
+// The pair list, one piece of at most 256 pairs of a chunk per wave and round;
+// f(pair index, live) for 64 pairs at a time with the whole wave active.
+// Chunks are filled to very different degrees (a wave's own chunk may hold a
+// few pairs of 1,024), so the waves walk what a piece holds and not its slots.
+template <class F>
+__device__ __forceinline__ void for_pairs(const uint32_t *fill, const uint32_t *n_chunks, uint32_t max_chunks,
+                                          uint32_t chunk_log2, F &&f)
 {
     const uint32_t nc = *n_chunks;
     if (nc > max_chunks) return;
-    const unsigned long long n = (unsigned long long)nc << chunk_log2;
-    const uint32_t cmask = (1u << chunk_log2) - 1u;
-    for (unsigned long long e = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; e < n;
-         e += (unsigned long long)gridDim.x * blockDim.x) {
-        if (((uint32_t)e & cmask) >= fill[e >> chunk_log2]) continue;
+    const uint32_t plog = chunk_log2 > 8u ? 8u : chunk_log2;
+    const uint64_t pieces = (uint64_t)nc << (chunk_log2 - plog);
+    const uint32_t lane = lane_id(), wpb = blockDim.x >> 6;
+    for (uint64_t u = blockIdx.x * (uint64_t)wpb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); u < pieces;
+         u += (uint64_t)gridDim.x * wpb) {
+        const uint64_t e0 = u << plog;
+        const uint32_t at = (uint32_t)e0 & ((1u << chunk_log2) - 1u), end = fill[e0 >> chunk_log2];
+        for (uint32_t k = 0; k < (1u << plog) && at + k < end; k += 64u) f(e0 + k + lane, at + k + lane < end);
+    }
+}
+
+__global__ void k_union_to_entries(uint2 *edges, const uint32_t *fill, const uint32_t *n_chunks, uint32_t max_chunks,
+                                   uint32_t chunk_log2, const uint32_t *pe, uint32_t *par_e, uint32_t *bmin)
+{
+    for_pairs(fill, n_chunks, max_chunks, chunk_log2, [&](uint64_t e, bool live) {
+        if (!live) return;
         const uint2 p = edges[e];
         const uint32_t px = pe[p.x], py = pe[p.y];
         const bool cx = px != IDB_NONE && (px & PE_CORE) != 0u, cy = py != IDB_NONE && (py & PE_CORE) != 0u;
@@ -2165,27 +1957,44 @@ __global__ void k_union_to_entries(uint2 *edges, const uint32_t *fill, const uin
             atomicMin(bmin + p.x, p.y);
         }
         edges[e] = q;
-    }
+    });
+}
+
+// The same for a pair list that already holds entries (idb_mx.hip): the core
+// flags are read per entry, so a wave's pairs, which come from one tile,
+// touch a few lines; only pairs that are not core-core are rewritten (dead),
+// and rows are looked up for border claims alone.  A link that the parent as
+// last seen already makes is left out (an older, larger parent only costs an
+// atomic that changes nothing).
+__global__ void k_union_link(uint2 *edges, const uint32_t *fill, const uint32_t *n_chunks, uint32_t max_chunks,
+                             uint32_t chunk_log2, const uint8_t *ecore, const uint32_t *erow, uint32_t *par_e,
+                             uint32_t *bmin)
+{
+    for_pairs(fill, n_chunks, max_chunks, chunk_log2, [&](uint64_t e, bool live) {
+        if (!live) return;
+        const uint2 p = edges[e];
+        const bool cx = ecore[p.x] != 0, cy = ecore[p.y] != 0;
+        if (cx && cy) {
+            const uint32_t lo = p.x < p.y ? p.x : p.y, hi = p.x < p.y ? p.y : p.x;
+            if (ld_cached(par_e + hi) > lo) atomicMin(par_e + hi, lo);
+            return;
+        }
+        edges[e] = make_uint2(IDB_NONE, IDB_NONE);
+        if (cx || cy) {
+            const uint32_t core = erow[cx ? p.x : p.y], border = erow[cx ? p.y : p.x];
+            if (ld_cached(bmin + border) > core) atomicMin(bmin + border, core);
+        }
+    });
 }
 
 __global__ void k_union_entries(const uint2 *edges, const uint32_t *fill, const uint32_t *n_chunks,
                                 uint32_t max_chunks, uint32_t chunk_log2, uint32_t *par_e)
 {
-    const uint32_t nc = *n_chunks;
-    if (nc > max_chunks) return;
-    const unsigned long long n = (unsigned long long)nc << chunk_log2;
-    const uint32_t cmask = (1u << chunk_log2) - 1u;
-    // The grid-stride step is a multiple of 64 and chunks hold a multiple of
-    // 64 pairs, so the lanes of a wave always hold consecutive slots of one
-    // chunk.  Consecutive pairs mostly share their first entry x (one query's
-    // hits); a run x-y1, x-y2, ... is joined as the chain x-y1, y1-y2, ...:
-    // the same component, without every lane queueing its exchange on the
-    // root of x.
-    const uint32_t lane = __lane_id();
-    for (unsigned long long base = (blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x) & ~63ull; base < n;
-         base += (unsigned long long)gridDim.x * blockDim.x) {
-        const unsigned long long e = base + lane;
-        const bool live = ((uint32_t)e & cmask) < fill[e >> chunk_log2];
+    // Consecutive pairs mostly share their first entry x (one query's hits); a
+    // run x-y1, x-y2, ... is joined as the chain x-y1, y1-y2, ...: the same
+    // component, without every lane queueing its exchange on the root of x.
+    for_pairs(fill, n_chunks, max_chunks, chunk_log2, [&](uint64_t e, bool live) {
+        const uint32_t lane = lane_id();
         uint2 p = make_uint2(IDB_NONE, IDB_NONE);
         if (live) p = edges[e];
         const bool cc = p.x != IDB_NONE;
@@ -2193,7 +2002,7 @@ __global__ void k_union_entries(const uint2 *edges, const uint32_t *fill, const 
         const uint32_t px = (uint32_t)__shfl_up((int)p.x, 1, 64), py = (uint32_t)__shfl_up((int)p.y, 1, 64);
         const bool pcc = __shfl_up((int)cc, 1, 64) != 0 && lane > 0;
         if (cc) union_cached(par_e, (pcc && px == p.x) ? py : p.x, p.y);
-    }
+    });
 }
 
 // Between the pre-link and the union: every entry points straight at its
@@ -2274,45 +2083,13 @@ __global__ void k_union_to_rows(const uint32_t *n_chunks, uint32_t max_chunks, c
 // every launch otherwise.
 uint32_t resident_blocks(const void *kernel, uint32_t block, size_t shm)
 {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) {
-        (void)hipGetLastError();
-        dev = 0;
-    }
-    static std::mutex m;
-    static std::map<std::tuple<int, const void *, uint32_t, size_t>, uint32_t> known;
-    const auto key = std::make_tuple(dev, kernel, block, shm);
-    {
-        std::lock_guard<std::mutex> g(m);
-        const auto it = known.find(key);
-        if (it != known.end()) return it->second;
-    }
-    int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, (int)block, shm) != hipSuccess || per_cu <= 0)
-        per_cu = 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-    (void)hipGetLastError();
-    const uint32_t r = (uint32_t)per_cu * (uint32_t)cus;
-    std::lock_guard<std::mutex> g(m);
-    known[key] = r;
-    return r;
+    return idb_resident_blocks(kernel, block, shm);
 }
-
 uint32_t grid_for(uint32_t n_tiles, uint32_t wpb, uint32_t resident, uint32_t mul = 1)
 {
-    uint32_t b = (n_tiles + wpb - 1) / wpb;
-    const uint32_t cap = resident * (mul ? mul : 1u);
-    if (b > cap) b = cap;
-    return b ? b : 1u;
+    return idb_grid_for(n_tiles, wpb, resident, mul);
 }
-
-// Waves per block: the tuned value when set, within [1, most].
-uint32_t pick_wpb(const idb_pair_args &a, uint32_t most)
-{
-    uint32_t w = a.tune_wpb ? a.tune_wpb : most;
-    return std::max(1u, std::min(w, most));
-}
+uint32_t pick_wpb(const idb_pair_args &a, uint32_t most) { return idb_pick_wpb(a, most); }
 
 template <int W, bool FUSE, int FILT>
 hipError_t launch_myers_w(const idb_pair_args &a, dim3 block, size_t shm, uint32_t wpb, hipStream_t s)
@@ -2372,6 +2149,7 @@ template <bool FUSE>
 hipError_t launch_myers(const idb_pair_args &a_in, uint32_t W, hipStream_t s)
 {
     if (a_in.n_tiles == 0) return hipSuccess;
+    if (a_in.e_feat) return FUSE ? idb_launch_mx_fuse(a_in, s) : idb_launch_mx_count(a_in, s);
     // Unless a shape was tuned: one wave per block, plain block order, and a
     // grid of 4x (one-word rows) or 8x (longer rows) the resident waves, so
     // that waves done early are replaced while heavy tiles run.  These are
@@ -2452,7 +2230,7 @@ hipError_t launch_count_ham_hw(const idb_pair_args &a_in, hipStream_t s)
     }
     const uint32_t wpb = pick_wpb(a, 4);
     const void *k = (const void *)k_count_ham<HWMAX, BITS>;
-    const dim3 block(64 * wpb), grid(grid_for(a.n_tiles, wpb, resident_blocks(k, 64 * wpb, 0), a.tune_grid_mul));
+    const dim3 block(64 * wpb), grid(idb_count_grid(a, a.n_tiles, wpb, resident_blocks(k, 64 * wpb, 0)));
     hipLaunchKernelGGL((k_count_ham<HWMAX, BITS>), grid, block, 0, s, a, wpb);
     return hipGetLastError();
 }
@@ -2497,7 +2275,7 @@ hipError_t launch_learned(const idb_pair_args &a_in, hipStream_t s)
     // pattern words of the longest row (the encoder reads up to 160 letters)
     const uint32_t W = std::max(1u, (a.S + 31) / 32);
     if (W > 5) return hipErrorInvalidValue;
-    const size_t per_wave = idb_myers_lds_per_wave(a.K, W) + (a.qgram_filter ? 2 * idb_qgram_lds_per_wave() : 0);
+    const size_t per_wave = idb_myers_lds_per_wave(a.K, W) + (a.qgram_filter ? idb_qgram_lds_per_wave() : 0);
     uint32_t wpb = (uint32_t)(std::min<size_t>(idb_lds_limit(), 65536) / per_wave);
     if (wpb > 4) wpb = 4;
     if (wpb == 0) return hipErrorInvalidValue;
@@ -2534,6 +2312,56 @@ hipError_t launch_pair_dist_w(const uint8_t *seq, const uint64_t *off, const uin
 }
 
 }  // namespace
+
+uint32_t idb_resident_blocks(const void *kernel, uint32_t block, size_t shm)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();
+        dev = 0;
+    }
+    static std::mutex m;
+    static std::map<std::tuple<int, const void *, uint32_t, size_t>, uint32_t> known;
+    const auto key = std::make_tuple(dev, kernel, block, shm);
+    {
+        std::lock_guard<std::mutex> g(m);
+        const auto it = known.find(key);
+        if (it != known.end()) return it->second;
+    }
+    int per_cu = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, (int)block, shm) != hipSuccess || per_cu <= 0)
+        per_cu = 1;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    (void)hipGetLastError();
+    const uint32_t r = (uint32_t)per_cu * (uint32_t)cus;
+    std::lock_guard<std::mutex> g(m);
+    known[key] = r;
+    return r;
+}
+
+uint32_t idb_grid_for(uint32_t n_tiles, uint32_t wpb, uint32_t resident, uint32_t mul)
+{
+    uint32_t b = (n_tiles + wpb - 1) / wpb;
+    const uint32_t cap = resident * (mul ? mul : 1u);
+    if (b > cap) b = cap;
+    return b ? b : 1u;
+}
+
+// The grid of a count pass: no more waves than own a chunk of the pair list
+// (every further one would claim a chunk for its few pairs).
+uint32_t idb_count_grid(const idb_pair_args &a, uint32_t n_tiles, uint32_t wpb, uint32_t resident)
+{
+    const uint32_t g = idb_grid_for(n_tiles, wpb, resident, a.tune_grid_mul);
+    return a.edges && a.chunk_base ? std::max(1u, std::min(g, a.chunk_base / wpb)) : g;
+}
+
+// Waves per block: the tuned value when set, within [1, most].
+uint32_t idb_pick_wpb(const idb_pair_args &a, uint32_t most)
+{
+    uint32_t w = a.tune_wpb ? a.tune_wpb : most;
+    return std::max(1u, std::min(w, most));
+}
 
 hipError_t idb_launch_count_learned(const idb_pair_args &a, hipStream_t s) { return launch_learned(a, s); }
 
@@ -2585,9 +2413,15 @@ hipError_t idb_launch_fuse_hamming(const idb_pair_args &a, hipStream_t s) { retu
 hipError_t idb_launch_union_edges(const idb_pair_args &a, const idb_union_args &u, hipStream_t s)
 {
     if (!a.edges || a.max_chunks == 0) return hipSuccess;
-    const uint32_t b1 = resident_blocks((const void *)k_union_to_entries, 256, 0);
-    hipLaunchKernelGGL(k_union_to_entries, dim3(b1), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks, a.max_chunks,
-                       a.chunk_log2, u.pe, u.par_e, u.bmin);
+    if (u.ecore) {
+        const uint32_t b1 = resident_blocks((const void *)k_union_link, 256, 0);
+        hipLaunchKernelGGL(k_union_link, dim3(b1), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks, a.max_chunks,
+                           a.chunk_log2, u.ecore, u.erow, u.par_e, u.bmin);
+    } else {
+        const uint32_t b1 = resident_blocks((const void *)k_union_to_entries, 256, 0);
+        hipLaunchKernelGGL(k_union_to_entries, dim3(b1), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks,
+                           a.max_chunks, a.chunk_log2, u.pe, u.par_e, u.bmin);
+    }
     const uint32_t eb = (u.n_entries + 255) / 256 < 2048u ? (u.n_entries + 255) / 256 : 2048u;
     hipLaunchKernelGGL(k_union_compress, dim3(eb ? eb : 1u), dim3(256), 0, s, a.n_chunks, a.max_chunks, u.par_e,
                        u.n_entries);

@@ -14,13 +14,11 @@
 //
 // Weights are bfloat16 copies of float32 master weights (Adam keeps the
 // master copy); activations are bfloat16, all products accumulate in float32.
-// Embeddings come from one fused kernel (k_encode).  In training, the three
-// convolutions, their data gradients and their weight gradients run on one
-// MFMA GEMM kernel (v_mfma_f32_32x32x16_bf16) whose operand loaders gather
-// im2col windows straight from the activations, so no im2col matrix is ever
-// materialised.  Row m of an activation matrix is position m % P of
-// sequence m / P; positions at or past the sequence's length are zero after
-// every layer (each row is convolved with its own zero padding).
+// Rows are packed back to back with two zero rows after each (the zero
+// padding of a 5-tap window), in tiles of 256.  One fused kernel (k_encode)
+// runs the forward pass of a tile in LDS, a second one (k_enc_bwd) the data
+// gradients; only what the weight gradients (k_wgrad) read goes through HBM.
+// All products run on v_mfma_f32_32x32x16_bf16.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -50,12 +48,6 @@ static_assert(N_PARAMS == IDB_ENC_PARAMS, "parameter count");
 __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-// tanh(u) = 1 - 2 / (exp(2u) + 1): one hardware exponential and one
-// reciprocal (exp overflows to inf for large u and gives 1; underflows to 0
-// for very negative u and gives -1).  Its error is far below the bfloat16
-// rounding every activation goes through.
-__device__ __forceinline__ float tanh_exp(float u) { return 1.f - __fdividef(2.f, __expf(2.f * u) + 1.f); }
-
 // 0.5 x (1 + tanh(u)) = x / (1 + exp(-2u)), u = k (x + 0.044715 x^3): one
 // hardware base-2 exponential and one reciprocal.  For very negative x the
 // exponential overflows to inf and the result is -0; for large x it is x.
@@ -65,468 +57,14 @@ __device__ __forceinline__ float gelu(float x)
     const float e = x * __builtin_fmaf(C3, x * x, C1);
     return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(e));
 }
+// Its derivative s + x s (1 - s) d(2u)/dx with s = 1 / (1 + exp(-2u)).
 __device__ __forceinline__ float gelu_grad(float x)
 {
-    const float th = tanh_exp(GELU_K * (x + 0.044715f * x * x * x));
-    return 0.5f * (1.f + th) + 0.5f * x * (1.f - th * th) * GELU_K * (1.f + 3.f * 0.044715f * x * x);
-}
-
-// ---------------------------------------------------------------------------
-// GEMM: out[m][n] = sum_k A[m][k] B[n][k] over a block tile of 128 x 128 with
-// k chunks of 64, double-buffered in LDS, with global loads two chunks ahead
-// of the chunk whose 16 MFMAs per wave are running.  Four waves own
-// 64 x 64 each (2 x 2 MFMA tiles of 32 x 32).  LDS rows hold 64 k values plus
-// 8 of padding (144 bytes), so the 16-byte fragment reads of 16 consecutive
-// rows hit disjoint banks.  Loaders fetch 8 consecutive k of one row (ROW) or
-// 8 consecutive rows at one k (COL, stored transposed) per 16-byte load.
-constexpr uint32_t GM = 128, GN = 128, GK = 64, LDK = GK + 8;
-constexpr uint32_t GCH = GM * GK / 8 / 256;  // 16-byte chunks per thread and operand
-
-// k at or past kend (the end of this block's k range) reads as zero.
-template <bool COL, class L>
-__device__ __forceinline__ void fetch_tile(const L &ld, uint32_t r0, uint32_t k0, uint32_t kend, uint32_t tid,
-                                           uint4 (&v)[GCH])
-{
-#pragma unroll
-    for (uint32_t i = 0; i < GCH; ++i) {
-        const uint32_t c = tid + i * 256;
-        const uint32_t k = COL ? k0 + (c >> 4) : k0 + (c & 7) * 8;
-        v[i] = make_uint4(0, 0, 0, 0);
-        if (k < kend) v[i] = COL ? ld.fetch(r0 + (c & 15) * 8, k) : ld.fetch(r0 + (c >> 3), k);
-    }
-}
-
-template <bool COL>
-__device__ __forceinline__ void store_tile(uint16_t *lds, const uint4 (&v)[GCH], uint32_t tid)
-{
-#pragma unroll
-    for (uint32_t i = 0; i < GCH; ++i) {
-        const uint32_t c = tid + i * 256;
-        if (!COL) {
-            *(uint4 *)(lds + (c >> 3) * LDK + (c & 7) * 8) = v[i];
-        } else {
-            const uint32_t r = (c & 15) * 8, k = c >> 4;
-            const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-#pragma unroll
-            for (uint32_t e = 0; e < 8; ++e) lds[(r + e) * LDK + k] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
-        }
-    }
-}
-
-template <class LA, class LB, class EP>
-__global__ __launch_bounds__(256, 2) void k_gemm(LA la, LB lb, EP ep, uint32_t M, uint32_t N, uint32_t K, uint32_t ksplit)
-{
-    __shared__ __align__(16) uint16_t As[2][GM * LDK];
-    __shared__ __align__(16) uint16_t Bs[2][GN * LDK];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t m0 = blockIdx.x * GM, n0 = blockIdx.y * GN;
-    const uint32_t kb = blockIdx.z * ksplit, ke = min(K, kb + ksplit);
-    const uint32_t wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    if (kb >= ke) return;
-    // Loads run two chunks ahead: chunk c + 1 sits in registers (ra, rb)
-    // while chunk c + 2 is in flight (na, nb) and chunk c is consumed from LDS.
-    uint4 ra[GCH], rb[GCH], na[GCH] = {}, nb[GCH] = {};
-    fetch_tile<LA::COL>(la, m0, kb, ke, tid, ra);
-    fetch_tile<LB::COL>(lb, n0, kb, ke, tid, rb);
-    store_tile<LA::COL>(As[0], ra, tid);
-    store_tile<LB::COL>(Bs[0], rb, tid);
-    fetch_tile<LA::COL>(la, m0, kb + GK, ke, tid, ra);
-    fetch_tile<LB::COL>(lb, n0, kb + GK, ke, tid, rb);
-    __syncthreads();
-    uint32_t buf = 0;
-    for (uint32_t k0 = kb; k0 < ke; k0 += GK) {
-        const bool more = k0 + GK < ke;
-        if (k0 + 2 * GK < ke) {
-            fetch_tile<LA::COL>(la, m0, k0 + 2 * GK, ke, tid, na);
-            fetch_tile<LB::COL>(lb, n0, k0 + 2 * GK, ke, tid, nb);
-        }
-#pragma unroll
-        for (uint32_t ks = 0; ks < GK / 16; ++ks) {
-            bf16x8 a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                a[i] = *(const bf16x8 *)(As[buf] + (wm + i * 32 + (lane & 31)) * LDK + ks * 16 + (lane >> 5) * 8);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                b[j] = *(const bf16x8 *)(Bs[buf] + (wn + j * 32 + (lane & 31)) * LDK + ks * 16 + (lane >> 5) * 8);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) {
-            store_tile<LA::COL>(As[buf ^ 1], ra, tid);
-            store_tile<LB::COL>(Bs[buf ^ 1], rb, tid);
-#pragma unroll
-            for (uint32_t i = 0; i < GCH; ++i) {
-                ra[i] = na[i];
-                rb[i] = nb[i];
-            }
-        }
-        __syncthreads();
-        buf ^= 1;
-    }
-    // result layout of the 32 x 32 MFMA: lane l holds column l % 32 and rows
-    // 8 (r / 4) + 4 (l / 32) + r % 4 for r = 0 .. 15
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) ep.tile(acc[i][j], m0 + wm + i * 32, n0 + wn + j * 32 + (lane & 31), lane, M, N);
-}
-
-// Row of element r of a lane's 32 x 32 result tile, relative to the tile.
-__device__ __forceinline__ uint32_t tile_row(int r, uint32_t lane) { return (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3); }
-
-// im2col window of an activation matrix X[rows][cin]: element (m, t * cin +
-// c) is X[PP s + q][c] with q = p + t - 2 (forward) or q = p - t + 2 (data
-// gradient), zero outside the PP positions of sequence s = m / PP.
-template <uint32_t PP>
-struct LdConv {
-    static constexpr bool COL = false;
-    const uint16_t *X;
-    uint32_t cin, M;  // cin a power of two
-    int flip;
-    __device__ uint4 fetch(uint32_t m, uint32_t k) const
-    {
-        if (m >= M) return make_uint4(0, 0, 0, 0);
-        const uint32_t sh = 31u - __builtin_clz(cin);
-        const int t = (int)(k >> sh), c = (int)(k & (cin - 1u)), p = (int)(m % PP);
-        const int q = flip ? p - t + 2 : p + t - 2;
-        if (q < 0 || q >= (int)PP) return make_uint4(0, 0, 0, 0);
-        return *(const uint4 *)(X + ((size_t)(m - (uint32_t)p) + q) * cin + c);
-    }
-};
-
-// Plain row-major matrix R[rows][ld], k contiguous.
-struct LdRows {
-    static constexpr bool COL = false;
-    const uint16_t *R;
-    uint32_t ld, rows;
-    __device__ uint4 fetch(uint32_t r, uint32_t k) const
-    {
-        if (r >= rows) return make_uint4(0, 0, 0, 0);
-        return *(const uint4 *)(R + (size_t)r * ld + k);
-    }
-};
-
-// Weight gradient, operand A: rows are output channels o, k runs over
-// activation rows m: dH[m][o] (8 consecutive o per load).
-struct LdGradT {
-    static constexpr bool COL = true;
-    const uint16_t *dH;
-    uint32_t M;
-    __device__ uint4 fetch(uint32_t o, uint32_t m) const
-    {
-        if (m >= M) return make_uint4(0, 0, 0, 0);
-        return *(const uint4 *)(dH + (size_t)m * C + o);
-    }
-};
-
-// Weight gradient, operand B: rows are im2col columns k' = t * cin + c, k runs
-// over activation rows m: X[PP s + p + t - 2][c] (8 consecutive c per load).
-template <uint32_t PP>
-struct LdConvT {
-    static constexpr bool COL = true;
-    const uint16_t *X;
-    uint32_t cin, M;  // cin a power of two
-    __device__ uint4 fetch(uint32_t kc, uint32_t m) const
-    {
-        if (m >= M || kc >= T * cin) return make_uint4(0, 0, 0, 0);
-        const uint32_t sh = 31u - __builtin_clz(cin);
-        const uint32_t p = m % PP;
-        const int t = (int)(kc >> sh), c = (int)(kc & (cin - 1u)), q = (int)p + t - 2;
-        if (q < 0 || q >= (int)PP) return make_uint4(0, 0, 0, 0);
-        return *(const uint4 *)(X + ((size_t)(m - p) + q) * cin + c);
-    }
-};
-
-// Epilogues get one 32 x 32 result tile per call: rows row0 .. row0 + 31
-// (within one sequence: row0 and PP are multiples of 32) and this lane's
-// column `col`.
-
-// Forward epilogue: bias, saved pre-activation, GELU, length mask.
-template <uint32_t PP>
-struct EpConvFwd {
-    const uint16_t *bias;
-    const uint32_t *len;
-    uint16_t *H, *A;
-    __device__ void tile(const f32x16 &v, uint32_t row0, uint32_t col, uint32_t lane, uint32_t M, uint32_t N) const
-    {
-        if (col >= N || row0 >= M) return;
-        const float b = bf2f(bias[col]);
-        // rows row0 + pl + d(r), d(r) = 8 (r / 4) + r % 4, within one sequence
-        const uint32_t pl = (lane >> 5) * 4;
-        const int32_t lim = (int32_t)len[row0 / PP] - (int32_t)(row0 % PP + pl);  // rows d < lim are letters
-        const size_t base = (size_t)(row0 + pl) * C + col;
-        uint16_t *a = A + base;
-        uint16_t *h = H + base;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int32_t d = (r >> 2) * 8 + (r & 3);
-            const float x = v[r] + b;
-            h[d * C] = f2bf(x);
-            a[d * C] = d < lim ? f2bf(gelu(x)) : (uint16_t)0;
-        }
-    }
-};
-
-// Data-gradient epilogue: masked, times GELU' of the previous layer's saved
-// pre-activation (bfloat16 out), or the embedding gradient (float out).
-template <uint32_t PP>
-struct EpConvBwd {
-    const uint16_t *Hprev;
-    const uint32_t *len;
-    uint32_t cin;
-    uint16_t *dHprev;
-    float *dX0;
-    __device__ void tile(const f32x16 &v, uint32_t row0, uint32_t col, uint32_t lane, uint32_t M, uint32_t N) const
-    {
-        if (col >= N || row0 >= M) return;
-        const uint32_t L = len[row0 / PP], p0 = row0 % PP;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t p = tile_row(r, lane);
-            const size_t at = (size_t)(row0 + p) * cin + col;
-            const bool valid = p0 + p < L;
-            if (dHprev) dHprev[at] = valid ? f2bf(v[r] * gelu_grad(bf2f(Hprev[at]))) : (uint16_t)0;
-            else dX0[at] = valid ? v[r] : 0.f;
-        }
-    }
-};
-
-struct EpAtomic {
-    float *G;
-    uint32_t ld;
-    __device__ void tile(const f32x16 &v, uint32_t row0, uint32_t col, uint32_t lane, uint32_t M, uint32_t N) const
-    {
-        if (col >= N) return;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t row = row0 + tile_row(r, lane);
-            if (row < M) atomicAdd(G + (size_t)row * ld + col, v[r]);
-        }
-    }
-};
-
-// ---------------------------------------------------------------------------
-// VALU kernels
-
-// Tokens of every row: vocabulary map, first P letters, token 0 past the end.
-__global__ void k_tokenize(const uint8_t *seq, const uint64_t *off, const uint32_t *len, uint32_t n,
-                           const uint8_t *vocab, uint32_t P, uint8_t *tok, uint32_t *tlen)
-{
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const uint32_t L = min(len[i], P);
-        const uint8_t *s = seq + off[i];
-        for (uint32_t p = 0; p < P; ++p) tok[(size_t)i * P + p] = p < L ? vocab[s[p]] : (uint8_t)0;
-        tlen[i] = L;
-    }
-}
-
-// Batch assembly: sequence b of the batch is row rows[b] (IDB_NONE: empty).
-__global__ void k_gather_rows(const uint8_t *tok, const uint32_t *tlen, const uint32_t *rows, uint32_t nb,
-                              uint32_t P, uint8_t *btok, uint32_t *blen)
-{
-    for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < nb; b += gridDim.x * blockDim.x) {
-        const uint32_t r = rows[b];
-        const uint32_t L = r == IDB_NONE ? 0u : tlen[r];
-        for (uint32_t p = 0; p < P; ++p) btok[(size_t)b * P + p] = r == IDB_NONE ? (uint8_t)0 : tok[(size_t)r * P + p];
-        blen[b] = L;
-    }
-}
-
-// Consecutive rows first .. first + nb - 1 (past n: empty).
-__global__ void k_iota_rows(uint32_t first, uint32_t n, uint32_t nb, uint32_t *rows)
-{
-    for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < nb; b += gridDim.x * blockDim.x)
-        rows[b] = first + b < n ? first + b : IDB_NONE;
-}
-
-// Pairs of a training batch: sequences 2 i and 2 i + 1 are the pair's rows.
-__global__ void k_pair_rows(const uint32_t *pairs, const uint32_t *order, uint64_t first, uint32_t nb, uint64_t n,
-                            uint32_t *rows, float *y, const float *labels)
-{
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += gridDim.x * blockDim.x) {
-        const uint64_t k = first + i;
-        if (k < n) {
-            const uint32_t q = order ? order[k] : (uint32_t)k;
-            rows[2 * i] = pairs[2 * (size_t)q];
-            rows[2 * i + 1] = pairs[2 * (size_t)q + 1];
-            y[i] = labels[q];
-        } else {
-            rows[2 * i] = rows[2 * i + 1] = IDB_NONE;
-            y[i] = -1.f;  // padding pair: no loss
-        }
-    }
-}
-
-__global__ void k_embed(const uint8_t *btok, const uint32_t *blen, uint32_t nseq, uint32_t P, const uint16_t *emb,
-                        uint16_t *X0)
-{
-    const uint32_t total = nseq * P * (C0 / 8);
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        const uint32_t m = i / (C0 / 8), c8 = (i % (C0 / 8)) * 8;
-        const bool valid = (m % P) < blen[m / P];
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (valid) v = *(const uint4 *)(emb + (size_t)btok[m] * C0 + c8);
-        *(uint4 *)(X0 + (size_t)m * C0 + c8) = v;
-    }
-}
-
-// Head: mean over the sequence's letters, projection, L2 norm.  One wave per
-// sequence: lanes hold channels l and l + 64, then output l.
-__global__ void k_head_fwd(const uint16_t *A3, const uint32_t *blen, uint32_t nseq, uint32_t P, const uint16_t *wp_b,
-                           const uint16_t *bp, float *pool, float *u, float *z)
-{
-    __shared__ float sp[4][C];
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (uint32_t s = blockIdx.x * 4 + w; s < nseq; s += gridDim.x * 4) {
-        const uint32_t L = blen[s];
-        float a0 = 0.f, a1 = 0.f;
-        for (uint32_t p = 0; p < L; ++p) {
-            a0 += bf2f(A3[((size_t)s * P + p) * C + lane]);
-            a1 += bf2f(A3[((size_t)s * P + p) * C + lane + 64]);
-        }
-        const float inv = L ? 1.f / (float)L : 0.f;
-        a0 *= inv;
-        a1 *= inv;
-        sp[w][lane] = a0;
-        sp[w][lane + 64] = a1;
-        pool[(size_t)s * C + lane] = a0;
-        pool[(size_t)s * C + lane + 64] = a1;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        float acc = bf2f(bp[lane]);
-        for (uint32_t o = 0; o < C; ++o) acc += bf2f(wp_b[(size_t)lane * C + o]) * sp[w][o];
-        float ss = acc * acc;
-#pragma unroll
-        for (int k = 32; k > 0; k >>= 1) ss += __shfl_xor(ss, k, 64);
-        const float nrm = fmaxf(sqrtf(ss), 1e-6f);
-        u[(size_t)s * D + lane] = acc;
-        z[(size_t)s * D + lane] = acc / nrm;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    }
-}
-
-// Contrastive loss of pair i (sequences 2i, 2i+1); one wave per pair.
-__global__ void k_pair_loss(const float *z, const float *y, uint32_t npairs, float margin, float inv_b, float *dz,
-                            float *loss)
-{
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    float lsum = 0.f;
-    for (uint32_t i = blockIdx.x * 4 + w; i < npairs; i += gridDim.x * 4) {
-        const float yi = y[i];
-        const float diff = z[(size_t)(2 * i) * D + lane] - z[(size_t)(2 * i + 1) * D + lane];
-        float d2 = diff * diff;
-#pragma unroll
-        for (int k = 32; k > 0; k >>= 1) d2 += __shfl_xor(d2, k, 64);
-        float g = 0.f;
-        if (yi >= 0.f) {
-            const float d = sqrtf(d2 + 1e-12f);
-            const float hinge = fmaxf(0.f, margin - d);
-            if (lane == 0) lsum += yi * d2 + (1.f - yi) * hinge * hinge;
-            g = (2.f * yi - (1.f - yi) * 2.f * hinge / d) * inv_b * diff;
-        }
-        dz[(size_t)(2 * i) * D + lane] = g;
-        dz[(size_t)(2 * i + 1) * D + lane] = -g;
-    }
-    if (lane == 0 && lsum != 0.f) atomicAdd(loss, lsum * inv_b);
-}
-
-// Head backward, one wave per sequence: du, dpool, and the last layer's
-// pre-activation gradient dH3 = (dpool / L) * GELU'(H3) at the valid letters.
-__global__ void k_head_bwd(const float *dz, const float *z, const float *u, const uint32_t *blen, uint32_t nseq,
-                           uint32_t P, const uint16_t *wp_b, const uint16_t *H3, float *du_out, uint16_t *dH3)
-{
-    __shared__ float sdu[4][D];
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (uint32_t s = blockIdx.x * 4 + w; s < nseq; s += gridDim.x * 4) {
-        const float zz = z[(size_t)s * D + lane], g = dz[(size_t)s * D + lane], uu = u[(size_t)s * D + lane];
-        float zg = zz * g, ss = uu * uu;
-#pragma unroll
-        for (int k = 32; k > 0; k >>= 1) {
-            zg += __shfl_xor(zg, k, 64);
-            ss += __shfl_xor(ss, k, 64);
-        }
-        const float nrm = fmaxf(sqrtf(ss), 1e-6f);
-        const float du = (g - zz * zg) / nrm;
-        du_out[(size_t)s * D + lane] = du;
-        sdu[w][lane] = du;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        const uint32_t L = blen[s];
-        const float inv = L ? 1.f / (float)L : 0.f;
-        float dp0 = 0.f, dp1 = 0.f;
-        for (uint32_t j = 0; j < D; ++j) {
-            dp0 += bf2f(wp_b[(size_t)j * C + lane]) * sdu[w][j];
-            dp1 += bf2f(wp_b[(size_t)j * C + lane + 64]) * sdu[w][j];
-        }
-        dp0 *= inv;
-        dp1 *= inv;
-        for (uint32_t p = 0; p < P; ++p) {
-            const size_t m = (size_t)s * P + p;
-            const bool valid = p < L;
-            dH3[m * C + lane] = valid ? f2bf(dp0 * gelu_grad(bf2f(H3[m * C + lane]))) : (uint16_t)0;
-            dH3[m * C + lane + 64] = valid ? f2bf(dp1 * gelu_grad(bf2f(H3[m * C + lane + 64]))) : (uint16_t)0;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    }
-}
-
-// Projection gradients: dWp[j][o] = sum_s du[s][j] pool[s][o], dbp[j] = sum_s du[s][j].
-__global__ void k_proj_grad(const float *du, const float *pool, uint32_t nseq, float *g_wp, float *g_bp)
-{
-    const uint32_t j = blockIdx.x, o = threadIdx.x;  // D blocks x C threads
-    float acc = 0.f, accb = 0.f;
-    for (uint32_t s = blockIdx.y; s < nseq; s += gridDim.y) {
-        const float d = du[(size_t)s * D + j];
-        acc += d * pool[(size_t)s * C + o];
-        accb += d;
-    }
-    atomicAdd(g_wp + (size_t)j * C + o, acc);
-    if (o == 0) atomicAdd(g_bp + j, accb);
-}
-
-// Bias gradient: column sums of dH[M][C].
-__global__ void k_bias_grad(const uint16_t *dH, uint32_t M, float *gb)
-{
-    const uint32_t o = threadIdx.x;  // C threads
-    float acc = 0.f;
-    for (uint32_t m = blockIdx.x; m < M; m += gridDim.x) acc += bf2f(dH[(size_t)m * C + o]);
-    atomicAdd(gb + o, acc);
-}
-
-// Embedding gradient: scatter-add of dX0 rows by token, through LDS.
-__global__ void k_emb_grad(const float *dX0, const uint8_t *btok, const uint32_t *blen, uint32_t M, uint32_t P,
-                           float *gemb)
-{
-    __shared__ float acc[NTOK * C0];
-    for (uint32_t i = threadIdx.x; i < NTOK * C0; i += blockDim.x) acc[i] = 0.f;
-    __syncthreads();
-    const uint32_t c = threadIdx.x & (C0 - 1);
-    for (uint32_t m = blockIdx.x * (blockDim.x / C0) + threadIdx.x / C0; m < M; m += gridDim.x * (blockDim.x / C0)) {
-        if ((m % P) >= blen[m / P]) continue;
-        atomicAdd(&acc[(uint32_t)btok[m] * C0 + c], dX0[(size_t)m * C0 + c]);
-    }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < NTOK * C0; i += blockDim.x)
-        if (acc[i] != 0.f) atomicAdd(gemb + i, acc[i]);
-}
-
-// Data-gradient weights: WT[c][t * C + o] = W[o][t * cin + c] (bfloat16).
-__global__ void k_transpose_w(const uint16_t *W, uint32_t cin, uint16_t *WT)
-{
-    const uint32_t total = C * T * cin;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        const uint32_t o = i / (T * cin), k = i % (T * cin), t = k / cin, c = k % cin;
-        WT[(size_t)c * (T * C) + t * C + o] = W[i];
-    }
+    constexpr float C1 = -2.f * GELU_K * 1.4426950408889634f, C3 = C1 * 0.044715f;
+    const float x2 = x * x;
+    const float s = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * __builtin_fmaf(C3, x2, C1)));
+    const float du2 = __builtin_fmaf(6.f * GELU_K * 0.044715f, x2, 2.f * GELU_K);
+    return s + x * du2 * (s - s * s);
 }
 
 __global__ void k_to_bf16(const float *src, uint32_t n, uint16_t *dst)
@@ -550,7 +88,7 @@ __global__ void k_adam(float *th, const float *g, float *m, float *v, uint32_t n
 }
 
 // ---------------------------------------------------------------------------
-// Inference: the whole encoder in one kernel.
+// The whole forward pass in one kernel.
 //
 // A block takes a tile of EM = 256 activation rows and keeps them in LDS
 // through all three convolutions (layer by layer, in place), so neither
@@ -567,8 +105,10 @@ __global__ void k_adam(float *th, const float *g, float *m, float *v, uint32_t n
 // in a row.  128 accumulators leave room for 2 waves per SIMD; at 71 KB of
 // activations two blocks share a CU, so one block's GELU (as many VALU cycles
 // as the MFMAs take) overlaps the other's products.
-// The k order and the arithmetic of every output are those of the training
-// forward pass (k_gemm), bit for bit.
+// In training (TRAIN) a block also writes what the backward pass reads: the
+// pre-activations in the lanes' own order (512 bytes per wave and store; k_enc_bwd
+// has the same lane mapping), the layers' inputs row by row in packed order,
+// the pooled means and the norms.
 // Measured: 200k protein rows (packed 1.25 Tflop) 5.22 -> 1.52 ms, 825 TFLOP/s
 // (a large bf16 product reaches 1,214 here); 20k rows of 24-150 letters
 // 2.98 -> 0.81 ms.
@@ -577,15 +117,29 @@ constexpr uint32_t EPW = 1024;                    // sequences per packing windo
 constexpr uint32_t EGRP = 8;                      // sequences per round of the head
 constexpr uint32_t EKS1 = T * C0 / 16, EKS = T * C / 16;  // k steps of layer 1, of layers 2 and 3
 constexpr size_t EPACK = (size_t)(EKS1 + 2 * EKS) * 4 * 64 * 8;  // packed weights (bfloat16)
+constexpr uint32_t BLAYER = EKS * 4 * 64 * 8, BPACK = 2 * BLAYER + EKS * 64 * 8;  // and transposed
+constexpr uint32_t EPAD = 2 * 2048;               // fragments loaded ahead past a pack's end
 
+// Where a training batch's sequences come from: sequence 2 i + h is row
+// pairs[2 q + h] of pair q = order[first + i] (or first + i).
+struct PairSource {
+    const uint32_t *pairs, *order;
+    const float *labels;
+    uint64_t first;
+    uint32_t *rows, *blen;  // out: row and length of every sequence
+    float *y;               // out: label of every pair
+};
+
+// A tile: first sequence, sequences, first row in packed order, packed rows.
 // Greedy packing of consecutive sequences into tiles, window by window:
-// tiles (first sequence, count) in any order, and every sequence's first row
-// within its tile.  At most EM + 2 rows per tile counting each sequence's two
-// zero rows (the last two lie in the tile's zero border).
-__global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t n, uint32_t P, uint2 *tiles,
-                                                  uint32_t *n_tiles, uint16_t *rstart)
+// tiles in any order, and every sequence's first row within its tile.  At
+// most EM + 2 rows per tile counting each sequence's two zero rows (the last
+// two lie in the tile's zero border).  count[0] = tiles, count[1] = rows.
+template <bool TRAIN>
+__global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t n, uint32_t P, uint4 *tiles,
+                                                  uint32_t *count, uint16_t *rstart, PairSource ps)
 {
-    __shared__ uint32_t S[EPW + 1], cut[EPW + 1], part[4], base_s;
+    __shared__ uint32_t S[EPW + 1], cut[EPW + 1], part[4], base_s, base_r;
     __shared__ uint16_t nxt[EPW];
     const uint32_t w0 = blockIdx.x * EPW, m = min(EPW, n - w0), tid = threadIdx.x, lane = tid & 63;
     constexpr uint32_t PER = EPW / 256;
@@ -593,7 +147,23 @@ __global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t 
 #pragma unroll
     for (uint32_t k = 0; k < PER; ++k) {
         const uint32_t i = tid * PER + k;
-        v[k] = i < m ? min(len[w0 + i], P) + 2u : 0u;
+        v[k] = 0u;
+        if (i < m) {
+            uint32_t L;
+            if (TRAIN) {
+                const uint32_t b = w0 + i;
+                const uint64_t at = ps.first + (b >> 1);
+                const uint32_t q = ps.order ? ps.order[at] : (uint32_t)at;
+                const uint32_t r = ps.pairs[2 * (size_t)q + (b & 1u)];
+                L = min(len[r], P);
+                ps.rows[b] = r;
+                ps.blen[b] = L;
+                if ((b & 1u) == 0) ps.y[b >> 1] = ps.labels[q];
+            } else {
+                L = min(len[w0 + i], P);
+            }
+            v[k] = L + 2u;
+        }
         sum += v[k];
     }
     uint32_t inc = sum;
@@ -628,11 +198,13 @@ __global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t 
         for (uint32_t i = 0; i < m; i = nxt[i]) cut[c++] = i;
         cut[c] = m;
         part[0] = c;
-        base_s = atomicAdd(n_tiles, c);
+        base_s = atomicAdd(count, c);
+        base_r = TRAIN ? atomicAdd(count + 1, S[m]) : 0u;
     }
     __syncthreads();
     const uint32_t c = part[0];
-    for (uint32_t t = tid; t < c; t += 256) tiles[base_s + t] = make_uint2(w0 + cut[t], cut[t + 1] - cut[t]);
+    for (uint32_t t = tid; t < c; t += 256)
+        tiles[base_s + t] = make_uint4(w0 + cut[t], cut[t + 1] - cut[t], base_r + S[cut[t]], S[cut[t + 1]] - S[cut[t]]);
     for (uint32_t i = tid; i < m; i += 256) {
         uint32_t lo = 0, hi = c;  // last tile that starts at or before i
         while (lo + 1 < hi) {
@@ -645,8 +217,10 @@ __global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t 
 
 // Weights in the order the encoder's waves read them: per layer and k step,
 // four 32-channel fragments of 64 lanes x 8 values; then the projection as
-// (input pair, output) words.
-__global__ void k_enc_pack(const uint16_t *theta_b, uint16_t *dst, uint32_t *wp2)
+// (input pair, output) words and as (output, input pair) words; then, for the
+// data gradients, layers 3 and 2 transposed (40 k steps of four fragments
+// each) and layer 1 (40 k steps of one fragment).
+__global__ void k_enc_pack(const uint16_t *theta_b, uint16_t *dst, uint32_t *wp2, uint16_t *bdst)
 {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < EPACK; i += gridDim.x * blockDim.x) {
         const uint32_t e = i & 7u, ln = (i >> 3) & 63u, ct = (i >> 9) & 3u;
@@ -666,13 +240,22 @@ __global__ void k_enc_pack(const uint16_t *theta_b, uint16_t *dst, uint32_t *wp2
         const uint32_t d = i % D, o = 2 * (i / D);
         wp2[i] = (uint32_t)theta_b[O_WP + d * C + o] | ((uint32_t)theta_b[O_WP + d * C + o + 1] << 16);
     }
+    // k step ks of a transposed layer: tap ks / 8, output channels 16 (ks % 8) ..
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < BPACK; i += gridDim.x * blockDim.x) {
+        const uint32_t e = i & 7u, ln = (i >> 3) & 63u;
+        const bool l1 = i >= 2 * BLAYER;
+        const uint32_t at = (l1 ? i - 2 * BLAYER : i % BLAYER) >> 9, ct = l1 ? 0u : at & 3u, ks = l1 ? at : at >> 2;
+        const uint32_t cin = l1 ? C0 : C, w = l1 ? O_W1 : (i < BLAYER ? O_W3 : O_W2);
+        const uint32_t o = (ks & 7u) * 16 + (ln >> 5) * 8 + e, c = ct * 32 + (ln & 31u);
+        bdst[i] = theta_b[w + o * (T * cin) + (ks >> 3) * cin + c];
+    }
 }
 
 struct EncArgs {
     const uint8_t *seq;
     const uint64_t *off;
     const uint32_t *len;
-    const uint2 *tiles;
+    const uint4 *tiles;
     const uint32_t *n_tiles;
     const uint16_t *rstart;
     const uint8_t *vocab;
@@ -681,10 +264,16 @@ struct EncArgs {
     uint32_t P;
     float *z;        // either may be null
     uint16_t *zb;
+    // training
+    const uint32_t *rows;  // row of each sequence (len is per sequence)
+    uint2 *H[3];           // pre-activations, lane order: 8192 words of 8 bytes per tile
+    uint16_t *X0, *A1, *A2;
+    float *pool, *nrm;
 };
 
-// One convolution over the tile: acc = W x window, CIN input channels.
-template <uint32_t CIN>
+// One convolution over the tile: acc = W x window, CIN input channels.  REV:
+// taps in the order of the data gradient (window row 4 - t for tap t).
+template <uint32_t CIN, bool REV = false>
 __device__ __forceinline__ void enc_conv(const uint16_t *X, const u32x4 *wp, uint32_t lane, f32x16 (&acc)[2][4])
 {
 #pragma unroll
@@ -703,7 +292,7 @@ __device__ __forceinline__ void enc_conv(const uint16_t *X, const u32x4 *wp, uin
     }
 #pragma unroll 1
     for (uint32_t t = 0; t < T; ++t) {
-        const uint16_t *xt = xr + t * EST;
+        const uint16_t *xt = xr + (REV ? T - 1 - t : t) * EST;
         const u32x4 *wt = wp + t * KT * 256;
 #pragma unroll
         for (uint32_t c = 0; c < KT; ++c) {
@@ -722,6 +311,25 @@ __device__ __forceinline__ void enc_conv(const uint16_t *X, const u32x4 *wp, uin
     }
 }
 
+// Rows [0, used) of the tile in LDS (its zero border included), to packed rows.
+__device__ __forceinline__ void enc_store_rows(const uint16_t *X, uint16_t *out, uint32_t used, uint32_t tid)
+{
+    for (uint32_t r = tid >> 4; r < used; r += 16)
+        *(u32x4 *)(out + (size_t)r * C + (tid & 15u) * 8) = *(const u32x4 *)(X + (r + 2) * EST + (tid & 15u) * 8);
+}
+
+// Index of the sequence that row r of a tile belongs to.
+__device__ __forceinline__ uint32_t seq_of_row(const uint16_t *s_row, uint32_t cnt, uint32_t r)
+{
+    uint32_t lo = 0, hi = cnt;
+    while (lo + 1 < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (s_row[mid] <= r) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+template <bool TRAIN>
 __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
 {
     __shared__ __align__(16) uint16_t X[(EM + 4) * EST];
@@ -740,23 +348,18 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
     for (uint32_t i = tid; i < 4 * EST; i += 256) X[(i < 2 * EST ? 0 : EM * EST) + i] = 0;
     const uint32_t nt = *a.n_tiles;
     for (uint32_t ti = blockIdx.x; ti < nt; ti += gridDim.x) {
-        const uint2 t = a.tiles[ti];
+        const uint4 t = a.tiles[ti];
         const uint32_t first = t.x, cnt = t.y;  // cnt <= EM / 2 + 1: two rows at least per sequence
         __syncthreads();
         if (tid < cnt) {
             s_len[tid] = min(a.len[first + tid], a.P);
             s_row[tid] = a.rstart[first + tid];
-            s_off[tid] = a.off[first + tid];
+            s_off[tid] = a.off[TRAIN ? a.rows[first + tid] : first + tid];
         }
         __syncthreads();
         {
             // embedding: thread = row
-            uint32_t lo = 0, hi = cnt;
-            while (lo + 1 < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (s_row[mid] <= tid) lo = mid; else hi = mid;
-            }
-            const uint32_t p = tid - s_row[lo];
+            const uint32_t lo = seq_of_row(s_row, cnt, tid), p = tid - s_row[lo];
             u32x4 e[4] = {};
             if (p < s_len[lo]) {
                 const u32x4 *src = (const u32x4 *)(a.theta_b + O_EMB + (uint32_t)a.vocab[a.seq[s_off[lo] + p]] * C0);
@@ -766,17 +369,22 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
             u32x4 *dst = (u32x4 *)(X + (tid + 2) * EST);
 #pragma unroll
             for (int k = 0; k < 4; ++k) dst[k] = e[k];
+            if (TRAIN) {
+                u32x4 *g = (u32x4 *)(a.X0 + (size_t)(t.z + tid) * C0);
+                if (tid < t.w)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) g[k] = e[k];
+                if (tid + EM < t.w)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) g[EM * C0 / 8 + k] = u32x4{};
+            }
         }
         // validity of this lane's four rows (row wr * 128 + 32 j + lane % 32)
         uint32_t valid = 0;
 #pragma unroll
         for (uint32_t j = 0; j < 4; ++j) {
             const uint32_t row = wr * 128 + 32 * j + (lane & 31u);
-            uint32_t lo = 0, hi = cnt;
-            while (lo + 1 < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (s_row[mid] <= row) lo = mid; else hi = mid;
-            }
+            const uint32_t lo = seq_of_row(s_row, cnt, row);
             if (row - s_row[lo] < s_len[lo]) valid |= 1u << j;
         }
         __syncthreads();
@@ -788,6 +396,7 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
             if (l == 0) enc_conv<C0>(Xw, wp, lane, acc);
             else enc_conv<C>(Xw, wp + (EKS1 + (l - 1) * EKS) * 256, lane, acc);
             __syncthreads();  // every wave has read the layer's input
+            uint2 *h = TRAIN ? a.H[l] + (size_t)ti * 8192 + wave * 2048 + lane : nullptr;
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -796,8 +405,12 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
                     const float4 b = *(const float4 *)(bias + l * C + ch);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const float g0 = gelu(acc[i][j][4 * q] + b.x), g1 = gelu(acc[i][j][4 * q + 1] + b.y),
-                                    g2 = gelu(acc[i][j][4 * q + 2] + b.z), g3 = gelu(acc[i][j][4 * q + 3] + b.w);
+                        const float x0 = acc[i][j][4 * q] + b.x, x1 = acc[i][j][4 * q + 1] + b.y,
+                                    x2 = acc[i][j][4 * q + 2] + b.z, x3 = acc[i][j][4 * q + 3] + b.w;
+                        if (TRAIN)
+                            h[((i * 4 + j) * 4 + q) * 64] = make_uint2((uint32_t)f2bf(x0) | ((uint32_t)f2bf(x1) << 16),
+                                                                       (uint32_t)f2bf(x2) | ((uint32_t)f2bf(x3) << 16));
+                        const float g0 = gelu(x0), g1 = gelu(x1), g2 = gelu(x2), g3 = gelu(x3);
                         const bool v = (valid >> j) & 1u;
                         uint2 o;
                         o.x = v ? (uint32_t)f2bf(g0) | ((uint32_t)f2bf(g1) << 16) : 0u;
@@ -806,6 +419,7 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
                     }
                 }
             __syncthreads();
+            if (TRAIN && l < 2) enc_store_rows(X, (l ? a.A2 : a.A1) + (size_t)t.z * C, t.w, tid);
         }
         // head, EGRP sequences a round: mean over the letters (a wave per
         // sequence, two channels per lane), projection, L2 norm
@@ -826,6 +440,7 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
                     a0 *= inv;
                     a1 *= inv;
                     *(float2 *)(&sp[r * 4 + wave][2 * lane]) = make_float2(a0, a1);
+                    if (TRAIN) *(float2 *)(a.pool + (size_t)(first + s) * C + 2 * lane) = make_float2(a0, a1);
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -856,10 +471,524 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
                 if (s < cnt) {
                     if (a.z) a.z[(size_t)(first + s) * D + lane] = zz;
                     if (a.zb) a.zb[(size_t)(first + s) * D + lane] = f2bf(zz);
+                    if (TRAIN && lane == 0) a.nrm[first + s] = nrm;
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Training: loss and head, data gradients, weight gradients, their sums.
+
+constexpr uint32_t HP = 16;                        // pairs per round of the head's backward pass
+constexpr uint32_t HPART = D * C + D + 4;          // one block's projection gradients and loss
+constexpr uint32_t HBLOCKS = 128;                  // most blocks of the head's backward pass
+constexpr uint32_t BPART = NTOK * C0 + 3 * C;      // one block's embedding and bias gradients
+
+// Contrastive loss of pair i (sequences 2i, 2i+1), back through the norm and
+// the projection to the pooled means (dp, already divided by the length), and
+// the projection's gradients.  A wave takes four pairs of a round of HP; the
+// block then adds the round's du x pool into 32 accumulators per thread.
+// Latency-bound (4,096 pairs are one or two rounds a block); the sums over
+// pairs stay in registers and leave as one partial per block, since one atomic
+// word per pair (the loss) took 49 us.  With the three kernels it replaces:
+// 4,096 pairs 306 -> 37 us.
+__global__ __launch_bounds__(256) void k_pair_head(const float *z, const float *nrm, const float *pool,
+                                                   const uint32_t *blen, const float *y, uint32_t npairs, float margin,
+                                                   float inv_b, const uint32_t *wp2, float *dp, float *part)
+{
+    __shared__ __align__(16) float sdu[2 * HP][D];
+    __shared__ __align__(16) float spool[2 * HP][C];
+    __shared__ uint32_t swp[D][C / 2 + 1];  // (output, input pair)
+    __shared__ float sloss[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    for (uint32_t i = tid; i < D * C / 2; i += 256) swp[i % D][i / D] = wp2[i];
+    float acc[4][8] = {}, accb = 0.f, lsum = 0.f;
+    const uint32_t tj = (tid >> 4) * 4, to = (tid & 15u) * 8;
+    for (uint32_t p0 = blockIdx.x * HP; p0 < npairs; p0 += gridDim.x * HP) {
+        __syncthreads();
+        const uint32_t ns = min(2 * HP, 2 * (npairs - p0));  // sequences of this round
+        for (uint32_t i = tid; i < 2 * HP * C / 4; i += 256) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (i / (C / 4) < ns) v = *(const float4 *)(pool + (size_t)2 * p0 * C + 4 * i);
+            *(float4 *)(&spool[0][0] + 4 * i) = v;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < HP / 4; ++k) {
+            const uint32_t q = w * (HP / 4) + k, i = p0 + q;
+            float du0 = 0.f, du1 = 0.f;
+            if (i < npairs) {
+                const float yi = y[i], z0 = z[(size_t)(2 * i) * D + lane], z1 = z[(size_t)(2 * i + 1) * D + lane];
+                const float n0 = nrm[2 * i], n1 = nrm[2 * i + 1], diff = z0 - z1;
+                float d2 = diff * diff;
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) d2 += __shfl_xor(d2, o, 64);
+                const float d = sqrtf(d2 + 1e-12f), hinge = fmaxf(0.f, margin - d);
+                lsum += yi * d2 + (1.f - yi) * hinge * hinge;
+                const float g = (2.f * yi - (1.f - yi) * 2.f * hinge / d) * inv_b * diff;  // dz0 = g, dz1 = -g
+                float a = z0 * g, b = z1 * g;
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) {
+                    a += __shfl_xor(a, o, 64);
+                    b += __shfl_xor(b, o, 64);
+                }
+                du0 = (g - z0 * a) / n0;
+                du1 = (z1 * b - g) / n1;
+            }
+            sdu[2 * q][lane] = du0;
+            sdu[2 * q + 1][lane] = du1;
+        }
+        __syncthreads();
+        // dp of this wave's eight sequences, two channels per lane
+        {
+            float d0[HP / 2] = {}, d1[HP / 2] = {};
+#pragma unroll 4
+            for (uint32_t j = 0; j < D; j += 4) {
+                uint32_t v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = swp[j + k][lane];
+#pragma unroll
+                for (uint32_t s = 0; s < HP / 2; ++s) {
+                    const float4 u = *(const float4 *)(&sdu[w * (HP / 2) + s][j]);
+                    const float uu[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        d0[s] += bf2f((uint16_t)v[k]) * uu[k];
+                        d1[s] += bf2f((uint16_t)(v[k] >> 16)) * uu[k];
+                    }
+                }
+            }
+#pragma unroll
+            for (uint32_t s = 0; s < HP / 2; ++s) {
+                const uint32_t q = w * (HP / 2) + s;
+                if (q < ns) {
+                    const uint32_t L = blen[2 * p0 + q];
+                    const float inv = L ? 1.f / (float)L : 0.f;
+                    *(float2 *)(dp + (size_t)(2 * p0 + q) * C + 2 * lane) = make_float2(d0[s] * inv, d1[s] * inv);
+                }
+            }
+        }
+#pragma unroll 4
+        for (uint32_t s = 0; s < 2 * HP; ++s) {
+            const float4 u = *(const float4 *)(&sdu[s][tj]);
+            const float4 a = *(const float4 *)(&spool[s][to]), b = *(const float4 *)(&spool[s][to + 4]);
+            const float uu[4] = {u.x, u.y, u.z, u.w}, pp[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int o = 0; o < 8; ++o) acc[i][o] += uu[i] * pp[o];
+            if (tid < D) accb += sdu[s][tid];
+        }
+    }
+    float *out = part + (size_t)blockIdx.x * HPART;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int o = 0; o < 8; o += 4)
+            *(float4 *)(out + (tj + i) * C + to + o) =
+                make_float4(acc[i][o], acc[i][o + 1], acc[i][o + 2], acc[i][o + 3]);
+    if (tid < D) out[D * C + tid] = accb;
+    if (lane == 0) sloss[w] = lsum;
+    __syncthreads();
+    if (tid < 4) out[D * C + D + tid] = sloss[tid] * inv_b;
+}
+
+struct BwdArgs {
+    const uint8_t *seq;
+    const uint64_t *off;
+    const uint32_t *rows, *len;   // row and length of each sequence
+    const uint4 *tiles;
+    const uint32_t *n_tiles;
+    const uint16_t *rstart;
+    const uint8_t *vocab;
+    const uint16_t *pack;         // transposed weights (k_enc_pack)
+    const uint2 *H[3];
+    const float *dp;
+    uint16_t *dH[3];              // out: pre-activation gradients, packed rows
+    float *part;                  // out: BPART sums per block
+};
+
+// Packed rows [0, used) of a pre-activation gradient to HBM, and its column
+// sums (the bias gradient) into sb.
+__device__ __forceinline__ void bwd_store_rows(const uint16_t *X, uint16_t *out, uint32_t used, uint32_t tid, float *sb)
+{
+    float sum[8] = {};
+    for (uint32_t r = tid >> 4; r < used; r += 16) {
+        const u32x4 v = *(const u32x4 *)(X + (r + 2) * EST + (tid & 15u) * 8);
+        *(u32x4 *)(out + (size_t)r * C + (tid & 15u) * 8) = v;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            sum[2 * k] += bf2f((uint16_t)v[k]);
+            sum[2 * k + 1] += bf2f((uint16_t)(v[k] >> 16));
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        sum[k] += __shfl_xor(sum[k], 16, 64);
+        sum[k] += __shfl_xor(sum[k], 32, 64);
+        if ((tid & 63u) < 16u) atomicAdd(&sb[(tid & 15u) * 8 + k], sum[k]);
+    }
+}
+
+// Four gradients times the GELU's derivative at four saved pre-activations,
+// as bfloat16; zero where the row is no letter.
+__device__ __forceinline__ uint2 times_grad(float a, float b, float c, float d, uint2 h, bool v)
+{
+    const float g0 = a * gelu_grad(bf2f((uint16_t)h.x)), g1 = b * gelu_grad(bf2f((uint16_t)(h.x >> 16))),
+                g2 = c * gelu_grad(bf2f((uint16_t)h.y)), g3 = d * gelu_grad(bf2f((uint16_t)(h.y >> 16)));
+    return make_uint2(v ? (uint32_t)f2bf(g0) | ((uint32_t)f2bf(g1) << 16) : 0u,
+                      v ? (uint32_t)f2bf(g2) | ((uint32_t)f2bf(g3) << 16) : 0u);
+}
+
+// Data gradients of a tile, in LDS as in k_encode (same tiles, same lane
+// mapping): dH3 from dp, then each layer's transposed convolution times the
+// GELU's derivative at the saved pre-activation, and the first layer's input
+// gradient added per token.  Gradients leave for k_wgrad row by row; bias and
+// embedding sums stay in LDS over a block's tiles.
+// MFMA-bound like k_encode.  4,096 pairs of protein rows: head's last part,
+// three data-gradient products, three bias sums and the embedding scatter
+// took 870 us as eight launches over padded rows; 204 us here.
+__global__ __launch_bounds__(256, 2) void k_enc_bwd(BwdArgs a)
+{
+    __shared__ __align__(16) uint16_t X[(EM + 4) * EST];
+    __shared__ float semb[C0 * (NTOK + 1)];  // [channel][token]
+    __shared__ float sbias[3 * C];
+    __shared__ uint32_t s_len[EM / 2 + 2], s_seq[EM / 2 + 2];
+    __shared__ uint16_t s_row[EM / 2 + 2];
+    __shared__ uint8_t s_tok[EM];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t wc = wave & 1u, wr = wave >> 1;
+    for (uint32_t i = tid; i < C0 * (NTOK + 1); i += 256) semb[i] = 0.f;
+    for (uint32_t i = tid; i < 3 * C; i += 256) sbias[i] = 0.f;
+    for (uint32_t i = tid; i < 4 * EST; i += 256) X[(i < 2 * EST ? 0 : EM * EST) + i] = 0;
+    const uint32_t nt = *a.n_tiles;
+    for (uint32_t ti = blockIdx.x; ti < nt; ti += gridDim.x) {
+        const uint4 t = a.tiles[ti];
+        const uint32_t first = t.x, cnt = t.y;
+        __syncthreads();
+        if (tid < cnt) {
+            s_len[tid] = a.len[first + tid];
+            s_row[tid] = a.rstart[first + tid];
+            s_seq[tid] = a.rows[first + tid];
+        }
+        __syncthreads();
+        {
+            const uint32_t q = seq_of_row(s_row, cnt, tid), p = tid - s_row[q];
+            s_tok[tid] = p < s_len[q] ? a.vocab[a.seq[a.off[s_seq[q]] + p]] : (uint8_t)255;
+        }
+        uint32_t valid = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t row = wr * 128 + 32 * j + (lane & 31u);
+            const uint32_t q = seq_of_row(s_row, cnt, row);
+            const bool v = row - s_row[q] < s_len[q];
+            if (v) valid |= 1u << j;
+            const float *dp = a.dp + (size_t)(first + q) * C + wc * 64 + 4 * (lane >> 5);
+            const uint2 *h = a.H[2] + (size_t)ti * 8192 + wave * 2048 + lane;
+            uint16_t *x = X + (2 + row) * EST + wc * 64 + 4 * (lane >> 5);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q2 = 0; q2 < 4; ++q2) {
+                    const uint2 hv = h[((i * 4 + j) * 4 + q2) * 64];
+                    const float4 d = *(const float4 *)(dp + i * 32 + 8 * q2);
+                    *(uint2 *)(x + i * 32 + 8 * q2) = times_grad(d.x, d.y, d.z, d.w, hv, v);
+                }
+        }
+        __syncthreads();
+        const uint16_t *Xw = X + wr * 128 * EST;
+        const u32x4 *wp = (const u32x4 *)a.pack + wc * 128 + lane;
+#pragma unroll 1
+        for (int l = 1; l >= 0; --l) {
+            bwd_store_rows(X, a.dH[l + 1] + (size_t)t.z * C, t.w, tid, sbias + (l + 1) * C);
+            f32x16 acc[2][4];
+            enc_conv<C, true>(Xw, wp + (1 - l) * (BLAYER / 8), lane, acc);
+            __syncthreads();  // every wave has read the layer's gradient
+            const uint2 *h = a.H[l] + (size_t)ti * 8192 + wave * 2048 + lane;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool v = (valid >> j) & 1u;
+                uint16_t *x = X + (2 + wr * 128 + 32 * j + (lane & 31u)) * EST + wc * 64 + 4 * (lane >> 5);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int q2 = 0; q2 < 4; ++q2)
+                        *(uint2 *)(x + i * 32 + 8 * q2) =
+                            times_grad(acc[i][j][4 * q2], acc[i][j][4 * q2 + 1], acc[i][j][4 * q2 + 2],
+                                       acc[i][j][4 * q2 + 3], h[((i * 4 + j) * 4 + q2) * 64], v);
+            }
+            __syncthreads();
+        }
+        bwd_store_rows(X, a.dH[0] + (size_t)t.z * C, t.w, tid, sbias);
+        // input gradient: 32 channels of this wave's 64 rows
+        f32x16 g[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) g[j][r] = 0.f;
+        const uint16_t *xr = X + (wave * 64 + (lane & 31u)) * EST + (lane >> 5) * 8;
+        const u32x4 *w1 = (const u32x4 *)a.pack + 2 * (BLAYER / 8) + lane;
+#pragma unroll 1
+        for (uint32_t tp = 0; tp < T; ++tp)
+#pragma unroll
+            for (uint32_t c = 0; c < C / 16; ++c) {
+                const bf16x8 w = __builtin_bit_cast(bf16x8, w1[(tp * (C / 16) + c) * 64]);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    g[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        w, *(const bf16x8 *)(xr + (T - 1 - tp + j * 32) * EST + c * 16), g[j], 0, 0, 0);
+            }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t tok = s_tok[wave * 64 + 32 * j + (lane & 31u)];
+            if (tok != 255u)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    atomicAdd(&semb[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * (NTOK + 1) + tok], g[j][r]);
+        }
+    }
+    __syncthreads();
+    float *out = a.part + (size_t)blockIdx.x * BPART;
+    for (uint32_t i = tid; i < NTOK * C0; i += 256) out[i] = semb[(i % C0) * (NTOK + 1) + i / C0];
+    for (uint32_t i = tid; i < 3 * C; i += 256) out[NTOK * C0 + i] = sbias[i];
+}
+
+// Weight gradients: dW[o][t][c] = sum over packed rows m of dH[m][o] X[m + t - 2][c]
+// (the zero rows between sequences make every window plain row offsets).  A
+// block owns 128 outputs x 64 channels x 5 taps of layer 3 or 2, or all of
+// layer 1, over one split of the rows: 10 MFMA tiles per wave, so that 7
+// fragments from LDS feed 10 products and a row is read 2.25 times.  Operands
+// have the rows as their inner dimension: fragments come by transposing LDS
+// reads of row-major chunks of 64 rows, a tap being a row offset.  Two groups
+// of four waves take the chunks in turn and add their sums at the end, which
+// halves the partial sums (k_train_sum adds the splits; atomics on one copy
+// of the gradients queue).
+// 4,096 pairs of protein rows (139k packed rows), three layers: 1,263 us as
+// im2col products over padded rows with transposing LDS stores and atomics,
+// 66 us here (780 TFLOP/s).
+constexpr uint32_t WROWS = 64, WA = C + 32, WB = 64 + 32;  // rows per chunk; LDS row strides
+constexpr uint32_t WPART = 4 * 10 * 16 * 64;               // sums of a block (layer 1: two halves)
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+constexpr size_t WLDS = sizeof(uint16_t) * 4 * (WROWS * WA + (WROWS + 4) * WB);  // two groups, two buffers
+
+struct WgradArgs {
+    const uint16_t *dH[3], *X[3];
+    const uint32_t *total;  // packed rows
+    uint32_t ns, ns1;       // splits of the rows for layers 3 and 2, for layer 1
+    float *part;            // [4 units x ns, then ns1][WPART]
+};
+
+// 32 x 16 fragment of a row-major LDS matrix, transposed: lane l gets column
+// c + l % 32, rows r + 8 (l / 32) .. + 7.  A transposing read takes four rows
+// of 16 columns per group of 16 lanes.
+template <uint32_t ST>
+__device__ __forceinline__ bf16x8 tr_frag(const uint16_t *lds, uint32_t r, uint32_t c, uint32_t lane)
+{
+    typedef __attribute__((address_space(3))) s16x4 lds4;
+    const uint16_t *p = lds + (r + (lane >> 5) * 8 + ((lane & 15u) >> 2)) * ST + c + ((lane >> 4) & 1u) * 16 + (lane & 3u) * 4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)p);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)(p + 4 * ST));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+__global__ __launch_bounds__(512, 2) void k_wgrad(WgradArgs a)
+{
+    extern __shared__ __align__(16) uint16_t wl[];
+    constexpr uint32_t BUF = WROWS * WA + (WROWS + 4) * WB;
+    const uint32_t tid = threadIdx.x & 255u, grp = threadIdx.x >> 8, lane = tid & 63u, w = tid >> 6;
+    const bool l1 = blockIdx.x >= 4 * a.ns;
+    const uint32_t u = l1 ? 4u : blockIdx.x / a.ns, split = l1 ? blockIdx.x - 4 * a.ns : blockIdx.x % a.ns;
+    const uint32_t layer = l1 ? 0u : 2u - (u >> 1), c0 = l1 ? 0u : (u & 1u) * 64, ldx = l1 ? C0 : C;
+    const uint32_t xw = l1 ? 4u : 8u;  // 16-byte words of an X row that this block takes
+    const uint16_t *dH = a.dH[layer], *Xg = a.X[layer] + c0;
+    const uint32_t M = *a.total;
+    const uint32_t per = ((M + (l1 ? a.ns1 : a.ns) - 1) / (l1 ? a.ns1 : a.ns) + 2 * WROWS - 1) / (2 * WROWS);  // chunk pairs
+    const uint64_t b0 = (uint64_t)split * per * (2 * WROWS);
+    const uint32_t m_end = (uint32_t)min((uint64_t)M, b0 + (uint64_t)per * (2 * WROWS));  // rows of this split
+    uint16_t *base = wl + grp * 2 * BUF;
+    const uint32_t wo = (w >> 1) * 64, wx = l1 ? 0u : (w & 1u) * 32;
+    f32x16 acc[2][T];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (uint32_t t = 0; t < T; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][t][r] = 0.f;
+    u32x4 ra[4], rb[3];
+    const auto fetch = [&](uint32_t it) {
+        const uint64_t m0 = b0 + (uint64_t)(2 * it + grp) * WROWS;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint64_t m = m0 + (tid >> 4) + 16 * k;
+            ra[k] = u32x4{};
+            if (m < m_end) ra[k] = *(const u32x4 *)(dH + m * C + (tid & 15u) * 8);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k) {
+            const uint32_t i = tid + 256 * k, r = i / xw;
+            const uint64_t m = m0 + r;  // row + 2
+            rb[k] = u32x4{};
+            if (r < WROWS + 4 && m >= 2 && m - 2 < M) rb[k] = *(const u32x4 *)(Xg + (m - 2) * ldx + (i % xw) * 8);
+        }
+    };
+    const auto stage = [&](uint16_t *buf) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) *(u32x4 *)(buf + ((tid >> 4) + 16 * k) * WA + (tid & 15u) * 8) = ra[k];
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k) {
+            const uint32_t i = tid + 256 * k, r = i / xw;
+            if (r < WROWS + 4) *(u32x4 *)(buf + WROWS * WA + r * WB + (i % xw) * 8) = rb[k];
+        }
+    };
+    const uint32_t n_it = b0 >= M ? 0u : (uint32_t)((m_end - b0 + 2 * WROWS - 1) / (2 * WROWS));
+    if (n_it) {
+        fetch(0);
+        stage(base);
+        if (n_it > 1) fetch(1);
+    }
+    __syncthreads();
+    for (uint32_t it = 0; it < n_it; ++it) {
+        if (it + 1 < n_it) stage(base + ((it + 1) & 1u) * BUF);
+        if (it + 2 < n_it) fetch(it + 2);
+        const uint16_t *A = base + (it & 1u) * BUF, *B = A + WROWS * WA;
+#pragma unroll
+        for (uint32_t ks = 0; ks < WROWS / 16; ++ks) {
+            if (l1 && ((ks ^ w) & 1u)) continue;  // layer 1: two waves share an output tile
+            const bf16x8 f0 = tr_frag<WA>(A, ks * 16, wo, lane), f1 = tr_frag<WA>(A, ks * 16, wo + 32, lane);
+#pragma unroll
+            for (uint32_t t = 0; t < T; ++t) {
+                const bf16x8 x = tr_frag<WB>(B, ks * 16 + t, wx, lane);
+                acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f0, x, acc[0][t], 0, 0, 0);
+                acc[1][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1, x, acc[1][t], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    // the second group's sums through LDS, five tiles at a time
+    float4 *sx = (float4 *)wl;
+    float4 *out = (float4 *)(a.part + (size_t)blockIdx.x * WPART);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (grp == 1)
+#pragma unroll
+            for (uint32_t t = 0; t < T; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    sx[((w * T + t) * 4 + q) * 64 + lane] =
+                        make_float4(acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]);
+        __syncthreads();
+        if (grp == 0)
+#pragma unroll
+            for (uint32_t t = 0; t < T; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 v = sx[((w * T + t) * 4 + q) * 64 + lane];
+                    out[((w * 10 + i * T + t) * 4 + q) * 64 + lane] =
+                        make_float4(acc[i][t][4 * q] + v.x, acc[i][t][4 * q + 1] + v.y, acc[i][t][4 * q + 2] + v.z,
+                                    acc[i][t][4 * q + 3] + v.w);
+                }
+        __syncthreads();
+    }
+}
+
+// Sums of the partials into the flat gradient (and the loss): 16 columns of
+// four floats by 16 row groups per block.  Bound by reading the partials
+// (4,096 protein pairs: 46 MB, 15 us).
+struct SumArgs {
+    const float *wpart, *hpart, *bpart;
+    uint32_t ns, ns1, hblocks, bblocks;
+    float *grad, *loss;
+};
+constexpr uint32_t SUM_W = 4 * WPART / 64, SUM_W1 = WPART / 128, SUM_H = (HPART + 63) / 64, SUM_B = BPART / 64;
+static_assert(BPART % 64 == 0 && HPART % 4 == 0 && WPART % 64 == 0, "sum blocks");
+
+__global__ __launch_bounds__(256) void k_train_sum(SumArgs a)
+{
+    __shared__ float4 sh[16][16];
+    const uint32_t col = threadIdx.x & 15u, row = threadIdx.x >> 4;
+    uint32_t b = blockIdx.x, kind = 0, n, c4, unit = 0;
+    size_t stride;
+    const float *src;
+    if (b < SUM_W) {
+        unit = b / (WPART / 64);
+        c4 = (b % (WPART / 64)) * 16 + col;
+        src = a.wpart + (size_t)unit * a.ns * WPART;
+        n = a.ns;
+        stride = WPART;
+    } else if ((b -= SUM_W) < SUM_W1) {
+        // two waves of a block hold the sums of the same outputs
+        kind = 1;
+        c4 = b * 16 + col;
+        c4 += c4 / 2560u * 2560u;
+        src = a.wpart + (size_t)4 * a.ns * WPART;
+        n = 2 * a.ns1;
+        stride = WPART;
+    } else if ((b -= SUM_W1) < SUM_H) {
+        kind = 2;
+        c4 = b * 16 + col;
+        src = a.hpart;
+        n = 4 * c4 < HPART ? a.hblocks : 0u;
+        stride = HPART;
+    } else {
+        b -= SUM_H;
+        kind = 3;
+        c4 = b * 16 + col;
+        src = a.bpart;
+        n = a.bblocks;
+        stride = BPART;
+    }
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (uint32_t r = row; r < n; r += 16) {
+        const size_t at = kind == 1 ? (r >> 1) * stride + (r & 1u) * (2560u * 4) : r * stride;
+        const float4 v = *(const float4 *)(src + at + 4 * (size_t)c4);
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+    }
+    sh[row][col] = s;
+    __syncthreads();
+    if (row) return;
+    for (uint32_t r = 1; r < 16; ++r) {
+        const float4 v = sh[r][col];
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+    }
+    const float v[4] = {s.x, s.y, s.z, s.w};
+    if (kind < 2) {
+        // word c4 of a block's sums: wave, tile, quarter, lane
+        const uint32_t lane = c4 & 63u, q = (c4 >> 6) & 3u, tile = (c4 >> 8) % 10u, w = (c4 >> 8) / 10u;
+        const uint32_t o = (w >> 1) * 64 + (tile / T) * 32 + 8 * q + 4 * (lane >> 5), t = tile % T;
+        if (kind == 0) {
+            const uint32_t c = (unit & 1u) * 64 + (w & 1u) * 32 + (lane & 31u);
+            float *g = a.grad + (unit < 2 ? O_W3 : O_W2) + (size_t)o * (T * C) + t * C + c;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) g[k * T * C] = v[k];
+        } else {
+            float *g = a.grad + O_W1 + (size_t)o * (T * C0) + t * C0 + (lane & 31u);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) g[k * T * C0] = v[k];
+        }
+    } else if (kind == 2) {
+        if (4 * c4 < D * C + D) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) a.grad[O_WP + 4 * c4 + k] = v[k];
+        } else if (4 * c4 < HPART) {
+            *a.loss = (v[0] + v[1]) + (v[2] + v[3]);
+        }
+    } else {
+        const uint32_t at = 4 * c4;
+        const uint32_t l = (at - NTOK * C0) / C, dst = at < NTOK * C0 ? O_EMB + at
+                                                   : (l == 0 ? O_B1 : (l == 1 ? O_B2 : O_B3)) + (at - NTOK * C0) % C;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a.grad[dst + k] = v[k];
     }
 }
 
@@ -892,34 +1021,32 @@ struct idb_encoder {
     uint8_t vocab[256];
     float *theta = nullptr, *grad = nullptr, *mom1 = nullptr, *mom2 = nullptr;
     uint16_t *theta_b = nullptr;
-    uint16_t *wt[3] = {nullptr, nullptr, nullptr};  // transposed conv weights for data gradients
     uint32_t adam_step = 0;
     std::string err;
-    // workspace
+    // workspace of a training step
     uint32_t cap_seq = 0;
-    uint8_t *btok = nullptr;
     uint32_t *blen = nullptr, *brows = nullptr;
-    uint16_t *X0 = nullptr, *A[3] = {nullptr, nullptr, nullptr}, *H[3] = {nullptr, nullptr, nullptr};
-    uint16_t *dHa = nullptr, *dHb = nullptr;
-    float *dX0 = nullptr, *pool = nullptr, *u = nullptr, *z = nullptr, *dz = nullptr, *du = nullptr, *y = nullptr;
+    uint16_t *X0 = nullptr, *A[2] = {nullptr, nullptr}, *dH[3] = {nullptr, nullptr, nullptr};
+    uint2 *H[3] = {nullptr, nullptr, nullptr};
+    float *pool = nullptr, *z = nullptr, *nrm = nullptr, *dp = nullptr, *y = nullptr;
+    float *wpart = nullptr, *hpart = nullptr, *bpart = nullptr;  // partial sums
+    uint4 *ttiles = nullptr;
+    uint16_t *trstart = nullptr;
     float *loss = nullptr;
-    // tokens of the last dataset (kept apart from the batch workspace)
-    uint8_t *tok = nullptr;
-    uint32_t *tlen = nullptr;
-    uint32_t tok_cap = 0;
     uint8_t *vocab_d = nullptr;
     // inference: weights in the fused kernel's order (packed again when the
     // parameters have changed), and the packing of the current rows
     uint16_t *pack = nullptr;
+    uint16_t *bpack = nullptr;
     uint32_t *wp2 = nullptr;
     bool pack_stale = true;
-    uint2 *tiles = nullptr;
+    uint4 *tiles = nullptr;
     uint16_t *rstart = nullptr;
     uint32_t *n_tiles = nullptr;
     uint32_t plan_cap = 0;
     float *zbuf = nullptr;
     uint32_t zbuf_cap = 0;
-    uint32_t enc_blocks = 0;
+    uint32_t enc_blocks = 0, cus = 1;
     std::vector<void *> fixed, ws;  // parameter and workspace allocations
 };
 
@@ -941,42 +1068,79 @@ void free_workspace(idb_encoder *e)
     e->cap_seq = 0;
 }
 
-// Workspace of a training step over nseq sequences.
+// Workspace of a training step over nseq sequences (an even number).  A
+// window's tiles hold at least EM + 2 over P + 2 sequences each but its last.
+constexpr uint32_t WSPLITS = 56;  // splits of the rows: 4 x 56 + 28 blocks fill 256 CUs
+
+uint32_t tile_capacity(uint32_t nseq, uint32_t P)
+{
+    const uint32_t windows = (nseq + EPW - 1) / EPW;
+    return std::min(nseq, nseq / ((EM + 2) / (P + 2)) + windows);
+}
+
 void ensure_workspace(idb_encoder *e, uint32_t nseq)
 {
     if (nseq <= e->cap_seq) return;
     free_workspace(e);
-    const size_t M = (size_t)nseq * e->P;
-    e->btok = dalloc<uint8_t>(e->ws, M);
+    const size_t M = (size_t)nseq * (e->P + 2), nt = tile_capacity(nseq, e->P);
     e->blen = dalloc<uint32_t>(e->ws, nseq);
     e->brows = dalloc<uint32_t>(e->ws, nseq);
     e->X0 = dalloc<uint16_t>(e->ws, M * C0);
+    for (int l = 0; l < 2; ++l) e->A[l] = dalloc<uint16_t>(e->ws, M * C);
     for (int l = 0; l < 3; ++l) {
-        e->A[l] = dalloc<uint16_t>(e->ws, M * C);
-        e->H[l] = dalloc<uint16_t>(e->ws, M * C);
+        e->dH[l] = dalloc<uint16_t>(e->ws, M * C);
+        e->H[l] = dalloc<uint2>(e->ws, nt * 8192);
     }
     e->pool = dalloc<float>(e->ws, (size_t)nseq * C);
-    e->u = dalloc<float>(e->ws, (size_t)nseq * D);
     e->z = dalloc<float>(e->ws, (size_t)nseq * D);
-    e->dHa = dalloc<uint16_t>(e->ws, M * C);
-    e->dHb = dalloc<uint16_t>(e->ws, M * C);
-    e->dX0 = dalloc<float>(e->ws, M * C0);
-    e->dz = dalloc<float>(e->ws, (size_t)nseq * D);
-    e->du = dalloc<float>(e->ws, (size_t)nseq * D);
-    e->y = dalloc<float>(e->ws, nseq / 2 + 1);
-    e->loss = dalloc<float>(e->ws, 1);
+    e->nrm = dalloc<float>(e->ws, nseq);
+    e->dp = dalloc<float>(e->ws, (size_t)nseq * C);
+    e->y = dalloc<float>(e->ws, nseq / 2);
+    e->ttiles = dalloc<uint4>(e->ws, nt);
+    e->trstart = dalloc<uint16_t>(e->ws, nseq);
     e->cap_seq = nseq;
 }
 
-void refresh_transposed(idb_encoder *e)
+// The packed weights of the current parameters, on e->stream.
+void ensure_pack(idb_encoder *e)
 {
-    const uint32_t cins[3] = {C0, C, C};
-    const uint32_t offs[3] = {O_W1, O_W2, O_W3};
-    for (int l = 0; l < 3; ++l)
-        hipLaunchKernelGGL(k_transpose_w, dim3(nblocks((size_t)C * T * cins[l])), dim3(256), 0, e->stream,
-                           e->theta_b + offs[l], cins[l], e->wt[l]);
-    hcheck(hipGetLastError(), "transpose launch");
-    e->pack_stale = true;
+    if (!e->pack) {
+        // (fragments are read ahead past a pack's end)
+        uint16_t *pack = dalloc<uint16_t>(e->fixed, EPACK + EPAD);
+        e->bpack = dalloc<uint16_t>(e->fixed, BPACK + EPAD);
+        e->wp2 = dalloc<uint32_t>(e->fixed, C / 2 * D);
+        e->n_tiles = dalloc<uint32_t>(e->fixed, 2);
+        hcheck(hipMemsetAsync(pack, 0, (EPACK + EPAD) * sizeof(uint16_t), e->stream), "memset");
+        hcheck(hipMemsetAsync(e->bpack, 0, (BPACK + EPAD) * sizeof(uint16_t), e->stream), "memset");
+        int dev = 0, cus = 0, per_cu = 0;
+        hcheck(hipGetDevice(&dev), "device");
+        hcheck(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device");
+        hcheck(hipFuncSetAttribute((const void *)k_wgrad, hipFuncAttributeMaxDynamicSharedMemorySize, (int)WLDS), "wgrad LDS");
+        hcheck(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_encode<false>, 256, 0), "occupancy");
+        e->cus = (uint32_t)std::max(cus, 1);
+        e->enc_blocks = (uint32_t)std::max(per_cu, 1) * e->cus;
+        e->pack = pack;
+    }
+    if (e->pack_stale) {
+        hipLaunchKernelGGL(k_enc_pack, dim3(256), dim3(256), 0, e->stream, e->theta_b, e->pack, e->wp2, e->bpack);
+        e->pack_stale = false;
+    }
+}
+
+void enc_args(const idb_encoder *e, EncArgs &a, const uint8_t *seq, const uint64_t *off, const uint32_t *len,
+              const uint4 *tiles, const uint16_t *rstart)
+{
+    a.seq = seq;
+    a.off = off;
+    a.len = len;
+    a.tiles = tiles;
+    a.n_tiles = e->n_tiles;
+    a.rstart = rstart;
+    a.vocab = e->vocab_d;
+    a.theta_b = e->theta_b;
+    a.pack = e->pack;
+    a.wp2 = e->wp2;
+    a.P = e->P;
 }
 
 // Embeddings of rows [0, n) of device data by the fused kernel, on e->stream:
@@ -986,23 +1150,7 @@ void embed_fused(idb_encoder *e, const uint8_t *seq, const uint64_t *off, const 
 {
     if (n == 0) return;
     hipStream_t s = e->stream;
-    if (!e->pack) {
-        // (AHEAD fragments are read past the last layer's end)
-        uint16_t *pack = dalloc<uint16_t>(e->fixed, EPACK + 2 * 2048);
-        e->wp2 = dalloc<uint32_t>(e->fixed, C / 2 * D);
-        e->n_tiles = dalloc<uint32_t>(e->fixed, 1);
-        hcheck(hipMemsetAsync(pack, 0, (EPACK + 2 * 2048) * sizeof(uint16_t), s), "memset");
-        int dev = 0, cus = 0, per_cu = 0;
-        hcheck(hipGetDevice(&dev), "device");
-        hcheck(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device");
-        hcheck(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_encode, 256, 0), "occupancy");
-        e->enc_blocks = (uint32_t)(std::max(per_cu, 1) * cus);
-        e->pack = pack;
-    }
-    if (e->pack_stale) {
-        hipLaunchKernelGGL(k_enc_pack, dim3(256), dim3(256), 0, s, e->theta_b, e->pack, e->wp2);
-        e->pack_stale = false;
-    }
+    ensure_pack(e);
     if (n > e->plan_cap) {
         hcheck(hipStreamSynchronize(s), "sync");
         (void)hipFree(e->tiles);
@@ -1010,108 +1158,19 @@ void embed_fused(idb_encoder *e, const uint8_t *seq, const uint64_t *off, const 
         e->tiles = nullptr;
         e->rstart = nullptr;
         e->plan_cap = 0;
-        hcheck(hipMalloc(&e->tiles, sizeof(uint2) * (size_t)n), "hipMalloc");
+        hcheck(hipMalloc(&e->tiles, sizeof(uint4) * (size_t)n), "hipMalloc");
         hcheck(hipMalloc(&e->rstart, sizeof(uint16_t) * (size_t)n), "hipMalloc");
         e->plan_cap = n;
     }
     hcheck(hipMemsetAsync(e->n_tiles, 0, sizeof(uint32_t), s), "memset");
-    hipLaunchKernelGGL(k_enc_plan, dim3((n + EPW - 1) / EPW), dim3(256), 0, s, len, n, e->P, e->tiles, e->n_tiles,
-                       e->rstart);
-    const EncArgs a{seq, off, len, e->tiles, e->n_tiles, e->rstart, e->vocab_d, e->theta_b, e->pack, e->wp2, e->P, z, zb};
-    hipLaunchKernelGGL(k_encode, dim3(std::min(e->enc_blocks, n)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_enc_plan<false>, dim3((n + EPW - 1) / EPW), dim3(256), 0, s, len, n, e->P, e->tiles, e->n_tiles,
+                       e->rstart, PairSource{});
+    EncArgs a{};
+    enc_args(e, a, seq, off, len, e->tiles, e->rstart);
+    a.z = z;
+    a.zb = zb;
+    hipLaunchKernelGGL(k_encode<false>, dim3(std::min(e->enc_blocks, n)), dim3(256), 0, s, a);
     hcheck(hipGetLastError(), "encoder launch");
-}
-
-// Training forward pass over the batch in e->btok / e->blen (nseq, a multiple of 4).
-template <uint32_t PP>
-void forward_p(idb_encoder *e, uint32_t nseq)
-{
-    hipStream_t s = e->stream;
-    const uint32_t M = nseq * PP;
-    hipLaunchKernelGGL(k_embed, dim3(nblocks((size_t)M * C0 / 8)), dim3(256), 0, s, e->btok, e->blen, nseq, PP,
-                       e->theta_b + O_EMB, e->X0);
-    const uint16_t *in = e->X0;
-    uint32_t cin = C0;
-    const uint32_t offs[3] = {O_W1, O_W2, O_W3}, boff[3] = {O_B1, O_B2, O_B3};
-    for (int l = 0; l < 3; ++l) {
-        uint16_t *out = e->A[l];
-        LdConv<PP> la{in, cin, M, 0};
-        LdRows lb{e->theta_b + offs[l], T * cin, C};
-        EpConvFwd<PP> ep{e->theta_b + boff[l], e->blen, e->H[l], out};
-        hipLaunchKernelGGL((k_gemm<LdConv<PP>, LdRows, EpConvFwd<PP>>), dim3((M + GM - 1) / GM, 1, 1), dim3(256), 0, s,
-                           la, lb, ep, M, C, T * cin, T * cin);
-        in = out;
-        cin = C;
-    }
-    hipLaunchKernelGGL(k_head_fwd, dim3(nblocks(nseq, 4)), dim3(256), 0, s, in, e->blen, nseq, PP, e->theta_b + O_WP,
-                       e->theta_b + O_BP, e->pool, e->u, e->z);
-    hcheck(hipGetLastError(), "encoder forward launch");
-}
-
-void forward(idb_encoder *e, uint32_t nseq)
-{
-    if (e->P == 160) forward_p<160>(e, nseq);
-    else forward_p<32>(e, nseq);
-}
-
-// Backward of sum(dz . z) into e->grad (zeroed here).
-template <uint32_t PP>
-void backward_p(idb_encoder *e, uint32_t nseq)
-{
-    hipStream_t s = e->stream;
-    const uint32_t M = nseq * PP;
-    hcheck(hipMemsetAsync(e->grad, 0, sizeof(float) * N_PARAMS, s), "memset");
-    hipLaunchKernelGGL(k_head_bwd, dim3(nblocks(nseq, 4)), dim3(256), 0, s, e->dz, e->z, e->u, e->blen, nseq, PP,
-                       e->theta_b + O_WP, e->H[2], e->du, e->dHa);
-    hipLaunchKernelGGL(k_proj_grad, dim3(D, 64), dim3(C), 0, s, e->du, e->pool, nseq, e->grad + O_WP, e->grad + O_BP);
-    const uint32_t offs[3] = {O_W1, O_W2, O_W3}, boff[3] = {O_B1, O_B2, O_B3}, cins[3] = {C0, C, C};
-    uint16_t *dH = e->dHa, *dHn = e->dHb;
-    // split the weight-gradient reduction over rows into chunks of 4096 rows
-    const uint32_t ks = 4096, nsplit = (M + ks - 1) / ks;
-    for (int l = 2; l >= 0; --l) {
-        const uint32_t cin = cins[l];
-        const uint16_t *Aprev = l ? e->A[l - 1] : e->X0;
-        LdGradT la{dH, M};
-        LdConvT<PP> lb{Aprev, cin, M};
-        EpAtomic ep{e->grad + offs[l], T * cin};
-        hipLaunchKernelGGL((k_gemm<LdGradT, LdConvT<PP>, EpAtomic>), dim3(1, (T * cin + GN - 1) / GN, nsplit), dim3(256),
-                           0, s, la, lb, ep, C, T * cin, M, ks);
-        hipLaunchKernelGGL(k_bias_grad, dim3(2048), dim3(C), 0, s, dH, M, e->grad + boff[l]);
-        LdConv<PP> la2{dH, C, M, 1};
-        LdRows lb2{e->wt[l], T * C, cin};
-        EpConvBwd<PP> ep2{l ? e->H[l - 1] : nullptr, e->blen, cin, l ? dHn : nullptr, l ? nullptr : e->dX0};
-        hipLaunchKernelGGL((k_gemm<LdConv<PP>, LdRows, EpConvBwd<PP>>), dim3((M + GM - 1) / GM, (cin + GN - 1) / GN, 1),
-                           dim3(256), 0, s, la2, lb2, ep2, M, cin, T * C, T * C);
-        std::swap(dH, dHn);
-    }
-    hipLaunchKernelGGL(k_emb_grad, dim3(256), dim3(256), 0, s, e->dX0, e->btok, e->blen, M, PP, e->grad + O_EMB);
-    hcheck(hipGetLastError(), "encoder backward launch");
-}
-
-void backward(idb_encoder *e, uint32_t nseq)
-{
-    if (e->P == 160) backward_p<160>(e, nseq);
-    else backward_p<32>(e, nseq);
-}
-
-void tokenize(idb_encoder *e, const idb_dataset *d)
-{
-    const uint32_t n = d->n_rows;
-    if (d->mem != IDB_MEM_DEVICE) throw Fail{IDB_ERR_ARG, "encoder inputs must be device memory here"};
-    if (n > e->tok_cap) {
-        (void)hipStreamSynchronize(e->stream);
-        (void)hipFree(e->tok);
-        (void)hipFree(e->tlen);
-        e->tok = nullptr;
-        e->tlen = nullptr;
-        e->tok_cap = 0;
-        hcheck(hipMalloc(&e->tok, (size_t)n * e->P), "hipMalloc");
-        hcheck(hipMalloc(&e->tlen, sizeof(uint32_t) * n), "hipMalloc");
-        e->tok_cap = n;
-    }
-    hipLaunchKernelGGL(k_tokenize, dim3(nblocks(n)), dim3(256), 0, e->stream, d->seq, d->off, d->len, n, e->vocab_d,
-                       e->P, e->tok, e->tlen);
-    hcheck(hipGetLastError(), "tokenize launch");
 }
 
 // Device copies of host inputs for the encoder entry points.
@@ -1144,24 +1203,50 @@ const idb_dataset *device_view(const idb_dataset *d, DevData &dd, hipStream_t s)
     return &dd.d;
 }
 
-uint32_t round4(uint32_t n) { return (n + 3u) & ~3u; }
-
-// One training step over pairs [first, first + nb) of the (ordered) pair list.
-float step(idb_encoder *e, const uint32_t *pairs_d, const float *labels_d, const uint32_t *order_d, uint64_t first,
-           uint32_t nb, uint64_t npairs, float margin, float inv_b, bool read_loss)
+// One training step over pairs [first, first + nb) of the (ordered) pair list:
+// the gradient into e->grad, the loss behind it.
+float step(idb_encoder *e, const idb_dataset *d, const uint32_t *pairs_d, const float *labels_d, const uint32_t *order_d,
+           uint64_t first, uint32_t nb, float margin, float inv_b, bool read_loss)
 {
     hipStream_t s = e->stream;
-    const uint32_t nseq = round4(2 * nb);
-    hipLaunchKernelGGL(k_iota_rows, dim3(nblocks(nseq)), dim3(256), 0, s, 0u, 0u, nseq, e->brows);
-    hipLaunchKernelGGL(k_pair_rows, dim3(nblocks(nb)), dim3(256), 0, s, pairs_d, order_d, first, nb, npairs, e->brows,
-                       e->y, labels_d);
-    hipLaunchKernelGGL(k_gather_rows, dim3(nblocks(nseq)), dim3(256), 0, s, e->tok, e->tlen, e->brows, nseq, e->P,
-                       e->btok, e->blen);
-    forward(e, nseq);
-    hcheck(hipMemsetAsync(e->loss, 0, sizeof(float), s), "memset");
-    hcheck(hipMemsetAsync(e->dz, 0, sizeof(float) * (size_t)nseq * D, s), "memset");
-    hipLaunchKernelGGL(k_pair_loss, dim3(nblocks(nb, 4)), dim3(256), 0, s, e->z, e->y, nb, margin, inv_b, e->dz, e->loss);
-    backward(e, nseq);
+    const uint32_t nseq = 2 * nb, nt = tile_capacity(nseq, e->P);
+    ensure_pack(e);
+    if (!e->wpart) {
+        e->hpart = dalloc<float>(e->fixed, (size_t)HBLOCKS * HPART);
+        e->bpart = dalloc<float>(e->fixed, (size_t)e->enc_blocks * BPART);
+        e->loss = dalloc<float>(e->fixed, 1);
+        e->wpart = dalloc<float>(e->fixed, (size_t)(4 * WSPLITS + WSPLITS / 2) * WPART);
+    }
+    hcheck(hipMemsetAsync(e->n_tiles, 0, 2 * sizeof(uint32_t), s), "memset");
+    const PairSource ps{pairs_d, order_d, labels_d, first, e->brows, e->blen, e->y};
+    hipLaunchKernelGGL(k_enc_plan<true>, dim3((nseq + EPW - 1) / EPW), dim3(256), 0, s, d->len, nseq, e->P, e->ttiles,
+                       e->n_tiles, e->trstart, ps);
+    EncArgs a{};
+    enc_args(e, a, d->seq, d->off, e->blen, e->ttiles, e->trstart);
+    a.z = e->z;
+    a.rows = e->brows;
+    for (int l = 0; l < 3; ++l) a.H[l] = e->H[l];
+    a.X0 = e->X0;
+    a.A1 = e->A[0];
+    a.A2 = e->A[1];
+    a.pool = e->pool;
+    a.nrm = e->nrm;
+    hipLaunchKernelGGL(k_encode<true>, dim3(std::min(e->enc_blocks, nt)), dim3(256), 0, s, a);
+    const uint32_t hb = std::min(HBLOCKS, (nb + HP - 1) / HP);
+    hipLaunchKernelGGL(k_pair_head, dim3(hb), dim3(256), 0, s, e->z, e->nrm, e->pool, e->blen, e->y, nb, margin, inv_b,
+                       e->wp2, e->dp, e->hpart);
+    BwdArgs b{d->seq, d->off, e->brows, e->blen, e->ttiles, e->n_tiles, e->trstart, e->vocab_d, e->bpack,
+              {e->H[0], e->H[1], e->H[2]}, e->dp, {e->dH[0], e->dH[1], e->dH[2]}, e->bpart};
+    const uint32_t bb = std::min(e->enc_blocks, nt);
+    hipLaunchKernelGGL(k_enc_bwd, dim3(bb), dim3(256), 0, s, b);
+    // splits of at least 512 rows
+    const uint32_t ns = (uint32_t)std::max<uint64_t>(2, std::min<uint64_t>(WSPLITS, (uint64_t)nseq * (e->P + 2) / 512));
+    const uint32_t ns1 = (ns + 1) / 2;
+    const WgradArgs wa{{e->dH[0], e->dH[1], e->dH[2]}, {e->X0, e->A[0], e->A[1]}, e->n_tiles + 1, ns, ns1, e->wpart};
+    hipLaunchKernelGGL(k_wgrad, dim3(4 * ns + ns1), dim3(512), WLDS, s, wa);
+    const SumArgs sa{e->wpart, e->hpart, e->bpart, ns, ns1, hb, bb, e->grad, e->loss};
+    hipLaunchKernelGGL(k_train_sum, dim3(SUM_W + SUM_W1 + SUM_H + SUM_B), dim3(256), 0, s, sa);
+    hcheck(hipGetLastError(), "training step launch");
     float l = 0.f;
     if (read_loss) {
         hcheck(hipMemcpyAsync(&l, e->loss, sizeof(float), hipMemcpyDeviceToHost, s), "loss");
@@ -1245,10 +1330,6 @@ int idb_encoder_create_positions(int device, const uint8_t *vocab, uint32_t posi
         e->theta_b = dalloc<uint16_t>(e->fixed, N_PARAMS);
         e->vocab_d = dalloc<uint8_t>(e->fixed, 256);
         hcheck(hipMemcpyAsync(e->vocab_d, e->vocab, 256, hipMemcpyHostToDevice, e->stream), "vocab");
-        uint16_t *wt = dalloc<uint16_t>(e->fixed, (size_t)C * T * (C0 + 2 * C));
-        e->wt[0] = wt;
-        e->wt[1] = wt + (size_t)C * T * C0;
-        e->wt[2] = e->wt[1] + (size_t)C * T * C;
         // N(0, 1) embedding, U(+-1/sqrt(fan_in)) weights, zero biases
         std::vector<float> h(N_PARAMS, 0.f);
         std::mt19937_64 rng(seed);
@@ -1266,7 +1347,6 @@ int idb_encoder_create_positions(int device, const uint8_t *vocab, uint32_t posi
         hcheck(hipMemsetAsync(e->mom1, 0, sizeof(float) * N_PARAMS, e->stream), "memset");
         hcheck(hipMemsetAsync(e->mom2, 0, sizeof(float) * N_PARAMS, e->stream), "memset");
         hipLaunchKernelGGL(k_to_bf16, dim3(nblocks(N_PARAMS)), dim3(256), 0, e->stream, e->theta, N_PARAMS, e->theta_b);
-        refresh_transposed(e);
         hcheck(hipStreamSynchronize(e->stream), "sync");
     });
     if (rc != IDB_OK) {
@@ -1284,8 +1364,6 @@ void idb_encoder_destroy(idb_encoder *e)
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     for (void *p : e->fixed) (void)hipFree(p);
     for (void *p : e->ws) (void)hipFree(p);
-    (void)hipFree(e->tok);
-    (void)hipFree(e->tlen);
     (void)hipFree(e->tiles);
     (void)hipFree(e->rstart);
     (void)hipFree(e->zbuf);
@@ -1310,7 +1388,7 @@ int idb_encoder_set_params(idb_encoder *e, const float *host)
     return guard(e, [&] {
         hcheck(hipMemcpyAsync(e->theta, host, sizeof(float) * N_PARAMS, hipMemcpyHostToDevice, e->stream), "copy");
         hipLaunchKernelGGL(k_to_bf16, dim3(nblocks(N_PARAMS)), dim3(256), 0, e->stream, e->theta, N_PARAMS, e->theta_b);
-        refresh_transposed(e);
+        e->pack_stale = true;
         hcheck(hipMemsetAsync(e->mom1, 0, sizeof(float) * N_PARAMS, e->stream), "memset");
         hcheck(hipMemsetAsync(e->mom2, 0, sizeof(float) * N_PARAMS, e->stream), "memset");
         e->adam_step = 0;
@@ -1353,11 +1431,10 @@ int idb_encoder_loss_grad(idb_encoder *e, const idb_dataset *d, const uint32_t *
             if (pairs[i] >= d->n_rows) throw Fail{IDB_ERR_ARG, "pair row out of range"};
         DevData dd;
         const idb_dataset *dv = device_view(d, dd, e->stream);
-        tokenize(e, dv);
         const uint32_t *pd = dd.up(pairs, 2 * (size_t)n_pairs, e->stream);
         const float *ld = dd.up(labels, n_pairs, e->stream);
-        ensure_workspace(e, round4(2 * n_pairs));
-        *loss = step(e, pd, ld, nullptr, 0, n_pairs, n_pairs, margin, 1.f / (float)n_pairs, true);
+        ensure_workspace(e, 2 * n_pairs);
+        *loss = step(e, dv, pd, ld, nullptr, 0, n_pairs, margin, 1.f / (float)n_pairs, true);
         hcheck(hipMemcpyAsync(grad_host, e->grad, sizeof(float) * N_PARAMS, hipMemcpyDeviceToHost, e->stream), "copy");
         hcheck(hipStreamSynchronize(e->stream), "sync");
     });
@@ -1373,11 +1450,10 @@ int idb_encoder_train(idb_encoder *e, const idb_dataset *d, const uint32_t *pair
             if (pairs[i] >= d->n_rows) throw Fail{IDB_ERR_ARG, "pair row out of range"};
         DevData dd;
         const idb_dataset *dv = device_view(d, dd, e->stream);
-        tokenize(e, dv);
         const uint32_t *pd = dd.up(pairs, 2 * (size_t)n_pairs, e->stream);
         const float *ld = dd.up(labels, n_pairs, e->stream);
         const uint32_t B = tp->batch_pairs;
-        ensure_workspace(e, round4(2 * B));
+        ensure_workspace(e, 2 * (uint32_t)std::min<uint64_t>(B, n_pairs));
         std::vector<uint32_t> order(n_pairs);
         std::iota(order.begin(), order.end(), 0u);
         std::mt19937_64 rng(tp->seed);
@@ -1403,7 +1479,7 @@ int idb_encoder_train(idb_encoder *e, const idb_dataset *d, const uint32_t *pair
                 const uint32_t nb = (uint32_t)std::min<uint64_t>(B, n_pairs - first);
                 const bool rd = steps == 0 || (tp->log_every && steps % tp->log_every == 0) ||
                                 (first + B >= n_pairs);
-                const float l = step(e, pd, ld, od, first, nb, n_pairs, tp->margin, 1.f / (float)nb, rd);
+                const float l = step(e, dv, pd, ld, od, first, nb, tp->margin, 1.f / (float)nb, rd);
                 if (rd) {
                     if (steps == 0) first_loss = l;
                     last = l;
@@ -1414,7 +1490,7 @@ int idb_encoder_train(idb_encoder *e, const idb_dataset *d, const uint32_t *pair
                 const float c1 = 1.f - std::pow(b1, (float)e->adam_step), c2 = 1.f - std::pow(b2, (float)e->adam_step);
                 hipLaunchKernelGGL(k_adam, dim3(nblocks(N_PARAMS)), dim3(256), 0, e->stream, e->theta, e->grad, e->mom1,
                                    e->mom2, N_PARAMS, tp->lr, b1, b2, 1e-8f, c1, c2, e->theta_b);
-                refresh_transposed(e);
+                e->pack_stale = true;
                 ++steps;
             }
         }

@@ -27,6 +27,7 @@
 #include <string>
 #include <vector>
 
+#include "copy_pool.h"
 #include "idb_internal.h"
 
 namespace {
@@ -90,7 +91,7 @@ __global__ void k_adam(float *th, const float *g, float *m, float *v, uint32_t n
 // ---------------------------------------------------------------------------
 // The whole forward pass in one kernel.
 //
-// A block takes a tile of EM = 256 activation rows and keeps them in LDS
+// A block takes a tile of EM = 64 RT activation rows (256 or 128) and keeps them in LDS
 // through all three convolutions (layer by layer, in place), so neither
 // activations nor im2col windows touch HBM.  Sequences are packed back to
 // back with two zero rows between them: a 5-tap window reaches two rows, so
@@ -112,13 +113,13 @@ __global__ void k_adam(float *th, const float *g, float *m, float *v, uint32_t n
 // Measured: 200k protein rows (packed 1.25 Tflop) 5.22 -> 1.52 ms, 825 TFLOP/s
 // (a large bf16 product reaches 1,214 here); 20k rows of 24-150 letters
 // 2.98 -> 0.81 ms.
-constexpr uint32_t EM = 256, EST = C + 8;         // rows per tile; LDS row stride (272 bytes: conflict-free)
+constexpr uint32_t EST = C + 8;                   // LDS row stride (272 bytes: conflict-free)
 constexpr uint32_t EPW = 1024;                    // sequences per packing window
 constexpr uint32_t EGRP = 8;                      // sequences per round of the head
 constexpr uint32_t EKS1 = T * C0 / 16, EKS = T * C / 16;  // k steps of layer 1, of layers 2 and 3
 constexpr size_t EPACK = (size_t)(EKS1 + 2 * EKS) * 4 * 64 * 8;  // packed weights (bfloat16)
 constexpr uint32_t BLAYER = EKS * 4 * 64 * 8, BPACK = 2 * BLAYER + EKS * 64 * 8;  // and transposed
-constexpr uint32_t EPAD = 2 * 2048;               // fragments loaded ahead past a pack's end
+constexpr uint32_t EPAD = 4 * 2048;               // fragments loaded ahead past a pack's end
 
 // Where a training batch's sequences come from: sequence 2 i + h is row
 // pairs[2 q + h] of pair q = order[first + i] (or first + i).
@@ -134,9 +135,11 @@ struct PairSource {
 // Greedy packing of consecutive sequences into tiles, window by window:
 // tiles in any order, and every sequence's first row within its tile.  At
 // most EM + 2 rows per tile counting each sequence's two zero rows (the last
-// two lie in the tile's zero border).  count[0] = tiles, count[1] = rows.
+// two lie in the tile's zero border).  Segments of wseg windows keep their
+// tiles from the place of their first sequence on: count[2 s] = tiles of
+// segment s, count[1] = packed rows (training, one segment).
 template <bool TRAIN>
-__global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t n, uint32_t P, uint4 *tiles,
+__global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t n, uint32_t P, uint32_t em, uint32_t wseg, uint4 *tiles,
                                                   uint32_t *count, uint16_t *rstart, PairSource ps)
 {
     __shared__ uint32_t S[EPW + 1], cut[EPW + 1], part[4], base_s, base_r;
@@ -188,7 +191,7 @@ __global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t 
         uint32_t lo = i + 1, hi = m;  // S[lo] - S[i] fits (one sequence always does)
         while (lo < hi) {
             const uint32_t mid = (lo + hi + 1) >> 1;
-            if (S[mid] - S[i] <= EM + 2u) lo = mid; else hi = mid - 1;
+            if (S[mid] - S[i] <= em + 2u) lo = mid; else hi = mid - 1;
         }
         nxt[i] = (uint16_t)lo;
     }
@@ -198,7 +201,8 @@ __global__ __launch_bounds__(256) void k_enc_plan(const uint32_t *len, uint32_t 
         for (uint32_t i = 0; i < m; i = nxt[i]) cut[c++] = i;
         cut[c] = m;
         part[0] = c;
-        base_s = atomicAdd(count, c);
+        const uint32_t seg = blockIdx.x / wseg;
+        base_s = seg * wseg * EPW + atomicAdd(count + 2 * seg, c);
         base_r = TRAIN ? atomicAdd(count + 1, S[m]) : 0u;
     }
     __syncthreads();
@@ -251,6 +255,14 @@ __global__ void k_enc_pack(const uint16_t *theta_b, uint16_t *dst, uint32_t *wp2
     }
 }
 
+// Rows of a tile: 64 RT.  Embedding takes 256 (RT = 4): two blocks a CU, and
+// the least padding (200k protein rows 1.58 ms, tiles of 128 rows 1.63).  A
+// training batch is a few tiles per CU, so that the spread of the tiles over
+// the CUs and the latency of one tile count: 128 rows (three blocks a CU)
+// where P fits, 4,096 protein pairs forward 135 -> 107 us, backward 223 ->
+// 176, 256 pairs 54 -> 39 and 84 -> 55.
+constexpr int enc_blocks_per_cu(int rt) { return rt == 4 ? 2 : 3; }
+
 struct EncArgs {
     const uint8_t *seq;
     const uint64_t *off;
@@ -273,22 +285,24 @@ struct EncArgs {
 
 // One convolution over the tile: acc = W x window, CIN input channels.  REV:
 // taps in the order of the data gradient (window row 4 - t for tap t).
-template <uint32_t CIN, bool REV = false>
-__device__ __forceinline__ void enc_conv(const uint16_t *X, const u32x4 *wp, uint32_t lane, f32x16 (&acc)[2][4])
+template <uint32_t CIN, int RT, bool REV = false>
+__device__ __forceinline__ void enc_conv(const uint16_t *X, const u32x4 *wp, uint32_t lane, f32x16 (&acc)[2][RT])
 {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < RT; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    constexpr uint32_t KT = CIN / 16, AHEAD = 2;  // k steps per tap; weight fragments loaded ahead
+    // k steps per tap; steps of weight fragments loaded ahead (four against
+    // two measured the same, 1.58 ms for 200k protein rows)
+    constexpr uint32_t KT = CIN / 16, AHEAD = CIN == C0 ? 2 : 4;
     const uint16_t *xr = X + (lane & 31u) * EST + (lane >> 5) * 8;
     u32x4 wq[AHEAD][2];
 #pragma unroll
     for (uint32_t a = 0; a < AHEAD; ++a) {
-        wq[a][0] = wp[a * 256];
-        wq[a][1] = wp[a * 256 + 64];
+        wq[a][0] = wp[a * 256 + lane];
+        wq[a][1] = wp[a * 256 + 64 + lane];
     }
 #pragma unroll 1
     for (uint32_t t = 0; t < T; ++t) {
@@ -299,10 +313,10 @@ __device__ __forceinline__ void enc_conv(const uint16_t *X, const u32x4 *wp, uin
             bf16x8 w0 = __builtin_bit_cast(bf16x8, wq[c % AHEAD][0]), w1 = __builtin_bit_cast(bf16x8, wq[c % AHEAD][1]);
             // (past the layer's last step: the next layer's first fragments,
             // or the buffer's padding)
-            wq[c % AHEAD][0] = wt[(c + AHEAD) * 256];
-            wq[c % AHEAD][1] = wt[(c + AHEAD) * 256 + 64];
+            wq[c % AHEAD][0] = wt[(c + AHEAD) * 256 + lane];
+            wq[c % AHEAD][1] = wt[(c + AHEAD) * 256 + 64 + lane];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < RT; ++j) {
                 const bf16x8 x = *(const bf16x8 *)(xt + j * 32 * EST + c * 16);
                 acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0, x, acc[0][j], 0, 0, 0);
                 acc[1][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1, x, acc[1][j], 0, 0, 0);
@@ -329,16 +343,17 @@ __device__ __forceinline__ uint32_t seq_of_row(const uint16_t *s_row, uint32_t c
     return lo;
 }
 
-template <bool TRAIN>
-__global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
+template <bool TRAIN, int RT>
+__global__ __launch_bounds__(256, enc_blocks_per_cu(RT)) void k_encode(EncArgs a)
 {
+    constexpr uint32_t EM = 64 * RT;
     __shared__ __align__(16) uint16_t X[(EM + 4) * EST];
     __shared__ __align__(16) float bias[3 * C];
     __shared__ __align__(16) float sp[EGRP][C];
     __shared__ uint32_t s_len[EM / 2 + 2];
     __shared__ uint16_t s_row[EM / 2 + 2];
     __shared__ uint64_t s_off[EM / 2 + 2];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wc = wave & 1u, wr = wave >> 1;  // this wave's 64 channels and 128 rows
     for (uint32_t i = tid; i < 3 * C; i += 256) {
         const uint32_t l = i / C, c = i % C;
@@ -357,7 +372,7 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
             s_off[tid] = a.off[TRAIN ? a.rows[first + tid] : first + tid];
         }
         __syncthreads();
-        {
+        if (EM == 256 || tid < EM) {
             // embedding: thread = row
             const uint32_t lo = seq_of_row(s_row, cnt, tid), p = tid - s_row[lo];
             u32x4 e[4] = {};
@@ -382,21 +397,21 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
         // validity of this lane's four rows (row wr * 128 + 32 j + lane % 32)
         uint32_t valid = 0;
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t row = wr * 128 + 32 * j + (lane & 31u);
+        for (uint32_t j = 0; j < RT; ++j) {
+            const uint32_t row = wr * (32 * RT) + 32 * j + (lane & 31u);
             const uint32_t lo = seq_of_row(s_row, cnt, row);
             if (row - s_row[lo] < s_len[lo]) valid |= 1u << j;
         }
         __syncthreads();
-        const uint16_t *Xw = X + wr * 128 * EST;
-        const u32x4 *wp = (const u32x4 *)a.pack + wc * 128 + lane;
+        const uint16_t *Xw = X + wr * (32 * RT) * EST;
+        const u32x4 *wp = (const u32x4 *)a.pack + wc * 128;
 #pragma unroll 1
         for (uint32_t l = 0; l < 3; ++l) {
-            f32x16 acc[2][4];
-            if (l == 0) enc_conv<C0>(Xw, wp, lane, acc);
-            else enc_conv<C>(Xw, wp + (EKS1 + (l - 1) * EKS) * 256, lane, acc);
+            f32x16 acc[2][RT];
+            if (l == 0) enc_conv<C0, RT>(Xw, wp, lane, acc);
+            else enc_conv<C, RT>(Xw, wp + (EKS1 + (l - 1) * EKS) * 256, lane, acc);
             __syncthreads();  // every wave has read the layer's input
-            uint2 *h = TRAIN ? a.H[l] + (size_t)ti * 8192 + wave * 2048 + lane : nullptr;
+            uint2 *h = TRAIN ? a.H[l] + (size_t)ti * (2048 * RT) + wave * (512 * RT) + lane : nullptr;
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -404,18 +419,18 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
                     const uint32_t ch = wc * 64 + i * 32 + 8 * q + 4 * (lane >> 5);
                     const float4 b = *(const float4 *)(bias + l * C + ch);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                    for (int j = 0; j < RT; ++j) {
                         const float x0 = acc[i][j][4 * q] + b.x, x1 = acc[i][j][4 * q + 1] + b.y,
                                     x2 = acc[i][j][4 * q + 2] + b.z, x3 = acc[i][j][4 * q + 3] + b.w;
                         if (TRAIN)
-                            h[((i * 4 + j) * 4 + q) * 64] = make_uint2((uint32_t)f2bf(x0) | ((uint32_t)f2bf(x1) << 16),
+                            h[((i * RT + j) * 4 + q) * 64] = make_uint2((uint32_t)f2bf(x0) | ((uint32_t)f2bf(x1) << 16),
                                                                        (uint32_t)f2bf(x2) | ((uint32_t)f2bf(x3) << 16));
                         const float g0 = gelu(x0), g1 = gelu(x1), g2 = gelu(x2), g3 = gelu(x3);
                         const bool v = (valid >> j) & 1u;
                         uint2 o;
                         o.x = v ? (uint32_t)f2bf(g0) | ((uint32_t)f2bf(g1) << 16) : 0u;
                         o.y = v ? (uint32_t)f2bf(g2) | ((uint32_t)f2bf(g3) << 16) : 0u;
-                        *(uint2 *)(X + (2 + wr * 128 + 32 * j + (lane & 31u)) * EST + ch) = o;
+                        *(uint2 *)(X + (2 + wr * (32 * RT) + 32 * j + (lane & 31u)) * EST + ch) = o;
                     }
                 }
             __syncthreads();
@@ -484,14 +499,14 @@ __global__ __launch_bounds__(256, 2) void k_encode(EncArgs a)
 
 constexpr uint32_t HP = 16;                        // pairs per round of the head's backward pass
 constexpr uint32_t HPART = D * C + D + 4;          // one block's projection gradients and loss
-constexpr uint32_t HBLOCKS = 128;                  // most blocks of the head's backward pass
+constexpr uint32_t HBLOCKS = 256;                  // most blocks of the head's backward pass
 constexpr uint32_t BPART = NTOK * C0 + 3 * C;      // one block's embedding and bias gradients
 
 // Contrastive loss of pair i (sequences 2i, 2i+1), back through the norm and
 // the projection to the pooled means (dp, already divided by the length), and
 // the projection's gradients.  A wave takes four pairs of a round of HP; the
 // block then adds the round's du x pool into 32 accumulators per thread.
-// Latency-bound (4,096 pairs are one or two rounds a block); the sums over
+// Latency-bound (4,096 pairs are one round a block); the sums over
 // pairs stay in registers and leave as one partial per block, since one atomic
 // word per pair (the loss) took 49 us.  With the three kernels it replaces:
 // 4,096 pairs 306 -> 37 us.
@@ -642,7 +657,7 @@ __device__ __forceinline__ uint2 times_grad(float a, float b, float c, float d, 
                       v ? (uint32_t)f2bf(g2) | ((uint32_t)f2bf(g3) << 16) : 0u);
 }
 
-// Data gradients of a tile, in LDS as in k_encode (same tiles, same lane
+// Data gradients of a tile, in LDS as in k_encode (same tiles and lane
 // mapping): dH3 from dp, then each layer's transposed convolution times the
 // GELU's derivative at the saved pre-activation, and the first layer's input
 // gradient added per token.  Gradients leave for k_wgrad row by row; bias and
@@ -650,15 +665,17 @@ __device__ __forceinline__ uint2 times_grad(float a, float b, float c, float d, 
 // MFMA-bound like k_encode.  4,096 pairs of protein rows: head's last part,
 // three data-gradient products, three bias sums and the embedding scatter
 // took 870 us as eight launches over padded rows; 204 us here.
-__global__ __launch_bounds__(256, 2) void k_enc_bwd(BwdArgs a)
+template <int RT>
+__global__ __launch_bounds__(256, enc_blocks_per_cu(RT)) void k_enc_bwd(BwdArgs a)
 {
+    constexpr uint32_t EM = 64 * RT;
     __shared__ __align__(16) uint16_t X[(EM + 4) * EST];
     __shared__ float semb[C0 * (NTOK + 1)];  // [channel][token]
     __shared__ float sbias[3 * C];
     __shared__ uint32_t s_len[EM / 2 + 2], s_seq[EM / 2 + 2];
     __shared__ uint16_t s_row[EM / 2 + 2];
     __shared__ uint8_t s_tok[EM];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wc = wave & 1u, wr = wave >> 1;
     for (uint32_t i = tid; i < C0 * (NTOK + 1); i += 256) semb[i] = 0.f;
     for (uint32_t i = tid; i < 3 * C; i += 256) sbias[i] = 0.f;
@@ -674,75 +691,82 @@ __global__ __launch_bounds__(256, 2) void k_enc_bwd(BwdArgs a)
             s_seq[tid] = a.rows[first + tid];
         }
         __syncthreads();
-        {
+        if (EM == 256 || tid < EM) {
             const uint32_t q = seq_of_row(s_row, cnt, tid), p = tid - s_row[q];
             s_tok[tid] = p < s_len[q] ? a.vocab[a.seq[a.off[s_seq[q]] + p]] : (uint8_t)255;
         }
         uint32_t valid = 0;
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t row = wr * 128 + 32 * j + (lane & 31u);
+        for (uint32_t j = 0; j < RT; ++j) {
+            const uint32_t row = wr * (32 * RT) + 32 * j + (lane & 31u);
             const uint32_t q = seq_of_row(s_row, cnt, row);
             const bool v = row - s_row[q] < s_len[q];
             if (v) valid |= 1u << j;
             const float *dp = a.dp + (size_t)(first + q) * C + wc * 64 + 4 * (lane >> 5);
-            const uint2 *h = a.H[2] + (size_t)ti * 8192 + wave * 2048 + lane;
+            const uint2 *h = a.H[2] + (size_t)ti * (2048 * RT) + wave * (512 * RT) + lane;
             uint16_t *x = X + (2 + row) * EST + wc * 64 + 4 * (lane >> 5);
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int q2 = 0; q2 < 4; ++q2) {
-                    const uint2 hv = h[((i * 4 + j) * 4 + q2) * 64];
+                    const uint2 hv = h[((i * RT + j) * 4 + q2) * 64];
                     const float4 d = *(const float4 *)(dp + i * 32 + 8 * q2);
                     *(uint2 *)(x + i * 32 + 8 * q2) = times_grad(d.x, d.y, d.z, d.w, hv, v);
                 }
         }
         __syncthreads();
-        const uint16_t *Xw = X + wr * 128 * EST;
-        const u32x4 *wp = (const u32x4 *)a.pack + wc * 128 + lane;
+        const uint16_t *Xw = X + wr * (32 * RT) * EST;
+        const u32x4 *wp = (const u32x4 *)a.pack + wc * 128;
 #pragma unroll 1
         for (int l = 1; l >= 0; --l) {
             bwd_store_rows(X, a.dH[l + 1] + (size_t)t.z * C, t.w, tid, sbias + (l + 1) * C);
-            f32x16 acc[2][4];
-            enc_conv<C, true>(Xw, wp + (1 - l) * (BLAYER / 8), lane, acc);
+            f32x16 acc[2][RT];
+            enc_conv<C, RT, true>(Xw, wp + (1 - l) * (BLAYER / 8), lane, acc);
             __syncthreads();  // every wave has read the layer's gradient
-            const uint2 *h = a.H[l] + (size_t)ti * 8192 + wave * 2048 + lane;
+            const uint2 *h = a.H[l] + (size_t)ti * (2048 * RT) + wave * (512 * RT) + lane;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < RT; ++j) {
                 const bool v = (valid >> j) & 1u;
-                uint16_t *x = X + (2 + wr * 128 + 32 * j + (lane & 31u)) * EST + wc * 64 + 4 * (lane >> 5);
+                uint16_t *x = X + (2 + wr * (32 * RT) + 32 * j + (lane & 31u)) * EST + wc * 64 + 4 * (lane >> 5);
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int q2 = 0; q2 < 4; ++q2)
                         *(uint2 *)(x + i * 32 + 8 * q2) =
                             times_grad(acc[i][j][4 * q2], acc[i][j][4 * q2 + 1], acc[i][j][4 * q2 + 2],
-                                       acc[i][j][4 * q2 + 3], h[((i * 4 + j) * 4 + q2) * 64], v);
+                                       acc[i][j][4 * q2 + 3], h[((i * RT + j) * 4 + q2) * 64], v);
             }
             __syncthreads();
         }
         bwd_store_rows(X, a.dH[0] + (size_t)t.z * C, t.w, tid, sbias);
-        // input gradient: 32 channels of this wave's 64 rows
-        f32x16 g[2];
+        // input gradient, 32 channels: row tiles wave and wave + 4
+        constexpr int NG = (2 * RT + 3) / 4;
+        f32x16 g[NG];
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NG; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) g[j][r] = 0.f;
-        const uint16_t *xr = X + (wave * 64 + (lane & 31u)) * EST + (lane >> 5) * 8;
-        const u32x4 *w1 = (const u32x4 *)a.pack + 2 * (BLAYER / 8) + lane;
+        const uint16_t *xr = X + (wave * 32 + (lane & 31u)) * EST + (lane >> 5) * 8;
+        const u32x4 *w1 = (const u32x4 *)a.pack + 2 * (BLAYER / 8);
+        u32x4 wq[C / 16];  // a tap's fragments, loaded a tap ahead (past the last: the padding)
+#pragma unroll
+        for (uint32_t c = 0; c < C / 16; ++c) wq[c] = w1[c * 64 + lane];
 #pragma unroll 1
         for (uint32_t tp = 0; tp < T; ++tp)
 #pragma unroll
             for (uint32_t c = 0; c < C / 16; ++c) {
-                const bf16x8 w = __builtin_bit_cast(bf16x8, w1[(tp * (C / 16) + c) * 64]);
+                const bf16x8 w = __builtin_bit_cast(bf16x8, wq[c]);
+                wq[c] = w1[((tp + 1) * (C / 16) + c) * 64 + lane];
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    g[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        w, *(const bf16x8 *)(xr + (T - 1 - tp + j * 32) * EST + c * 16), g[j], 0, 0, 0);
+                for (int j = 0; j < NG; ++j)
+                    if (wave + 4 * j < 2 * RT)
+                        g[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            w, *(const bf16x8 *)(xr + (T - 1 - tp + j * 128) * EST + c * 16), g[j], 0, 0, 0);
             }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t tok = s_tok[wave * 64 + 32 * j + (lane & 31u)];
+        for (int j = 0; j < NG; ++j) {
+            if (wave + 4 * j >= 2 * RT) continue;
+            const uint32_t tok = s_tok[(wave + 4 * j) * 32 + (lane & 31u)];
             if (tok != 255u)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
@@ -1011,6 +1035,12 @@ void hcheck(hipError_t e, const char *what)
 
 }  // namespace
 
+// Embeddings leave for the host in segments of rows, so that copying one
+// overlaps computing the next: at most ENC_SEGS segments per launch group of
+// ENC_GROUP rows, ENC_SLOTS of them staged at a time (64 MB pinned at most).
+constexpr uint32_t ENC_SEGS = 16, ENC_SLOTS = 4, ENC_GROUP = 1u << 20;
+constexpr size_t ENC_STAGE_MAX = 64u << 20;  // most input bytes that are staged (and kept on the device)
+
 // ---------------------------------------------------------------------------
 // Encoder state: parameters, optimiser moments, and a workspace sized for the
 // largest batch seen so far.
@@ -1032,7 +1062,6 @@ struct idb_encoder {
     float *wpart = nullptr, *hpart = nullptr, *bpart = nullptr;  // partial sums
     uint4 *ttiles = nullptr;
     uint16_t *trstart = nullptr;
-    float *loss = nullptr;
     uint8_t *vocab_d = nullptr;
     // inference: weights in the fused kernel's order (packed again when the
     // parameters have changed), and the packing of the current rows
@@ -1046,7 +1075,14 @@ struct idb_encoder {
     uint32_t plan_cap = 0;
     float *zbuf = nullptr;
     uint32_t zbuf_cap = 0;
-    uint32_t enc_blocks = 0, cus = 1;
+    // host transfers: the second compute stream and the copy stream of an
+    // embedding call, pinned staging (inputs and gradients, then the ring of
+    // embedding segments), and the device copy of the inputs
+    hipStream_t side = nullptr, copy = nullptr;
+    hipEvent_t ev_in = nullptr, ev_enc[ENC_SLOTS] = {}, ev_copy[ENC_SLOTS] = {};
+    uint8_t *pin = nullptr, *ring = nullptr, *inbuf = nullptr;
+    size_t pin_cap = 0, ring_cap = 0, in_cap = 0;
+    uint32_t cus = 1;
     std::vector<void *> fixed, ws;  // parameter and workspace allocations
 };
 
@@ -1072,10 +1108,12 @@ void free_workspace(idb_encoder *e)
 // window's tiles hold at least EM + 2 over P + 2 sequences each but its last.
 constexpr uint32_t WSPLITS = 56;  // splits of the rows: 4 x 56 + 28 blocks fill 256 CUs
 
+int train_rt(uint32_t P) { return P + 2 <= 66u ? 2 : 4; }
+
 uint32_t tile_capacity(uint32_t nseq, uint32_t P)
 {
     const uint32_t windows = (nseq + EPW - 1) / EPW;
-    return std::min(nseq, nseq / ((EM + 2) / (P + 2)) + windows);
+    return std::min(nseq, nseq / ((64u * train_rt(P) + 2) / (P + 2)) + windows);
 }
 
 void ensure_workspace(idb_encoder *e, uint32_t nseq)
@@ -1089,7 +1127,7 @@ void ensure_workspace(idb_encoder *e, uint32_t nseq)
     for (int l = 0; l < 2; ++l) e->A[l] = dalloc<uint16_t>(e->ws, M * C);
     for (int l = 0; l < 3; ++l) {
         e->dH[l] = dalloc<uint16_t>(e->ws, M * C);
-        e->H[l] = dalloc<uint2>(e->ws, nt * 8192);
+        e->H[l] = dalloc<uint2>(e->ws, nt * 2048 * train_rt(e->P));
     }
     e->pool = dalloc<float>(e->ws, (size_t)nseq * C);
     e->z = dalloc<float>(e->ws, (size_t)nseq * D);
@@ -1109,16 +1147,14 @@ void ensure_pack(idb_encoder *e)
         uint16_t *pack = dalloc<uint16_t>(e->fixed, EPACK + EPAD);
         e->bpack = dalloc<uint16_t>(e->fixed, BPACK + EPAD);
         e->wp2 = dalloc<uint32_t>(e->fixed, C / 2 * D);
-        e->n_tiles = dalloc<uint32_t>(e->fixed, 2);
+        e->n_tiles = dalloc<uint32_t>(e->fixed, 2 * ENC_SEGS);
         hcheck(hipMemsetAsync(pack, 0, (EPACK + EPAD) * sizeof(uint16_t), e->stream), "memset");
         hcheck(hipMemsetAsync(e->bpack, 0, (BPACK + EPAD) * sizeof(uint16_t), e->stream), "memset");
-        int dev = 0, cus = 0, per_cu = 0;
+        hcheck(hipFuncSetAttribute((const void *)k_wgrad, hipFuncAttributeMaxDynamicSharedMemorySize, (int)WLDS), "wgrad LDS");
+        int dev = 0, cus = 0;
         hcheck(hipGetDevice(&dev), "device");
         hcheck(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device");
-        hcheck(hipFuncSetAttribute((const void *)k_wgrad, hipFuncAttributeMaxDynamicSharedMemorySize, (int)WLDS), "wgrad LDS");
-        hcheck(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_encode<false>, 256, 0), "occupancy");
         e->cus = (uint32_t)std::max(cus, 1);
-        e->enc_blocks = (uint32_t)std::max(per_cu, 1) * e->cus;
         e->pack = pack;
     }
     if (e->pack_stale) {
@@ -1128,13 +1164,13 @@ void ensure_pack(idb_encoder *e)
 }
 
 void enc_args(const idb_encoder *e, EncArgs &a, const uint8_t *seq, const uint64_t *off, const uint32_t *len,
-              const uint4 *tiles, const uint16_t *rstart)
+              const uint4 *tiles, const uint16_t *rstart, const uint32_t *n_tiles)
 {
     a.seq = seq;
     a.off = off;
     a.len = len;
     a.tiles = tiles;
-    a.n_tiles = e->n_tiles;
+    a.n_tiles = n_tiles;
     a.rstart = rstart;
     a.vocab = e->vocab_d;
     a.theta_b = e->theta_b;
@@ -1143,16 +1179,14 @@ void enc_args(const idb_encoder *e, EncArgs &a, const uint8_t *seq, const uint64
     a.P = e->P;
 }
 
-// Embeddings of rows [0, n) of device data by the fused kernel, on e->stream:
-// float32 (z) and/or bfloat16 (zb), 64 per row.
-void embed_fused(idb_encoder *e, const uint8_t *seq, const uint64_t *off, const uint32_t *len, uint32_t n, float *z,
-                 uint16_t *zb)
+// The packing of n rows of device data, in segments of `rows` rows (a whole
+// number of windows), on e->stream.  All segments are planned ahead: a plan
+// between two segments would wait for the first one's blocks to leave the CUs.
+void embed_plan(idb_encoder *e, const uint32_t *len, uint32_t n, uint32_t rows)
 {
-    if (n == 0) return;
-    hipStream_t s = e->stream;
     ensure_pack(e);
     if (n > e->plan_cap) {
-        hcheck(hipStreamSynchronize(s), "sync");
+        hcheck(hipStreamSynchronize(e->stream), "sync");
         (void)hipFree(e->tiles);
         (void)hipFree(e->rstart);
         e->tiles = nullptr;
@@ -1162,14 +1196,23 @@ void embed_fused(idb_encoder *e, const uint8_t *seq, const uint64_t *off, const 
         hcheck(hipMalloc(&e->rstart, sizeof(uint16_t) * (size_t)n), "hipMalloc");
         e->plan_cap = n;
     }
-    hcheck(hipMemsetAsync(e->n_tiles, 0, sizeof(uint32_t), s), "memset");
-    hipLaunchKernelGGL(k_enc_plan<false>, dim3((n + EPW - 1) / EPW), dim3(256), 0, s, len, n, e->P, e->tiles, e->n_tiles,
-                       e->rstart, PairSource{});
+    hcheck(hipMemsetAsync(e->n_tiles, 0, 2 * ENC_SEGS * sizeof(uint32_t), e->stream), "memset");
+    hipLaunchKernelGGL(k_enc_plan<false>, dim3((n + EPW - 1) / EPW), dim3(256), 0, e->stream, len, n, e->P, 256u,
+                       (rows + EPW - 1) / EPW, e->tiles, e->n_tiles, e->rstart, PairSource{});
+    hcheck(hipGetLastError(), "plan launch");
+}
+
+// Embeddings of planned segment seg (`rows` rows each, n in all) by the fused
+// kernel on stream s: float32 (z) and/or bfloat16 (zb), 64 per row.
+void embed_segment(idb_encoder *e, const uint8_t *seq, const uint64_t *off, const uint32_t *len, uint32_t n,
+                   uint32_t rows, uint32_t seg, float *z, uint16_t *zb, hipStream_t s)
+{
+    const uint32_t first = seg * rows, m = std::min(rows, n - first);
     EncArgs a{};
-    enc_args(e, a, seq, off, len, e->tiles, e->rstart);
+    enc_args(e, a, seq, off, len, e->tiles + first, e->rstart, e->n_tiles + 2 * seg);
     a.z = z;
     a.zb = zb;
-    hipLaunchKernelGGL(k_encode<false>, dim3(std::min(e->enc_blocks, n)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((k_encode<false, 4>), dim3(std::min(e->cus * enc_blocks_per_cu(4), m)), dim3(256), 0, s, a);
     hcheck(hipGetLastError(), "encoder launch");
 }
 
@@ -1203,6 +1246,101 @@ const idb_dataset *device_view(const idb_dataset *d, DevData &dd, hipStream_t s)
     return &dd.d;
 }
 
+// Pinned memory of at least `bytes` bytes (false: none to be had, the copies
+// then go to the caller's arrays directly).
+bool pinned(uint8_t **p, size_t *cap, size_t bytes)
+{
+    if (*cap >= bytes) return true;
+    if (*p) (void)hipHostFree(*p);
+    *p = nullptr;
+    *cap = 0;
+    if (hipHostMalloc((void **)p, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+        return false;
+    }
+    *cap = bytes;
+    return true;
+}
+
+// Host inputs of one call on the device: by one copy from pinned staging into
+// a buffer that the encoder keeps (five allocations, frees and copies of
+// pageable arrays took 0.2 ms a call), or, past ENC_STAGE_MAX bytes, by
+// separate copies into memory of the call.
+struct Upload {
+    idb_encoder *e;
+    DevData dd;
+    CopyPool::Job jobs[5];
+    const void **out[5];
+    uint32_t n = 0;
+    explicit Upload(idb_encoder *enc) : e(enc) {}
+    template <typename T>
+    void add(const T *h, size_t count, const T **dst)
+    {
+        if (count && !h) throw Fail{IDB_ERR_ARG, "missing input array"};
+        jobs[n] = {nullptr, h, count * sizeof(T)};
+        out[n++] = (const void **)dst;
+    }
+    void run()
+    {
+        size_t at[5], total = 0;
+        for (uint32_t k = 0; k < n; ++k) {
+            at[k] = total;
+            total += (jobs[k].bytes + 255) & ~(size_t)255;
+        }
+        total += 256;
+        const bool staged = total <= ENC_STAGE_MAX && pinned(&e->pin, &e->pin_cap, total);
+        if (staged && e->in_cap < total) {
+            (void)hipFree(e->inbuf);
+            e->inbuf = nullptr;
+            e->in_cap = 0;
+            hcheck(hipMalloc((void **)&e->inbuf, total), "hipMalloc");
+            e->in_cap = total;
+        }
+        for (uint32_t k = 0; k < n; ++k) {
+            if (staged) *out[k] = e->inbuf + at[k];
+            else *out[k] = dd.up((const uint8_t *)jobs[k].src, jobs[k].bytes, e->stream);
+            if (staged) jobs[k].dst = e->pin + at[k];
+        }
+        if (!staged) return;
+        CopyPool::get().run(jobs, n);
+        hcheck(hipMemcpyAsync(e->inbuf, e->pin, total, hipMemcpyHostToDevice, e->stream), "input copy");
+    }
+    void add_rows(const idb_dataset *d, idb_dataset &v)
+    {
+        v = *d;
+        if (d->mem == IDB_MEM_DEVICE) return;
+        v.mem = IDB_MEM_DEVICE;
+        add(d->seq, d->seq_bytes, &v.seq);
+        add(d->off, d->n_rows, &v.off);
+        add(d->len, d->n_rows, &v.len);
+    }
+};
+
+// Streams and events of a call in several segments.
+void embed_streams(idb_encoder *e)
+{
+    if (e->copy) return;
+    if (!e->ev_in) hcheck(hipEventCreateWithFlags(&e->ev_in, hipEventDisableTiming), "event");
+    for (uint32_t k = 0; k < ENC_SLOTS; ++k) {
+        if (!e->ev_enc[k]) hcheck(hipEventCreateWithFlags(&e->ev_enc[k], hipEventDisableTiming), "event");
+        if (!e->ev_copy[k]) hcheck(hipEventCreateWithFlags(&e->ev_copy[k], hipEventDisableTiming), "event");
+    }
+    if (!e->side) hcheck(hipStreamCreateWithFlags(&e->side, hipStreamNonBlocking), "stream");
+    hcheck(hipStreamCreateWithFlags(&e->copy, hipStreamNonBlocking), "stream");
+}
+
+// Nothing of a call is in flight any more when it returns, also by an error.
+struct Drain {
+    idb_encoder *e;
+    ~Drain()
+    {
+        (void)hipStreamSynchronize(e->stream);
+        if (e->side) (void)hipStreamSynchronize(e->side);
+        if (e->copy) (void)hipStreamSynchronize(e->copy);
+    }
+};
+
 // One training step over pairs [first, first + nb) of the (ordered) pair list:
 // the gradient into e->grad, the loss behind it.
 float step(idb_encoder *e, const idb_dataset *d, const uint32_t *pairs_d, const float *labels_d, const uint32_t *order_d,
@@ -1210,19 +1348,19 @@ float step(idb_encoder *e, const idb_dataset *d, const uint32_t *pairs_d, const 
 {
     hipStream_t s = e->stream;
     const uint32_t nseq = 2 * nb, nt = tile_capacity(nseq, e->P);
+    const int rt = train_rt(e->P);
     ensure_pack(e);
     if (!e->wpart) {
         e->hpart = dalloc<float>(e->fixed, (size_t)HBLOCKS * HPART);
-        e->bpart = dalloc<float>(e->fixed, (size_t)e->enc_blocks * BPART);
-        e->loss = dalloc<float>(e->fixed, 1);
+        e->bpart = dalloc<float>(e->fixed, (size_t)e->cus * enc_blocks_per_cu(rt) * BPART);
         e->wpart = dalloc<float>(e->fixed, (size_t)(4 * WSPLITS + WSPLITS / 2) * WPART);
     }
     hcheck(hipMemsetAsync(e->n_tiles, 0, 2 * sizeof(uint32_t), s), "memset");
     const PairSource ps{pairs_d, order_d, labels_d, first, e->brows, e->blen, e->y};
-    hipLaunchKernelGGL(k_enc_plan<true>, dim3((nseq + EPW - 1) / EPW), dim3(256), 0, s, d->len, nseq, e->P, e->ttiles,
+    hipLaunchKernelGGL(k_enc_plan<true>, dim3((nseq + EPW - 1) / EPW), dim3(256), 0, s, d->len, nseq, e->P, 64u * rt, ~0u, e->ttiles,
                        e->n_tiles, e->trstart, ps);
     EncArgs a{};
-    enc_args(e, a, d->seq, d->off, e->blen, e->ttiles, e->trstart);
+    enc_args(e, a, d->seq, d->off, e->blen, e->ttiles, e->trstart, e->n_tiles);
     a.z = e->z;
     a.rows = e->brows;
     for (int l = 0; l < 3; ++l) a.H[l] = e->H[l];
@@ -1231,25 +1369,27 @@ float step(idb_encoder *e, const idb_dataset *d, const uint32_t *pairs_d, const 
     a.A2 = e->A[1];
     a.pool = e->pool;
     a.nrm = e->nrm;
-    hipLaunchKernelGGL(k_encode<true>, dim3(std::min(e->enc_blocks, nt)), dim3(256), 0, s, a);
+    const dim3 bb(std::min(e->cus * enc_blocks_per_cu(rt), nt));
+    if (rt == 2) hipLaunchKernelGGL((k_encode<true, 2>), bb, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_encode<true, 4>), bb, dim3(256), 0, s, a);
     const uint32_t hb = std::min(HBLOCKS, (nb + HP - 1) / HP);
     hipLaunchKernelGGL(k_pair_head, dim3(hb), dim3(256), 0, s, e->z, e->nrm, e->pool, e->blen, e->y, nb, margin, inv_b,
                        e->wp2, e->dp, e->hpart);
     BwdArgs b{d->seq, d->off, e->brows, e->blen, e->ttiles, e->n_tiles, e->trstart, e->vocab_d, e->bpack,
               {e->H[0], e->H[1], e->H[2]}, e->dp, {e->dH[0], e->dH[1], e->dH[2]}, e->bpart};
-    const uint32_t bb = std::min(e->enc_blocks, nt);
-    hipLaunchKernelGGL(k_enc_bwd, dim3(bb), dim3(256), 0, s, b);
+    if (rt == 2) hipLaunchKernelGGL(k_enc_bwd<2>, bb, dim3(256), 0, s, b);
+    else hipLaunchKernelGGL(k_enc_bwd<4>, bb, dim3(256), 0, s, b);
     // splits of at least 512 rows
     const uint32_t ns = (uint32_t)std::max<uint64_t>(2, std::min<uint64_t>(WSPLITS, (uint64_t)nseq * (e->P + 2) / 512));
     const uint32_t ns1 = (ns + 1) / 2;
     const WgradArgs wa{{e->dH[0], e->dH[1], e->dH[2]}, {e->X0, e->A[0], e->A[1]}, e->n_tiles + 1, ns, ns1, e->wpart};
     hipLaunchKernelGGL(k_wgrad, dim3(4 * ns + ns1), dim3(512), WLDS, s, wa);
-    const SumArgs sa{e->wpart, e->hpart, e->bpart, ns, ns1, hb, bb, e->grad, e->loss};
+    const SumArgs sa{e->wpart, e->hpart, e->bpart, ns, ns1, hb, bb.x, e->grad, e->grad + N_PARAMS};
     hipLaunchKernelGGL(k_train_sum, dim3(SUM_W + SUM_W1 + SUM_H + SUM_B), dim3(256), 0, s, sa);
     hcheck(hipGetLastError(), "training step launch");
     float l = 0.f;
     if (read_loss) {
-        hcheck(hipMemcpyAsync(&l, e->loss, sizeof(float), hipMemcpyDeviceToHost, s), "loss");
+        hcheck(hipMemcpyAsync(&l, e->grad + N_PARAMS, sizeof(float), hipMemcpyDeviceToHost, s), "loss");
         hcheck(hipStreamSynchronize(s), "sync");
     }
     return l;
@@ -1268,6 +1408,9 @@ int guard(idb_encoder *e, F &&f)
     } catch (const std::bad_alloc &) {
         if (e) e->err = "host allocation failed";
         return IDB_ERR_OOM;
+    } catch (const std::exception &x) {
+        if (e) e->err = x.what();
+        return IDB_ERR_HIP;
     }
 }
 
@@ -1282,7 +1425,10 @@ hipError_t idb_encoder_embed_rows(idb_encoder *e, const uint8_t *seq, const uint
         hipStream_t keep = e->stream;
         e->stream = s;
         try {
-            embed_fused(e, seq, off, len, n, nullptr, zb);
+            if (n) {
+                embed_plan(e, len, n, n);
+                embed_segment(e, seq, off, len, n, n, 0, nullptr, zb, s);
+            }
         } catch (...) {
             e->stream = keep;
             throw;
@@ -1324,7 +1470,7 @@ int idb_encoder_create_positions(int device, const uint8_t *vocab, uint32_t posi
     const int rc = guard(e, [&] {
         hcheck(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "stream");
         e->theta = dalloc<float>(e->fixed, N_PARAMS);
-        e->grad = dalloc<float>(e->fixed, N_PARAMS);
+        e->grad = dalloc<float>(e->fixed, N_PARAMS + 1);  // and the loss
         e->mom1 = dalloc<float>(e->fixed, N_PARAMS);
         e->mom2 = dalloc<float>(e->fixed, N_PARAMS);
         e->theta_b = dalloc<uint16_t>(e->fixed, N_PARAMS);
@@ -1367,6 +1513,18 @@ void idb_encoder_destroy(idb_encoder *e)
     (void)hipFree(e->tiles);
     (void)hipFree(e->rstart);
     (void)hipFree(e->zbuf);
+    (void)hipFree(e->inbuf);
+    if (e->side) (void)hipStreamSynchronize(e->side);
+    if (e->copy) (void)hipStreamSynchronize(e->copy);
+    if (e->pin) (void)hipHostFree(e->pin);
+    if (e->ring) (void)hipHostFree(e->ring);
+    if (e->ev_in) (void)hipEventDestroy(e->ev_in);
+    for (uint32_t k = 0; k < ENC_SLOTS; ++k) {
+        if (e->ev_enc[k]) (void)hipEventDestroy(e->ev_enc[k]);
+        if (e->ev_copy[k]) (void)hipEventDestroy(e->ev_copy[k]);
+    }
+    if (e->side) (void)hipStreamDestroy(e->side);
+    if (e->copy) (void)hipStreamDestroy(e->copy);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
 }
@@ -1400,25 +1558,68 @@ int idb_encoder_embed(idb_encoder *e, const idb_dataset *d, float *z_host)
 {
     if (!e || !d || !z_host) return IDB_ERR_ARG;
     return guard(e, [&] {
-        DevData dd;
-        const idb_dataset *dv = device_view(d, dd, e->stream);
-        // a million rows (256 MB of embeddings) at a time
-        const uint32_t n = d->n_rows, chunk = 1u << 20;
-        if (std::min(n, chunk) > e->zbuf_cap) {
-            hcheck(hipStreamSynchronize(e->stream), "sync");
+        const uint32_t n = d->n_rows;
+        if (n == 0) return;
+        Upload up(e);
+        idb_dataset v;
+        up.add_rows(d, v);
+        const Drain drain{e};
+        if (std::min(n, ENC_GROUP) > e->zbuf_cap) {
             (void)hipFree(e->zbuf);
             e->zbuf = nullptr;
             e->zbuf_cap = 0;
-            hcheck(hipMalloc(&e->zbuf, sizeof(float) * D * std::min(n, chunk)), "hipMalloc");
-            e->zbuf_cap = std::min(n, chunk);
+            hcheck(hipMalloc(&e->zbuf, sizeof(float) * D * std::min(n, ENC_GROUP)), "hipMalloc");
+            e->zbuf_cap = std::min(n, ENC_GROUP);
         }
-        for (uint32_t first = 0; first < n; first += chunk) {
-            const uint32_t cnt = std::min(chunk, n - first);
-            embed_fused(e, dv->seq, dv->off + first, dv->len + first, cnt, e->zbuf, nullptr);
-            hcheck(hipMemcpyAsync(z_host + (size_t)first * D, e->zbuf, sizeof(float) * cnt * D, hipMemcpyDeviceToHost,
-                                  e->stream), "copy");
+        up.run();
+        // Segments of a whole number of packing windows, 4,096 (1 MB) to 65,536
+        // rows; neighbours run on two streams, so that one's last tiles share
+        // the chip with the next one's first.
+        for (uint32_t g0 = 0; g0 < n; g0 += ENC_GROUP) {
+            const uint32_t cnt = std::min(ENC_GROUP, n - g0);
+            const uint32_t rows = std::min(ENC_GROUP / ENC_SEGS, std::max(4u * EPW, ((cnt + 7) / 8 + EPW - 1) / EPW * EPW));
+            const uint32_t segs = (cnt + rows - 1) / rows;
+            const size_t slot = sizeof(float) * D * std::min(rows, cnt);
+            const bool staged = slot <= ENC_STAGE_MAX / ENC_SLOTS &&
+                                pinned(&e->ring, &e->ring_cap, slot * std::min(segs, ENC_SLOTS));
+            embed_plan(e, v.len + g0, cnt, rows);
+            if (segs > 1) {
+                embed_streams(e);
+                hcheck(hipEventRecord(e->ev_in, e->stream), "event");
+                hcheck(hipStreamWaitEvent(e->side, e->ev_in, 0), "event");
+            }
+            // while the GPU computes, the caller's pages of the next segment are
+            // made present
+            const auto present = [&](uint32_t seg) {
+                if (!staged || seg >= segs) return;
+                const CopyPool::Job job{z_host + (size_t)(g0 + seg * rows) * D, nullptr,
+                                        sizeof(float) * D * std::min(rows, cnt - seg * rows)};
+                CopyPool::get().run(&job, 1);
+            };
+            uint32_t issued = 0;
+            for (uint32_t done = 0; done < segs; ++done) {
+                for (; issued < segs && issued < done + ENC_SLOTS; ++issued) {
+                    const uint32_t first = issued * rows, m = std::min(rows, cnt - first), k = issued % ENC_SLOTS;
+                    hipStream_t s = issued & 1u ? e->side : e->stream, cs = segs > 1 ? e->copy : s;
+                    embed_segment(e, v.seq, v.off + g0, v.len + g0, cnt, rows, issued, e->zbuf, nullptr, s);
+                    if (segs > 1) {
+                        hcheck(hipEventRecord(e->ev_enc[k], s), "event");
+                        hcheck(hipStreamWaitEvent(cs, e->ev_enc[k], 0), "event");
+                    }
+                    void *dst = staged ? (void *)(e->ring + k * slot) : (void *)(z_host + (size_t)(g0 + first) * D);
+                    hcheck(hipMemcpyAsync(dst, e->zbuf + (size_t)first * D, sizeof(float) * D * m, hipMemcpyDeviceToHost,
+                                          cs), "copy");
+                    if (segs > 1) hcheck(hipEventRecord(e->ev_copy[k], cs), "event");
+                }
+                const uint32_t first = done * rows, m = std::min(rows, cnt - first), k = done % ENC_SLOTS;
+                if (done == 0) present(0);
+                present(done + 1);
+                hcheck(segs > 1 ? hipEventSynchronize(e->ev_copy[k]) : hipStreamSynchronize(e->stream), "sync");
+                if (!staged) continue;
+                const CopyPool::Job job{z_host + (size_t)(g0 + first) * D, e->ring + k * slot, sizeof(float) * D * m};
+                CopyPool::get().run(&job, 1);
+            }
         }
-        hcheck(hipStreamSynchronize(e->stream), "sync");
     });
 }
 
@@ -1429,14 +1630,31 @@ int idb_encoder_loss_grad(idb_encoder *e, const idb_dataset *d, const uint32_t *
     return guard(e, [&] {
         for (uint32_t i = 0; i < 2 * n_pairs; ++i)
             if (pairs[i] >= d->n_rows) throw Fail{IDB_ERR_ARG, "pair row out of range"};
-        DevData dd;
-        const idb_dataset *dv = device_view(d, dd, e->stream);
-        const uint32_t *pd = dd.up(pairs, 2 * (size_t)n_pairs, e->stream);
-        const float *ld = dd.up(labels, n_pairs, e->stream);
+        Upload up(e);
+        idb_dataset v;
+        const uint32_t *pd = nullptr;
+        const float *ld = nullptr;
+        up.add_rows(d, v);
+        up.add(pairs, 2 * (size_t)n_pairs, &pd);
+        up.add(labels, (size_t)n_pairs, &ld);
+        const Drain drain{e};
         ensure_workspace(e, 2 * n_pairs);
-        *loss = step(e, dv, pd, ld, nullptr, 0, n_pairs, margin, 1.f / (float)n_pairs, true);
-        hcheck(hipMemcpyAsync(grad_host, e->grad, sizeof(float) * N_PARAMS, hipMemcpyDeviceToHost, e->stream), "copy");
-        hcheck(hipStreamSynchronize(e->stream), "sync");
+        up.run();
+        (void)step(e, &v, pd, ld, nullptr, 0, n_pairs, margin, 1.f / (float)n_pairs, false);
+        const size_t bytes = sizeof(float) * (N_PARAMS + 1);
+        const CopyPool::Job present{grad_host, nullptr, bytes - sizeof(float)};
+        CopyPool::get().run(&present, 1);  // the caller's pages, while the GPU computes
+        if (pinned(&e->ring, &e->ring_cap, bytes)) {
+            hcheck(hipMemcpyAsync(e->ring, e->grad, bytes, hipMemcpyDeviceToHost, e->stream), "copy");
+            hcheck(hipStreamSynchronize(e->stream), "sync");
+            std::memcpy(loss, e->ring + bytes - sizeof(float), sizeof(float));
+            const CopyPool::Job job{grad_host, e->ring, bytes - sizeof(float)};
+            CopyPool::get().run(&job, 1);
+        } else {
+            hcheck(hipMemcpyAsync(loss, e->grad + N_PARAMS, sizeof(float), hipMemcpyDeviceToHost, e->stream), "copy");
+            hcheck(hipMemcpyAsync(grad_host, e->grad, bytes - sizeof(float), hipMemcpyDeviceToHost, e->stream), "copy");
+            hcheck(hipStreamSynchronize(e->stream), "sync");
+        }
     });
 }
 

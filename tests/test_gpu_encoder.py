@@ -68,3 +68,20 @@ def test_embeddings_follow_new_parameters(gpu_ctx):
     b.set_params(a.get_params())
     zt = a.embed(rep)
     assert np.array_equal(zt, b.embed(rep)) and not np.array_equal(zt, zb)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [4096, 4097, 40_961])
+def test_segmented_embeddings(gpu_ctx, n):
+    """Calls of one segment, of a last segment of one row, and of more
+    segments than are staged at a time: bit for bit those of short calls."""
+    from immunodbscan_amd import learned
+
+    rep = synth.generate(configs.c2_params(n_rows=n, n_seeds=n // 10, seed=12))
+    enc = learned.Encoder(learned.vocab_for(synth.LETTERS[synth.AA]), seed=3)
+    z = enc.embed(rep)
+    part = learned.Encoder(learned.vocab_for(synth.LETTERS[synth.AA]), seed=3)
+    for a in range(0, n, 3000):
+        rows = np.arange(a, min(n, a + 3000))
+        assert np.array_equal(part.embed(rep.subset(rows)), z[rows]), a
+    assert np.array_equal(enc.embed(rep), z)

@@ -76,7 +76,7 @@ enum Slot {
     S_KEY, S_GSLOT, S_HTAB, S_REP, S_COPIES, S_CNT, S_CORE, S_PAR, S_BMIN,
     S_FLAG, S_UNIQ, S_NUM, S_MEMB, S_EOFF, S_EKEY, S_EROW, S_EKEY2, S_EROW2,
     S_ELEN, S_ECP, S_ECHK, S_ECODES, S_EPK, S_BSTART, S_QBOFF, S_TCNT, S_TOFF, S_TILES,
-    S_LAB, S_RANK, S_RFLAG, S_QBCNT, S_BFLAG, S_TLUT_C, S_SMALL, S_WORK, S_TMP,
+    S_LAB, S_RANK, S_RFLAG, S_QBCNT, S_BFLAG, S_TLUT_C, S_SMALL, S_TMP,
     S_OUT_CID, S_OUT_CORE, S_OUT_COP, S_OUT_UNQ, S_OUT_CNT, S_USTART, S_EDGES, S_ENT, S_FILL, S_ZB, S_PAIRS,
     S_DIST, S_CNT2, S_EQG, S_RSCNT, S_PE, S_PARE, S_CMINE, S_GCALLS, S_GOFF, S_GLEN, S_GOUT, S_GHDR, S_GWORDS,
     S_ELOW, S_SCAN, S_ROWREC, S_META, S_FEAT, S_VREC, S_INV, S_CNTE, S_ECORE, S_COUNT
@@ -96,8 +96,8 @@ struct idb_ctx {
     // Pinned staging of host-memory inputs and outputs (grown on demand).
     uint8_t *xfer = nullptr;
     size_t xfer_cap = 0;
-    hipEvent_t ev[IDB_N_STAGES + 1] = {};
-    hipEvent_t kev[4] = {};       // around the count and the fuse kernels
+    hipEvent_t kev[6] = {};       // around the count and the fuse kernels and the embedding (learned, tuned, pair-list runs)
+    int clock_khz = 100000;       // rate of the device's wall clock
     // autotuner: best count-kernel launch shape per kernel and shape class
     struct Tuned {
         uint32_t wpb, grid_mul, no_xcd, trials;
@@ -382,7 +382,7 @@ __global__ void k_dedup_insert(const uint8_t *seq, const uint64_t *off, const ui
 __global__ void k_dedup_resolve(const uint2 *tab, const uint32_t *gslot, uint32_t n, uint32_t *rep, uint32_t *copies,
                                 uint8_t *flag, int32_t *cnt, uint32_t *par, uint32_t *bmin, uint32_t *rflag,
                                 uint32_t *pe, const uint64_t *off, const int32_t *vb, uint32_t vw, const int32_t *jb,
-                                uint32_t jw, uint4 *rrec)
+                                uint32_t jw, uint4 *rrec, unsigned long long *stamps)
 {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint2 g = tab[gslot[i]];
@@ -404,6 +404,7 @@ __global__ void k_dedup_resolve(const uint2 *tab, const uint32_t *gslot, uint32_
         rflag[i] = 0u;
         pe[i] = IDB_NONE;
     }
+    idb_stamp_end(stamps + IDB_T_DEDUP);
 }
 
 __device__ __forceinline__ uint32_t popc_words(const int32_t *w, uint32_t n)
@@ -414,8 +415,10 @@ __device__ __forceinline__ uint32_t popc_words(const int32_t *w, uint32_t n)
 }
 
 __global__ void k_membership(const uint32_t *uniq, const uint32_t *num, const int32_t *vb, uint32_t vw,
-                             const int32_t *jb, uint32_t jw, uint32_t single, uint32_t cap, uint64_t *memb)
+                             const int32_t *jb, uint32_t jw, uint32_t single, uint32_t cap, uint64_t *memb,
+                             unsigned long long *stamps)
 {
+    idb_stamp_start(stamps ? stamps + IDB_T_UNIQ : nullptr);
     const uint32_t U = num[0];
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k <= cap; k += gridDim.x * blockDim.x) {
         if (k >= U) {
@@ -432,8 +435,12 @@ __global__ void k_membership(const uint32_t *uniq, const uint32_t *num, const in
 __global__ void k_emit_entries(const uint32_t *uniq, const uint32_t *num, const uint64_t *eoff, const int32_t *vb,
                                uint32_t vw, const int32_t *jb, uint32_t jw, const uint32_t *len, const uint32_t *rid,
                                uint32_t single, uint32_t gj, uint32_t gvj, uint32_t lb, uint64_t *ekey, uint32_t *erow,
-                               uint4 *rrec)
+                               uint4 *rrec, const uint32_t *lut_host, uint32_t lut_words, uint32_t *lut)
 {
+    // the length tables and the letter map, from pinned memory, for the
+    // kernels after this one
+    if (blockIdx.x == gridDim.x - 1)
+        for (uint32_t k = threadIdx.x; k < lut_words; k += blockDim.x) lut[k] = lut_host[k];
     const uint32_t U = num[0];
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < U; k += gridDim.x * blockDim.x) {
         const uint32_t u = uniq[k];
@@ -760,33 +767,74 @@ __global__ void k_tile_counts(const uint32_t *qboff, const uint32_t *nb_dev, con
     }
 }
 
-// Sizes the host needs, gathered on the device so that one read-back brings
-// them: sz[0..1] = entries (eoff[U], when there are bucket memberships),
-// sz[5] = uniques; later sz[2] = buckets, sz[3] = query blocks, sz[4] and
-// sz[6] = tiles (low and high words).
-__global__ void k_size_entries(const uint64_t *eoff, const uint32_t *num, uint32_t *sz)
+// Sizes the host needs, gathered so that one wait brings them: small[100, 102)
+// = entries (eoff[U], when there are bucket memberships), small[105] =
+// uniques; later small[102] = buckets, [103] = query blocks, [104] and [106] =
+// tiles (low and high words).
+// One block; small[0, IDB_SMALL_READ) with these sizes also goes to `host`
+// (pinned memory): a copy command for it took 5 to 8 us more per read-back.
+__global__ __launch_bounds__(256) void k_size_entries(const uint64_t *eoff, const uint32_t *num, uint32_t *small,
+                                                      uint32_t *host, unsigned long long *stamps)
 {
-    const uint32_t U = num[0];
+    const uint32_t i = threadIdx.x, U = num[0];
     const uint64_t e = eoff ? eoff[U] : 0u;
-    sz[0] = (uint32_t)e;
-    sz[1] = (uint32_t)(e >> 32);
-    sz[5] = U;
+    uint32_t v = i < IDB_SMALL_READ ? small[i] : 0u;
+    if (i == 100) v = (uint32_t)e;
+    if (i == 101) v = (uint32_t)(e >> 32);
+    if (i == 105) v = U;
+    if (i >= 100 && i < 106) small[i] = v;
+    if (i < IDB_SMALL_READ) host[i] = v;
+    if (i == 0 && !eoff) stamps[IDB_T_UNIQ] = wall_clock64();
 }
 
-__global__ void k_size_tiles(const uint32_t *num, const uint32_t *qboff, const uint64_t *toff, uint32_t *sz)
+__global__ void k_size_tiles(const uint32_t *num, const uint32_t *qboff, const uint64_t *toff, uint32_t *sz,
+                             uint32_t *host)
 {
     const uint32_t B = num[1], QB = qboff[B];
     const uint64_t T = toff[QB];
-    sz[2] = B;
-    sz[3] = QB;
-    sz[4] = (uint32_t)T;
-    sz[6] = (uint32_t)(T >> 32);
+    host[0] = sz[2] = B;
+    host[1] = sz[3] = QB;
+    host[2] = sz[4] = (uint32_t)T;
+    host[3] = sz[5];
+    host[4] = sz[6] = (uint32_t)(T >> 32);
+}
+
+// A run's first kernel: its small words cleared, its first time stamp.
+__global__ __launch_bounds__(256) void k_begin(uint32_t *small)
+{
+    for (uint32_t i = threadIdx.x; i < IDB_SMALL_TOTAL; i += 256) small[i] = 0u;
+    __syncthreads();
+    if (threadIdx.x == 0) ((unsigned long long *)(small + IDB_SMALL_STAMPS))[IDB_T_BEGIN] = wall_clock64();
+}
+
+// A run's last kernel: everything the host reads of it, in pinned memory
+// (four copies of a few words into pageable memory and one more after the
+// last wait took 20 to 50 us each).
+__global__ __launch_bounds__(256) void k_finish(const uint32_t *small, const uint32_t *n_clusters,
+                                                const uint32_t *scan_err, const uint32_t *ustart, uint32_t n_ustart,
+                                                uint32_t *host)
+{
+    const uint32_t i = threadIdx.x;
+    host[i] = small[i];  // IDB_SMALL_WORDS
+    const unsigned long long *work = (const unsigned long long *)(small + IDB_SMALL_WORK);
+    unsigned long long *h64 = (unsigned long long *)(host + IDB_FIN_WORK);
+    if (i < IDB_WORK_U64) {
+        unsigned long long t = 0;
+        for (uint32_t k = 0; k < IDB_WORK_COPIES; ++k) t += work[k * IDB_WORK_U64 + i];
+        h64[i] = t;
+    }
+    if (i < IDB_N_STAMPS)
+        h64[IDB_WORK_U64 + i] = i == IDB_T_END ? (unsigned long long)wall_clock64()
+                                               : ((const unsigned long long *)(small + IDB_SMALL_STAMPS))[i];
+    if (i == 0) host[IDB_FIN_ERR] = *scan_err;
+    if (i == 1) host[IDB_FIN_CLUSTERS] = *n_clusters;
+    for (uint32_t k = i; k < n_ustart; k += 256) host[IDB_FIN_USTART + k] = ustart[k];
 }
 
 __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, const uint32_t *bstart, uint32_t E,
                              const uint16_t *elen, const uint16_t *hilen, uint32_t banded, uint32_t split,
                              const uint64_t *ekey, uint32_t lb, uint32_t gvj, const uint64_t *toff, idb_tile *tiles,
-                             uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t chunk_base)
+                             uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t chunk_base, unsigned long long *stamps)
 {
     // the pair list's chunks that belong to the count pass's waves
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < chunk_base; i += gridDim.x * blockDim.x) {
@@ -823,6 +871,7 @@ __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, cons
             tiles[o++] = t;
         }
     }
+    idb_stamp_end(stamps + IDB_T_TILES);
 }
 
 // The pair list's starting state (k_emit_tiles writes it too).
@@ -855,6 +904,8 @@ __device__ __forceinline__ void block_add(uint32_t v, uint32_t *dst)
 __global__ void k_core_flags(const int32_t *cnt, uint32_t n, int32_t minpts, int32_t *core, uint32_t *pe,
                              uint32_t *small)
 {
+    unsigned long long *stamps = (unsigned long long *)(small + IDB_SMALL_STAMPS);
+    idb_stamp_start(stamps + IDB_T_COUNT);
     uint32_t local = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const int32_t c = cnt[i] >= minpts;
@@ -866,6 +917,7 @@ __global__ void k_core_flags(const int32_t *cnt, uint32_t n, int32_t minpts, int
         local += (uint32_t)c;
     }
     block_add(local, small + IDB_SMALL_CORES + (blockIdx.x & 15u));  // 16 counters
+    idb_stamp_end(stamps + IDB_T_CORE);
 }
 
 __device__ __forceinline__ uint32_t find_root(const uint32_t *par, uint32_t x)
@@ -881,8 +933,10 @@ __device__ __forceinline__ uint32_t find_root(const uint32_t *par, uint32_t x)
 // R9/R10: label root of every unique row (its component root, its border
 // core's root, or none) and root flags for R12.
 __global__ void k_roots(const uint32_t *uniq, const uint32_t *num, const int32_t *core, const uint32_t *par,
-                        const uint32_t *bmin, uint32_t *lab, uint32_t *rflag, uint32_t n)
+                        const uint32_t *bmin, uint32_t *lab, uint32_t *rflag, uint32_t n,
+                        unsigned long long *stamps)
 {
+    idb_stamp_start(stamps + IDB_T_GROW);
     const uint32_t U = num[0];
     if (blockIdx.x == 0 && threadIdx.x == 0) rflag[n] = 0u;  // the renumbering scan's last slot
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < U; k += gridDim.x * blockDim.x) {
@@ -931,6 +985,8 @@ __global__ void k_labels(const uint32_t *rep, const uint32_t *lab, const uint32_
                          uint32_t n, uint32_t *cid, int32_t *core_out, uint32_t *cop_out, uint32_t *cnt_out,
                          uint32_t *unq_out, uint32_t *small)
 {
+    unsigned long long *stamps = (unsigned long long *)(small + IDB_SMALL_STAMPS);
+    idb_stamp_start(stamps + IDB_T_ROOTS);
     uint32_t noise = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint32_t l = lab[rep[i]];
@@ -947,6 +1003,7 @@ __global__ void k_labels(const uint32_t *rep, const uint32_t *lab, const uint32_
         if (unq_out) unq_out[i] = 0u;  // the uniques' positions are written next
     }
     block_add(noise, small + IDB_SMALL_NOISE + (blockIdx.x & 15u));  // 16 counters
+    idb_stamp_end(stamps + IDB_T_LABELS);
 }
 
 // First unique position of every repertoire (binary search over uniques).
@@ -1029,6 +1086,14 @@ void *scan_workspace(idb_ctx *c, uint64_t max_n)
         c->scan_gen = 0;
     }
     return w;
+}
+
+// What the last kernel wrote to the context's pinned read-back area.
+void wait_pinned(idb_ctx *c, void *dst, size_t bytes)
+{
+    check(c, hipGetLastError(), "launch");
+    check(c, hipStreamSynchronize(c->stream), "readback sync");
+    std::memcpy(dst, c->pinned, bytes);
 }
 
 // Small read-backs go through the context's pinned staging area (a direct
@@ -1136,7 +1201,7 @@ unsigned bits_for(uint64_t v)
     return b;
 }
 
-void record(idb_ctx *c, int k) { check(c, hipEventRecord(c->ev[k], c->stream), "event record"); }
+
 
 // roctx ranges named after the reference's stage timers
 // (cuda/PSDBSCAN.hcu:1301-1354): one outer range for the whole run and one
@@ -1251,7 +1316,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
 {
     const bool learned = x && x->enc;
     const bool force_large = (p->flags & IDB_FLAG_FORCE_LARGE_PATHS) != 0;
-    float encoder_ms = 0.f;
     const uint32_t N = d->n_rows;
     const uint32_t vw = d->v_width, jw = d->j_width;
     if (o->mem != IDB_MEM_HOST && o->mem != IDB_MEM_DEVICE) fail(c, IDB_ERR_ARG, "outputs.mem must be host or device");
@@ -1273,8 +1337,13 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         return;
     }
     hipStream_t s = c->stream;
-    record(c, 0);
     StageRanges rng;
+    // the run's small words, statistics and time stamps, cleared
+    uint32_t *small = buf<uint32_t>(c, S_SMALL, IDB_SMALL_TOTAL);
+    unsigned long long *stamps = (unsigned long long *)(small + IDB_SMALL_STAMPS);
+    unsigned long long *work = (unsigned long long *)(small + IDB_SMALL_WORK);
+    uint32_t *pin = (uint32_t *)c->pinned;
+    hipLaunchKernelGGL(k_begin, dim3(1), dim3(256), 0, s, small);
     // scans run over at most N + 1 rows or E + 1 entries, E <= 4N + 4096
     c->scan_ws = scan_workspace(c, 4ull * N + 4098);
     rng.stage("Identify Duplicates");
@@ -1297,8 +1366,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
     }
 
     // --- Identify Duplicates
-    uint32_t *small = buf<uint32_t>(c, S_SMALL, IDB_SMALL_WORDS);
-    check(c, hipMemsetAsync(small, 0, IDB_SMALL_WORDS * sizeof(uint32_t), s), "memset");
     uint64_t *key = buf<uint64_t>(c, S_KEY, N);
     // 32 key bits are plenty to group duplicates (colliding rows are told apart
     // by the byte comparison)
@@ -1323,15 +1390,13 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
     // row records for the entry records, when a row's gene words fit in four
     uint4 *rrec = (vw + jw <= 4) ? buf<uint4>(c, S_ROWREC, 2 * (size_t)N) : nullptr;
     hipLaunchKernelGGL(k_dedup_resolve, dim3(blocks_for(N)), dim3(256), 0, s, htab, gslot, N, rep, copies, flag, cnt, par,
-                       bmin, rflag, pe, off, vb, vw, jb, jw, rrec);
-    record(c, 1);
+                       bmin, rflag, pe, off, vb, vw, jb, jw, rrec, stamps);
     rng.stage("Determine copies");
 
     // --- Determine copies: uniques
     uint32_t *uniq = buf<uint32_t>(c, S_UNIQ, N);
     uint32_t *num = buf<uint32_t>(c, S_NUM, 4);
     select_flagged(c, N, flag, uniq, num);
-    record(c, 2);
     rng.stage("Identify core points");
 
     // --- Identify core points: buckets, tiles, count pass
@@ -1345,12 +1410,13 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
     uint32_t E = 0, U = 0;
     if (vw > 0 && jw > 0) {
         hipLaunchKernelGGL(k_membership, dim3(blocks_for((uint64_t)N + 1)), dim3(256), 0, s, uniq, num, vb, vw, jb, jw,
-                           0u, N, memb);
+                           0u, N, memb, stamps);
         exclusive_scan_total<uint64_t>(c, memb, eoff, (size_t)N + 1);
     }
-    hipLaunchKernelGGL(k_size_entries, dim3(1), dim3(64), 0, s, (vw > 0 && jw > 0) ? eoff : nullptr, num, sz);
-    uint32_t hs[IDB_SMALL_GENES + 16];
-    readback(c, hs, small, sizeof(hs));
+    hipLaunchKernelGGL(k_size_entries, dim3(1), dim3(256), 0, s, (vw > 0 && jw > 0) ? eoff : nullptr, num, small, pin,
+                       stamps);
+    uint32_t hs[IDB_SMALL_READ];
+    wait_pinned(c, hs, sizeof(hs));
     uint32_t lw[9] = {};  // letter-set words and the longest row, over the row scan's 8 copies
     for (uint32_t cpy = 0; cpy < 8; ++cpy)
         for (uint32_t t = 0; t < 9; ++t) {
@@ -1410,7 +1476,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         if (vw > 0 && jw > 0 && (E64 > 4ull * U + 4096 || gvj64 * std::max(n_reps, 1u) >= (1ull << 47))) {
             single = 1;
             hipLaunchKernelGGL(k_membership, dim3(blocks_for((uint64_t)N + 1)), dim3(256), 0, s, uniq, num, vb, vw, jb,
-                               jw, 1u, N, memb);
+                               jw, 1u, N, memb, (unsigned long long *)nullptr);
             exclusive_scan_total<uint64_t>(c, memb, eoff, (size_t)N + 1);
             E64 = U;
         }
@@ -1441,9 +1507,10 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         }
         hl[l] = (int16_t)std::min<uint32_t>(h, 32767u);
     }
-    // the three length tables and the letter map in one upload from pinned
-    // memory: [count t | fuse t | band end] as int16 per length, then 256 codes
-    const size_t tl = sizeof(int16_t) * (maxlen + 1), lut_bytes = 3 * tl + 256;
+    // the three length tables and the letter map, taken up from pinned memory
+    // by k_emit_entries: [count t | fuse t | band end] as int16 per length, then 256 codes
+    const size_t tl = sizeof(int16_t) * (maxlen + 1), lut_bytes = (3 * tl + 256 + 3) & ~(size_t)3;
+    const uint32_t lut_words = (uint32_t)(lut_bytes / 4);
     uint8_t *lut = buf<uint8_t>(c, S_TLUT_C, lut_bytes);
     int16_t *tlut_c = (int16_t *)lut, *tlut_f = (int16_t *)(lut + tl);
     uint16_t *hilen = (uint16_t *)(lut + 2 * tl);
@@ -1454,11 +1521,9 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         std::memcpy(up + tl, tf.data(), tl);
         std::memcpy(up + 2 * tl, hl.data(), tl);
         std::memcpy(up + 3 * tl, cmap_h, 256);
-        check(c, hipMemcpyAsync(lut, up, lut_bytes, hipMemcpyHostToDevice, s), "lut");
     }
+    const uint32_t *lut_up = (const uint32_t *)((uint8_t *)c->pinned + IDB_STAGE_BYTES);
 
-    unsigned long long *work = buf<unsigned long long>(c, S_WORK, IDB_WORK_U64 * IDB_WORK_COPIES);
-    check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "memset");
     unsigned long long edge_cap = 0;
     uint32_t B = 0, T = 0;
     idb_pair_args a{};
@@ -1469,7 +1534,8 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         uint32_t *erow = buf<uint32_t>(c, S_EROW, E), *erow2 = buf<uint32_t>(c, S_EROW2, E);
         const uint32_t lb = std::max(1u, bits_for(maxlen));
         hipLaunchKernelGGL(k_emit_entries, dim3(blocks_for(U)), dim3(256), 0, s, uniq, num, eoff, vb, vw, jb, jw, len, rid,
-                           single, gj, gvj, lb, ekey, erow, rrec);
+                           single, gj, gvj, lb, ekey, erow, rrec, lut_up,
+                           lut_words, (uint32_t *)lut);
         const uint64_t max_bucket = single ? std::max(n_reps, 1u) : gvj64 * std::max(n_reps, 1u);
         const unsigned ebits = lb + bits_for(max_bucket);
         bool sorted = false, in_first = false;
@@ -1533,6 +1599,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             mr.ecore = buf<uint8_t>(c, S_ECORE, E);
             mr.par_e = par_e;
             mr.n_cores = small + IDB_SMALL_CORES;
+            mr.stamps = stamps;
             ua.ecore = mr.ecore;
             ua.erow = srow;
             a.mx_planes = planes;
@@ -1577,9 +1644,9 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         hipLaunchKernelGGL(k_tile_counts, dim3(blocks_for((uint64_t)E + 1)), dim3(256), 0, s, qboff, num + 1, bstart, E,
                            elen, hilen, banded ? 1u : 0u, qsplit, tcount);
         exclusive_scan_total<uint64_t>(c, tcount, toff, (size_t)E + 1);
-        hipLaunchKernelGGL(k_size_tiles, dim3(1), dim3(64), 0, s, num, qboff, toff, sz);
+        hipLaunchKernelGGL(k_size_tiles, dim3(1), dim3(64), 0, s, num, qboff, toff, sz, pin);
         uint32_t bqt[5];  // sz[2 .. 6]: buckets, query blocks, tiles (low), uniques, tiles (high)
-        readback(c, bqt, sz + 2, sizeof(bqt));
+        wait_pinned(c, bqt, sizeof(bqt));
         B = bqt[0];
         const uint64_t T64 = (uint64_t)bqt[2] | ((uint64_t)bqt[4] << 32);
         // Tile indices are 32-bit in the pair kernels, and a wave's next
@@ -1650,16 +1717,14 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                                                     a.max_chunks / 4);
         hipLaunchKernelGGL(k_emit_tiles, dim3(blocks_for(std::max<uint64_t>(bqt[1], a.chunk_base))), dim3(256), 0, s,
                            qboff, num + 1, bstart, E, elen, hilen, banded ? 1u : 0u, qsplit, skey, lb, gvj, toff, tiles,
-                           a.n_chunks, a.chunk_fill, a.chunk_base);
+                           a.n_chunks, a.chunk_fill, a.chunk_base, stamps);
         if (learned) {
             // embeddings of every row, then proposals verified by Myers
             uint16_t *zb = buf<uint16_t>(c, S_ZB, (size_t)N * 64);
-            check(c, hipEventRecord(c->kev[2], s), "event record");
+            check(c, hipEventRecord(c->kev[4], s), "event record");
             if (idb_encoder_embed_rows(x->enc, seq, off, len, N, zb, s) != hipSuccess)
                 fail(c, IDB_ERR_HIP, std::string("encoder: ") + idb_encoder_error(x->enc));
-            check(c, hipEventRecord(c->kev[3], s), "event record");
-            check(c, hipEventSynchronize(c->kev[3]), "event sync");
-            check(c, hipEventElapsedTime(&encoder_ms, c->kev[2], c->kev[3]), "event time");
+            check(c, hipEventRecord(c->kev[5], s), "event record");
             a.zb = zb;
             a.min_sim = x->min_sim;
         }
@@ -1682,7 +1747,9 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
     // the side stream into their places in the pinned staging while the
     // clustering runs, so that only clone ids (and counts) are left for the
     // end.
-    const bool early_out = !dev_out && c->side && xfer_ready(c, ob * n_out);
+    // A megabyte of outputs is where this starts to pay: the copies, events and
+    // waits take some 40 us of the host, the transfer of 1 MB 25 us.
+    const bool early_out = !dev_out && c->side && ob * n_out > (1u << 20) && xfer_ready(c, ob * n_out);
     if (early_out) {
         check(c, hipMemsetAsync(unq_o, 0, sizeof(uint32_t) * N, s), "memset");
         if (n_reps > 0)
@@ -1701,16 +1768,20 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
     // grows it and runs the learned pass again (below).
     const bool graph = (p->flags & IDB_FLAG_GRAPH) && !(x && x->pairs_out) && !learned;
     bool from_edges = false;
+    // Kernel times by events where passes are repeated or something runs between
+    // them; by the kernels' own time stamps otherwise (an event leaves a gap of
+    // about 5 us on the stream).
+    const bool ev_times = learned || (x && x->pairs_out) || (p->flags & IDB_FLAG_AUTOTUNE);
 
     // Everything after the sizing steps.  As a graph (g) the union / fuse
     // choice is made on the device (each kernel checks the chunk counter) and
     // no event is recorded inside.
     auto tail = [&](bool g) {
         if (E > 0) {
-            if (!g) check(c, hipEventRecord(c->kev[0], s), "event record");
+            if (!g && ev_times) check(c, hipEventRecord(c->kev[0], s), "event record");
             if (learned) check(c, idb_launch_count_learned(a, s), "learned count kernel launch");
             else check(c, ham ? idb_launch_count_hamming(a, s) : idb_launch_count_myers(a, W, s), "count kernel launch");
-            if (!g) check(c, hipEventRecord(c->kev[1], s), "event record");
+            if (!g && ev_times) check(c, hipEventRecord(c->kev[1], s), "event record");
         }
         if (mr.inv) {
             mr.core = core;
@@ -1725,7 +1796,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             check(c, hipMemcpyAsync(c->xfer + ob, core, sizeof(int32_t) * N, hipMemcpyDeviceToHost, c->side),
                   "output copy");
         }
-        if (!g) record(c, 3);
         rng.stage("Grow clusters");
 
         // --- Grow clusters: union over the recorded neighbour pairs, or a
@@ -1743,13 +1813,13 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             // growth; the host learns which ran from the final statistics.
             // Learned runs and callers of the pair list decide on the host.
             if (g || !(learned || (x && x->pairs_out))) {
-                if (!g) check(c, hipEventRecord(c->kev[2], s), "event record");
+                if (!g && ev_times) check(c, hipEventRecord(c->kev[2], s), "event record");
                 check(c, idb_launch_union_edges(a, ua, s), "union kernel launch");
                 if (!learned) {
                     f.fuse_if_overflow = 1;
                     check(c, ham ? idb_launch_fuse_hamming(f, s) : idb_launch_fuse_myers(f, W, s), "fuse kernel launch");
                 }
-                if (!g) check(c, hipEventRecord(c->kev[3], s), "event record");
+                if (!g && ev_times) check(c, hipEventRecord(c->kev[3], s), "event record");
             } else {
                 uint32_t n_chunks = 0;
                 readback(c, &n_chunks, small + 12, sizeof(n_chunks));
@@ -1814,15 +1884,14 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                 check(c, hipEventRecord(c->kev[3], s), "event record");
             }
         }
-        if (!g) record(c, 4);
         rng.stage("Reduction of cluster information tree structure");
 
         // --- Reduction of cluster information tree structure
-        hipLaunchKernelGGL(k_roots, dim3(blocks_for(U)), dim3(256), 0, s, uniq, num, core, par, bmin, lab, rflag, N);
+        hipLaunchKernelGGL(k_roots, dim3(blocks_for(U)), dim3(256), 0, s, uniq, num, core, par, bmin, lab, rflag, N,
+                           stamps);
         if (p->tree_stats)
             hipLaunchKernelGGL(k_tree_depth, dim3(blocks_for(N)), dim3(256), 0, s, rep, core, par, bmin, N, small + 16,
                                small + 12, a.max_chunks, E > 0 ? 1u : 0u);
-        if (!g) record(c, 5);
         rng.stage("Re-number clusters and identify noise");
 
         // --- Re-number clusters and identify noise
@@ -1838,7 +1907,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                                unq_o);
         }
         check(c, hipGetLastError(), "tail launch");
-        if (!g) record(c, 6);
     };
 
     if (graph) {
@@ -1872,7 +1940,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         }
         (void)hipGraphDestroy(gr);
         check(c, hipGraphLaunch(c->gexec, s), "graph launch");
-        for (int k = 3; k <= 6; ++k) record(c, k);
     } else {
         tail(false);
     }
@@ -1897,21 +1964,24 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             check(c, hipMemcpyAsync(o->neighbour_count, cnt_o, sizeof(uint32_t) * N, hipMemcpyDeviceToHost, s),
                   "output copy");
     }
-    record(c, 7);
+    // (more repertoires than the read-back area holds come in a copy of their own)
+    const bool us_pinned = n_reps + 1ull <= IDB_FIN_USTART_MAX;
     std::vector<uint32_t> us;
-    if (n_reps > 0) {
-        us.resize(n_reps + 1);
+    if (n_reps > 0) us.resize(n_reps + 1);
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(256), 0, s, small, rank + N,
+                       (const uint32_t *)((uint8_t *)c->scan_ws + idb_scan_error_offset()), ustart,
+                       n_reps > 0 && us_pinned ? n_reps + 1 : 0u, pin);
+    check(c, hipGetLastError(), "finish launch");
+    if (n_reps > 0 && !us_pinned)
         check(c, hipMemcpyAsync(us.data(), ustart, sizeof(uint32_t) * (n_reps + 1), hipMemcpyDeviceToHost, s), "ustart");
-    }
-    uint32_t fin[IDB_SMALL_WORDS];
-    unsigned long long wkc[IDB_WORK_U64 * IDB_WORK_COPIES], wk[IDB_WORK_U64] = {};
-    check(c, hipMemcpyAsync(fin, small, sizeof(fin), hipMemcpyDeviceToHost, s), "stats");
-    check(c, hipMemcpyAsync(wkc, work, sizeof(wkc), hipMemcpyDeviceToHost, s), "stats");
-    uint32_t scan_err = 0;
-    check(c, hipMemcpyAsync(&scan_err, (uint8_t *)c->scan_ws + idb_scan_error_offset(), sizeof(scan_err),
-                            hipMemcpyDeviceToHost, s), "stats");
     check(c, hipStreamSynchronize(s), "final sync");
     if (early_out) check(c, hipStreamSynchronize(c->side), "final sync");
+    const uint32_t *fin = pin;
+    unsigned long long wk[IDB_WORK_U64], ts[IDB_N_STAMPS];
+    std::memcpy(wk, pin + IDB_FIN_WORK, sizeof(wk));
+    std::memcpy(ts, (uint8_t *)(pin + IDB_FIN_WORK) + sizeof(wk), sizeof(ts));
+    if (n_reps > 0 && us_pinned) std::memcpy(us.data(), pin + IDB_FIN_USTART, sizeof(uint32_t) * (n_reps + 1));
+    const uint32_t scan_err = pin[IDB_FIN_ERR], n_clusters = pin[IDB_FIN_CLUSTERS];
     if (scan_err) fail(c, IDB_ERR_HIP, "a scan's look-back did not end (the run's sizes are not valid)");
     if (staged_out) {
         CopyPool::Job jobs[5] = {{o->clone_id, c->xfer, (size_t)N * 4}, {o->core, c->xfer + ob, (size_t)N * 4},
@@ -1919,7 +1989,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                                  {o->neighbour_count, c->xfer + 4 * ob, (size_t)N * 4}};
         CopyPool::get().run(jobs, n_out);
     }
-    for (uint32_t k = 0; k < IDB_WORK_U64 * IDB_WORK_COPIES; ++k) wk[k % IDB_WORK_U64] += wkc[k];
     if (E > 0 && (graph || !(learned || (x && x->pairs_out)))) {
         from_edges = fin[12] <= a.max_chunks;
         if (learned && !from_edges)
@@ -1928,6 +1997,9 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
     if (n_uniques_h)
         for (uint32_t r = 0; r < n_reps; ++r) n_uniques_h[r] = us[r + 1] - us[r];
     if (st) {
+        const auto span = [&](int a, int b) {
+            return ts[b] > ts[a] ? (float)((double)(ts[b] - ts[a]) / c->clock_khz) : 0.f;
+        };
         st->n_uniques = U;
         st->n_cores = 0;
         st->n_noise = 0;
@@ -1956,27 +2028,27 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             for (const auto &kv : c->tuned)
                 if (kv.second.wpb == a.tune_wpb && kv.second.grid_mul == a.tune_grid_mul) st->tuned_trials = kv.second.trials;
         st->graph_used = graph ? 1u : 0u;
-        st->encoder_ms = encoder_ms;
+        if (learned && E > 0) (void)hipEventElapsedTime(&st->encoder_ms, c->kev[4], c->kev[5]);
         if (E > 0 && T > 0 && !graph) {
-            (void)hipEventElapsedTime(&st->count_kernel_ms, c->kev[0], c->kev[1]);
-            (void)hipEventElapsedTime(&st->fuse_kernel_ms, c->kev[2], c->kev[3]);
+            if (ev_times) {
+                (void)hipEventElapsedTime(&st->count_kernel_ms, c->kev[0], c->kev[1]);
+                (void)hipEventElapsedTime(&st->fuse_kernel_ms, c->kev[2], c->kev[3]);
+            } else {
+                st->count_kernel_ms = span(IDB_T_TILES, IDB_T_COUNT);
+                st->fuse_kernel_ms = span(IDB_T_CORE, IDB_T_GROW);
+            }
         }
         if (p->tree_stats)
             for (int k = 0; k <= 50; ++k) st->tree_depth[k] = fin[16 + k];
         // Stage slots follow the reference's timers; duplicate-tree reduction
         // is part of the duplicate stage here (representatives are direct).
+        // A graph's time is the core-point stage's.
+        if (graph) ts[IDB_T_CORE] = ts[IDB_T_GROW] = ts[IDB_T_ROOTS] = ts[IDB_T_LABELS];
+        const int at[8] = {IDB_T_BEGIN, IDB_T_DEDUP, IDB_T_UNIQ, IDB_T_CORE, IDB_T_GROW, IDB_T_ROOTS, IDB_T_LABELS, IDB_T_END};
         const int from[8] = {0, 1, 1, 2, 3, 4, 5, 0}, to[8] = {1, 1, 2, 3, 4, 5, 6, 7};
-        for (int k = 0; k < 8; ++k) {
-            float ms = 0.f;
-            if (from[k] != to[k]) (void)hipEventElapsedTime(&ms, c->ev[from[k]], c->ev[to[k]]);
-            st->stage_ms[k] = ms;
-        }
+        for (int k = 0; k < 8; ++k) st->stage_ms[k] = from[k] != to[k] ? span(at[from[k]], at[to[k]]) : 0.f;
     }
-    if (st) {
-        uint32_t ncl = 0;
-        check(c, hipMemcpy(&ncl, rank + N, sizeof(uint32_t), hipMemcpyDeviceToHost), "stats");
-        st->n_clusters = ncl;
-    }
+    if (st) st->n_clusters = n_clusters;
 }
 
 }  // namespace
@@ -2005,12 +2077,9 @@ int idb_create(idb_ctx **out, int device)
         delete c;
         return IDB_ERR_HIP;
     }
-    for (int k = 0; k <= IDB_N_STAGES; ++k)
-        if (hipEventCreate(&c->ev[k]) != hipSuccess) {
-            delete c;
-            return IDB_ERR_HIP;
-        }
-    for (int k = 0; k < 4; ++k)
+    (void)hipDeviceGetAttribute(&c->clock_khz, hipDeviceAttributeWallClockRate, device);
+    if (c->clock_khz <= 0) c->clock_khz = 100000;
+    for (int k = 0; k < 6; ++k)
         if (hipEventCreate(&c->kev[k]) != hipSuccess) {
             delete c;
             return IDB_ERR_HIP;
@@ -2032,9 +2101,7 @@ void idb_destroy(idb_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (int s = 0; s < S_COUNT; ++s)
         if (c->ptr[s]) (void)hipFree(c->ptr[s]);
-    for (int k = 0; k <= IDB_N_STAGES; ++k)
-        if (c->ev[k]) (void)hipEventDestroy(c->ev[k]);
-    for (int k = 0; k < 4; ++k)
+    for (int k = 0; k < 6; ++k)
         if (c->kev[k]) (void)hipEventDestroy(c->kev[k]);
     if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->xfer) (void)hipHostFree(c->xfer);

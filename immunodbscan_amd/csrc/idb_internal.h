@@ -70,7 +70,8 @@ hipError_t idb_sort_small(uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1
 #define IDB_STAGE_BYTES 32768u    // each half of a context's pinned staging area
 #define IDB_XFER_MAX_BYTES (256ull << 20)  // most pinned staging a context keeps for host inputs and outputs
 // The run's small device words (zeroed at the start of a run): [12] chunks
-// handed out, [16, 67) the depth histogram, [100, 106) sizes for the host,
+// handed out, [16, 67) the depth histogram, [68, 88) time stamps, [100, 107)
+// sizes for the host,
 // then 8 copies of the row scan's 9 words (letter set, longest row) and 16
 // partial counts each of core and noise rows (copies keep blocks from
 // queueing their atomics on one word).
@@ -79,12 +80,31 @@ hipError_t idb_sort_small(uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1
 #define IDB_SMALL_NOISE 216u
 #define IDB_SMALL_GENES 232u      // 8 copies of (highest V gene + 1, highest J gene + 1), row scan
 #define IDB_SMALL_WORDS 256u
+#define IDB_SMALL_READ (IDB_SMALL_GENES + 16u)  // words the host reads for the sizing
 // The run's device counters: 8 64-bit statistics
 #define IDB_WORK_U64 8u
 // ... kept in IDB_WORK_COPIES copies (a kernel block adds into copy
 // blockIdx & (copies - 1)), so that the waves' closing atomics do not queue
 // on one word; readers sum the copies.
 #define IDB_WORK_COPIES 16u
+// Time stamps of the device's wall clock among the small words (a kernel's
+// start or end: see idb_stamp_start); the counters behind the small words.
+enum {
+    IDB_T_BEGIN, IDB_T_DEDUP, IDB_T_UNIQ, IDB_T_TILES, IDB_T_COUNT, IDB_T_CORE, IDB_T_GROW, IDB_T_ROOTS, IDB_T_LABELS,
+    IDB_T_END, IDB_N_STAMPS
+};
+#define IDB_SMALL_STAMPS 68u
+#define IDB_SMALL_WORK IDB_SMALL_WORDS
+#define IDB_SMALL_TOTAL (IDB_SMALL_WORK + 2u * IDB_WORK_U64 * IDB_WORK_COPIES)
+// A run's results for the host in pinned memory (words): the small words, the
+// counters' sums and the stamps, the scans' error word, the clusters, then the
+// repertoires' first uniques.
+#define IDB_FIN_WORK IDB_SMALL_WORDS
+#define IDB_FIN_ERR (IDB_FIN_WORK + 64u)
+#define IDB_FIN_CLUSTERS (IDB_FIN_ERR + 1u)
+#define IDB_FIN_USTART (IDB_FIN_ERR + 16u)
+#define IDB_FIN_USTART_MAX (IDB_STAGE_BYTES / 4u - IDB_FIN_USTART)
+static_assert(2 * (IDB_WORK_U64 + IDB_N_STAMPS) <= 64 && IDB_SMALL_READ <= 256 && IDB_SMALL_STAMPS + 2 * IDB_N_STAMPS <= 100, "word layout");
 #define IDB_MAX_W 8               // Myers 32-bit words per pattern (<= 256 letters)
 #define IDB_MAX_HW 64             // Hamming packed words per row
 #define IDB_MAX_LEN 65535u
@@ -160,6 +180,17 @@ struct idb_pair_args {
     // grid_mul, and plain block order instead of the XCD-grouped one
     uint32_t tune_wpb, tune_grid_mul, no_xcd_order;
 };
+
+// Time stamps inside kernels: at the start by the first block, at the end by
+// one block in 32 (the latest counts).
+__device__ __forceinline__ void idb_stamp_start(unsigned long long *at)
+{
+    if (at && blockIdx.x == 0 && threadIdx.x == 0) *at = wall_clock64();
+}
+__device__ __forceinline__ void idb_stamp_end(unsigned long long *at)
+{
+    if ((blockIdx.x & 31u) == 0 && threadIdx.x == 0) atomicMax(at, (unsigned long long)wall_clock64());
+}
 
 // Bytes k .. k+15 of a row of length L as one 16-byte value, zero past the
 // row's end.  Every load stays inside the row: a short tail is read as the
@@ -277,6 +308,7 @@ struct idb_mx_rows_args {
     uint32_t *pe;
     uint8_t *ecore;
     uint32_t *par_e, *n_cores;
+    unsigned long long *stamps;
 };
 hipError_t idb_launch_mx_fill(const idb_mx_fill_args &f, hipStream_t s);
 hipError_t idb_launch_mx_rows(const idb_mx_rows_args &r, hipStream_t s);

@@ -559,8 +559,10 @@ __global__ __launch_bounds__(256) void k_mx_fill(const uint64_t *ekey, const uin
 __global__ __launch_bounds__(256) void k_mx_rows(const uint32_t *uniq, const uint32_t *num, const uint64_t *eoff,
                                                  const uint32_t *inv, const int32_t *cnt_e, const uint32_t *copies,
                                                  uint32_t n, int32_t minpts, int32_t *cnt, int32_t *core, uint32_t *pe,
-                                                 uint8_t *ecore, uint32_t *par_e, uint32_t *n_cores)
+                                                 uint8_t *ecore, uint32_t *par_e, uint32_t *n_cores,
+                                                 unsigned long long *stamps)
 {
+    idb_stamp_start(stamps + IDB_T_COUNT);
     __shared__ uint32_t part[4];
     const uint32_t U = num[0], step = gridDim.x * blockDim.x, i0 = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t local = 0;
@@ -599,6 +601,7 @@ __global__ __launch_bounds__(256) void k_mx_rows(const uint32_t *uniq, const uin
         const uint32_t t = part[0] + part[1] + part[2] + part[3];
         if (t) atomicAdd(n_cores + (blockIdx.x & 15u), t);  // 16 counters
     }
+    idb_stamp_end(stamps + IDB_T_CORE);
 }
 
 template <class G, bool FUSE>
@@ -665,7 +668,7 @@ hipError_t idb_launch_mx_rows(const idb_mx_rows_args &r, hipStream_t s)
 {
     const uint32_t blocks = std::max<uint32_t>(1u, std::min<uint32_t>((r.n + 255u) / 256u, 2048u));
     hipLaunchKernelGGL(k_mx_rows, dim3(blocks), dim3(256), 0, s, r.uniq, r.num, r.eoff, r.inv, r.cnt_e, r.copies, r.n,
-                       r.min_pts, r.cnt, r.core, r.pe, r.ecore, r.par_e, r.n_cores);
+                       r.min_pts, r.cnt, r.core, r.pe, r.ecore, r.par_e, r.n_cores, r.stamps);
     return hipGetLastError();
 }
 

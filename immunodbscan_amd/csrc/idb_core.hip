@@ -1713,7 +1713,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         // start from an empty list); at most a quarter of the list is given
         // out this way, so that partly filled chunks do not make it overflow.
         a.chunk_base = learned ? 0u
-                               : std::min<uint32_t>((uint32_t)std::min<uint64_t>(4ull * T, 32768u),
+                               : std::min<uint32_t>((uint32_t)std::min<uint64_t>(8ull * T, 32768u),
                                                     a.max_chunks / 4);
         hipLaunchKernelGGL(k_emit_tiles, dim3(blocks_for(std::max<uint64_t>(bqt[1], a.chunk_base))), dim3(256), 0, s,
                            qboff, num + 1, bstart, E, elen, hilen, banded ? 1u : 0u, qsplit, skey, lb, gvj, toff, tiles,

@@ -98,6 +98,19 @@ __device__ __forceinline__ void tile_load(const idb_pair_args &a, const idb_tile
     }
 }
 
+// Part ti of the tiles, each taken in 2^sub_log2 parts of its queries: shape
+// bits 17 and up hold the part's first query within the tile.  A part past
+// the tile's queries has none.
+__device__ __forceinline__ idb_tile sub_tile(const idb_pair_args &a, uint32_t ti)
+{
+    idb_tile t = tile_rec(a, ti >> a.sub_log2);
+    const uint32_t part = IDB_TILE >> a.sub_log2, qoff = (ti & ((1u << a.sub_log2) - 1u)) * part;
+    const int32_t rest = (int32_t)(t.shape & 0xFFu) - (int32_t)qoff;  // (signed: see k_mx)
+    t.q0 += qoff;
+    t.shape = (t.shape & 0x1FF00u) | (uint32_t)max(0, min((int32_t)part, rest)) | (qoff << 17);
+    return t;
+}
+
 // Hit bookkeeping of the batched Myers path (one pair per lane).
 // Counts go to the tile's LDS accumulators of query qi and target tl.
 template <bool FUSE>
@@ -491,12 +504,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FILT == 2 &
 
     // static order; the next tile's data and the record of the one after are
     // loaded while the current tile runs
-    const uint32_t T = a.n_tiles;
+    const uint32_t T = a.n_tiles << a.sub_log2;
     uint32_t ti = wave0;
     uint32_t ti1 = step_tile(ti, total_waves, T);
-    idb_tile rec1 = ti1 < T ? tile_rec(a, ti1) : idb_tile{};
+    idb_tile rec1 = ti1 < T ? sub_tile(a, ti1) : idb_tile{};
     TilePre<FILT == 1> cur{};
-    if (ti < T) tile_load<FILT == 1>(a, tile_rec(a, ti), lane, cur);
+    if (ti < T) tile_load<FILT == 1>(a, sub_tile(a, ti), lane, cur);
     const bool wide = a.S > 16;
     while (ti < T) {
         // The tile's records (loaded one tile ago) are waited for once; its
@@ -507,6 +520,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FILT == 2 &
         const idb_tile tile = cur.tile;
         const uint32_t qn = tile.shape & 0xFFu, tn = (tile.shape >> 8) & 0xFFu;
         const bool diag = (tile.shape >> 16) & 1u;
+        const uint32_t qoff = tile.shape >> 17;  // the part's first query within its tile
         const bool tvalid = lane < tn;
         const uint32_t p = tile.t0 + (tvalid ? lane : 0u);
         const idb_entry te = entry_of(cur.te0, cur.te1), qe = entry_of(cur.qe0, cur.qe1);
@@ -560,7 +574,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FILT == 2 &
         uint32_t qlen = 0;  // queued pairs (FILT)
         // query qi pairs with this lane iff qi < dlim (upper triangle on the
         // diagonal tile, nothing past the tile's targets)
-        const uint32_t dlim = !tvalid ? 0u : (diag ? lane : 64u);
+        const uint32_t dlim = !tvalid ? 0u : (diag ? lane - min(lane, qoff) : 64u);
         const uint32_t ny1 = ~te.pres1;
         // per-tile counters fit 32 bits: at most 4096 pairs of 16-bit lengths
         uint32_t tg = 0, tgl = 0, tm = 0;
@@ -604,7 +618,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FILT == 2 &
         TilePre<FILT == 1> nxt{};
         if (ti1 < T) tile_load<FILT == 1>(a, rec1, lane, nxt);
         const uint32_t ti2 = step_tile(ti1, total_waves, T);
-        const idb_tile rec2 = ti2 < T ? tile_rec(a, ti2) : idb_tile{};
+        const idb_tile rec2 = ti2 < T ? sub_tile(a, ti2) : idb_tile{};
 
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         if (FILT == 1 && !FUSE) {
@@ -2092,14 +2106,24 @@ uint32_t grid_for(uint32_t n_tiles, uint32_t wpb, uint32_t resident, uint32_t mu
 uint32_t pick_wpb(const idb_pair_args &a, uint32_t most) { return idb_pick_wpb(a, most); }
 
 template <int W, bool FUSE, int FILT>
-hipError_t launch_myers_w(const idb_pair_args &a, dim3 block, size_t shm, uint32_t wpb, hipStream_t s)
+hipError_t launch_myers_w(const idb_pair_args &a_in, dim3 block, size_t shm, uint32_t wpb, hipStream_t s)
 {
     const void *k = (const void *)k_pairs_myers<W, FUSE, FILT>;
     if (shm > 65536) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
     }
-    const dim3 grid(grid_for(a.n_tiles, wpb, resident_blocks(k, block.x, shm), a.tune_grid_mul));
+    const uint32_t resident = resident_blocks(k, block.x, shm);
+    // Few tiles (buckets of a small table) leave most of the chip idle behind
+    // the waves of the fullest ones: they are taken in up to 8 parts of their
+    // queries each, while the parts are no more than twice the resident waves
+    // (nucleotide rows, relative threshold: 300 tiles 166 -> 63 us, 600 tiles
+    // 170 -> 84 us, 1,950 tiles 272 -> 215 us, where one round of waves as the
+    // limit left it at 279).
+    idb_pair_args a = a_in;
+    if (!FUSE)
+        while (a.sub_log2 < 3 && ((uint64_t)a.n_tiles << (a.sub_log2 + 1)) <= 2ull * resident * wpb) ++a.sub_log2;
+    const dim3 grid(grid_for(a.n_tiles << a.sub_log2, wpb, resident, a.tune_grid_mul));
     hipLaunchKernelGGL((k_pairs_myers<W, FUSE, FILT>), grid, block, shm, s, a, wpb);
     return hipGetLastError();
 }

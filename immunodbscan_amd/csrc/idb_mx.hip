@@ -523,14 +523,22 @@ __global__ __launch_bounds__(256) void k_mx_fill(const uint64_t *ekey, const uin
                 uint32_t a0 = 0, a1 = 0;
                 for (uint32_t k0 = 32 * wd; k0 < 32 * wd + 32 && k0 < L; k0 += 16) {
                     const uint4 v = row16(s, L, k0);
+                    // (all 16 letters, those past the row's end masked: the
+                    // letter map's LDS reads then run ahead of the profile)
                     const uint32_t nb = min(16u, L - k0);
-                    for (uint32_t b = 0; b < nb; ++b) {
-                        const uint32_t code = cm[byte_of(v, b)] & 3u;
-                        a0 |= (code & 1u) << ((k0 + b) & 31u);
-                        a1 |= (code >> 1) << ((k0 + b) & 31u);
-                        hist = ((hist << 2) | code) & 63u;
-                        if (k0 + b >= 2) idb_qmask_add(g, hist);
+                    uint32_t code[16], p0 = 0, p1 = 0;
+#pragma unroll
+                    for (uint32_t b = 0; b < 16; ++b) code[b] = cm[byte_of(v, b)] & 3u;
+#pragma unroll
+                    for (uint32_t b = 0; b < 16; ++b) {
+                        p0 |= (code[b] & 1u) << b;
+                        p1 |= (code[b] >> 1) << b;
+                        hist = ((hist << 2) | code[b]) & 63u;
+                        if (b < nb && k0 + b >= 2) idb_qmask_add(g, hist);
                     }
+                    const uint32_t in = (1u << nb) - 1u;
+                    a0 |= (p0 & in) << (k0 & 31u);
+                    a1 |= (p1 & in) << (k0 & 31u);
                 }
                 vrec[(size_t)wd * E + e] = a0;
                 vrec[(size_t)(W + wd) * E + e] = a1;

@@ -1283,6 +1283,7 @@ struct Upload {
     }
     void run()
     {
+        if (n == 0) return;
         size_t at[5], total = 0;
         for (uint32_t k = 0; k < n; ++k) {
             at[k] = total;

@@ -46,7 +46,6 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12  # int32 lanes x clock: 39.3 T ops/s
 HBM_PEAK_GBS = 8000.0
 
 
@@ -60,12 +59,11 @@ def myers_ops_per_letter(W: int) -> int:
     return 20 * W + 4 * (W - 1)
 
 
-# absent-letter filter per pair: per direction an AND-NOT of the letter-set
-# planes and a bit count, then a maximum and the threshold compare
-FILTER_OPS_PER_PAIR = 6
-# 3-gram profile bound per pair: 16 four-byte absolute-difference sums, the
-# scaled threshold and the compare
-QGRAM_OPS_PER_PAIR = 18
+# the count pass's exact lower bound on the matrix cores: two products per
+# gated pair of 4-bit feature vectors (64 wide for protein rows, 192 for
+# nucleotide rows)
+BOUND_DIMS = {1: 64, 2: 192}
+MFMA_F4_PEAK_TFLOPS = 10000.0
 
 
 def count_kernel_ops(s: dict, vw: int, jw: int) -> int:
@@ -76,18 +74,16 @@ def count_kernel_ops(s: dict, vw: int, jw: int) -> int:
     return s["gated_pairs"] * gate_ops + s["myers_letters"] * myers_ops_per_letter(W)
 
 
-def filter_ops(s: dict) -> int:
-    """Ops of the exact lower bound that runs before Myers (absent letters
-    or 3-grams), which the work model does not count."""
-    if s["band_filter"] == 1:
-        return s["gated_pairs"] * FILTER_OPS_PER_PAIR
-    if s["band_filter"] == 2:
-        return s["gated_pairs"] * QGRAM_OPS_PER_PAIR
-    return 0
+def bound_roofline(s: dict, ms: float) -> dict:
+    """The bound's products against the dense 4-bit matrix peak; deciding the
+    pairs that pass (diagonals on bit planes) is not in these flops."""
+    flops = s["gated_pairs"] * 4 * BOUND_DIMS.get(s["band_filter"], 0)
+    achieved = flops / (ms * 1e-3) / 1e12
+    return {"bound": "mfma", "achieved": achieved, "peak": MFMA_F4_PEAK_TFLOPS, "unit": "TFLOP/s",
+            "frac": achieved / MFMA_F4_PEAK_TFLOPS, "bound_flops": flops}
 
 
-ENC_FLOPS_PER_ROW = 2 * 32 * (5 * 32 * 128 + 2 * 5 * 128 * 128)  # three conv layers, 32 positions
-ENC160_FLOPS_PER_ROW = 5 * ENC_FLOPS_PER_ROW  # the nucleotide encoder: 160 positions
+ENC_FLOPS_PER_LETTER = 2 * 5 * (32 * 128 + 2 * 128 * 128)  # three conv layers of five taps
 MFMA_BF16_PEAK_TFLOPS = 2500.0
 
 
@@ -140,7 +136,7 @@ def learned_section(args, cl, exact_rep, exact_ms, exact_res) -> dict:
         s = res.stats
         n = rep.n
         enc_ms = s["encoder_ms"]
-        flops = ENC_FLOPS_PER_ROW * n
+        flops = ENC_FLOPS_PER_LETTER * int(rep.length.clip(max=32).sum())
         return {
             "workload": tag,
             "rows": n,
@@ -161,7 +157,7 @@ def learned_section(args, cl, exact_rep, exact_ms, exact_res) -> dict:
             "encoder_roofline": {"bound": "mfma", "achieved": flops / (enc_ms * 1e-3) / 1e12,
                                  "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                                  "frac": flops / (enc_ms * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS,
-                                 "flops_per_row": ENC_FLOPS_PER_ROW},
+                                 "flops_per_letter": ENC_FLOPS_PER_LETTER},
         }
 
     if args.learned_c2:
@@ -307,17 +303,6 @@ def genes_section(args) -> dict:
     }
 
 
-def pmc_traffic(rows: int):
-    """HBM bytes per launch of the count kernel from the committed PMC
-    profile of this workload (FETCH_SIZE and WRITE_SIZE passes, each scaled
-    by a 256 MiB device copy measured in the same run); None for other sizes."""
-    path = os.path.join(ROOT, "profiles", "c2_count_kernel_pmc.json")
-    if rows != 200_000 or not os.path.exists(path):
-        return None
-    with open(path) as f:
-        return float(json.load(f)["traffic_bytes"])
-
-
 def large_section(args, threads: int) -> dict:
     import numpy as np
 
@@ -352,9 +337,7 @@ def large_section(args, threads: int) -> dict:
         "myers_words": W,
         "filter": "3-gram profile bound" if s["band_filter"] == 2 else s["band_filter"],
         "stage_ms": s["stage_ms"],
-        "count_kernel_roofline": {"bound": "valu", "achieved": ops / (kms * 1e-3) / 1e12, "peak": VALU_PEAK_TOPS,
-                                  "unit": "TOP/s", "frac": ops / (kms * 1e-3) / 1e12 / VALU_PEAK_TOPS,
-                                  "kernel_ms": kms, "algorithmic_ops": ops, "filter_ops": filter_ops(s)},
+        "count_kernel_roofline": {**bound_roofline(s, kms), "kernel_ms": kms, "algorithmic_ops": ops},
         "cpu_baseline": None if cpu_v is None else {
             "value": cpu_v, "unit": "pairs/s", "cores": threads, "kind": "port",
             "sample": f"literal all-pairs clustering of the first {sub_n} rows in {dt:.1f} s; extrapolated"},
@@ -386,7 +369,7 @@ def large_learned(args, rep, exact_ms, exact_res) -> dict:
     res = lrun.result()
     s = res.stats
     enc_ms = s["encoder_ms"]
-    flops = ENC160_FLOPS_PER_ROW * rep.n
+    flops = ENC_FLOPS_PER_LETTER * int(rep.length.clip(max=160).sum())
     log(f"large learned: {ms:.1f} ms/step against exact {exact_ms:.1f}")
     return {
         "training": {"pairs": int(len(labels)), "positive_fraction": float(labels.mean()), **tstats,
@@ -412,7 +395,7 @@ def large_learned(args, rep, exact_ms, exact_res) -> dict:
         "encoder_roofline": {"bound": "mfma", "achieved": flops / (enc_ms * 1e-3) / 1e12,
                              "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                              "frac": flops / (enc_ms * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS,
-                             "flops_per_row": ENC160_FLOPS_PER_ROW},
+                             "flops_per_letter": ENC_FLOPS_PER_LETTER},
     }
 
 
@@ -595,11 +578,8 @@ def main() -> int:
     dms, _ = timed(drun, args.steps, args.warmup)
     log(f"device-resident: {dms:.3f} ms/step")
 
-    W = max(1, (s["max_len"] + 31) // 32)
     ops = count_kernel_ops(s, rep.vw, rep.jw)
-    fops = filter_ops(s)
     kms = float(np.mean(cnt_ms))
-    achieved = ops / (kms * 1e-3) / 1e12
     out = {
         "metric": "CDR3 pairs/sec & seqs clustered/sec, exact vs learned filter, 1 MI355X",
         "value": pairs / (ms * 1e-3),
@@ -636,19 +616,12 @@ def main() -> int:
         "noise": s["n_noise"],
         "stage_ms": s["stage_ms"],
         "roofline": {
-            "kernel": ("k_count1<true> (one-word count pass, constant threshold)" if W == 1 and s["band_filter"]
-                       else f"k_pairs_myers<{W},false,{1 if s['band_filter'] else 0}> (count pass)"),
-            "bound": "valu",
-            "achieved": achieved,
-            "peak": VALU_PEAK_TOPS,
-            "unit": "TOP/s",
-            "frac": achieved / VALU_PEAK_TOPS,
-            "traffic": pmc_traffic(n),
+            "kernel": "k_mx (count pass: the bound on matrix cores, pairs that pass on bit planes)",
+            **bound_roofline(s, kms),
+            "traffic": None,
             "kernel_ms": kms,
             "algorithmic_ops": ops,
             "work_model": "gated pairs x (2(Vw+Jw)+2) + Myers text letters x (20W+4(W-1))",
-            "filter_ops": fops,
-            "frac_with_filter_ops": (ops + fops) / (kms * 1e-3) / 1e12 / VALU_PEAK_TOPS,
         },
     }
     run_sections(args, out, threads, cl, rep, dms, drun.result())

@@ -2399,12 +2399,18 @@ uint32_t idb_grid_for(uint32_t n_tiles, uint32_t wpb, uint32_t resident, uint32_
     return b ? b : 1u;
 }
 
-// The grid of a count pass: no more waves than own a chunk of the pair list
-// (every further one would claim a chunk for its few pairs).
+// The grid of a count pass.  Waves past chunk_base claim a chunk for their few
+// pairs, so where the owned chunks cover the resident waves the grid stops at
+// them (200k protein rows: count pass 156 us without owned chunks, 105 with).
+// A shorter list (a small requested capacity, little scratch) says nothing
+// about the work: there the whole grid runs and its waves claim (1M protein
+// rows at a capacity of 256 pairs: 395 ms on the single block that the owned
+// chunks allowed, 1.5 ms on the whole grid).
 uint32_t idb_count_grid(const idb_pair_args &a, uint32_t n_tiles, uint32_t wpb, uint32_t resident)
 {
     const uint32_t g = idb_grid_for(n_tiles, wpb, resident, a.tune_grid_mul);
-    return a.edges && a.chunk_base ? std::max(1u, std::min(g, a.chunk_base / wpb)) : g;
+    const uint32_t own = a.edges ? a.chunk_base / wpb : 0u;
+    return own >= resident ? std::min(g, own) : g;
 }
 
 // Waves per block: the tuned value when set, within [1, most].

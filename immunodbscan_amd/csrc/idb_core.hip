@@ -28,6 +28,7 @@
 #include <string_view>
 #include <array>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <atomic>
 #include <condition_variable>
@@ -1689,6 +1690,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         // took the count pass from 3.40 to 3.15 ms).
         edge_cap = p->edge_capacity ? p->edge_capacity : std::max<unsigned long long>(1ull << 22, 64ull * E);
         edge_cap = std::min<unsigned long long>(edge_cap, 1ull << 31);
+        unsigned long long scratch_pairs = 0;  // allocation-free runs: most pairs that fit
         if (c->noalloc) {
             // Allocation-free run: the pair list gets what the scratch holds
             // after the buffers still to come (core flags, labels, output
@@ -1699,22 +1701,31 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             const size_t used = (c->na_used + 255) & ~(size_t)255;
             const size_t later = 28ull * N + (1ull << 20);
             const size_t room = IDB_NOALLOC_SCRATCH_BYTES > used + later ? IDB_NOALLOC_SCRATCH_BYTES - used - later : 0;
-            edge_cap = std::min<unsigned long long>(edge_cap, room / 12);
+            scratch_pairs = room / 12;
+            edge_cap = std::min<unsigned long long>(edge_cap, scratch_pairs);
             if (edge_cap < IDB_TILE) fail(c, IDB_ERR_UNSUPPORTED, "the allocation-free run's scratch is too small for this input");
         }
         a.chunk_log2 = (force_large || edge_cap >= (1ull << 24)) ? 10u : (edge_cap >= (1ull << 20) ? 8u : 6u);
         a.max_chunks = c->noalloc ? (uint32_t)std::max<unsigned long long>(1ull, edge_cap >> a.chunk_log2)
                                   : (uint32_t)((edge_cap + (1ull << a.chunk_log2) - 1) >> a.chunk_log2);
+        // Waves own their first chunk, at most a quarter of the list; the owned
+        // chunks come on top of the capacity, since one that its wave leaves
+        // empty holds no pairs.  (In an allocation-free run they are part of a
+        // list that already takes all the scratch.)  Not in learned runs, which
+        // may repeat their pass and start from an empty list, and not for a
+        // caller of the pairs, who would be sent the empty chunks (6,000 protein
+        // rows: 976 us a call with them, 490 without).  There the list grows by
+        // a chunk per part of a tile, so that the chunks that the waves leave
+        // partly filled do not count against the capacity either.
+        const uint32_t parts = (uint32_t)std::min<uint64_t>(8ull * T, 32768u);
+        const bool to_caller = x && x->pairs_out;
+        const uint32_t own = learned ? 0u : (to_caller ? parts : std::min(parts, a.max_chunks / 4));
+        a.chunk_base = to_caller ? 0u : own;
         edge_cap = (unsigned long long)a.max_chunks << a.chunk_log2;
-        a.edges = buf<uint2>(c, S_EDGES, edge_cap);
+        a.max_chunks += c->noalloc ? std::min(own, (uint32_t)((scratch_pairs >> a.chunk_log2) - a.max_chunks)) : own;
+        a.edges = buf<uint2>(c, S_EDGES, (size_t)a.max_chunks << a.chunk_log2);
         a.chunk_fill = buf<uint32_t>(c, S_FILL, a.max_chunks);
         a.n_chunks = small + 12;
-        // Waves own their first chunk (learned runs may repeat their pass and
-        // start from an empty list); at most a quarter of the list is given
-        // out this way, so that partly filled chunks do not make it overflow.
-        a.chunk_base = learned ? 0u
-                               : std::min<uint32_t>((uint32_t)std::min<uint64_t>(8ull * T, 32768u),
-                                                    a.max_chunks / 4);
         hipLaunchKernelGGL(k_emit_tiles, dim3(blocks_for(std::max<uint64_t>(bqt[1], a.chunk_base))), dim3(256), 0, s,
                            qboff, num + 1, bstart, E, elen, hilen, banded ? 1u : 0u, qsplit, skey, lb, gvj, toff, tiles,
                            a.n_chunks, a.chunk_fill, a.chunk_base, stamps);
@@ -1851,11 +1862,12 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                 if (x && x->pairs_out) {
                     if (!from_edges) fail(c, IDB_ERR_OOM, "neighbour pair list overflow: raise edge_capacity");
                     std::vector<uint32_t> fill(n_chunks);
-                    std::vector<uint2> ed((size_t)n_chunks << a.chunk_log2);
+                    const size_t ne = (size_t)n_chunks << a.chunk_log2;
+                    std::unique_ptr<uint2[]> ed(new uint2[ne]);  // (not zeroed)
                     if (n_chunks) {
                         check(c, hipMemcpyAsync(fill.data(), a.chunk_fill, sizeof(uint32_t) * n_chunks,
                                                 hipMemcpyDeviceToHost, s), "pairs copy");
-                        check(c, hipMemcpyAsync(ed.data(), a.edges, sizeof(uint2) * ed.size(), hipMemcpyDeviceToHost, s),
+                        check(c, hipMemcpyAsync(ed.get(), a.edges, sizeof(uint2) * ne, hipMemcpyDeviceToHost, s),
                               "pairs copy");
                         check(c, hipStreamSynchronize(s), "pairs sync");
                     }
@@ -1868,6 +1880,9 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                         check(c, hipStreamSynchronize(s), "pairs sync");
                     }
                     uint64_t k = 0;
+                    for (const uint32_t f : fill) k += f;
+                    if (k > edge_cap) fail(c, IDB_ERR_OOM, "neighbour pair list overflow: raise edge_capacity");
+                    k = 0;
                     for (uint32_t ch = 0; ch < n_chunks; ++ch)
                         for (uint32_t i = 0; i < fill[ch]; ++i, ++k) {
                             if (k >= x->pairs_cap) continue;

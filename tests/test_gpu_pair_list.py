@@ -35,3 +35,44 @@ def test_short_list_leaves_the_count_pass_its_grid(gpu_ctx, name, rep, cl):
             assert np.array_equal(getattr(got, k), getattr(full, k)), (cap, k)
         assert got.stats["fuse_from_edges"] == 0
         assert t < 8 * t_full, cap
+
+
+def pairs_of(ctx, rep, cl, capacity):
+    import ctypes as C
+
+    from immunodbscan_amd import _lib
+
+    cap = 1 << 20
+    out = np.zeros((cap, 2), np.uint32)
+    n = C.c_uint64()
+    ctx.check(_lib.lib.idb_neighbour_pairs(ctx.handle, engine._dataset(rep),
+                                           engine._params(cl, False, 0, edge_capacity=capacity), out.ctypes.data, cap,
+                                           C.byref(n)))
+    pairs = out[: n.value]
+    return pairs[np.lexsort((pairs[:, 1], pairs[:, 0]))]
+
+
+RELATIVE = configs.Clustering(eps=0.15, abs_k=-1, min_pts=2, use_hamming=False)
+
+
+@pytest.mark.parametrize("rep,cl,factor", [
+    (lambda: configs.c1_params(60, 6, 5), RELATIVE, 2.0),
+    (lambda: configs.c1_params(700, 70, 5), RELATIVE, 2.0),
+    (lambda: configs.c1_params(6_000, 600, 5), RELATIVE, 2.0),
+    (lambda: configs.c1_params(6_000, 600, 5), configs.C1, 2.0),
+    (lambda: configs.c2_params(6_000, 600, 5), configs.C2, 2.0),
+    (lambda: configs.c5_params(300, 1, 5), configs.C5, 1.25),
+])
+def test_neighbour_pairs_within_the_capacity(gpu_ctx, rep, cl, factor):
+    """A list of some more pairs than there are holds them, however few of them
+    each wave finds; a list of fewer is refused."""
+    from immunodbscan_amd import _lib
+
+    rep = synth.generate(rep())
+    want = pairs_of(gpu_ctx, rep, cl, 0)
+    assert len(want) > 64
+    assert np.array_equal(pairs_of(gpu_ctx, rep, cl, int(factor * len(want)) + 1), want)
+    with pytest.raises(_lib.IdbError, match="raise edge_capacity"):
+        pairs_of(gpu_ctx, rep, cl, len(want) // 2)
+    with pytest.raises(_lib.IdbError, match="raise edge_capacity"):
+        pairs_of(gpu_ctx, rep, cl, 64)

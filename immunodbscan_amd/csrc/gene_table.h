@@ -33,7 +33,34 @@ struct idb_gene_table {
     std::vector<uint32_t> nodes;
 };
 
-#define IDB_GENE_NAME_MAX 1024u     // longer names never match
+#define IDB_GENE_NAME_MAX 1024u         // longer names never match
+#define IDB_GENE_TABLE_NARROW 32768u    // entries of a table that goes to LDS (16-bit byte offsets)
+#define IDB_GENE_TABLE_MAX (1u << 20)   // entries of the largest table that is built
+
+// The automaton while building its table costs less than testing every name:
+// measured, the per-name kernel takes 0.45 us per name (a wave's walk over the
+// names) + 0.081 ns per call and name, the automaton about 11 us + 4.5 ns per
+// table entry (mostly its construction on the host).  104 V genes: 58 against
+// 70 us from 100 calls on, 74 us against 8.75 ms at 1M; 37 D genes: even at
+// 5,000 calls; 6 J genes: from about 15,000 calls (31.5 against 36.6 us at
+// 20,000).  The largest table that is worth building for n calls:
+inline uint32_t idb_gene_table_cap(uint32_t n, uint32_t n_genes)
+{
+    const int64_t worth = 100ll * n_genes + (int64_t)((uint64_t)n * n_genes * 18u / 1000u) - 2500;
+    return (uint32_t)std::max<int64_t>(0, std::min<int64_t>(IDB_GENE_TABLE_MAX, worth));
+}
+
+// LDS of a block that keeps the table there: class map, 16-bit entries, nodes.
+inline size_t idb_gene_table_lds(const idb_gene_table &t)
+{
+    return 256 + ((size_t)t.entries + 1) / 2 * 4 + 4 * t.nodes.size();
+}
+
+// True for a table that goes to LDS (of which a block may have lds_limit bytes).
+inline bool idb_gene_table_narrow(const idb_gene_table &t, size_t lds_limit)
+{
+    return t.entries <= IDB_GENE_TABLE_NARROW && t.nodes.size() <= 4096 && idb_gene_table_lds(t) <= lds_limit;
+}
 
 // False when the table would hold more than `cap` entries or a name holds a
 // zero byte.

@@ -2316,22 +2316,13 @@ int idb_gene_bitsets_gpu(idb_ctx *c, uint32_t mem, uint32_t n, const uint8_t *ca
             ld = stage_in<uint32_t>(c, S_GLEN, call_len, n, mem);
             outd = buf<int32_t>(c, S_GOUT, (size_t)n * width);
         }
-        // The automaton while building its table costs less than testing every
-        // name: measured, the per-name kernel takes 0.45 us per name (a wave's
-        // walk over the names) + 0.081 ns per call and name, the automaton
-        // about 11 us + 4.5 ns per table entry (mostly its construction on the
-        // host).  104 V genes: 58 against 70 us from 100 calls on, 74 us
-        // against 8.75 ms at 1M; 37 D genes: even at 5,000 calls; 6 J genes:
-        // from about 15,000 calls (31.5 against 36.6 us at 20,000).
-        const int64_t worth = 100ll * n_genes + (int64_t)((uint64_t)n * n_genes * 18u / 1000u) - 2500;
-        const uint32_t cap = (uint32_t)std::max<int64_t>(0, std::min<int64_t>(IDB_GENE_TABLE_MAX, worth));
         // (host copies that the stream may still read at the end of their block)
         idb_gene_table t;
         std::vector<uint8_t> big;
         std::vector<idb_gene_hdr> hdr;
         std::vector<uint32_t> words;
-        if (n_genes && idb_gene_table_build(n_genes, genes, gene_off, gene_len, cap, t)) {
-            const bool narrow = t.entries <= IDB_GENE_TABLE_NARROW && t.nodes.size() <= 4096;
+        if (n_genes && idb_gene_table_build(n_genes, genes, gene_off, gene_len, idb_gene_table_cap(n, n_genes), t)) {
+            const bool narrow = idb_gene_table_narrow(t, idb_lds_limit());
             const size_t nodes_at = 256, trans_at = (nodes_at + 4 * t.nodes.size() + 15) & ~(size_t)15;
             const size_t bytes = trans_at + (narrow ? ((size_t)t.entries + 1) / 2 * 4 : 4 * (size_t)t.entries + 4);
             // built in the pinned staging area when it fits (the previous

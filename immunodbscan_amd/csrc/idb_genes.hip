@@ -349,9 +349,18 @@ hipError_t idb_launch_gene_scan(const uint8_t *calls, const uint64_t *off, const
     const uint32_t threads = lds <= 19000 ? 256u : (lds <= 39000 ? 512u : 1024u);
     const dim3 grid(idb_gene_scan_blocks(n, threads, lds)), block(threads);
     const uint32_t wide = width == 4 && ((uintptr_t)out & 15u) == 0 ? 1u : 0u;
+    // 16-bit tables of a few hundred names pass 64 KB (up to 82 KB: 32,768
+    // entries and 4,096 nodes), which a kernel has to ask for
 #define IDB_GS(TE, NW)                                                                                            \
-    hipLaunchKernelGGL((k_gene_scan<TE, NW>), grid, block, lds, s, calls, off, len, n, cls, (const TE *)trans,    \
-                       nodes, ncls, entries, out_min, n_nodes, max_len, out, width, wide)
+    do {                                                                                                          \
+        if (lds > 65536) {                                                                                        \
+            const hipError_t e = hipFuncSetAttribute((const void *)k_gene_scan<TE, NW>,                           \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);       \
+            if (e != hipSuccess) return e;                                                                        \
+        }                                                                                                         \
+        hipLaunchKernelGGL((k_gene_scan<TE, NW>), grid, block, lds, s, calls, off, len, n, cls, (const TE *)trans, \
+                           nodes, ncls, entries, out_min, n_nodes, max_len, out, width, wide);                    \
+    } while (0)
     if (narrow) {
         if (width <= 4) IDB_GS(uint16_t, 4);
         else IDB_GS(uint16_t, 0);

@@ -40,8 +40,6 @@
 struct idb_gene_hdr {
     uint32_t w0, w1, len, woff;
 };
-#define IDB_GENE_TABLE_NARROW 32768u    // entries of a table that goes to LDS (16-bit byte offsets)
-#define IDB_GENE_TABLE_MAX (1u << 20)   // entries of the largest table that is built
 #define IDB_GENE_MAX_WIDTH 256u   // bit words per row (8,192 gene names)
 
 // Entry order for runs of up to IDB_SORT_SMALL_MAX entries: stable radix

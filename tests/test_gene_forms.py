@@ -1,0 +1,92 @@
+"""The gene scan's forms at the edges of what they take, each case checked to
+run the form that it is meant for (tests/cpp/gene_form.cpp applies the same
+rule to the same names)."""
+from __future__ import annotations
+
+import os
+import random
+import subprocess
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def form_of(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("genes") / "gene_form")
+    subprocess.run(["g++", "-O1", "-std=c++17", os.path.join(ROOT, "tests", "cpp", "gene_form.cpp"), "-o", exe],
+                   check=True)
+
+    def form(n_calls, names):
+        r = subprocess.run([exe], input=b"%d %d\n" % (n_calls, len(names)) + b"".join(n + b"\n" for n in names),
+                           capture_output=True, check=True)
+        kind, entries, lds = r.stdout.split()
+        return kind.decode(), int(entries), int(lds)
+
+    return form
+
+
+def names_with(rng, k, letters, states):
+    """k names over the letters whose automaton has exactly `states` states."""
+    prefixes, names = {b""}, []
+    for left in range(k, 0, -1):
+        room = states - len(prefixes)
+        n = bytes(rng.choice(letters) for _ in range(min(room, room // left + 4)))
+        names.append(n or rng.choice(names))  # (no room: a name twice)
+        prefixes |= {n[:i] for i in range(1, len(n) + 1)}
+    while len(prefixes) < states:  # the first name, letter by letter
+        names[0] += rng.choice(letters).to_bytes(1, "little")
+        prefixes.add(names[0])
+    assert len(prefixes) == states
+    return names
+
+
+def calls_of(rng, n, names, letters):
+    calls = []
+    for _ in range(n):
+        c = bytes(rng.choice(letters) for _ in range(rng.choice([0, 1, 15, 16, 17, 40])))
+        for _ in range(rng.randrange(0, 3)):
+            c += rng.choice(names) + b"-"
+        calls.append(c)
+    for L in (2047, 2048, 2049, 5000):
+        c = bytearray(b"~" * L)
+        for _ in range(12):
+            g = rng.choice(names)
+            p = rng.randrange(0, L - len(g) + 1)
+            c[p:p + len(g)] = g
+        calls[rng.randrange(n)] = bytes(c)
+    return calls
+
+
+LETTERS = b"ABCDEFGHIJ"  # table rows of 12 entries
+# names, states, calls, form, LDS of a block: the largest 16-bit tables (64 KB
+# of LDS are passed at 32,384 entries for 128 names), and 32-bit ones, for bit
+# words in registers (at most 128 names) and in memory
+FORMS = [(128, 2698, 12000, "16", 65520), (128, 2699, 12000, "16", 65544), (128, 2730, 12000, "16", 66288),
+         (600, 2730, 3000, "16", 68176), (128, 2731, 16000, "32", 256), (128, 3600, 16000, "32", 256),
+         (300, 2731, 3000, "32", 256)]
+
+
+def test_forms_are_the_ones_named(form_of):
+    for k, states, n, kind, lds in FORMS:
+        rng = random.Random(k + states)
+        got = form_of(n, names_with(rng, k, LETTERS, states))
+        assert got == (kind, 12 * states, lds), (k, states)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,states,n,kind,lds", FORMS)
+def test_forms(gpu_ctx, form_of, k, states, n, kind, lds):
+    from immunodbscan_amd.interlink import gene_bitsets_gpu
+
+    rng = random.Random(k + states)
+    names = names_with(rng, k, LETTERS, states)
+    assert form_of(n, names)[0] == kind
+    calls = calls_of(rng, n, names, LETTERS)
+    print(f"case genes {kind} bit, {k} names, {states} states, {lds} bytes of LDS", flush=True)
+    got, _ = gene_bitsets_gpu(calls, names)
+    assert np.array_equal(got, O.gene_bitsets(calls, names))

@@ -2321,7 +2321,13 @@ int idb_gene_bitsets_gpu(idb_ctx *c, uint32_t mem, uint32_t n, const uint8_t *ca
         std::vector<uint8_t> big;
         std::vector<idb_gene_hdr> hdr;
         std::vector<uint32_t> words;
-        if (n_genes && idb_gene_table_build(n_genes, genes, gene_off, gene_len, idb_gene_table_cap(n, n_genes), t)) {
+        const bool scan =
+            n_genes && idb_gene_table_build(n_genes, genes, gene_off, gene_len, idb_gene_table_cap(n, n_genes), t);
+        if (scan && t.nodes.empty()) {
+            // no name that could match (all are empty or too long): no walk
+            // (1,000 strings of 6,000 bytes: 59 ms)
+            check(c, hipMemsetAsync(outd, 0, sizeof(int32_t) * (size_t)n * width, s), "bitset clear");
+        } else if (scan) {
             const bool narrow = idb_gene_table_narrow(t, idb_lds_limit());
             const size_t nodes_at = 256, trans_at = (nodes_at + 4 * t.nodes.size() + 15) & ~(size_t)15;
             const size_t bytes = trans_at + (narrow ? ((size_t)t.entries + 1) / 2 * 4 : 4 * (size_t)t.entries + 4);
@@ -2333,7 +2339,7 @@ int idb_gene_bitsets_gpu(idb_ctx *c, uint32_t mem, uint32_t n, const uint8_t *ca
                 h = big.data();
             }
             std::memcpy(h, t.cls, sizeof(t.cls));
-            if (!t.nodes.empty()) std::memcpy(h + nodes_at, t.nodes.data(), 4 * t.nodes.size());
+            std::memcpy(h + nodes_at, t.nodes.data(), 4 * t.nodes.size());
             // offsets in bytes; list heads as they are
             auto fill = [&](auto *e) {
                 for (uint32_t r = 0; r < t.entries; r += t.stride) {

@@ -90,3 +90,22 @@ def test_forms(gpu_ctx, form_of, k, states, n, kind, lds):
     print(f"case genes {kind} bit, {k} names, {states} states, {lds} bytes of LDS", flush=True)
     got, _ = gene_bitsets_gpu(calls, names)
     assert np.array_equal(got, O.gene_bitsets(calls, names))
+
+
+@pytest.mark.gpu
+def test_names_that_cannot_match_cost_no_walk(gpu_ctx):
+    """Only empty and too long names: no bits, and no pass over long calls (the
+    walk with every lane started at its string's first byte took 59 ms)."""
+    import time
+
+    from immunodbscan_amd.interlink import gene_bitsets_gpu
+
+    names = [b""] * 20 + [b"x" * 1100] * 20
+    calls = [b"x" * 6000] * 1000
+    best = 1e9
+    for _ in range(4):
+        t0 = time.perf_counter()
+        got, _ = gene_bitsets_gpu(calls, names)
+        best = min(best, time.perf_counter() - t0)
+    assert got.shape == (1000, 2) and not got.any()
+    assert best < 0.03  # with 6 MB of calls packed and copied

@@ -31,7 +31,8 @@
 
 namespace {
 
-constexpr uint32_t GS_LONG = 2048;           // longer call strings are walked by a whole wave
+constexpr uint32_t GS_LONG = 2048;           // longer call strings may be walked by a whole wave
+constexpr uint32_t GS_LANE = 1u << 20;       // ... and still longer ones always are
 
 // A lane's walk over one call string, with offsets in bytes (one add-shift
 // per lookup).  A byte where a name ends only notes the state, in a queue of
@@ -107,7 +108,12 @@ struct GeneWalk {
 // wave instructions, 33 us of issue; 47 MB of calls at the copy rate: 14 us).
 // A string longer than GS_LONG is cut into 64 segments walked by the lanes of
 // its wave, each starting max_len - 1 bytes early at the root state (a name
-// that ends in the segment starts no earlier).
+// that ends in the segment starts no earlier), where that is the shorter way:
+// the wave walks its long strings one after the other, at twice the time per
+// byte (it reads byte by byte), while a string per lane runs beside the
+// others'.  104 V genes, strings of 2,100 bytes: a single one 39 us a call by
+// the wave, 100 of them 541 us that way and 179 a lane each; 1,000 of 40,000
+// bytes 12.4 and 3.0 ms.
 template <typename TE, int NW>
 __global__ __launch_bounds__(1024) void k_gene_scan(const uint8_t *calls, const uint64_t *off, const uint32_t *len,
                                                     uint32_t n, const uint8_t *__restrict__ cls_g,
@@ -142,7 +148,14 @@ __global__ __launch_bounds__(1024) void k_gene_scan(const uint8_t *calls, const 
         int32_t *ro = out + (size_t)row * width;
         if (!NW && valid)
             for (uint32_t k = 0; k < width; ++k) ro[k] = 0;
-        const bool is_long = L > GS_LONG;
+        bool is_long = L > GS_LONG;
+        if (const uint64_t lm = __ballot(is_long)) {
+            uint32_t longest = L;
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) longest = max(longest, (uint32_t)__shfl_xor((int)longest, d, 64));
+            const uint64_t by_wave = 2ull * (uint32_t)__popcll(lm) * (longest / 64u + max_len);
+            is_long = is_long && (longest > GS_LANE || by_wave < longest);
+        }
         if (!NW) __threadfence();  // the zeros are in place before any bit is set
         GeneWalk<TE, NW> wk{tr, cls, nodes, head_at, out_b, ro};
         if (!is_long) {

@@ -109,3 +109,90 @@ def test_names_that_cannot_match_cost_no_walk(gpu_ctx):
         best = min(best, time.perf_counter() - t0)
     assert got.shape == (1000, 2) and not got.any()
     assert best < 0.03  # with 6 MB of calls packed and copied
+
+
+AB = b"ABCDEFGHIJKLMNOPQRSTUVWXYZ"
+
+
+def arrays_of(calls, names, width):
+    from immunodbscan_amd.interlink import pack_strings
+
+    return pack_strings(calls), pack_strings(names), np.zeros((len(calls), width), np.int32)
+
+
+def scan(ctx, calls, names, out):
+    from immunodbscan_amd import _lib
+
+    ctx.check(_lib.lib.idb_gene_bitsets_gpu(ctx.handle, _lib.IDB_MEM_HOST, len(calls[2]), *(a.ctypes.data for a in calls),
+                                            len(names[2]), *(a.ctypes.data for a in names), out.ctypes.data,
+                                            out.shape[1]))
+
+
+def gene_names(*lists):
+    return [ln for x in lists for ln in open(os.path.join(ROOT, "tests", "golden", x + "genes.txt"), "rb").read().split(b"\n")
+            if ln]
+
+
+# calls around a wave's 64 rows and a block's; every 50th string is a long one
+@pytest.mark.gpu
+@pytest.mark.parametrize("lists", [("VH",), ("VH", "DH")])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 2047, 2048, 2049, 4097, 20_000, 140_001])
+def test_some_long_strings(gpu_ctx, form_of, lists, n):
+    rng = random.Random(n)
+    names = gene_names(*lists)
+    assert form_of(n, names)[0] == "16"
+    pool = calls_of(rng, 250, names, AB)
+    for i in range(0, 250, 50):
+        pool[i] = (pool[i] + b"~" * 2100 + rng.choice(names)) * 2
+    calls = [pool[i % 250] for i in range(n)]
+    want = O.gene_bitsets(pool, names)
+    cs, ns, out = arrays_of(calls, names, (len(names) + 31) // 32)
+    scan(gpu_ctx, cs, ns, out)
+    assert np.array_equal(out, want[np.arange(n) % 250])
+
+
+# waves of 1 to 64 long strings: by the wave and a lane each, on both sides of the rule
+@pytest.mark.gpu
+@pytest.mark.parametrize("lists", [("VH",), ("VH", "DH")])
+@pytest.mark.parametrize("m", [1, 10, 20, 22, 23, 24, 26, 30, 40, 63, 64])
+def test_waves_of_long_strings(gpu_ctx, form_of, lists, m):
+    rng = random.Random(m)
+    names = gene_names(*lists)
+    pool = calls_of(rng, 64, names, AB)
+    for i in rng.sample(range(64), m):
+        c = bytearray(b"~" * rng.choice([2049, 2100, 3000]))
+        for _ in range(40):
+            g = rng.choice(names)
+            p = rng.randrange(0, len(c) - len(g) + 1)
+            c[p:p + len(g)] = g
+        pool[i] = bytes(c)
+    assert form_of(len(pool) * 3, names)[0] == "16"
+    want = O.gene_bitsets(pool, names)
+    cs, ns, out = arrays_of(pool * 3, names, (len(names) + 31) // 32)
+    scan(gpu_ctx, cs, ns, out)
+    assert np.array_equal(out, np.concatenate([want] * 3))
+
+
+@pytest.mark.gpu
+def test_many_long_strings_run_beside_each_other(gpu_ctx, form_of):
+    """A hundred strings of 2,100 bytes, a lane each, against one that its whole
+    wave walks (64 of them one after the other took 14 times as long as one)."""
+    import time
+
+    rng = random.Random(2)
+    names = gene_names("VH")
+    string = bytes(rng.choice(AB) for _ in range(2100))
+    assert form_of(1, names)[0] == form_of(100, names)[0] == "16"
+
+    def best(n):
+        cs, ns, out = arrays_of([string] * n, names, 4)
+        t = 1e9
+        for _ in range(20):
+            t0 = time.perf_counter()
+            scan(gpu_ctx, cs, ns, out)
+            t = min(t, time.perf_counter() - t0)
+        return t
+
+    one, many = best(1), best(100)
+    print(f"one {one * 1e6:.0f} us, a hundred {many * 1e6:.0f}", flush=True)
+    assert many < 8 * one

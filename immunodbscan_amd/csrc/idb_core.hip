@@ -2321,8 +2321,9 @@ int idb_gene_bitsets_gpu(idb_ctx *c, uint32_t mem, uint32_t n, const uint8_t *ca
         std::vector<uint8_t> big;
         std::vector<idb_gene_hdr> hdr;
         std::vector<uint32_t> words;
-        const bool scan =
-            n_genes && idb_gene_table_build(n_genes, genes, gene_off, gene_len, idb_gene_table_cap(n, n_genes), t);
+        const uint32_t cap = idb_gene_table_cap(n, n_genes);
+        const bool scan = n_genes && idb_gene_table_in_reach(n_genes, genes, gene_off, gene_len, cap) &&
+                          idb_gene_table_build(n_genes, genes, gene_off, gene_len, cap, t);
         if (scan && t.nodes.empty()) {
             // no name that could match (all are empty or too long): no walk
             // (1,000 strings of 6,000 bytes: 59 ms)

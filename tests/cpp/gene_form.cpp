@@ -23,7 +23,9 @@ int main()
     }
     data.push_back(0);
     idb_gene_table t;
-    if (!idb_gene_table_build(k, data.data(), off.data(), len.data(), idb_gene_table_cap(n, k), t)) {
+    const uint32_t cap = idb_gene_table_cap(n, k);
+    if (!idb_gene_table_in_reach(k, data.data(), off.data(), len.data(), cap) ||
+        !idb_gene_table_build(k, data.data(), off.data(), len.data(), cap, t)) {
         std::puts("names 0 0");
         return 0;
     }

@@ -30,6 +30,14 @@ def form_of(tmp_path_factory):
     return form
 
 
+def test_reach_of_tables(tmp_path):
+    exe = str(tmp_path / "reach")
+    subprocess.run(["g++", "-O1", "-fsanitize=address,undefined", "-std=c++17",
+                    os.path.join(ROOT, "tests", "cpp", "test_gene_reach.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe, os.path.join(ROOT, "tests", "golden")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
 def names_with(rng, k, letters, states):
     """k names over the letters whose automaton has exactly `states` states."""
     prefixes, names = {b""}, []

@@ -2405,7 +2405,7 @@ uint32_t idb_grid_for(uint32_t n_tiles, uint32_t wpb, uint32_t resident, uint32_
 // A shorter list (a small requested capacity, little scratch) says nothing
 // about the work: there the whole grid runs and its waves claim (1M protein
 // rows at a capacity of 256 pairs: 395 ms on the single block that the owned
-// chunks allowed, 1.5 ms on the whole grid).
+// chunks allowed, 0.97 ms on the whole grid).
 uint32_t idb_count_grid(const idb_pair_args &a, uint32_t n_tiles, uint32_t wpb, uint32_t resident)
 {
     const uint32_t g = idb_grid_for(n_tiles, wpb, resident, a.tune_grid_mul);

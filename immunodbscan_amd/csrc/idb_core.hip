@@ -103,7 +103,7 @@ struct idb_ctx {
     struct Tuned {
         uint32_t wpb, grid_mul, no_xcd, trials;
     };
-    std::map<std::array<uint32_t, 6>, Tuned> tuned;
+    std::map<std::array<uint32_t, 8>, Tuned> tuned;
     hipGraphExec_t gexec = nullptr;  // the tail graph, updated in place
     void *scan_ws = nullptr;         // the current call's scan workspace (idb_scan.hip)
     uint32_t scan_gen = 0;           // scans launched on it since it was zeroed
@@ -1229,14 +1229,20 @@ struct StageRanges {
 // LDS allows), grid of 1, 2, 4 or 8 times the resident blocks, XCD-grouped or
 // plain block order.  Each candidate runs the real count pass on the real
 // tiles twice (counts restored from a snapshot in between) and the fastest by
-// HIP events is kept for this kernel and shape class (kernel, words, code
-// width, filter, alphabet, log2 tiles) for the context's lifetime.
+// HIP events is kept for this kernel and shape class (the pass, the kernel that
+// runs it, words, code width, filter, alphabet, log2 tiles) for the context's
+// lifetime.
 void autotune(idb_ctx *c, idb_pair_args &a, uint32_t N, uint32_t E, uint32_t W, bool ham, bool learned, uint32_t *small,
               unsigned long long *work)
 {
     uint32_t lt = 0;
     while (lt < 31 && (1u << (lt + 1)) <= a.n_tiles) ++lt;
-    const std::array<uint32_t, 6> key{learned ? 2u : (ham ? 1u : 0u), ham ? a.HW : W, a.bits, a.band_filter, a.K, lt};
+    // the kernel: a matrix-core form by planes, words and threshold class, or the
+    // general ones by whether the threshold is one for all pairs
+    const uint32_t kernel = a.e_feat ? 2u + (a.mx_planes << 8) + (a.mx_words << 12) + ((uint32_t)std::max(a.t_const, 1) << 16)
+                                     : (a.t_const >= 0 ? 1u : 0u);
+    const std::array<uint32_t, 8> key{learned ? 2u : (ham ? 1u : 0u), kernel, ham ? a.HW : W, a.bits, a.band_filter,
+                                      a.qgram_filter | (a.single_bucket << 1), a.K, lt};
     auto it = c->tuned.find(key);
     if (it == c->tuned.end()) {
         hipStream_t s = c->stream;
@@ -1248,26 +1254,26 @@ void autotune(idb_ctx *c, idb_pair_args &a, uint32_t N, uint32_t E, uint32_t W, 
         idb_ctx::Tuned best{0, 0, 0, 0};
         float best_ms = 1e30f;
         uint32_t trials = 0;
-        const uint32_t base = a.chunk_base;
-        a.chunk_base = 0;  // trials start from an empty list
+        // a trial's starting state: the counts, the statistics and the pair list as
+        // the run itself finds them (the grid depends on the owned chunks)
+        const auto reset = [&] {
+            check(c, hipMemcpyAsync(acc, snap, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s), "tune reset");
+            check(c, hipMemsetAsync(small + 12, 0, sizeof(uint32_t), s), "tune reset");
+            check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "tune reset");
+            if (a.chunk_base)
+                hipLaunchKernelGGL(k_chunk_start, dim3(blocks_for(a.chunk_base)), dim3(256), 0, s, a.n_chunks,
+                                   a.chunk_fill, a.chunk_base);
+        };
         for (uint32_t wpb : {1u, 2u, 4u})
             for (uint32_t mul : {1u, 2u, 4u, 8u})
                 for (uint32_t nx : {0u, 1u}) {
                     a.tune_wpb = wpb;
                     a.tune_grid_mul = mul;
                     a.no_xcd_order = nx;
-                    check(c, hipMemcpyAsync(acc, snap, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s), "tune reset");
-                    check(c, hipMemsetAsync(small + 12, 0, sizeof(uint32_t), s), "tune reset");
-                    check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "tune reset");
                     // best of two runs per shape
                     float ms = 1e30f;
                     for (int rep = 0; rep < 2; ++rep) {
-                        if (rep) {
-                            check(c, hipMemcpyAsync(acc, snap, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s),
-                                  "tune reset");
-                            check(c, hipMemsetAsync(small + 12, 0, sizeof(uint32_t), s), "tune reset");
-                            check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "tune reset");
-                        }
+                        reset();
                         check(c, hipEventRecord(c->kev[0], s), "event record");
                         const hipError_t e = learned ? idb_launch_count_learned(a, s)
                                                      : (ham ? idb_launch_count_hamming(a, s)
@@ -1286,12 +1292,7 @@ void autotune(idb_ctx *c, idb_pair_args &a, uint32_t N, uint32_t E, uint32_t W, 
                     }
                 }
         best.trials = trials;
-        check(c, hipMemcpyAsync(acc, snap, sizeof(int32_t) * nacc, hipMemcpyDeviceToDevice, s), "tune reset");
-        check(c, hipMemsetAsync(small + 12, 0, sizeof(uint32_t), s), "tune reset");
-        check(c, hipMemsetAsync(work, 0, IDB_WORK_U64 * IDB_WORK_COPIES * sizeof(unsigned long long), s), "tune reset");
-        a.chunk_base = base;
-        if (base)
-            hipLaunchKernelGGL(k_chunk_start, dim3(blocks_for(base)), dim3(256), 0, s, a.n_chunks, a.chunk_fill, base);
+        reset();
         it = c->tuned.emplace(key, best).first;
     }
     a.tune_wpb = it->second.wpb;

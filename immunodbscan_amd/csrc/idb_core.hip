@@ -835,7 +835,7 @@ __global__ __launch_bounds__(256) void k_finish(const uint32_t *small, const uin
 __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, const uint32_t *bstart, uint32_t E,
                              const uint16_t *elen, const uint16_t *hilen, uint32_t banded, uint32_t split,
                              const uint64_t *ekey, uint32_t lb, uint32_t gvj, const uint64_t *toff, idb_tile *tiles,
-                             uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t chunk_base, unsigned long long *stamps)
+                             uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t chunk_base)
 {
     // the pair list's chunks that belong to the count pass's waves
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < chunk_base; i += gridDim.x * blockDim.x) {
@@ -872,7 +872,6 @@ __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, cons
             tiles[o++] = t;
         }
     }
-    idb_stamp_end(stamps + IDB_T_TILES);
 }
 
 // The pair list's starting state (k_emit_tiles writes it too).
@@ -1683,6 +1682,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         a.e_low = elow;
         a.cnt = cnt;
         a.work = work;
+        a.stamps = stamps;
         // Neighbour pairs found by the count pass are kept for the fuse step;
         // if they overflow the list, the fuse pass re-evaluates the tiles.
         // Waves own chunks of 256 pairs (64 for small requested capacities,
@@ -1729,7 +1729,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         a.n_chunks = small + 12;
         hipLaunchKernelGGL(k_emit_tiles, dim3(blocks_for(std::max<uint64_t>(bqt[1], a.chunk_base))), dim3(256), 0, s,
                            qboff, num + 1, bstart, E, elen, hilen, banded ? 1u : 0u, qsplit, skey, lb, gvj, toff, tiles,
-                           a.n_chunks, a.chunk_fill, a.chunk_base, stamps);
+                           a.n_chunks, a.chunk_fill, a.chunk_base);
         if (learned) {
             // embeddings of every row, then proposals verified by Myers
             uint16_t *zb = buf<uint16_t>(c, S_ZB, (size_t)N * 64);
@@ -2050,8 +2050,9 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                 (void)hipEventElapsedTime(&st->count_kernel_ms, c->kev[0], c->kev[1]);
                 (void)hipEventElapsedTime(&st->fuse_kernel_ms, c->kev[2], c->kev[3]);
             } else {
-                st->count_kernel_ms = span(IDB_T_TILES, IDB_T_COUNT);
-                st->fuse_kernel_ms = span(IDB_T_CORE, IDB_T_GROW);
+                // (to the start of the next kernel)
+                st->count_kernel_ms = span(IDB_T_COUNT_START, IDB_T_COUNT);
+                st->fuse_kernel_ms = span(IDB_T_FUSE_START, IDB_T_GROW);
             }
         }
         if (p->tree_stats)

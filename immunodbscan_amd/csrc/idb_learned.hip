@@ -502,9 +502,10 @@ constexpr uint32_t HPART = D * C + D + 4;          // one block's projection gra
 constexpr uint32_t HBLOCKS = 256;                  // most blocks of the head's backward pass
 constexpr uint32_t BPART = NTOK * C0 + 3 * C;      // one block's embedding and bias gradients
 
-// Contrastive loss of pair i (sequences 2i, 2i+1), back through the norm and
-// the projection to the pooled means (dp, already divided by the length), and
-// the projection's gradients.  A wave takes four pairs of a round of HP; the
+// Contrastive loss of pair i (sequences 2i, 2i+1; none where the label is below
+// zero or no number), back through the norm and the projection to the pooled
+// means (dp, already divided by the length), and the projection's gradients.
+// A wave takes four pairs of a round of HP; the
 // block then adds the round's du x pool into 32 accumulators per thread.
 // Latency-bound (4,096 pairs are one round a block); the sums over
 // pairs stay in registers and leave as one partial per block, since one atomic
@@ -540,9 +541,12 @@ __global__ __launch_bounds__(256) void k_pair_head(const float *z, const float *
                 float d2 = diff * diff;
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) d2 += __shfl_xor(d2, o, 64);
-                const float d = sqrtf(d2 + 1e-12f), hinge = fmaxf(0.f, margin - d);
-                lsum += yi * d2 + (1.f - yi) * hinge * hinge;
-                const float g = (2.f * yi - (1.f - yi) * 2.f * hinge / d) * inv_b * diff;  // dz0 = g, dz1 = -g
+                float g = 0.f;  // dz0 = g, dz1 = -g
+                if (yi >= 0.f) {
+                    const float d = sqrtf(d2 + 1e-12f), hinge = fmaxf(0.f, margin - d);
+                    lsum += yi * d2 + (1.f - yi) * hinge * hinge;
+                    g = (2.f * yi - (1.f - yi) * 2.f * hinge / d) * inv_b * diff;
+                }
                 float a = z0 * g, b = z1 * g;
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) {

@@ -835,7 +835,7 @@ __global__ __launch_bounds__(256) void k_finish(const uint32_t *small, const uin
 __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, const uint32_t *bstart, uint32_t E,
                              const uint16_t *elen, const uint16_t *hilen, uint32_t banded, uint32_t split,
                              const uint64_t *ekey, uint32_t lb, uint32_t gvj, const uint64_t *toff, idb_tile *tiles,
-                             uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t chunk_base)
+                             uint32_t *n_chunks, uint32_t *chunk_fill, uint32_t chunk_base, unsigned long long *stamps)
 {
     // the pair list's chunks that belong to the count pass's waves
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < chunk_base; i += gridDim.x * blockDim.x) {
@@ -872,6 +872,7 @@ __global__ void k_emit_tiles(const uint32_t *qboff, const uint32_t *nb_dev, cons
             tiles[o++] = t;
         }
     }
+    idb_stamp_end(stamps + IDB_T_TILES);
 }
 
 // The pair list's starting state (k_emit_tiles writes it too).
@@ -1023,7 +1024,7 @@ __global__ void k_ustart(const uint32_t *uniq, const uint32_t *num, const uint32
 }
 
 __global__ void k_uniques_out(const uint32_t *uniq, const uint32_t *num, const uint32_t *rid, const uint32_t *rstart,
-                              const uint32_t *ustart, uint32_t *out)
+                              const uint32_t *ustart, uint32_t *out, unsigned long long *stamps)
 {
     const uint32_t U = num[0];
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < U; k += gridDim.x * blockDim.x) {
@@ -1035,6 +1036,7 @@ __global__ void k_uniques_out(const uint32_t *uniq, const uint32_t *num, const u
             out[rstart[r] + (k - ustart[r])] = u - rstart[r];
         }
     }
+    if (stamps) idb_stamp_end(stamps + IDB_T_TILES);  // (the last kernel before the count pass)
 }
 
 // Grid-stride kernels run at most 8 blocks per CU: enough to fill the chip,
@@ -1682,7 +1684,6 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         a.e_low = elow;
         a.cnt = cnt;
         a.work = work;
-        a.stamps = stamps;
         // Neighbour pairs found by the count pass are kept for the fuse step;
         // if they overflow the list, the fuse pass re-evaluates the tiles.
         // Waves own chunks of 256 pairs (64 for small requested capacities,
@@ -1729,7 +1730,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         a.n_chunks = small + 12;
         hipLaunchKernelGGL(k_emit_tiles, dim3(blocks_for(std::max<uint64_t>(bqt[1], a.chunk_base))), dim3(256), 0, s,
                            qboff, num + 1, bstart, E, elen, hilen, banded ? 1u : 0u, qsplit, skey, lb, gvj, toff, tiles,
-                           a.n_chunks, a.chunk_fill, a.chunk_base);
+                           a.n_chunks, a.chunk_fill, a.chunk_base, stamps);
         if (learned) {
             // embeddings of every row, then proposals verified by Myers
             uint16_t *zb = buf<uint16_t>(c, S_ZB, (size_t)N * 64);
@@ -1767,14 +1768,18 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
         if (n_reps > 0)
             hipLaunchKernelGGL(k_ustart, dim3(blocks_for((uint64_t)n_reps + 1)), dim3(256), 0, s, uniq, num, rstart,
                                n_reps, ustart);
-        hipLaunchKernelGGL(k_uniques_out, dim3(blocks_for(U)), dim3(256), 0, s, uniq, num, rid, rstart, ustart, unq_o);
+        hipLaunchKernelGGL(k_uniques_out, dim3(blocks_for(U)), dim3(256), 0, s, uniq, num, rid, rstart, ustart, unq_o,
+                           stamps);
         check(c, hipEventRecord(c->side_ev[0], s), "event record");
-        check(c, hipStreamWaitEvent(c->side, c->side_ev[0], 0), "side wait");
-        check(c, hipMemcpyAsync(c->xfer + 2 * ob, copies, sizeof(uint32_t) * N, hipMemcpyDeviceToHost, c->side),
-              "output copy");
-        check(c, hipMemcpyAsync(c->xfer + 3 * ob, unq_o, sizeof(uint32_t) * N, hipMemcpyDeviceToHost, c->side),
-              "output copy");
     }
+    // (the host calls of a transfer, some 15 us, are made when the next kernel
+    // has been launched: before it they would leave the device idle)
+    const auto send = [&](int ev, uint32_t slot, const void *src) {
+        if (!early_out) return;
+        if (ev >= 0) check(c, hipStreamWaitEvent(c->side, c->side_ev[ev], 0), "side wait");
+        check(c, hipMemcpyAsync(c->xfer + slot * ob, src, sizeof(uint32_t) * N, hipMemcpyDeviceToHost, c->side),
+              "output copy");
+    };
     if (E > 0 && T > 0 && (p->flags & IDB_FLAG_AUTOTUNE)) autotune(c, a, N, E, W, ham, learned, small, work);
     // Learned runs stay uncaptured: when their pair list overflows, the host
     // grows it and runs the learned pass again (below).
@@ -1795,6 +1800,10 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             else check(c, ham ? idb_launch_count_hamming(a, s) : idb_launch_count_myers(a, W, s), "count kernel launch");
             if (!g && ev_times) check(c, hipEventRecord(c->kev[1], s), "event record");
         }
+        if (!g) {
+            send(0, 2, copies);
+            send(-1, 3, unq_o);
+        }
         if (mr.inv) {
             mr.core = core;
             check(c, idb_launch_mx_rows(mr, s), "row launch");
@@ -1802,12 +1811,9 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
             hipLaunchKernelGGL(k_core_flags, dim3(blocks_for(N)), dim3(256), 0, s, cnt, N, (int32_t)p->min_pts, core,
                                pe, small);
         }
-        if (!g && early_out) {
-            check(c, hipEventRecord(c->side_ev[1], s), "event record");
-            check(c, hipStreamWaitEvent(c->side, c->side_ev[1], 0), "side wait");
-            check(c, hipMemcpyAsync(c->xfer + ob, core, sizeof(int32_t) * N, hipMemcpyDeviceToHost, c->side),
-                  "output copy");
-        }
+        if (!g && early_out) check(c, hipEventRecord(c->side_ev[1], s), "event record");
+        const bool waits = E > 0 && !g && (learned || (x && x->pairs_out));  // for a read-back, in the growth
+        if (!g && waits) send(1, 1, core);
         rng.stage("Grow clusters");
 
         // --- Grow clusters: union over the recorded neighbour pairs, or a
@@ -1900,6 +1906,7 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                 check(c, hipEventRecord(c->kev[3], s), "event record");
             }
         }
+        if (!g && !waits) send(1, 1, core);
         rng.stage("Reduction of cluster information tree structure");
 
         // --- Reduction of cluster information tree structure
@@ -1920,12 +1927,14 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                 hipLaunchKernelGGL(k_ustart, dim3(blocks_for((uint64_t)n_reps + 1)), dim3(256), 0, s, uniq, num, rstart,
                                    n_reps, ustart);
             hipLaunchKernelGGL(k_uniques_out, dim3(blocks_for(U)), dim3(256), 0, s, uniq, num, rid, rstart, ustart,
-                               unq_o);
+                               unq_o, (unsigned long long *)nullptr);
         }
         check(c, hipGetLastError(), "tail launch");
     };
 
     if (graph) {
+        send(0, 2, copies);
+        send(-1, 3, unq_o);
         hipGraph_t gr = nullptr;
         check(c, hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed), "begin capture");
         try {
@@ -2050,9 +2059,10 @@ void run(idb_ctx *c, const idb_dataset *d, const uint32_t *rstart_h, uint32_t n_
                 (void)hipEventElapsedTime(&st->count_kernel_ms, c->kev[0], c->kev[1]);
                 (void)hipEventElapsedTime(&st->fuse_kernel_ms, c->kev[2], c->kev[3]);
             } else {
-                // (to the start of the next kernel)
-                st->count_kernel_ms = span(IDB_T_COUNT_START, IDB_T_COUNT);
-                st->fuse_kernel_ms = span(IDB_T_FUSE_START, IDB_T_GROW);
+                // (between the kernels before and after: a stamp of their own at
+                // the start cost k_count_ham 17 registers, 62 -> 79)
+                st->count_kernel_ms = span(IDB_T_TILES, IDB_T_COUNT);
+                st->fuse_kernel_ms = span(IDB_T_CORE, IDB_T_GROW);
             }
         }
         if (p->tree_stats)

@@ -68,7 +68,7 @@ hipError_t idb_sort_small(uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1
 #define IDB_STAGE_BYTES 32768u    // each half of a context's pinned staging area
 #define IDB_XFER_MAX_BYTES (256ull << 20)  // most pinned staging a context keeps for host inputs and outputs
 // The run's small device words (zeroed at the start of a run): [12] chunks
-// handed out, [16, 67) the depth histogram, [68, 90) time stamps, [100, 107)
+// handed out, [16, 67) the depth histogram, [68, 88) time stamps, [100, 107)
 // sizes for the host,
 // then 8 copies of the row scan's 9 words (letter set, longest row) and 16
 // partial counts each of core and noise rows (copies keep blocks from
@@ -88,8 +88,8 @@ hipError_t idb_sort_small(uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1
 // Time stamps of the device's wall clock among the small words (a kernel's
 // start or end: see idb_stamp_start); the counters behind the small words.
 enum {
-    IDB_T_BEGIN, IDB_T_DEDUP, IDB_T_UNIQ, IDB_T_COUNT, IDB_T_CORE, IDB_T_GROW, IDB_T_ROOTS, IDB_T_LABELS,
-    IDB_T_END, IDB_T_COUNT_START, IDB_T_FUSE_START, IDB_N_STAMPS
+    IDB_T_BEGIN, IDB_T_DEDUP, IDB_T_UNIQ, IDB_T_TILES, IDB_T_COUNT, IDB_T_CORE, IDB_T_GROW, IDB_T_ROOTS, IDB_T_LABELS,
+    IDB_T_END, IDB_N_STAMPS
 };
 #define IDB_SMALL_STAMPS 68u
 #define IDB_SMALL_WORK IDB_SMALL_WORDS
@@ -174,7 +174,6 @@ struct idb_pair_args {
     uint32_t mx_planes, mx_words; // planes per letter (5 or 2), words per plane
     int32_t *cnt_e;               // their count output, per entry; their pair list holds entries
     uint32_t sub_log2;            // tiles are taken in 2^sub_log2 parts of their queries
-    unsigned long long *stamps;   // the run's time stamps
     // launch shape (0 = default): waves per block, grid = resident blocks x
     // grid_mul, and plain block order instead of the XCD-grouped one
     uint32_t tune_wpb, tune_grid_mul, no_xcd_order;

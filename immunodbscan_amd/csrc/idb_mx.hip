@@ -217,7 +217,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G::W > 5 ? 
     __shared__ int32_t acc_all[4][G::PER_TILE ? 2 * IDB_TILE : 1];
     const uint32_t lane = lane_id();
     const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (!FUSE) idb_stamp_start(a.stamps + IDB_T_COUNT_START);
     if (FUSE && fuse_skipped(a)) return;
     __shared__ unsigned long long stat_sum[5];
     if (threadIdx.x < 5) stat_sum[threadIdx.x] = 0;

@@ -482,7 +482,6 @@ template <int W, bool FUSE, int FILT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FILT == 2 && W >= 3 ? 3 : 4))) void k_pairs_myers(
     idb_pair_args a, uint32_t wpb)
 {
-    if (!FUSE) idb_stamp_start(a.stamps + IDB_T_COUNT_START);
     extern __shared__ uint32_t lds[];
     const uint32_t lane = lane_id();
     const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, kept in a scalar register
@@ -998,7 +997,6 @@ __host__ __device__ inline size_t idb_count1_lds_per_wave(uint32_t K)
 template <bool TCONST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_count1(idb_pair_args a, uint32_t wpb)
 {
-    idb_stamp_start(a.stamps + IDB_T_COUNT_START);
     extern __shared__ uint32_t lds[];
     const uint32_t lane = lane_id();
     const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1579,7 +1577,6 @@ __global__ void k_pair_dist(const uint8_t *seq, const uint64_t *off, const uint3
 template <int HWMAX, int BITS, bool FUSE>
 __global__ __launch_bounds__(256) void k_pairs_hamming(idb_pair_args a, uint32_t wpb)
 {
-    if (!FUSE) idb_stamp_start(a.stamps + IDB_T_COUNT_START);
     const uint32_t lane = lane_id();
     const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, kept in a scalar register
     const uint32_t total_waves = gridDim.x * wpb;
@@ -1713,7 +1710,6 @@ __global__ __launch_bounds__(256) void k_pairs_hamming(idb_pair_args a, uint32_t
 template <int HWMAX, int BITS>
 __global__ __launch_bounds__(256) void k_count_ham(idb_pair_args a, uint32_t wpb)
 {
-    idb_stamp_start(a.stamps + IDB_T_COUNT_START);
     const uint32_t lane = lane_id();
     const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t total_waves = gridDim.x * wpb;
@@ -1957,10 +1953,8 @@ __device__ __forceinline__ void for_pairs(const uint32_t *fill, const uint32_t *
 }
 
 __global__ void k_union_to_entries(uint2 *edges, const uint32_t *fill, const uint32_t *n_chunks, uint32_t max_chunks,
-                                   uint32_t chunk_log2, const uint32_t *pe, uint32_t *par_e, uint32_t *bmin,
-                                   unsigned long long *stamps)
+                                   uint32_t chunk_log2, const uint32_t *pe, uint32_t *par_e, uint32_t *bmin)
 {
-    idb_stamp_start(stamps + IDB_T_FUSE_START);
     for_pairs(fill, n_chunks, max_chunks, chunk_log2, [&](uint64_t e, bool live) {
         if (!live) return;
         const uint2 p = edges[e];
@@ -1988,9 +1982,8 @@ __global__ void k_union_to_entries(uint2 *edges, const uint32_t *fill, const uin
 // atomic that changes nothing).
 __global__ void k_union_link(uint2 *edges, const uint32_t *fill, const uint32_t *n_chunks, uint32_t max_chunks,
                              uint32_t chunk_log2, const uint8_t *ecore, const uint32_t *erow, uint32_t *par_e,
-                             uint32_t *bmin, unsigned long long *stamps)
+                             uint32_t *bmin)
 {
-    idb_stamp_start(stamps + IDB_T_FUSE_START);
     for_pairs(fill, n_chunks, max_chunks, chunk_log2, [&](uint64_t e, bool live) {
         if (!live) return;
         const uint2 p = edges[e];
@@ -2480,11 +2473,11 @@ hipError_t idb_launch_union_edges(const idb_pair_args &a, const idb_union_args &
     if (u.ecore) {
         const uint32_t b1 = resident_blocks((const void *)k_union_link, 256, 0);
         hipLaunchKernelGGL(k_union_link, dim3(b1), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks, a.max_chunks,
-                           a.chunk_log2, u.ecore, u.erow, u.par_e, u.bmin, a.stamps);
+                           a.chunk_log2, u.ecore, u.erow, u.par_e, u.bmin);
     } else {
         const uint32_t b1 = resident_blocks((const void *)k_union_to_entries, 256, 0);
         hipLaunchKernelGGL(k_union_to_entries, dim3(b1), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks,
-                           a.max_chunks, a.chunk_log2, u.pe, u.par_e, u.bmin, a.stamps);
+                           a.max_chunks, a.chunk_log2, u.pe, u.par_e, u.bmin);
     }
     const uint32_t eb = (u.n_entries + 255) / 256 < 2048u ? (u.n_entries + 255) / 256 : 2048u;
     hipLaunchKernelGGL(k_union_compress, dim3(eb ? eb : 1u), dim3(256), 0, s, a.n_chunks, a.max_chunks, u.par_e,

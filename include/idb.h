@@ -116,8 +116,8 @@ typedef struct {
     uint64_t gated_letters;       /* text letters of the count pass's gated pairs    */
     uint64_t myers_pairs;         /* gated pairs that reached Myers (after the band filter) */
     uint64_t myers_letters;       /* text letters those Myers runs consumed          */
-    float count_kernel_ms;        /* count-pass kernel: from its first block to the start of the next
-                                     kernel, on the device's clock                   */
+    float count_kernel_ms;        /* count-pass kernel, between the kernels before and after it,
+                                     on the device's clock                           */
     float fuse_kernel_ms;         /* cluster growth (or the fuse pass), likewise     */
     uint32_t tree_depth[51];      /* union-find depth histogram when tree_stats      */
     float stage_ms[IDB_N_STAGES]; /* with IDB_FLAG_GRAPH the graph's time is the core-point stage's */

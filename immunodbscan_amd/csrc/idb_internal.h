@@ -191,13 +191,18 @@ __device__ __forceinline__ void idb_stamp_end(unsigned long long *at)
 }
 
 // Bytes k .. k+15 of a row of length L as one 16-byte value, zero past the
-// row's end.  Every load stays inside the row: a short tail is read as the
-// row's last 16 bytes and shifted down, rows under 16 bytes byte by byte.
-// Unaligned 16-byte global loads are legal on gfx950.  Only 32-bit shifts: a
-// 64-bit shift whose amount the compiler puts into the last of a wave's vector
-// registers now and then comes out wrong, and one kernel was compiled so (the
-// gene scan with a 32-bit table and bit words in memory: of 400,000 rows, 600
-// to 700 lost the name at their end).  tests/test_code_objects.py looks for it.
+// row's end (k a multiple of 16).  Every load stays inside the row: a short
+// tail is read as the row's last 16 bytes and shifted down, a row of 8 to 15
+// bytes as its first and its last eight, shorter rows byte by byte.  Unaligned
+// global loads are legal on gfx950.
+// Only 32-bit shifts: a 64-bit shift whose amount the compiler puts into the
+// last of a wave's vector registers now and then comes out wrong, and one
+// kernel was compiled so (the gene scan with a 32-bit table and bit words in
+// memory: of 400,000 rows, 600 to 750 lost the name at their end).
+// tests/test_code_objects.py looks for it.  Against 64-bit shifts and bytes for
+// all rows under 16 (the kernels that read rows this way, us): 2.56M nucleotide
+// rows 690 -> 680, 2M protein rows 535 -> 427, 2M long nucleotide rows 794 -> 789,
+// 1M gene calls 51.7 -> 50.9.
 __device__ __forceinline__ uint4 row16(const uint8_t *s, uint32_t L, uint32_t k)
 {
     uint4 v;
@@ -205,24 +210,28 @@ __device__ __forceinline__ uint4 row16(const uint8_t *s, uint32_t L, uint32_t k)
         __builtin_memcpy(&v, s + k, 16);
         return v;
     }
-    const uint32_t r = L - k;  // 1 .. 15 bytes left
     if (L >= 16) {
         __builtin_memcpy(&v, s + L - 16, 16);
-        const uint32_t d = 16 - r;  // bytes to drop
+        const uint32_t d = 16 - (L - k);  // bytes to drop
         if (d & 8u) v = make_uint4(v.z, v.w, 0u, 0u);
         if (d & 4u) v = make_uint4(v.y, v.z, v.w, 0u);
-        const uint32_t sh = 8 * (d & 3u);
-        return make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, sh), __builtin_amdgcn_alignbit(v.z, v.y, sh),
-                          __builtin_amdgcn_alignbit(v.w, v.z, sh), v.w >> sh);
+        return make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, d), __builtin_amdgcn_alignbyte(v.z, v.y, d),
+                          __builtin_amdgcn_alignbyte(v.w, v.z, d), __builtin_amdgcn_alignbyte(0u, v.w, d));
+    }
+    if (L >= 8) {
+        uint32_t h[2], t[2];
+        __builtin_memcpy(h, s, 8);
+        __builtin_memcpy(t, s + L - 8, 8);
+        const uint32_t d = 16 - L, x = d & 4u ? t[1] : t[0], y = d & 4u ? 0u : t[1];
+        return make_uint4(h[0], h[1], L > 8 ? __builtin_amdgcn_alignbyte(y, x, d) : 0u,
+                          L > 8 ? __builtin_amdgcn_alignbyte(0u, y, d) : 0u);
     }
     v = make_uint4(0u, 0u, 0u, 0u);
-    for (uint32_t b = 0; b < r; ++b) {
-        const uint32_t c = (uint32_t)s[k + b] << (8 * (b & 3u));
-        if (b < 8) {
-            if (b < 4) v.x |= c; else v.y |= c;
-        } else {
-            if (b < 12) v.z |= c; else v.w |= c;
-        }
+#pragma unroll 1
+    for (uint32_t b = 0; b < L; ++b) {
+        const uint32_t c = (uint32_t)s[b] << (8 * (b & 3u));
+        v.x |= b < 4 ? c : 0u;
+        v.y |= b < 4 ? 0u : c;
     }
     return v;
 }

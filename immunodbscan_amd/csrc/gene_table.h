@@ -80,6 +80,9 @@ inline bool idb_gene_table_in_reach(uint32_t n_genes, const uint8_t *genes, cons
         return idb_gene_fresh(genes + gene_off[a], gene_len[a], genes + gene_off[b], gene_len[b]);
     };
     const auto reach = [&](double per_name) { return per_name * n_genes * (classes + 2u) <= 1.3 * cap; };
+    uint64_t letters = 1;  // a state per letter and an entry per byte value are the most there can be
+    for (uint32_t g = 0; g < n_genes; ++g) letters += usable(g) ? gene_len[g] : 0u;
+    if (letters * 257u <= cap) return true;
     const uint32_t step = (n_genes + 63u) / 64u;
     for (uint32_t g = step / 2; g < n_genes; g += step) {
         if (!usable(g)) continue;

@@ -166,8 +166,8 @@ struct idb_pair_args {
     const uint16_t *zb;           // learned filter: bfloat16 embedding (64) per row
     float min_sim;                // learned filter: proposal threshold on z_x . z_y
     // matrix-core passes (idb_mx.hip), null otherwise: 4-bit features, length |
-    // lower-gene flag << 16, records (protein rows: 5 planes, row, copies,
-    // length per entry; nucleotide rows: plane word w of entry e at
+    // lower-gene flag << 16, records (protein rows: 5 planes, a spare word,
+    // copies, length per entry; nucleotide rows: plane word w of entry e at
     // w * n_entries + e, then the copies), rows
     const uint32_t *e_feat, *e_meta, *e_vrec, *e_row;
     uint32_t n_entries;

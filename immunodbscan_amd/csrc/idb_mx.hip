@@ -46,7 +46,7 @@ struct MxCfg {
     static constexpr int NP = NP_, W = W_, T = T_;
     static constexpr int KC = NP_ == 2 ? 3 : 1;
     static constexpr bool PER_TILE = NP_ == 2;             // records staged in LDS, queues emptied per tile
-    // record words: planes, row, copies, length in memory (protein rows);
+    // record words: planes, a spare word, copies, length in memory (protein rows);
     // planes, length, copies in LDS (nucleotide rows: an odd number of
     // 16-byte units, so that random records spread over the banks)
     static constexpr int VS = NP_ == 2 ? (W_ == 1 ? 4 : (W_ <= 5 ? 12 : 20)) : 8;
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(256) void k_mx_fill(const uint64_t *ekey, const uin
             f4[1] = make_uint4(d[4], d[5], d[6], d[7]);
             uint4 *r4 = (uint4 *)(vrec + (size_t)e * 8);
             r4[0] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-            r4[1] = make_uint4(pl[4], u, r0.z, L);
+            r4[1] = make_uint4(pl[4], 0u, r0.z, L);
         } else {
             uint32_t g[6] = {0u, 0u, 0u, 0u, 0u, 0u}, hist = 0;
             for (uint32_t wd = 0; wd < W; ++wd) {

@@ -1337,12 +1337,12 @@ __global__ __launch_bounds__(256) void k_pairs_learned(idb_pair_args a, uint32_t
     const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, kept in a scalar register
     const uint32_t K = a.K;
     // per wave: Peq, edge stage, queue, count accumulators, query records,
-    // then (3-gram bound) the tile's query and target profiles
+    // then (3-gram bound) the tile's query and target level masks
     const uint32_t QGW = a.qgram_filter ? 2u * IDB_TILE * IDB_QMASK_WORDS : 0u;
     uint32_t *peq = lds + (size_t)wib * (idb_myers_lds_per_wave(K, W) / sizeof(uint32_t) + QGW);
     uint32_t *qgp = peq + idb_myers_lds_per_wave(K, W) / sizeof(uint32_t);
     uint32_t *tgp = qgp + IDB_TILE * IDB_QMASK_WORDS;
-    EdgeStage est{(uint2 *)(peq + K * W * 64), 0u, IDB_NONE, 0u, 0u};
+    EdgeStage est{(uint2 *)(peq + K * W * 64), 0u, IDB_NONE, 0u};
     uint16_t *queue = (uint16_t *)(peq + K * W * 64 + 2 * IDB_TILE);
     int32_t *qacc = (int32_t *)(peq + K * W * 64 + 3 * IDB_TILE);
     int32_t *tacc = qacc + IDB_TILE;
@@ -1364,7 +1364,7 @@ __global__ __launch_bounds__(256) void k_pairs_learned(idb_pair_args a, uint32_t
         qacc[lane] = 0;
         tacc[lane] = 0;
         if (a.qgram_filter) {
-            // profiles of the tile's queries and targets (64 bytes each)
+            // level masks of the tile's queries and targets (32 bytes each)
             const uint4 *qs = (const uint4 *)(a.e_qg + (size_t)(tile.q0 + (lane < qn ? lane : 0u)) * IDB_QMASK_WORDS);
             const uint4 *ts = (const uint4 *)(a.e_qg + (size_t)p * IDB_QMASK_WORDS);
 #pragma unroll
@@ -1584,7 +1584,7 @@ __global__ __launch_bounds__(256) void k_pairs_hamming(idb_pair_args a, uint32_t
     const uint32_t HW = a.HW;
     __shared__ uint2 stage[4][IDB_TILE];
     __shared__ int32_t qacc_s[4][IDB_TILE];
-    EdgeStage est{stage[wib], 0u, IDB_NONE, 0u, 0u};
+    EdgeStage est{stage[wib], 0u, IDB_NONE, 0u};
     int32_t *qacc = qacc_s[wib];
     if (FUSE && fuse_skipped(a)) return;
     constexpr bool QREG = HWMAX <= 8;
@@ -2118,20 +2118,6 @@ __global__ void k_union_to_rows(const uint32_t *n_chunks, uint32_t max_chunks, c
     }
 }
 
-// Blocks that fit on the device at once for this kernel and shape.
-// Blocks of `kernel` resident on the whole device, remembered per (device,
-// kernel, block size, LDS bytes): the occupancy query is a runtime call on
-// every launch otherwise.
-uint32_t resident_blocks(const void *kernel, uint32_t block, size_t shm)
-{
-    return idb_resident_blocks(kernel, block, shm);
-}
-uint32_t grid_for(uint32_t n_tiles, uint32_t wpb, uint32_t resident, uint32_t mul = 1)
-{
-    return idb_grid_for(n_tiles, wpb, resident, mul);
-}
-uint32_t pick_wpb(const idb_pair_args &a, uint32_t most) { return idb_pick_wpb(a, most); }
-
 template <int W, bool FUSE, int FILT>
 hipError_t launch_myers_w(const idb_pair_args &a_in, dim3 block, size_t shm, uint32_t wpb, hipStream_t s)
 {
@@ -2140,7 +2126,7 @@ hipError_t launch_myers_w(const idb_pair_args &a_in, dim3 block, size_t shm, uin
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
     }
-    const uint32_t resident = resident_blocks(k, block.x, shm);
+    const uint32_t resident = idb_resident_blocks(k, block.x, shm);
     // Few tiles (buckets of a small table) leave most of the chip idle behind
     // the waves of the fullest ones: they are taken in up to 8 parts of their
     // queries each, while the parts are no more than twice the resident waves
@@ -2150,7 +2136,7 @@ hipError_t launch_myers_w(const idb_pair_args &a_in, dim3 block, size_t shm, uin
     idb_pair_args a = a_in;
     if (!FUSE)
         while (a.sub_log2 < 3 && ((uint64_t)a.n_tiles << (a.sub_log2 + 1)) <= 2ull * resident * wpb) ++a.sub_log2;
-    const dim3 grid(grid_for(a.n_tiles << a.sub_log2, wpb, resident, a.tune_grid_mul));
+    const dim3 grid(idb_grid_for(a.n_tiles << a.sub_log2, wpb, resident, a.tune_grid_mul));
     hipLaunchKernelGGL((k_pairs_myers<W, FUSE, FILT>), grid, block, shm, s, a, wpb);
     return hipGetLastError();
 }
@@ -2180,7 +2166,7 @@ hipError_t launch_count1_t(const idb_pair_args &a, uint32_t wpb, hipStream_t s)
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
     }
-    const dim3 block(64 * wpb), grid(grid_for(a.n_tiles, wpb, resident_blocks(k, block.x, shm), a.tune_grid_mul));
+    const dim3 block(64 * wpb), grid(idb_grid_for(a.n_tiles, wpb, idb_resident_blocks(k, block.x, shm), a.tune_grid_mul));
     hipLaunchKernelGGL(k_count1<TCONST>, grid, block, shm, s, a, wpb);
     return hipGetLastError();
 }
@@ -2192,7 +2178,7 @@ hipError_t launch_count1(const idb_pair_args &a, hipStream_t s)
     uint32_t wpb = (uint32_t)(std::min<size_t>(idb_lds_limit(), 65536) / per_wave);
     if (wpb > 4) wpb = 4;
     if (wpb == 0) return hipErrorInvalidValue;
-    wpb = pick_wpb(a, wpb);
+    wpb = idb_pick_wpb(a, wpb);
     return a.t_const >= 0 ? launch_count1_t<true>(a, wpb, s) : launch_count1_t<false>(a, wpb, s);
 }
 
@@ -2223,7 +2209,7 @@ hipError_t launch_myers(const idb_pair_args &a_in, uint32_t W, hipStream_t s)
     if (wpb > 4) wpb = 4;
     if (wpb == 0) wpb = per_wave <= limit ? 1u : 0u;
     if (wpb == 0) return hipErrorInvalidValue;
-    wpb = pick_wpb(a, wpb);
+    wpb = idb_pick_wpb(a, wpb);
     const dim3 block(64 * wpb);
     const size_t shm = per_wave * wpb;
     if (W == 1 && a.band_filter) {
@@ -2246,9 +2232,9 @@ hipError_t launch_hamming_hw(const idb_pair_args &a_in, hipStream_t s)
         a.tune_grid_mul = 4;
         a.no_xcd_order = 1;
     }
-    const uint32_t wpb = pick_wpb(a, 4);
+    const uint32_t wpb = idb_pick_wpb(a, 4);
     const void *k = (const void *)k_pairs_hamming<HWMAX, BITS, FUSE>;
-    const dim3 block(64 * wpb), grid(grid_for(a.n_tiles, wpb, resident_blocks(k, 64 * wpb, 0), a.tune_grid_mul));
+    const dim3 block(64 * wpb), grid(idb_grid_for(a.n_tiles, wpb, idb_resident_blocks(k, 64 * wpb, 0), a.tune_grid_mul));
     hipLaunchKernelGGL((k_pairs_hamming<HWMAX, BITS, FUSE>), grid, block, 0, s, a, wpb);
     return hipGetLastError();
 }
@@ -2279,9 +2265,9 @@ hipError_t launch_count_ham_hw(const idb_pair_args &a_in, hipStream_t s)
         a.tune_grid_mul = 4;
         a.no_xcd_order = 1;
     }
-    const uint32_t wpb = pick_wpb(a, 4);
+    const uint32_t wpb = idb_pick_wpb(a, 4);
     const void *k = (const void *)k_count_ham<HWMAX, BITS>;
-    const dim3 block(64 * wpb), grid(idb_count_grid(a, a.n_tiles, wpb, resident_blocks(k, 64 * wpb, 0)));
+    const dim3 block(64 * wpb), grid(idb_count_grid(a, a.n_tiles, wpb, idb_resident_blocks(k, 64 * wpb, 0)));
     hipLaunchKernelGGL((k_count_ham<HWMAX, BITS>), grid, block, 0, s, a, wpb);
     return hipGetLastError();
 }
@@ -2330,7 +2316,7 @@ hipError_t launch_learned(const idb_pair_args &a_in, hipStream_t s)
     uint32_t wpb = (uint32_t)(std::min<size_t>(idb_lds_limit(), 65536) / per_wave);
     if (wpb > 4) wpb = 4;
     if (wpb == 0) return hipErrorInvalidValue;
-    wpb = pick_wpb(a, wpb);
+    wpb = idb_pick_wpb(a, wpb);
     const size_t shm = per_wave * wpb;
     const void *k = W == 1   ? (const void *)k_pairs_learned<1>
                     : W == 2 ? (const void *)k_pairs_learned<2>
@@ -2341,7 +2327,7 @@ hipError_t launch_learned(const idb_pair_args &a_in, hipStream_t s)
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
     }
-    const dim3 block(64 * wpb), grid(grid_for(a.n_tiles, wpb, resident_blocks(k, block.x, shm), a.tune_grid_mul));
+    const dim3 block(64 * wpb), grid(idb_grid_for(a.n_tiles, wpb, idb_resident_blocks(k, block.x, shm), a.tune_grid_mul));
     switch (W) {
     case 1: hipLaunchKernelGGL(k_pairs_learned<1>, grid, block, shm, s, a, wpb); break;
     case 2: hipLaunchKernelGGL(k_pairs_learned<2>, grid, block, shm, s, a, wpb); break;
@@ -2364,6 +2350,9 @@ hipError_t launch_pair_dist_w(const uint8_t *seq, const uint64_t *off, const uin
 
 }  // namespace
 
+// Blocks of `kernel` resident on the whole device, remembered per (device,
+// kernel, block size, LDS bytes): the occupancy query is a runtime call on
+// every launch otherwise.
 uint32_t idb_resident_blocks(const void *kernel, uint32_t block, size_t shm)
 {
     int dev = 0;
@@ -2471,18 +2460,18 @@ hipError_t idb_launch_union_edges(const idb_pair_args &a, const idb_union_args &
 {
     if (!a.edges || a.max_chunks == 0) return hipSuccess;
     if (u.ecore) {
-        const uint32_t b1 = resident_blocks((const void *)k_union_link, 256, 0);
+        const uint32_t b1 = idb_resident_blocks((const void *)k_union_link, 256, 0);
         hipLaunchKernelGGL(k_union_link, dim3(b1), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks, a.max_chunks,
                            a.chunk_log2, u.ecore, u.erow, u.par_e, u.bmin);
     } else {
-        const uint32_t b1 = resident_blocks((const void *)k_union_to_entries, 256, 0);
+        const uint32_t b1 = idb_resident_blocks((const void *)k_union_to_entries, 256, 0);
         hipLaunchKernelGGL(k_union_to_entries, dim3(b1), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks,
                            a.max_chunks, a.chunk_log2, u.pe, u.par_e, u.bmin);
     }
     const uint32_t eb = (u.n_entries + 255) / 256 < 2048u ? (u.n_entries + 255) / 256 : 2048u;
     hipLaunchKernelGGL(k_union_compress, dim3(eb ? eb : 1u), dim3(256), 0, s, a.n_chunks, a.max_chunks, u.par_e,
                        u.n_entries);
-    const uint32_t b2 = resident_blocks((const void *)k_union_entries, 256, 0);
+    const uint32_t b2 = idb_resident_blocks((const void *)k_union_entries, 256, 0);
     hipLaunchKernelGGL(k_union_entries, dim3(b2), dim3(256), 0, s, a.edges, a.chunk_fill, a.n_chunks, a.max_chunks,
                        a.chunk_log2, u.par_e, a.chunk_base + (uint32_t)((4ull * u.n_entries) >> a.chunk_log2));
     const uint32_t rb = (u.n_rows + 255) / 256 < 2048u ? (u.n_rows + 255) / 256 : 2048u;

@@ -107,7 +107,6 @@ struct EdgeStage {
     uint32_t n;       // staged pairs (wave-uniform)
     uint32_t chunk;   // the wave's current chunk, IDB_NONE before the first
     uint32_t fill;    // pairs written into it
-    uint32_t total;   // pairs this wave produced
 };
 
 // This block's copy of the run's statistics counters.
@@ -123,7 +122,7 @@ __device__ __forceinline__ unsigned long long *work_copy(const idb_pair_args &a)
 // instead of per wave; the 2.6M-row batch's Hamming pass 517 -> 407 us).
 __device__ __forceinline__ EdgeStage edge_stage(const idb_pair_args &a, uint2 *buf, uint32_t wave)
 {
-    return {buf, 0u, a.edges && wave < a.chunk_base ? wave : IDB_NONE, 0u, 0u};
+    return {buf, 0u, a.edges && wave < a.chunk_base ? wave : IDB_NONE, 0u};
 }
 
 // Adds the waves' statistics (lane 0's values) to the run's, one atomic per
@@ -161,7 +160,6 @@ __device__ __forceinline__ void flush_edges(const idb_pair_args &a, EdgeStage &s
     if (st.chunk < a.max_chunks && lane < st.n)
         a.edges[((size_t)st.chunk << a.chunk_log2) + st.fill + lane] = st.buf[lane];
     st.fill += st.n;
-    st.total += st.n;
     st.n = 0;
 }
 

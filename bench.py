@@ -616,9 +616,8 @@ def main() -> int:
         "noise": s["n_noise"],
         "stage_ms": s["stage_ms"],
         "roofline": {
-            "kernel": "k_mx (count pass: the bound on matrix cores, pairs that pass on bit planes)",
+            "kernel": "count pass",
             **bound_roofline(s, kms),
-            "traffic": None,
             "kernel_ms": kms,
             "algorithmic_ops": ops,
             "work_model": "gated pairs x (2(Vw+Jw)+2) + Myers text letters x (20W+4(W-1))",

@@ -104,15 +104,16 @@ __global__ void k_adam(float *th, const float *g, float *m, float *v, uint32_t n
 // cycles) take 4 row fragments from LDS (50% of its bandwidth over the 4
 // waves) and 2 weight fragments from L2, packed so that a wave reads 1 KB
 // in a row.  128 accumulators leave room for 2 waves per SIMD; at 71 KB of
-// activations two blocks share a CU, so one block's GELU (as many VALU cycles
-// as the MFMAs take) overlaps the other's products.
+// activations two blocks share a CU, so one block's GELU overlaps the other's
+// products (200k protein rows: 388M VALU instructions, 632 us of issue, beside
+// 513 us of MFMAs).
 // In training (TRAIN) a block also writes what the backward pass reads: the
 // pre-activations in the lanes' own order (512 bytes per wave and store; k_enc_bwd
 // has the same lane mapping), the layers' inputs row by row in packed order,
 // the pooled means and the norms.
-// Measured: 200k protein rows (packed 1.25 Tflop) 5.22 -> 1.52 ms, 825 TFLOP/s
-// (a large bf16 product reaches 1,214 here); 20k rows of 24-150 letters
-// 2.98 -> 0.81 ms.
+// Measured: 200k protein rows (1.29 Tflop of MFMAs) 5.22 -> 1.60 ms, 806 TFLOP/s
+// (a large bf16 product reaches 1,205 here); 20k rows of 24-150 letters in the
+// five segments of an embedding call 2.98 -> 1.07 ms.
 constexpr uint32_t EST = C + 8;                   // LDS row stride (272 bytes: conflict-free)
 constexpr uint32_t EPW = 1024;                    // sequences per packing window
 constexpr uint32_t EGRP = 8;                      // sequences per round of the head
@@ -259,8 +260,8 @@ __global__ void k_enc_pack(const uint16_t *theta_b, uint16_t *dst, uint32_t *wp2
 // the least padding (200k protein rows 1.58 ms, tiles of 128 rows 1.63).  A
 // training batch is a few tiles per CU, so that the spread of the tiles over
 // the CUs and the latency of one tile count: 128 rows (three blocks a CU)
-// where P fits, 4,096 protein pairs forward 135 -> 107 us, backward 223 ->
-// 176, 256 pairs 54 -> 39 and 84 -> 55.
+// where P fits, 4,096 protein pairs forward 135 -> 105 us, backward 204 ->
+// 157, 256 pairs 54 -> 39 and 84 -> 55.
 constexpr int enc_blocks_per_cu(int rt) { return rt == 4 ? 2 : 3; }
 
 struct EncArgs {
@@ -510,7 +511,7 @@ constexpr uint32_t BPART = NTOK * C0 + 3 * C;      // one block's embedding and 
 // Latency-bound (4,096 pairs are one round a block); the sums over
 // pairs stay in registers and leave as one partial per block, since one atomic
 // word per pair (the loss) took 49 us.  With the three kernels it replaces:
-// 4,096 pairs 306 -> 37 us.
+// 4,096 pairs 306 -> 24 us.
 __global__ __launch_bounds__(256) void k_pair_head(const float *z, const float *nrm, const float *pool,
                                                    const uint32_t *blen, const float *y, uint32_t npairs, float margin,
                                                    float inv_b, const uint32_t *wp2, float *dp, float *part)
@@ -668,7 +669,7 @@ __device__ __forceinline__ uint2 times_grad(float a, float b, float c, float d, 
 // embedding sums stay in LDS over a block's tiles.
 // MFMA-bound like k_encode.  4,096 pairs of protein rows: head's last part,
 // three data-gradient products, three bias sums and the embedding scatter
-// took 870 us as eight launches over padded rows; 204 us here.
+// took 870 us as eight launches over padded rows; 157 us here.
 template <int RT>
 __global__ __launch_bounds__(256, enc_blocks_per_cu(RT)) void k_enc_bwd(BwdArgs a)
 {
@@ -795,7 +796,7 @@ __global__ __launch_bounds__(256, enc_blocks_per_cu(RT)) void k_enc_bwd(BwdArgs 
 // of the gradients queue).
 // 4,096 pairs of protein rows (139k packed rows), three layers: 1,263 us as
 // im2col products over padded rows with transposing LDS stores and atomics,
-// 66 us here (780 TFLOP/s).
+// 68 us here (753 TFLOP/s).
 constexpr uint32_t WROWS = 64, WA = C + 32, WB = 64 + 32;  // rows per chunk; LDS row strides
 constexpr uint32_t WPART = 4 * 10 * 16 * 64;               // sums of a block (layer 1: two halves)
 typedef short s16x4 __attribute__((ext_vector_type(4)));

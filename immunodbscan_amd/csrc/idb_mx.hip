@@ -18,12 +18,12 @@
 // rows keep their queue across tiles, so that batches are full, and read their
 // 32-byte records from memory.  Nucleotide rows have ~260 such pairs a tile:
 // the tile's records are staged in LDS (gathered from memory, 64 bytes per
-// row and pair, the pass took 4.6 ms instead of 3.55 on 2M rows) and a first
-// look at their substitutions decides most pairs.
-// Measured (count kernel): 2M protein rows 9.28 -> 2.08 ms (320 VALU
+// row and pair, the pass took 4.6 ms instead of 3.55 on 2M rows
+// at the time) and a first look at their substitutions decides most pairs.
+// Measured (count kernel): 2M protein rows 9.28 -> 2.07 ms (320 VALU
 // instructions per tile of 4,096 pairs, 1.7 ms of issue; the rest is the
-// tiles' loads), 200k protein rows 0.225 -> 0.083 ms, 2M nucleotide rows of
-// 24-154 letters 15.8 -> 3.55 ms.
+// tiles' loads), 200k protein rows 0.225 -> 0.080 ms, 2M nucleotide rows of
+// 24-154 letters 15.8 -> 3.17 ms (2.6 ms of VALU issue).
 #include <algorithm>
 #include <type_traits>
 

@@ -144,7 +144,8 @@ int idb_gene_bitsets(uint32_t n, const uint8_t *calls, const uint64_t *call_off,
                      int32_t *out, uint32_t width);
 
 /* R2 gene bitsets on the device, with the same result as idb_gene_bitsets:
- * one wave per call string tests every gene name.  Replaces
+ * a multi-name automaton reads every call string once, or, for few names or
+ * calls, one wave per call string tests every name.  Replaces
  * bitset_container's constructor and its per-gene find_string_occurences
  * launches (cuda/BitsetVector.inl:27-45, 118-209).  calls, call_off,
  * call_len and out are in host memory (mem = IDB_MEM_HOST) or in device
@@ -255,8 +256,9 @@ int idb_encoder_get_params(idb_encoder *enc, float *params);
 int idb_encoder_set_params(idb_encoder *enc, const float *params);
 /* z (n_rows x 64 floats) of every row of data. */
 int idb_encoder_embed(idb_encoder *enc, const idb_dataset *data, float *z);
-/* Contrastive loss over the pairs (label 1: neighbours, 0: not) and its
- * gradient with respect to the flat parameters; no update. */
+/* Contrastive loss over the pairs (label 1: neighbours, 0: not, below 0: no
+ * loss, as in training) and its gradient with respect to the flat parameters;
+ * no update. */
 int idb_encoder_loss_grad(idb_encoder *enc, const idb_dataset *data, const uint32_t *pairs, const float *labels,
                           uint32_t n_pairs, float margin, float *loss, float *grad);
 /* Adam training over shuffled batches of the labelled pairs, on the device. */

@@ -18,8 +18,8 @@
 // rows keep their queue across tiles, so that batches are full, and read their
 // 32-byte records from memory.  Nucleotide rows have ~260 such pairs a tile:
 // the tile's records are staged in LDS (gathered from memory, 64 bytes per
-// row and pair, the pass took 4.6 ms instead of 3.55 on 2M rows
-// at the time) and a first look at their substitutions decides most pairs.
+// row and pair, the pass took 4.6 ms instead of 3.55 on 2M rows when it was
+// written) and a first look at their substitutions decides most pairs.
 // Measured (count kernel): 2M protein rows 9.28 -> 2.07 ms (320 VALU
 // instructions per tile of 4,096 pairs, 1.7 ms of issue; the rest is the
 // tiles' loads), 200k protein rows 0.225 -> 0.080 ms, 2M nucleotide rows of
@@ -622,8 +622,8 @@ hipError_t launch_mx_g(const idb_pair_args &a_in, hipStream_t s)
     const uint32_t resident = idb_resident_blocks(k, 64 * wpb, 0);
     // Launch shape, measured (count kernel).  Grid: 8x the resident blocks once
     // a wave has 16 tiles (2M protein rows 2.20 -> 2.08 ms, 2M nucleotide rows
-    // 3.90 -> 3.55 ms), else 2x (200k protein rows 0.083 against 0.107 ms at
-    // 4x).  Few tiles are taken in 2 or 4 parts each, while the parts fit
+    // 3.90 -> 3.55 ms when it was set), else 2x (200k protein rows 0.083 against
+    // 0.107 ms at 4x).  Few tiles are taken in 2 or 4 parts each, while the parts fit
     // half the resident waves (protein rows: 442 tiles 33 -> 17 us, 1,202
     // tiles 32 -> 25 us in 2 parts but 33 us in 4) or twice of them
     // (nucleotide rows, whose batches are longer: 471 tiles 69 -> 32 us,
